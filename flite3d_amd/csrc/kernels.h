@@ -3889,15 +3889,15 @@ __global__ void k_restrict_finish(LevelDev<R> K, DevParams P) {
 
 // ---------------------------------------------------------------------------
 // monitor reductions (writeResiduals MG:1302-1445, calculateLiftAndDrag
-// DEF:14710-14806), all on the device: a fixed grid of MON_BLOCKS blocks
-// strides over the nodes and the wall nodes, each thread accumulating its
-// share in stride order; wavefront butterflies and one LDS step reduce the
-// block to a record of MON_REC doubles; k_monitor_final reduces the records
-// in block order.  The order of every sum is fixed, so the results are
-// reproducible bit for bit.  Record: sum (u - uprev)^2 [7], max |u - uprev|
-// [7], host index of that maximum [7] (smallest index on ties), force
-// integrals [8] (lift, drag, latF, frictionDrag, latM, longM, pressureLift,
-// pressureDrag, before the 2/referenceArea factor).
+// DEF:14710-14806), all on the device: up to MON_BLOCKS blocks stride over
+// the nodes and the wall nodes, each thread accumulating its share in stride
+// order; wavefront butterflies and one LDS step reduce the block to a record
+// of MON_REC doubles; the last block reduces the records.  The order of
+// every sum is fixed, so the results are reproducible bit for bit.  Record:
+// sum (u - uprev)^2 [7], max |u - uprev| [7], host index of that maximum [7]
+// (smallest index on ties), force integrals [8] (lift, drag, latF,
+// frictionDrag, latM, longM, pressureLift, pressureDrag, before the
+// 2/referenceArea factor).
 // ---------------------------------------------------------------------------
 constexpr int MON_BLOCKS = 512;
 constexpr int MON_REC = 29;
@@ -3958,43 +3958,38 @@ __device__ __forceinline__ void maxloc(double &m, int &k, double m2, int k2) {
   }
 }
 
-// block-wide reduction of one sum and of one (max, index) pair: butterflies
-// inside each wavefront, then the NTHR/64 wavefront results in order
-__device__ __forceinline__ double block_sum(double v, double *lds) {
+// one wavefront's sum and (max, smallest index) by xor butterflies: every
+// lane ends with the same bits
+__device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
-  const int w = threadIdx.x >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) lds[w] = v;
-  __syncthreads();
-  double t = 0;
-  for (int q = 0; q < NTHR / 64; ++q) t += lds[q];
-  return t;
+  return v;
 }
-
-__device__ __forceinline__ void block_maxloc(double &m, int &k, double *lds, int *ildx) {
+__device__ __forceinline__ void wave_maxloc(double &m, int &k) {
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) maxloc(m, k, __shfl_xor(m, s, 64), __shfl_xor(k, s, 64));
-  const int w = threadIdx.x >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) {
-    lds[w] = m;
-    ildx[w] = k;
-  }
-  __syncthreads();
-  m = lds[0];
-  k = ildx[0];
-  for (int q = 1; q < NTHR / 64; ++q) maxloc(m, k, lds[q], ildx[q]);
 }
 
+// One launch: every block reduces its share to a record (block b's quantity
+// q at part[MON_BLOCKS q + b]), and the block that finishes last reduces the
+// records, each quantity by one wavefront, to `out` (MON_REC doubles in host
+// memory the device can write).  `ticket` counts the finished blocks and
+// wraps back to zero with the last one.  The records pass between the XCDs'
+// L2 caches through agent-scope stores and loads on both sides of the
+// ticket.  A launch this small is latency alone, so the quantities share one
+// barrier.  A barrier pair for each (16 us), a second launch of one block for
+// the records (28 us) and the copy of the result made the call 66 us on 729
+// nodes; it is 33 us now, most of it the launch and the wait.
 template <typename R>
 __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParams P, ForceFrame F, int nres,
                                                          const int *host_index, const int *wall_nodes, int nw,
-                                                         const R *warea, double *part, int bsel) {
+                                                         const R *warea, double *part, unsigned *ticket, double *out,
+                                                         int bsel) {
   L.to_batch(bsel);
   P.to_batch(bsel);
-  __shared__ double lds[NTHR / 64];
-  __shared__ int ildx[NTHR / 64];
+  constexpr int NW = NTHR / 64;
+  __shared__ double lds[MON_REC][NW];
+  __shared__ bool last;
   const int n = L.n, stride = gridDim.x * NTHR;
   double sum[7], mx[7];
   int mi[7];
@@ -4021,49 +4016,60 @@ __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParam
 #pragma unroll
     for (int c = 0; c < 8; ++c) f[c] += o[c];
   }
-  double *rec = part + (size_t)MON_REC * blockIdx.x;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
   for (int j = 0; j < 7; ++j) {
-    double t = block_sum(sum[j], lds);
-    double m = mx[j];
-    int k = mi[j];
-    block_maxloc(m, k, lds, ildx);
-    if (threadIdx.x == 0) {
-      rec[j] = t;
-      rec[7 + j] = m;
-      rec[14 + j] = double(k);
+    const double t = wave_sum(sum[j]);
+    wave_maxloc(mx[j], mi[j]);
+    if (lane == 0) {
+      lds[j][wave] = t;
+      lds[7 + j][wave] = mx[j];
+      lds[14 + j][wave] = double(mi[j]);
     }
   }
+#pragma unroll
   for (int c = 0; c < 8; ++c) {
-    double t = block_sum(f[c], lds);
-    if (threadIdx.x == 0) rec[21 + c] = t;
+    const double t = wave_sum(f[c]);
+    if (lane == 0) lds[21 + c][wave] = t;
   }
-}
-
-// the MON_BLOCKS records to one, in block order (one block of NTHR threads)
-__global__ __launch_bounds__(NTHR) void k_monitor_final(const double *part, int nrec, double *out) {
-  __shared__ double lds[NTHR / 64];
-  __shared__ int ildx[NTHR / 64];
-  for (int q = 0; q < MON_REC; ++q) {
-    const bool is_max = q >= 7 && q < 14, is_idx = q >= 14 && q < 21;
-    if (is_idx) continue;
+  __syncthreads();
+  const int q = threadIdx.x;
+  if (q < MON_REC) {
+    double v = 0;
+    if (q >= 7 && q < 21) {  // the maxima, and the indices that go with them
+      const int j = q < 14 ? q : q - 7;
+      double m = lds[j][0];
+      int k = (int)lds[j + 7][0];
+      for (int w = 1; w < NW; ++w) maxloc(m, k, lds[j][w], (int)lds[j + 7][w]);
+      v = q < 14 ? m : double(k);
+    } else {
+      for (int w = 0; w < NW; ++w) v += lds[q][w];
+    }
+    __hip_atomic_store(part + (size_t)MON_BLOCKS * q + blockIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0) last = atomicInc(ticket, gridDim.x - 1) == gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  const int nrec = gridDim.x;
+  auto rec = [&](int r, int b) {
+    return __hip_atomic_load(part + (size_t)MON_BLOCKS * r + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  for (int r = wave; r < MON_REC; r += NW) {
+    if (r >= 14 && r < 21) continue;
     double v = 0;
     int k = 0x7fffffff;
-    for (int b = threadIdx.x; b < nrec; b += NTHR) {
-      const double *r = part + (size_t)MON_REC * b;
-      if (is_max)
-        maxloc(v, k, r[q], (int)r[q + 7]);
-      else
-        v += r[q];
+    for (int b = lane; b < nrec; b += 64) {
+      if (r >= 7 && r < 14) maxloc(v, k, rec(r, b), (int)rec(r + 7, b));
+      else v += rec(r, b);
     }
-    if (is_max) {
-      block_maxloc(v, k, lds, ildx);
-      if (threadIdx.x == 0) {
-        out[q] = v;
-        out[q + 7] = double(k);
-      }
-    } else {
-      double t = block_sum(v, lds);
-      if (threadIdx.x == 0) out[q] = t;
+    if (r >= 7 && r < 14) wave_maxloc(v, k);
+    else v = wave_sum(v);
+    if (lane == 0) {
+      out[r] = v;
+      if (r >= 7 && r < 14) out[r + 7] = double(k);
     }
   }
 }

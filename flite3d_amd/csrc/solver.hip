@@ -185,8 +185,9 @@ struct Level {
   // transfer from the next finer level (coarse levels)
   int *f2c = nullptr, *cptr = nullptr, *clist = nullptr;
   double *rw = nullptr;
-  // monitor records: MON_BLOCKS block records and the total (MON_REC doubles each)
+  // monitor records: MON_BLOCKS block records (MON_REC doubles each), and the count of finished blocks
   double *m_part = nullptr;
+  unsigned *m_ticket = nullptr;
   double *abuf = nullptr;  // adjoint side shares, 10 per side (allocated on first use)
   double *vmesh = nullptr;  // viscous mesh-adjoint shares, 3 per side and boundary side (first use)
   // second-order linearisation (allocated on first use): per-side adjoint
@@ -245,6 +246,7 @@ struct flite_ctx {
   std::vector<flite_params> hp_b;  // per condition (batched contexts)
   double *cond_dev = nullptr;      // per-condition Mach and inflow state on the device
   int sel = 0;                     // condition that field/state/monitor calls act on
+  double *mon_host = nullptr;      // the monitor's MON_REC results, in pinned host memory the kernel writes
   std::vector<std::unique_ptr<Level>> lev;
   // coarse levels of the other precision (flite_set_coarse_precision),
   // built on first use and swapped with lev[1..] on every switch
@@ -295,8 +297,8 @@ int check_launch() {
   return 0;
 }
 
-// Device scratch of flite_monitor_noalloc: the MON_BLOCKS block records and
-// the total, MON_REC doubles each (119 KB), held on every GPU the library
+// Device scratch of flite_monitor_noalloc: the MON_BLOCKS block records, MON_REC
+// doubles each (119 KB), held on every GPU the library
 // runs on until the process ends.  In host code `scratch` names a host-side
 // stand-in, not a device address: each GPU's copy is found once per device
 // with hipGetSymbolAddress (scratch_setup, called by flite_ctx_create with
@@ -305,7 +307,7 @@ constexpr int SCRATCH_DEVICES = 64;
 std::mutex g_scratch_mu;
 double *g_scratch_dev[SCRATCH_DEVICES] = {};
 }  // namespace
-static __device__ __align__(256) double scratch[MON_REC * (MON_BLOCKS + 1)];
+static __device__ __align__(256) double scratch[MON_REC * MON_BLOCKS];
 namespace {
 
 int scratch_setup(int dev) {
@@ -941,7 +943,8 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
   TRY(al_real(&L.jst, c->hp.flux_type != 4 ? (size_t)(8 * (size_t)n) * NB : 1));
   TRY(al_real(&L.uold, c->hp.flow_type != 0 ? (size_t)(6 * (size_t)n) * NB : 1));
   TRY(al_real(&L.uold2, c->hp.flow_type != 0 ? (size_t)(6 * (size_t)n) * NB : 1));
-  TRY(P.alloc(&L.m_part, (size_t)MON_REC * (MON_BLOCKS + 1)));
+  TRY(P.alloc(&L.m_part, (size_t)MON_REC * MON_BLOCKS));
+  TRY(P.alloc(&L.m_ticket, 1));
   // transfer operators from the finer level
   if (level > 1) {
     Level &F = *c->lev[level - 2];
@@ -1682,6 +1685,7 @@ int flite_ctx_create(const flite_params *p, int n_levels, int n_batch, flite_ctx
   c->staged.resize(n_levels);
   c->staged_ok.assign(n_levels, 0);
   HIPTRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+  HIPTRY(hipHostMalloc((void **)&c->mon_host, MON_REC * sizeof(double), hipHostMallocDefault));
   *out = c.release();
   return 0;
 }
@@ -1698,6 +1702,7 @@ void flite_ctx_destroy(flite_ctx *c) {
   c->lev.clear();
   c->lev_alt.clear();
   if (c->cond_dev) (void)hipFree(c->cond_dev);
+  if (c->mon_host) (void)hipHostFree(c->mon_host);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -1984,9 +1989,9 @@ int flite_apply(flite_ctx *c, int level, int op) {
 }  // extern "C"
 
 namespace {
-// the monitor's reductions on the device into part (MON_BLOCKS + 1 records
-// of MON_REC doubles: the blocks' records, then the total), the total
-// copied into tot; res, maxres, maxidx and forces formed from it
+// the monitor's reductions on the device, the blocks' records in part, the
+// total in the context's host record; res, maxres, maxidx and forces formed
+// from it.  One block per NTHR nodes, as many as fill the chip twice.
 int monitor_into(flite_ctx *c, double *part, double res[7], double maxres[7], int maxidx[7], double forces[9]) {
   Level &L = *c->lev[0];
   int nres = c->P.sa ? 6 : 5;
@@ -2008,17 +2013,14 @@ int monitor_into(flite_ctx *c, double *part, double res[7], double maxres[7], in
   F.groundplane = hp.groundplane;
   for (int k = 0; k < 3; ++k) F.datum[k] = hp.datum[k];
   int nw = (int)L.wall_dev.size();
-  double *total = part + (size_t)MON_REC * MON_BLOCKS;
   TRY(with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
-    hipLaunchKernelGGL(k_monitor_reduce<R>, dim3(MON_BLOCKS), dim3(NTHR), 0, c->stream, V, P, F, nres, L.host_index,
-                       L.wall_nodes, nw, (const R *)L.warea, part, bsel);
-    hipLaunchKernelGGL(k_monitor_final, dim3(1), dim3(NTHR), 0, c->stream, (const double *)part, MON_BLOCKS, total);
+    hipLaunchKernelGGL(k_monitor_reduce<R>, dim3(std::min(MON_BLOCKS, nblk(L.n))), dim3(NTHR), 0, c->stream, V, P, F,
+                       nres, L.host_index, L.wall_nodes, nw, (const R *)L.warea, part, L.m_ticket, c->mon_host, bsel);
     return check_launch();
   }));
-  double tot[MON_REC];
-  HIPTRY(hipMemcpyAsync(tot, total, sizeof(tot), hipMemcpyDeviceToHost, c->stream));
   TRY(sync(c));
+  const double *tot = c->mon_host;
   for (int j = 0; j < 7; ++j) { res[j] = 0; maxres[j] = 0; maxidx[j] = 0; }
   for (int j = 0; j < nres; ++j) {
     res[j] = std::sqrt(tot[j]);
@@ -2059,7 +2061,7 @@ int flite_monitor_noalloc(flite_ctx *c, double res[7], double maxres[7], int max
                                "builds it)");
   if (c->device < 0 || c->device >= SCRATCH_DEVICES || !g_scratch_dev[c->device])
     return fail(FLITE_E_STATE, "no monitor scratch on this context's device");
-  // the scratch holds MON_BLOCKS + 1 records whatever the level's size: the
+  // the scratch holds MON_BLOCKS records whatever the level's size: the
   // reduction's blocks stride over the nodes, so no size exceeds it
   return monitor_into(c, g_scratch_dev[c->device], res, maxres, maxidx, forces);
 }
