@@ -428,30 +428,57 @@ __device__ __forceinline__ bool gb_stage(const LevelDev<R> &L, R *sn, int blk) {
   return true;
 }
 
-// ---------------------------------------------------------------------------
 // node preparation: makePressureField (DEF:13612-13630) + gather records
 // ---------------------------------------------------------------------------
 template <typename R>
-__global__ void k_prep(LevelDev<R> L, DevParams P) {
+__device__ __forceinline__ R state_pressure(const DevParams &P, const R *q) {
+  R pp = R(P.gamma - 1.0) * (q[4] - R(0.5) * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0]);
+  return pp > R(0.1) ? pp : R(0.1);
+}
+
+// pressure and gather record of node i for the state q[6]
+template <typename R>
+__device__ __forceinline__ void write_record(const LevelDev<R> &L, const DevParams &P, int i, const R *q, R mu) {
+  R pp = state_pressure(P, q);
+  L.p[i] = pp;
+  R *g = L.rec0 + 8 * (size_t)i;
+  g[0] = q[0];
+  g[1] = q[1] / q[0];
+  g[2] = q[2] / q[0];
+  g[3] = q[3] / q[0];
+  g[4] = q[4];
+  g[5] = pp;
+  g[6] = P.sa ? q[5] : R(0);
+  g[7] = mu;
+}
+
+// What a smoothing step starts from: the pressure and gather record of the
+// state q[6] and the state itself as the step's previous one (ncopy
+// components), and with `zero` an empty dissipation.  Every kernel that
+// leaves a level's state ready for its next smoothing step does this in the
+// same launch (k_restrict_forcing, k_map_state, k_prolong).
+template <typename R>
+__device__ __forceinline__ void begin_step(const LevelDev<R> &L, const DevParams &P, int i, const R *q, R mu,
+                                           int ncopy, int zero) {
+  const size_t n = L.n;
+  write_record(L, P, i, q, mu);
+  for (int c = 0; c < ncopy; ++c) L.uprev[c * n + i] = q[c];
+  if (zero)
+    for (int c = 0; c < 5; ++c) L.diss[c * n + i] = R(0);
+}
+
+// pressure and records of the current state; ncopy > 0 and zero as begin_step
+template <typename R>
+__global__ void k_prep(LevelDev<R> L, DevParams P, int ncopy, int zero) {
   int bb_;
   int i = btid(L.nb, bb_);
   L.to_batch(bb_);
   P.to_batch(bb_);
   if (i >= L.n) return;
-  int n = L.n;
-  R r = L.u[i], m1 = L.u[n + i], m2 = L.u[2 * n + i], m3 = L.u[3 * n + i], E = L.u[4 * n + i];
-  R pp = R(P.gamma - 1.0) * (E - R(0.5) * (m1 * m1 + m2 * m2 + m3 * m3) / r);
-  pp = pp > R(0.1) ? pp : R(0.1);
-  L.p[i] = pp;
-  R *q = L.rec0 + 8 * (size_t)i;
-  q[0] = r;
-  q[1] = m1 / r;
-  q[2] = m2 / r;
-  q[3] = m3 / r;
-  q[4] = E;
-  q[5] = pp;
-  q[6] = P.sa ? L.u[5 * n + i] : R(0);
-  q[7] = L.mu[i];
+  const size_t n = L.n;
+  R q[6];
+  for (int c = 0; c < 6; ++c) q[c] = L.u[c * n + i];
+  begin_step(L, P, i, q, L.mu[i], ncopy, zero);
 }
 
 // gather records from the current state without recomputing p (parity ops)
@@ -1304,10 +1331,11 @@ __global__ void k_jst_sums(LevelDev<R> L, DevParams P) {
 //           d2 = d0 k2 max(nu_a, nu_b), d4 = dim(d0 k4, d2);
 //   matrix: dr4, dr2 <- |w| |A| dr4, |w| |A| dr2 (Roe matrix along w in
 //           Turkel's form, Harten's fix), d2 = k2 max(nu), d4 = dim(k4, d2);
-// D_a += -dr4 d4 + dr2 d2 and D_b += dr4 d4 - dr2 d2, gathered per node and
-// added to the dissipation array (k4: coarse-grid factor below grid 1).
+// D_a += -dr4 d4 + dr2 d2 and D_b += dr4 d4 - dr2 d2, gathered per node into
+// the dissipation array (`add`: on top of the viscous term there; k4:
+// coarse-grid factor below grid 1).
 template <typename R, bool MATRIX>
-__global__ void k_jst_flux(LevelDev<R> L, DevParams P) {
+__global__ void k_jst_flux(LevelDev<R> L, DevParams P, int add) {
   int bb_;
   int i = btid(L.nb, bb_);
   L.to_batch(bb_);
@@ -1385,7 +1413,7 @@ __global__ void k_jst_flux(LevelDev<R> L, DevParams P) {
     }
   });
 #pragma unroll
-  for (int c = 0; c < 5; ++c) L.diss[c * n + i] += acc[c];
+  for (int c = 0; c < 5; ++c) L.diss[c * n + i] = (add ? L.diss[c * n + i] : R(0)) + acc[c];
 }
 
 // makeSASourceTerm (DEF:9285-9370) of one node on any arithmetic type: the
@@ -3724,18 +3752,7 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
     if (!S.next_record) return;
     // pressure and gather record of the new state, as k_prep forms them, so
     // the next stage starts without a separate pass
-    R pp = R(P.gamma - 1.0) * (q[4] - R(0.5) * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0]);
-    pp = pp > R(0.1) ? pp : R(0.1);
-    L.p[i] = pp;
-    R *g = L.rec0 + 8 * (size_t)i;
-    g[0] = q[0];
-    g[1] = q[1] / q[0];
-    g[2] = q[2] / q[0];
-    g[3] = q[3] / q[0];
-    g[4] = q[4];
-    g[5] = pp;
-    g[6] = P.sa ? q[5] : R(0);
-    g[7] = L.mu[i];
+    write_record(L, P, i, q, L.mu[i]);
   } else if (MODE == MODE_COARSE) {
     outer_bc(L, P, i, q, pi);
     for (int c = 0; c < 6; ++c) {
@@ -3798,92 +3815,182 @@ __global__ void k_bc_state(LevelDev<R> L, DevParams P, R *a, int outer) {
 // members of each coarse node: out[c*nc+k] = sum_i rw_i in[c*nf+i].  In the
 // nested device order the members of coarse node k are the contiguous fine
 // range [cptr[k], cptr[k+1]); SUB lanes per coarse node read it coalesced.
+//
+// The transfers are node-local once the members are summed, so each is one
+// launch with all that follows it at the node: the boundary conditions, the
+// pressure and records, the forcing, the correction of the fine members.  On
+// the small levels a launch costs 4-5 us whatever it does; as separate
+// kernels (restriction of u and mu, pressure, conditions, copy, pressure,
+// zero dissipation | restriction, forcing | restriction, conditions,
+// correction, prolongation) a restriction took 9 launches more and a
+// prolongation 3.  Every lane of a group ends its sum with the same bits
+// (lsum), so the correction is formed on all of them.
+struct Transfer {
+  const int *cptr;
+  const double *rw;
+  int nf;  // fine nodes
+};
+
+// sum over the members of coarse node k of NC components of `in`
+template <int SUB, int NC, typename RF>
+__device__ __forceinline__ void restrict_sum(const Transfer &T, const RF *in, int k, int sub, double *acc) {
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = 0;
+  for (int i = T.cptr[k] + sub; i < T.cptr[k + 1]; i += SUB) {
+    double r = T.rw[i];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] += r * double(in[(size_t)c * T.nf + i]);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = lsum<SUB>(acc[c]);
+}
+
+// six components of a state array
 template <typename RF, typename RC, int SUB>
-__global__ void k_restrict(const int *cptr, const double *rw, const RF *in, RC *out, int nc, int nf, int ncomp,
-                           int nb, long long in_bs, long long out_bs) {
+__global__ void k_restrict(Transfer T, const RF *in, RC *out, int nc, int nb) {
   int k, sub, bb_;
   node_lanes<SUB>(nb, bb_, k, sub);
   if (k >= nc) return;
-  in += (size_t)bb_ * (size_t)in_bs;
-  out += (size_t)bb_ * (size_t)out_bs;
-  double acc[6] = {0, 0, 0, 0, 0, 0};
-  for (int i = cptr[k] + sub; i < cptr[k + 1]; i += SUB) {
-    double r = rw[i];
-#pragma unroll
-    for (int c = 0; c < 6; ++c)
-      if (c < ncomp) acc[c] += r * double(in[(size_t)c * nf + i]);
-  }
-#pragma unroll
-  for (int c = 0; c < 6; ++c) acc[c] = lsum<SUB>(acc[c]);
+  double acc[6];
+  restrict_sum<SUB, 6>(T, in + (size_t)bb_ * 6 * (size_t)T.nf, k, sub, acc);
   if (sub) return;
+  out += (size_t)bb_ * 6 * (size_t)nc;
 #pragma unroll
-  for (int c = 0; c < 6; ++c)
-    if (c < ncomp) out[(size_t)c * nc + k] = RC(acc[c]);
+  for (int c = 0; c < 6; ++c) out[(size_t)c * nc + k] = RC(acc[c]);
 }
 
-// prolongateGrid (DEF:12432-12570) after the coarse correction rhs_H is
-// formed: inject, relax, add, BCs, clamps on the fine level
-template <typename RF, typename RC>
-__global__ void k_prolong_fine(LevelDev<RF> F, DevParams P, const int *f2c, const RC *crhs, int nc, int ncomp_add) {
-  int bb_;
-  int i = btid(F.nb, bb_);
+// mapFineToCoarse of u, ready for the coarse level's smoothing step
+template <typename RF, typename RC, int SUB>
+__global__ void k_map_state(LevelDev<RC> K, DevParams P, Transfer T, const RF *fu, int ncopy) {
+  int k, sub, bb_;
+  node_lanes<SUB>(K.nb, bb_, k, sub);
+  K.to_batch(bb_);
+  P.to_batch(bb_);
+  if (k >= K.n) return;
+  double acc[6];
+  restrict_sum<SUB, 6>(T, fu + (size_t)bb_ * 6 * (size_t)T.nf, k, sub, acc);
+  if (sub) return;
+  RC q[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    q[c] = RC(acc[c]);
+    K.u[(size_t)c * K.n + k] = q[c];
+  }
+  begin_step(K, P, k, q, K.mu[k], ncopy, 0);
+}
+
+// start of restrictGrid (DEF:12158-12184): u and the laminar viscosity
+// restricted, the boundary conditions on the restricted state (with its own
+// pressure), which is also kept as the previous one; pressure and records
+template <typename RF, typename RC, int SUB>
+__global__ void k_restrict_state(LevelDev<RC> K, DevParams P, Transfer T, const RF *fu, const RF *fmu, int zero) {
+  int k, sub, bb_;
+  node_lanes<SUB>(K.nb, bb_, k, sub);
+  K.to_batch(bb_);
+  P.to_batch(bb_);
+  if (k >= K.n) return;
+  double acc[6], am[1];
+  restrict_sum<SUB, 6>(T, fu + (size_t)bb_ * 6 * (size_t)T.nf, k, sub, acc);
+  restrict_sum<SUB, 1>(T, fmu + (size_t)bb_ * (size_t)T.nf, k, sub, am);
+  if (sub) return;
+  RC q[6], mu = RC(am[0]);
+#pragma unroll
+  for (int c = 0; c < 6; ++c) q[c] = RC(acc[c]);
+  K.mu[k] = mu;
+  RC pp = state_pressure(P, q);
+  bc_solution(K, P, k, q, q[0]);
+  outer_bc(K, P, k, q, pp);
+#pragma unroll
+  for (int c = 0; c < 6; ++c) K.u[(size_t)c * K.n + k] = q[c];
+  begin_step(K, P, k, q, mu, 6, zero);
+}
+
+// end of restrictGrid (DEF:12362-12428): the fine increment restricted to
+// rhs_H, BC'd as an increment, sourceTerm -= rhs_H, u_H += rhs_H; with
+// `begin` also the start of the coarse level's smoothing step
+template <typename RF, typename RC, int SUB>
+__global__ void k_restrict_forcing(LevelDev<RC> K, DevParams P, Transfer T, const RF *frhs, int begin) {
+  int k, sub, bb_;
+  node_lanes<SUB>(K.nb, bb_, k, sub);
+  K.to_batch(bb_);
+  P.to_batch(bb_);
+  if (k >= K.n) return;
+  double acc[6];
+  restrict_sum<SUB, 6>(T, frhs + (size_t)bb_ * 6 * (size_t)T.nf, k, sub, acc);
+  if (sub) return;
+  const size_t n = K.n;
+  RC r[6], q[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) r[c] = RC(acc[c]);
+  bc_increment(K, P, k, r);
+  const int nc = P.sa ? 6 : 5;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    K.rhs[c * n + k] = r[c];
+    q[c] = K.u[c * n + k];
+    if (c < nc) {
+      K.src[c * n + k] -= r[c];
+      q[c] += r[c];
+      K.u[c * n + k] = q[c];
+    }
+  }
+  if (begin) begin_step(K, P, k, q, K.mu[k], nc, 0);
+}
+
+// prolongateGrid (DEF:12432-12570): the coarse correction v_H = u_H -
+// BC(R u_h), BC'd as an increment, then on the fine members: inject, relax,
+// add, boundary conditions, clamps; with `begin` also the start of the fine
+// level's smoothing step
+template <typename RF, typename RC, int SUB>
+__global__ void k_prolong(LevelDev<RF> F, LevelDev<RC> K, DevParams P, Transfer T, int ncomp_add, int begin, int zero) {
+  int k, sub, bb_;
+  node_lanes<SUB>(K.nb, bb_, k, sub);
   F.to_batch(bb_);
-  P.to_batch(bb_);
-  crhs += (size_t)bb_ * 6 * (size_t)nc;
-  if (i >= F.n) return;
-  int n = F.n;
-  int k = f2c[i];
-  RF d[6];
-  for (int c = 0; c < 6; ++c) d[c] = RF(crhs[(size_t)c * nc + k]);
-  for (int c = 0; c < 5; ++c) d[c] = RF(P.prolong_relax) * d[c];
-  d[5] = RF(P.turb_prolong_relax) * d[5];
-  if (F.ncls[i] & NC_BFIRST)
-    for (int c = 0; c < 5; ++c) d[c] = RF(P.mg_bc_relax) * d[c];
-  for (int c = 0; c < 6; ++c) F.rhs[(size_t)c * n + i] = d[c];
-  RF q[6];
-  for (int c = 0; c < 6; ++c) q[c] = F.u[(size_t)c * n + i];
-  for (int c = 0; c < ncomp_add; ++c) q[c] = q[c] + d[c];
-  bc_solution(F, P, i, q, q[0]);
-  outer_bc(F, P, i, q, F.p[i]);
-  if (P.sa) q[5] = q[5] > RF(0) ? q[5] : RF(0);
-  q[0] = q[0] > RF(P.min_rho) ? q[0] : RF(P.min_rho);
-  for (int c = 0; c < 6; ++c) F.u[(size_t)c * n + i] = q[c];
-}
-
-// coarse correction v_H = u_H - BC(R u_h), BC'd as an increment
-template <typename R>
-__global__ void k_coarse_correction(LevelDev<R> K, DevParams P) {
-  int bb_;
-  int i = btid(K.nb, bb_);
   K.to_batch(bb_);
   P.to_batch(bb_);
-  if (i >= K.n) return;
-  int n = K.n;
-  R r[6];
-  for (int c = 0; c < 6; ++c) r[c] = K.u[(size_t)c * n + i] - K.uprev[(size_t)c * n + i];
+  if (k >= K.n) return;
+  const size_t nc = K.n, n = F.n;
+  double acc[6];
+  restrict_sum<SUB, 6>(T, F.u, k, sub, acc);
+  RC q[6], r[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) q[c] = RC(acc[c]);
+  bc_solution(K, P, k, q, K.u[k]);
+  outer_bc(K, P, k, q, K.p[k]);
+#pragma unroll
+  for (int c = 0; c < 6; ++c) r[c] = K.u[c * nc + k] - q[c];
   if (!P.sa) r[5] = 0;
-  bc_increment(K, P, i, r);
-  for (int c = 0; c < 6; ++c) K.rhs[(size_t)c * n + i] = r[c];
-}
-
-// end of restrictGrid: rhs_H BC'd as increment, sourceTerm -= rhs_H,
-// u_H += rhs_H (DEF:12362-12428)
-template <typename R>
-__global__ void k_restrict_finish(LevelDev<R> K, DevParams P) {
-  int bb_;
-  int i = btid(K.nb, bb_);
-  K.to_batch(bb_);
-  P.to_batch(bb_);
-  if (i >= K.n) return;
-  int n = K.n;
-  R r[6];
-  for (int c = 0; c < 6; ++c) r[c] = K.rhs[(size_t)c * n + i];
-  bc_increment(K, P, i, r);
-  int nc = P.sa ? 6 : 5;
-  for (int c = 0; c < 6; ++c) K.rhs[(size_t)c * n + i] = r[c];
-  for (int c = 0; c < nc; ++c) {
-    K.src[(size_t)c * n + i] -= r[c];
-    K.u[(size_t)c * n + i] += r[c];
+  bc_increment(K, P, k, r);
+  if (sub == 0) {
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      K.uprev[c * nc + k] = q[c];
+      K.rhs[c * nc + k] = r[c];
+    }
+  }
+  for (int i = T.cptr[k] + sub; i < T.cptr[k + 1]; i += SUB) {
+    RF d[6], v[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) d[c] = RF(r[c]);
+#pragma unroll
+    for (int c = 0; c < 5; ++c) d[c] = RF(P.prolong_relax) * d[c];
+    d[5] = RF(P.turb_prolong_relax) * d[5];
+    if (F.ncls[i] & NC_BFIRST)
+#pragma unroll
+      for (int c = 0; c < 5; ++c) d[c] = RF(P.mg_bc_relax) * d[c];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      F.rhs[c * n + i] = d[c];
+      v[c] = F.u[c * n + i];
+      if (c < ncomp_add) v[c] = v[c] + d[c];
+    }
+    bc_solution(F, P, i, v, v[0]);
+    outer_bc(F, P, i, v, F.p[i]);
+    if (P.sa) v[5] = v[5] > RF(0) ? v[5] : RF(0);
+    v[0] = v[0] > RF(P.min_rho) ? v[0] : RF(P.min_rho);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) F.u[c * n + i] = v[c];
+    if (begin) begin_step(F, P, i, v, F.mu[i], P.sa ? 6 : 5, zero);
   }
 }
 

@@ -1057,13 +1057,13 @@ int ensure_built(flite_ctx *c) {
 // ---------------------------------------------------------------------------
 // operations
 // ---------------------------------------------------------------------------
-int op_prep(flite_ctx *c, Level &L, bool compute_p) {
+int op_prep(flite_ctx *c, Level &L, bool compute_p, int ncopy = 0, bool zero = false) {
   DevParams P = c->P;
   Timed tm(c, "prep", L.gnum);
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
     if (compute_p) {
-      hipLaunchKernelGGL(k_prep<R>, dim3(nblk(L.n) * L.nbatch), dim3(NTHR), 0, c->stream, V, P);
+      hipLaunchKernelGGL(k_prep<R>, dim3(nblk(L.n) * L.nbatch), dim3(NTHR), 0, c->stream, V, P, ncopy, int(zero));
     } else {
       hipLaunchKernelGGL(k_pack<R>, dim3(nblk(L.n) * L.nbatch), dim3(NTHR), 0, c->stream, V, P);
     }
@@ -1198,22 +1198,27 @@ int op_zero_diss(flite_ctx *c, Level &L) {
   });
 }
 
-// makeArtificialDissipation2 (DEF:11484-11993) in two steps: op_dissipation
-// zeroes the array (as the routine does first), op_jst adds the JST terms
-// once the local time steps exist.  The reference computes the time steps
-// before the dissipation and subtracts the viscous term after it
-// (DEF:1023-1047).  Here the viscous gather writes dissipation = -viscous
-// (ViscFluxPart), so op_jst always runs after it and adds its node totals:
-// -viscous + JST is the reference's JST - viscous, each a single addition.
-int op_dissipation(flite_ctx *c, Level &L) { return op_zero_diss(c, L); }
-
+// makeArtificialDissipation2 (DEF:11484-11993).  The reference zeroes the
+// array, computes the time steps before the dissipation and subtracts the
+// viscous term after it (DEF:1023-1047).  Here the viscous gather writes
+// dissipation = -viscous (ViscFluxPart), so op_jst always runs after it and
+// adds its node totals: -viscous + JST is the reference's JST - viscous, each
+// a single addition.  Without a viscous term the JST totals overwrite the
+// array; with neither, the step's start zeroes it (zero_dissipation).
 bool jst_active(const flite_ctx *c, const Level &L) {
   const flite_params &hp = c->hp;
   if (hp.flux_type == 4 && L.gnum == 1) return false;  // DEF:11506
   return !(hp.fourth_order_dissipation_factor == 0.0 && hp.second_order_dissipation_factor == 0.0);  // DEF:11508
 }
 
-int op_jst(flite_ctx *c, Level &L) {
+bool viscous(const flite_ctx *c) { return c->hp.reynolds_number > 0.0; }
+
+// no kernel of the step writes the level's dissipation: its start must
+bool zero_dissipation(const flite_ctx *c, const Level &L) {
+  return !viscous(c) && !(jst_active(c, L) && L.ne > 0);
+}
+
+int op_jst(flite_ctx *c, Level &L, bool add) {
   if (!jst_active(c, L) || L.ne == 0) return 0;
   DevParams P = c->P;
   Timed tm(c, "dissipation", L.gnum);
@@ -1221,8 +1226,8 @@ int op_jst(flite_ctx *c, Level &L) {
     using R = std::remove_pointer_t<decltype(V.u)>;
     dim3 g(nblk(L.n) * L.nbatch), b(NTHR);
     hipLaunchKernelGGL(k_jst_sums<R>, g, b, 0, c->stream, V, P);
-    if (P.matdiss) hipLaunchKernelGGL((k_jst_flux<R, true>), g, b, 0, c->stream, V, P);
-    else hipLaunchKernelGGL((k_jst_flux<R, false>), g, b, 0, c->stream, V, P);
+    if (P.matdiss) hipLaunchKernelGGL((k_jst_flux<R, true>), g, b, 0, c->stream, V, P, int(add));
+    else hipLaunchKernelGGL((k_jst_flux<R, false>), g, b, 0, c->stream, V, P, int(add));
     return check_launch();
   });
 }
@@ -1311,40 +1316,59 @@ int op_bc_state(flite_ctx *c, Level &L, void *a, int outer) {
   });
 }
 
-// mapFineToCoarse of ncomp columns from array fa of F into array ka of K
-int op_restrict_array(flite_ctx *c, Level &F, Level &K, const void *fa, void *ka, int ncomp) {
-  auto go = [&](auto *fin, auto *kout) {
-    using RF = std::remove_const_t<std::remove_pointer_t<decltype(fin)>>;
-    using RC = std::remove_pointer_t<decltype(kout)>;
-    constexpr int SUB = 4;  // about 8 fine members per coarse node
-    long long per = ncomp == 1 ? 1 : 6;  // components allocated per node of the array
-    hipLaunchKernelGGL((k_restrict<RF, RC, SUB>), dim3(nblk((long long)K.n * SUB) * K.nbatch), dim3(NTHR), 0,
-                       c->stream, K.cptr, K.rw, fin, kout, K.n, F.n, ncomp, K.nbatch, per * F.n, per * K.n);
-    return check_launch();
-  };
-  if (F.fp32 && K.fp32) return go((const float *)fa, (float *)ka);
-  if (!F.fp32 && K.fp32) return go((const double *)fa, (float *)ka);
-  if (F.fp32 && !K.fp32) return go((const float *)fa, (double *)ka);
-  return go((const double *)fa, (double *)ka);
+constexpr int TRANSFER_SUB = 4;  // lanes per coarse node: about 8 fine members each
+
+Transfer transfer(const Level &F, const Level &K) { return Transfer{K.cptr, K.rw, F.n}; }
+
+dim3 transfer_grid(const Level &K) { return dim3(nblk((long long)K.n * TRANSFER_SUB) * K.nbatch); }
+
+// f(fine level's view, coarse level's view), each in its own precision
+template <typename FN>
+int with_levels(const Level &F, const Level &K, FN f) {
+  return with_level(F, [&](auto FV) { return with_level(K, [&](auto KV) { return f(FV, KV); }); });
 }
 
-int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss) {
+// mapFineToCoarse of the six components of array fa of F into array ka of K
+int op_restrict_array(flite_ctx *c, Level &F, Level &K, const void *fa, void *ka) {
+  return with_levels(F, K, [&](auto FV, auto KV) {
+    using RF = std::remove_pointer_t<decltype(FV.u)>;
+    using RC = std::remove_pointer_t<decltype(KV.u)>;
+    hipLaunchKernelGGL((k_restrict<RF, RC, TRANSFER_SUB>), transfer_grid(K), dim3(NTHR), 0, c->stream, transfer(F, K),
+                       (const RF *)fa, (RC *)ka, K.n, K.nbatch);
+    return check_launch();
+  });
+}
+
+// mapFineToCoarse of u, with the start of the coarse level's smoothing step
+int op_map_state(flite_ctx *c, Level &F, Level &K) {
+  DevParams P = c->P;
+  return with_levels(F, K, [&](auto FV, auto KV) {
+    using RF = std::remove_pointer_t<decltype(FV.u)>;
+    using RC = std::remove_pointer_t<decltype(KV.u)>;
+    hipLaunchKernelGGL((k_map_state<RF, RC, TRANSFER_SUB>), transfer_grid(K), dim3(NTHR), 0, c->stream, KV, P,
+                       transfer(F, K), (const RF *)F.u, P.sa ? 6 : 5);
+    return check_launch();
+  });
+}
+
+// begun: an earlier launch has done the step's start (begin_step).
+// record_last: the last stage leaves the records of its state too, for a
+// restriction that follows within the cycle.
+int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss, bool begun, bool record_last) {
   const flite_params &hp = c->hp;
+  if (!begun) TRY(op_prep(c, L, true, c->P.sa ? 6 : 5, calc_diss && zero_dissipation(c, L)));
   if (calc_diss) {
-    TRY(op_prep(c, L, true));
-    TRY(op_dissipation(c, L));
-    if (hp.reynolds_number > 0.0) {
+    if (viscous(c)) {
       // makeTimeSteps, makeViscosityTerm, makeTurbulentTimeSteps, makeSADiffusion
       TRY(op_step_terms(c, L, true, true));
     } else {
       TRY(op_timesteps(c, L));
     }
-    TRY(op_jst(c, L));
+    TRY(op_jst(c, L, viscous(c)));
   }
   for (int k = 1; k <= hp.rk_stages; ++k) {
     // stage k > 1 starts from the pressure and records the previous stage
-    // kernel wrote with the new state; stage 1 after the frozen terms too
-    if (k == 1 && !calc_diss) TRY(op_prep(c, L, true));
+    // kernel wrote with the new state
     TRY(op_grad(c, L));
     TRY(op_flux(c, L));
     StageArgs S;
@@ -1354,40 +1378,43 @@ int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss) {
     S.calc_turb = 1;
     S.fas = L.gnum > 1;
     S.has_src = L.gnum > 1;
-    S.next_record = k < hp.rk_stages;
+    S.next_record = k < hp.rk_stages || record_last;
     TRY(op_stage(c, L, MODE_STAGE, S));
   }
   return 0;
 }
 
-int do_time_iterations(flite_ctx *c, int level, int steps, bool calc_diss) {
+int do_time_iterations(flite_ctx *c, int level, int steps, bool calc_diss, bool begun = false,
+                       bool record_last = false) {
   Level &L = *c->lev[level - 1];
-  for (int s = 0; s < steps; ++s) {
-    TRY(op_copy(c, L, L.uprev, L.u, c->P.sa ? 6 : 5));
-    TRY(do_single_iteration(c, L, calc_diss));
-  }
+  for (int s = 0; s < steps; ++s)
+    TRY(do_single_iteration(c, L, calc_diss, begun && s == 0, record_last && s + 1 == steps));
   return 0;
 }
 
-int do_restrict(flite_ctx *c, int fine_level) {
+// recorded: the fine level's records and (where no kernel writes it) zero
+// dissipation are those of its state already.  begin: a smoothing step of
+// the coarse level follows.
+int do_restrict(flite_ctx *c, int fine_level, bool recorded = false, bool begin = false) {
   Level &F = *c->lev[fine_level - 1];
   Level &K = *c->lev[fine_level];
   const flite_params &hp = c->hp;
-  bool visc = hp.reynolds_number > 0.0;
+  const bool visc = viscous(c);
+  DevParams P = c->P;
   // coarse part (DEF:12158-12234)
-  TRY(op_restrict_array(c, F, K, F.u, K.u, 6));
-  TRY(op_restrict_array(c, F, K, F.mu, K.mu, 1));
-  TRY(op_prep(c, K, true));
-  TRY(op_bc_state(c, K, K.u, 1));
-  TRY(op_copy(c, K, K.uprev, K.u, 6));
-  TRY(op_prep(c, K, true));
-  TRY(op_dissipation(c, K));
+  TRY(with_levels(F, K, [&](auto FV, auto KV) {
+    using RF = std::remove_pointer_t<decltype(FV.u)>;
+    using RC = std::remove_pointer_t<decltype(KV.u)>;
+    hipLaunchKernelGGL((k_restrict_state<RF, RC, TRANSFER_SUB>), transfer_grid(K), dim3(NTHR), 0, c->stream, KV, P,
+                       transfer(F, K), (const RF *)F.u, (const RF *)F.mu, int(zero_dissipation(c, K)));
+    return check_launch();
+  }));
   if (visc) {
     TRY(op_step_terms(c, K, true, true));
   } else {
     TRY(op_timesteps(c, K));
   }
-  TRY(op_jst(c, K));
+  TRY(op_jst(c, K, visc));
   TRY(op_flux(c, K));
   StageArgs S;
   S.alpha = 1.0;
@@ -1398,50 +1425,36 @@ int do_restrict(flite_ctx *c, int fine_level) {
   S.has_src = 1;
   TRY(op_stage(c, K, MODE_COARSE, S));
   // fine part (DEF:12236-12361)
-  TRY(op_prep(c, F, true));
-  TRY(op_dissipation(c, F));
+  if (!recorded) TRY(op_prep(c, F, true, 0, zero_dissipation(c, F)));
   if (visc) TRY(op_step_terms(c, F, false, false));
-  TRY(op_jst(c, F));  // with the time steps of the last smoothing step
+  TRY(op_jst(c, F, visc));  // with the time steps of the last smoothing step
   TRY(op_grad(c, F));
   TRY(op_flux(c, F));
   S.has_src = F.gnum > 1;
   TRY(op_stage(c, F, MODE_FINE, S));
   // coarse forcing (DEF:12362-12428)
-  TRY(op_restrict_array(c, F, K, F.rhs, K.rhs, 6));
-  DevParams P = c->P;
-  TRY(with_level(K, [&](auto V) {
-    using R = std::remove_pointer_t<decltype(V.u)>;
-    hipLaunchKernelGGL(k_restrict_finish<R>, dim3(nblk(K.n) * K.nbatch), dim3(NTHR), 0, c->stream, V, P);
+  return with_levels(F, K, [&](auto FV, auto KV) {
+    using RF = std::remove_pointer_t<decltype(FV.u)>;
+    using RC = std::remove_pointer_t<decltype(KV.u)>;
+    hipLaunchKernelGGL((k_restrict_forcing<RF, RC, TRANSFER_SUB>), transfer_grid(K), dim3(NTHR), 0, c->stream, KV, P,
+                       transfer(F, K), (const RF *)F.rhs, int(begin));
     return check_launch();
-  }));
-  return 0;
+  });
 }
 
-int do_prolongate(flite_ctx *c, int coarse_level) {
+// begin: a smoothing step of the fine level follows
+int do_prolongate(flite_ctx *c, int coarse_level, bool begin = false) {
   Level &K = *c->lev[coarse_level - 1];
   Level &F = *c->lev[coarse_level - 2];
   DevParams P = c->P;
-  TRY(op_restrict_array(c, F, K, F.u, K.uprev, 6));
-  TRY(op_bc_state(c, K, K.uprev, 1));
-  TRY(with_level(K, [&](auto V) {
-    using R = std::remove_pointer_t<decltype(V.u)>;
-    hipLaunchKernelGGL(k_coarse_correction<R>, dim3(nblk(K.n) * K.nbatch), dim3(NTHR), 0, c->stream, V, P);
-    return check_launch();
-  }));
   int ncomp = (F.gnum < c->hp.number_of_turbulence_grids && P.sa) ? 6 : 5;
-  auto go = [&](auto FV, auto *crhs) {
+  return with_levels(F, K, [&](auto FV, auto KV) {
     using RF = std::remove_pointer_t<decltype(FV.u)>;
-    using RC = std::remove_pointer_t<decltype(crhs)>;
-    hipLaunchKernelGGL((k_prolong_fine<RF, RC>), dim3(nblk(F.n) * F.nbatch), dim3(NTHR), 0, c->stream, FV, P, K.f2c,
-                       (const RC *)crhs, K.n, ncomp);
+    using RC = std::remove_pointer_t<decltype(KV.u)>;
+    hipLaunchKernelGGL((k_prolong<RF, RC, TRANSFER_SUB>), transfer_grid(K), dim3(NTHR), 0, c->stream, FV, KV, P,
+                       transfer(F, K), ncomp, int(begin), int(zero_dissipation(c, F)));
     return check_launch();
-  };
-  if (F.fp32) {
-    auto FV = F.view<float>();
-    return K.fp32 ? go(FV, (float *)K.rhs) : go(FV, (double *)K.rhs);
-  }
-  auto FV = F.view<double>();
-  return K.fp32 ? go(FV, (float *)K.rhs) : go(FV, (double *)K.rhs);
+  });
 }
 
 int do_cycle(flite_ctx *c, int cycle) {
@@ -1454,7 +1467,7 @@ int do_cycle(flite_ctx *c, int cycle) {
     for (int i = 1; i < ng; ++i) {
       Level &F = *c->lev[i - 1];
       TRY(op_copy(c, F, F.uprev, F.u, 6));
-      TRY(op_restrict_array(c, F, *c->lev[i], F.u, c->lev[i]->u, 6));
+      TRY(op_restrict_array(c, F, *c->lev[i], F.u, c->lev[i]->u));
     }
     Level &Kc = *c->lev[ng - 1];
     TRY(with_level(Kc, [&](auto V) {
@@ -1465,27 +1478,31 @@ int do_cycle(flite_ctx *c, int cycle) {
     }));
     TRY(do_time_iterations(c, ng, nrs, true));
   } else if (hp.multigrid_scheme == 1) {
+    const bool more = nrs > 0;  // a smoothing step follows each transfer
     for (int i = 1; i < ng; ++i) {
-      TRY(do_time_iterations(c, i, nrs, i == 1));
-      TRY(do_restrict(c, i));
+      TRY(do_time_iterations(c, i, nrs, i == 1, more && i > 1, true));
+      TRY(do_restrict(c, i, more));
       Level &F = *c->lev[i - 1];
-      TRY(op_restrict_array(c, F, *c->lev[i], F.u, c->lev[i]->u, 6));
+      TRY(op_map_state(c, F, *c->lev[i]));
     }
-    TRY(do_time_iterations(c, ng, nrs, ng == 1));
+    TRY(do_time_iterations(c, ng, nrs, ng == 1, more && ng > 1));
     for (int i = ng; i >= 2; --i) {
-      TRY(do_prolongate(c, i));
-      TRY(do_time_iterations(c, i - 1, nrs, (i - 1) == 1));
+      TRY(do_prolongate(c, i, more));
+      TRY(do_time_iterations(c, i - 1, nrs, (i - 1) == 1, more));
     }
   } else if (hp.multigrid_scheme == 3) {
+    const bool more = nrs > 0;
     int sweeps = ng == 1 ? 1 : ng - 1, finest = 1;
     for (int s = 1; s <= sweeps; ++s) {
       for (int j = finest; j <= ng - 1; ++j) {
-        TRY(do_time_iterations(c, j, nrs, j == finest));
-        TRY(do_restrict(c, j));
+        // the previous sweep's prolongation or this one's restriction has
+        // started the step
+        TRY(do_time_iterations(c, j, nrs, j == finest, more && (s > 1 || j > finest), true));
+        TRY(do_restrict(c, j, more, more));
       }
-      TRY(do_time_iterations(c, ng, nrs, ng == 1));
+      TRY(do_time_iterations(c, ng, nrs, ng == 1, more && ng > 1));
       finest = finest == 1 ? (ng >= 2 ? ng - 1 : ng) : finest - 1;
-      for (int j = ng; j >= finest + 1; --j) TRY(do_prolongate(c, j));
+      for (int j = ng; j >= finest + 1; --j) TRY(do_prolongate(c, j, more && s < sweeps && j == finest + 1));
     }
   } else {
     return fail(FLITE_E_UNSUPPORTED, "multigrid scheme not implemented");
@@ -1506,8 +1523,8 @@ int preamble(flite_ctx *c) {
       return check_launch();
     }));
     if (l > 0) {
-      TRY(op_restrict_array(c, *c->lev[l - 1], L, c->lev[l - 1]->u, L.u, 6));
-      if (c->hp.flow_type != 0) TRY(op_restrict_array(c, *c->lev[l - 1], L, c->lev[l - 1]->uold, L.uold, 6));
+      TRY(op_restrict_array(c, *c->lev[l - 1], L, c->lev[l - 1]->u, L.u));
+      if (c->hp.flow_type != 0) TRY(op_restrict_array(c, *c->lev[l - 1], L, c->lev[l - 1]->uold, L.uold));
     }
   }
   return sync(c);
@@ -1911,7 +1928,7 @@ int flite_map_u_fine_to_coarse(flite_ctx *c, int fine_level) {
   TRY(check_ctx(c));
   if (fine_level < 1 || fine_level >= c->nl) return fail(FLITE_E_ARG, "fine_level out of range");
   Level &F = *c->lev[fine_level - 1];
-  TRY(op_restrict_array(c, F, *c->lev[fine_level], F.u, c->lev[fine_level]->u, 6));
+  TRY(op_restrict_array(c, F, *c->lev[fine_level], F.u, c->lev[fine_level]->u));
   return sync(c);
 }
 
@@ -1956,7 +1973,7 @@ int flite_apply(flite_ctx *c, int level, int op) {
     case FLITE_OP_PRESSURE:
     case FLITE_OP_PRESSURE_ABS: TRY(op_prep(c, L, true)); break;
     case FLITE_OP_TIMESTEPS: TRY(op_prep(c, L, false)); TRY(op_timesteps(c, L)); break;
-    case FLITE_OP_DISSIPATION: TRY(op_dissipation(c, L)); TRY(op_jst(c, L)); break;
+    case FLITE_OP_DISSIPATION: TRY(op_zero_diss(c, L)); TRY(op_jst(c, L, false)); break;
     case FLITE_OP_VISCOUS:
       if (!(c->hp.reynolds_number > 0.0)) return fail(FLITE_E_ARG, "viscous term needs ReynoldsNumber > 0");
       TRY(op_prep(c, L, false));
