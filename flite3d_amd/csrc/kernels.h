@@ -113,10 +113,26 @@ struct LevelDev {
   int ngb;
   const int *gb_first, *gb_nptr, *gb_node;
   const unsigned short *ell_loc;
+  // node blocks of the one-launch stages (k_stage_blk): block k's header is
+  // sb_head[8 k ..] = {first node, nodes, first staged entry, staged nodes,
+  // first task, tasks, first incidence, incidences}.  Staged nodes: the
+  // block's own, then their other neighbours.  Task t: sb_loc[t] = both ends'
+  // staged positions (12 bits each) | kind << 24 (0: an interior side, k + 1:
+  // a boundary side of indicator k (k <= 0 as 0: they are walls alike), seen
+  // from its first listed end), sb_w[3]
+  // (SoA, stride sb_ntask) its weight; sb_inc[sb_iptr[i] ..] = node i's tasks
+  // within the block (task << 1 | 1 when the node is the side's second end)
+  int nsb;
+  long long sb_ntask;
+  const int *sb_head, *sb_node, *sb_iptr;
+  const unsigned *sb_loc;
+  const unsigned short *sb_inc;
+  const R *sb_w;
   const R *vol, *xyz, *wd, *nrm;  // nrm: 3 per node AoS
   const int *ncls;
   R *u, *uprev, *rhs, *diss, *src, *p, *dt, *dtt, *mu, *vort, *divg, *tdiff;
   R *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;  // tau, dnu: VREC-strided, one shared record
+  R *rec1;  // the next state's gather records while a walking stage reads rec0 (null: no such stage)
   R *jst;  // JST node record (8 per node): L(U) 5, pressure switch, side count, pad
   R *uold, *uold2;  // solutions at the last two physical times (6 per node, unsteady only)
   // moving meshes (null on a fixed mesh): GCL weight per side and 2 per
@@ -142,6 +158,7 @@ struct LevelDev {
     divg += bn;
     tdiff += bn;
     rec0 += 8 * bn;
+    if (rec1) rec1 += 8 * bn;
     grec += (size_t)b * (size_t)gstride;
     tau += VREC * bn;
     dnu += VREC * bn;
@@ -436,12 +453,13 @@ __device__ __forceinline__ R state_pressure(const DevParams &P, const R *q) {
   return pp > R(0.1) ? pp : R(0.1);
 }
 
-// pressure and gather record of node i for the state q[6]
+// pressure and gather record (into rec) of node i for the state q[6]
 template <typename R>
-__device__ __forceinline__ void write_record(const LevelDev<R> &L, const DevParams &P, int i, const R *q, R mu) {
+__device__ __forceinline__ void write_record(const LevelDev<R> &L, const DevParams &P, int i, const R *q, R mu,
+                                             R *rec) {
   R pp = state_pressure(P, q);
   L.p[i] = pp;
-  R *g = L.rec0 + 8 * (size_t)i;
+  R *g = rec + 8 * (size_t)i;
   g[0] = q[0];
   g[1] = q[1] / q[0];
   g[2] = q[2] / q[0];
@@ -461,7 +479,7 @@ template <typename R>
 __device__ __forceinline__ void begin_step(const LevelDev<R> &L, const DevParams &P, int i, const R *q, R mu,
                                            int ncopy, int zero) {
   const size_t n = L.n;
-  write_record(L, P, i, q, mu);
+  write_record(L, P, i, q, mu, L.rec0);
   for (int c = 0; c < ncopy; ++c) L.uprev[c * n + i] = q[c];
   if (zero)
     for (int c = 0; c < 5; ++c) L.diss[c * n + i] = R(0);
@@ -1116,6 +1134,18 @@ __device__ __forceinline__ void farfield_roe(const double *inf, const R *q, R gm
   f[4] = R(0.5) * (fr5 + fl5) - R(0.5) * (rl3 * du5 + cc1 * hi + cc2 * ucp);
 }
 
+// the boundary flux of one end's state along the side's unit normal
+template <typename R>
+__device__ __forceinline__ void bside_state_flux(const DevParams &P, int ind, const R *q, R rnx, R rny, R rnz, R *f) {
+  if (ind <= 2 || ind == 9) {
+    phys_flux(q, rnx, rny, rnz, f);
+  } else {
+    double inf[6];
+    P.inflow_row(ind - 3, inf);
+    farfield_roe(inf, q, R(P.gamma - 1.0), rnx, rny, rnz, f);
+  }
+}
+
 // boundary-side loop of makeRHS (DEF:2116-2446): contributions to both ends,
 // bbuf[10*s + 5*end + c]
 template <typename R>
@@ -1160,16 +1190,8 @@ __global__ void k_bflux(LevelDev<R> L, DevParams P) {
   const R *A = L.rec0 + 8 * (size_t)ia;
   const R *B = L.rec0 + 8 * (size_t)ib;
   R f1[5], f2[5];
-  if (ind <= 2 || ind == 9) {
-    phys_flux(A, rnx, rny, rnz, f1);
-    phys_flux(B, rnx, rny, rnz, f2);
-  } else {
-    R gm1 = R(P.gamma - 1.0);
-    double inf[6];
-    P.inflow_row(ind - 3, inf);
-    farfield_roe(inf, A, gm1, rnx, rny, rnz, f1);
-    farfield_roe(inf, B, gm1, rnx, rny, rnz, f2);
-  }
+  bside_state_flux(P, ind, A, rnx, rny, rnz, f1);
+  bside_state_flux(P, ind, B, rnx, rny, rnz, f2);
 #pragma unroll
   for (int c = 0; c < 5; ++c) {
     if (P.bterm == 1) {
@@ -1191,27 +1213,16 @@ __global__ void k_bflux(LevelDev<R> L, DevParams P) {
 // the textbook fluxes |w| (F_1 + F_2 + D) along w/|w|: the reference reads
 // their densities (and Roe's enthalpies) before assigning them and subtracts
 // the upwind term D, which reverses its sign; both are repaired here.
-// fbuf[6 e + c] as k_flux (component 5: SA convection from the records).
-template <typename R, int FT, bool SA>
-__global__ void k_flux_simple(LevelDev<R> L, DevParams P) {
-  int bb_;
-  int e = btid(L.nb, bb_);
-  L.to_batch(bb_);
-  P.to_batch(bb_);
-  if (e >= L.ne) return;
-  const size_t n = L.n;
-  int ia = L.ea[e], ib = L.eb[e];
-  R wx = L.w[3 * e], wy = L.w[3 * e + 1], wz = L.w[3 * e + 2];
-  R r1 = L.u[ia], ru1 = L.u[n + ia], rv1 = L.u[2 * n + ia], rw1 = L.u[3 * n + ia], E1 = L.u[4 * n + ia];
-  R r2 = L.u[ib], ru2 = L.u[n + ib], rv2 = L.u[2 * n + ib], rw2 = L.u[3 * n + ib], E2 = L.u[4 * n + ib];
-  R pr1 = L.p[ia], pr2 = L.p[ib];
+template <typename R>
+__device__ __forceinline__ void simple_flux(const DevParams &P, int ft, const R *U1, R pr1, const R *U2, R pr2, R wx,
+                                            R wy, R wz, R wg, R *f) {
+  R r1 = U1[0], ru1 = U1[1], rv1 = U1[2], rw1 = U1[3], E1 = U1[4];
+  R r2 = U2[0], ru2 = U2[1], rv2 = U2[2], rw2 = U2[3], E2 = U2[4];
   R rinv1 = R(1) / r1, rinv2 = R(1) / r2;
   R u1 = rinv1 * ru1, v1 = rinv1 * rv1, w1 = rinv1 * rw1, rh1 = E1 + pr1;
   R u2 = rinv2 * ru2, v2 = rinv2 * rv2, w2 = rinv2 * rw2, rh2 = E2 + pr2;
-  R f[5];
-  const R wg = L.gcl ? L.gcl[e] / R(P.dtp) : R(0);
   const R us[5] = {r1 + r2, ru1 + ru2, rv1 + rv2, rw1 + rw2, E1 + E2};
-  if constexpr (FT == 1) {
+  if (ft == 1) {
     f[0] = wx * (ru1 + ru2) + wy * (rv1 + rv2) + wz * (rw1 + rw2);
     f[1] = wx * (ru1 * u1 + pr1 + ru2 * u2 + pr2) + wy * (ru1 * v1 + ru2 * v2) + wz * (ru1 * w1 + ru2 * w2);
     f[2] = wx * (rv1 * u1 + rv2 * u2) + wy * (rv1 * v1 + pr1 + rv2 * v2 + pr2) + wz * (rv1 * w1 + rv2 * w2);
@@ -1231,7 +1242,7 @@ __global__ void k_flux_simple(LevelDev<R> L, DevParams P) {
       R F2[5] = {r2 * nv2, pr2 * rnx + ru2 * nv2, pr2 * rny + rv2 * nv2, pr2 * rnz + rw2 * nv2, rh2 * nv2};
       R du[5] = {r1 - r2, ru1 - ru2, rv1 - rv2, rw1 - rw2, E1 - E2};
       R D[5];
-      if constexpr (FT == 2) {
+      if (ft == 2) {
         R c1 = sqrt(R(P.gamma) * pr1 * rinv1), c2 = sqrt(R(P.gamma) * pr2 * rinv2);
         R l1 = fabs(nv1 + c1), l12 = fabs(nv2 + c2);
         if (l1 < l12) l1 = l12;
@@ -1269,6 +1280,27 @@ __global__ void k_flux_simple(LevelDev<R> L, DevParams P) {
         for (int c = 0; c < 5; ++c) f[c] -= us[c] * wg;
     }
   }
+}
+
+// fbuf[6 e + c] as k_flux (component 5: SA convection from the records).
+template <typename R, int FT, bool SA>
+__global__ void k_flux_simple(LevelDev<R> L, DevParams P) {
+  int bb_;
+  int e = btid(L.nb, bb_);
+  L.to_batch(bb_);
+  P.to_batch(bb_);
+  if (e >= L.ne) return;
+  const size_t n = L.n;
+  int ia = L.ea[e], ib = L.eb[e];
+  R wx = L.w[3 * e], wy = L.w[3 * e + 1], wz = L.w[3 * e + 2];
+  R ua[5], ub[5], f[5];
+#pragma unroll
+  for (int c = 0; c < 5; ++c) {
+    ua[c] = L.u[c * n + ia];
+    ub[c] = L.u[c * n + ib];
+  }
+  const R wg = L.gcl ? L.gcl[e] / R(P.dtp) : R(0);
+  simple_flux(P, FT, ua, L.p[ia], ub, L.p[ib], wx, wy, wz, wg, f);
   R *o = L.fbuf + 6 * (size_t)e;
 #pragma unroll
   for (int c = 0; c < 5; ++c) o[c] = f[c];
@@ -3093,6 +3125,12 @@ struct TimeStepPart {
   static constexpr bool AUX = false;
   R lam, lamv, cc, am, gam;
   bool visc;
+  // a state's convective speed through a face: |w.v| + |w| c
+  static __device__ __forceinline__ R speed(const DevParams &P, const R *q, R wx, R wy, R wz, R al) {
+    R c = R(P.gamma) * q[5] / q[0];
+    c = c > R(0.001) ? c : R(0.001);
+    return fabs(wx * q[1] + wy * q[2] + wz * q[3]) + sqrt(c * al);
+  }
   __device__ void init(const LevelDev<R> &, const DevParams &P, int, const R *qi) {
     gam = R(P.gamma);
     cc = gam * qi[5] / qi[0];
@@ -3507,7 +3545,7 @@ __global__ void k_mu_record(LevelDev<R> L) {
 
 // makeSASourceTerm (DEF:9285-9370) for node i; returns the rhs(:,6) increment
 template <typename R>
-__device__ __forceinline__ double sa_source(LevelDev<R> &L, const DevParams &P, int i) {
+__device__ __forceinline__ double sa_source(const LevelDev<R> &L, const DevParams &P, int i) {
   const int n = L.n;
   double mu = L.mu[i];
   if (mu < 0.1 / P.Re) {
@@ -3641,6 +3679,8 @@ __device__ __forceinline__ void gather_rhs(const LevelDev<R> &L, int i, int sub,
   }
 }
 
+enum { FLUX_SIDES = 0, FLUX_PARTIALS = 1, FLUX_BLOCK = 2 };  // where a stage takes the interior fluxes from
+
 // Stage kernel modes
 //   MODE_RHS      rhs = makeRHS (+ makeSARHS/Source if SA)                 (parity)
 //   MODE_STAGE    singleIteration RK stage body (DEF:1074-1180)
@@ -3660,18 +3700,12 @@ struct StageArgs {
                              // reference's makePressureField leaves it)
 };
 
-template <typename R, int MODE, bool SA, int SUB>
-__global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
-  int i, sub;
-  int bb_;
-  node_lanes<SUB>(L.nb, bb_, i, sub);
-  L.to_batch(bb_);
-  P.to_batch(bb_);
-  if (i >= L.n) return;
-  int n = L.n;
-  R r[6];
-  gather_rhs<R, SA, SUB>(L, i, sub, S.partials, r);
-  if (sub) return;
+// the stage at node i from its convective residual r[6]; rec: where the
+// next state's gather record goes
+template <typename R, int MODE, bool SA>
+__device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams &P, const StageArgs &S, int i, R *r,
+                                           R *rec) {
+  const int n = L.n;
   bool sa_on = SA && S.calc_turb;
   if (sa_on) r[5] += R(sa_source(L, P, i));
   if (MODE == MODE_RHS) {
@@ -3752,7 +3786,7 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
     if (!S.next_record) return;
     // pressure and gather record of the new state, as k_prep forms them, so
     // the next stage starts without a separate pass
-    write_record(L, P, i, q, L.mu[i]);
+    write_record(L, P, i, q, L.mu[i], rec);
   } else if (MODE == MODE_COARSE) {
     outer_bc(L, P, i, q, pi);
     for (int c = 0; c < 6; ++c) {
@@ -3773,6 +3807,135 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
     for (int c = 0; c < 5; ++c) L.rhs[(size_t)c * n + i] = q[c] - up[c];
     L.rhs[5 * (size_t)n + i] = SA ? q[5] - up[5] : R(0);
   }
+}
+
+template <typename R, int MODE, bool SA, int SUB>
+__global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
+  int i, sub;
+  int bb_;
+  node_lanes<SUB>(L.nb, bb_, i, sub);
+  L.to_batch(bb_);
+  P.to_batch(bb_);
+  if (i >= L.n) return;
+  R r[6];
+  gather_rhs<R, SA, SUB>(L, i, sub, S.partials, r);
+  if (sub) return;
+  stage_node<R, MODE, SA>(L, P, S, i, r, L.rec0);
+}
+
+// One launch per stage: the residual of a block of consecutive nodes and
+// their update.  The block stages the records of its nodes and of their
+// neighbours in LDS, each thread evaluates one task from them (an interior
+// side that touches the block, or a boundary side seen from one of the
+// block's nodes), the fluxes take the records' place in LDS, and the threads
+// of a node sum its tasks and advance it.  A side between two blocks is
+// evaluated by both, in its stored orientation, so both ends still take the
+// same bits with opposite signs; that is about 1.4 times the arithmetic of
+// the sides, for two launches less (side fluxes, boundary fluxes) and no
+// partial sums through memory.  The neighbours' records are read while other
+// blocks write theirs, so the next state's go to rec1 and the host swaps the
+// two.  Latency bounds it (a launch and a chain of four loads), so one task
+// a thread and blocks as large as that allows.  Per stage, FP64 without SA,
+// against the three launches: 8.8 us for 18 on 1.3k nodes, 23.5 for 27 on
+// 33k.  (A walk of each node's own sides, every flux at both ends, measured
+// 14 and 40 us.)  Second-order sides stay with k_flux_blk: their records are
+// five times as long and their arithmetic twice, so the repeated sides cost
+// more than the launches.
+// STEP: the nodes' local time steps (makeTimeSteps, inviscid) from the same
+// tasks.
+constexpr int SB_NODES = 32, SB_TASKS = NTHR, SB_CAP = 224, SB_INC = 512, SB_SUB = NTHR / SB_NODES;
+constexpr int SB_S = 7;  // LDS stride of a record (not mu) and of a task's result, odd
+
+template <typename R, int MODE, bool SA, bool HLLC, bool STEP>
+__global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, StageArgs S) {
+  static_assert(SB_CAP <= SB_TASKS && !(SA && STEP), "one LDS area serves the records and the results");
+  __shared__ R sn[SB_TASKS * SB_S];
+  __shared__ unsigned short sinc[SB_INC];
+  const int lb = xcd_block(), bb_ = lb % L.nb, blk = lb / L.nb, t = threadIdx.x;
+  L.to_batch(bb_);
+  P.to_batch(bb_);
+  if (blk >= L.nsb) return;
+  const int4 h0 = reinterpret_cast<const int4 *>(L.sb_head)[2 * blk];
+  const int4 h1 = reinterpret_cast<const int4 *>(L.sb_head)[2 * blk + 1];
+  const int *nodes = L.sb_node + h0.z;
+  // this thread's task and node: their words are requested before the staging
+  const bool active = t < h1.y;
+  unsigned loc = 0;
+  R wx = 0, wy = 0, wz = 0;
+  if (active) {
+    loc = L.sb_loc[h1.x + t];
+    wx = L.sb_w[h1.x + t];
+    wy = L.sb_w[L.sb_ntask + h1.x + t];
+    wz = L.sb_w[2 * L.sb_ntask + h1.x + t];
+  }
+  const int me = t / SB_SUB, sub = t % SB_SUB, i = h0.x + me;
+  int q0 = 0, q1 = 0;
+  if (me < h0.y) {
+    q0 = L.sb_iptr[i] - h1.z;
+    q1 = L.sb_iptr[i + 1] - h1.z;
+  }
+#pragma unroll
+  for (int q = 0; q < SB_INC / NTHR; ++q)
+    if (t + q * NTHR < h1.w) sinc[t + q * NTHR] = L.sb_inc[h1.z + t + q * NTHR];
+  fb_stage<SB_CAP, 8, 8, 0, SB_S, R, SB_S>(sn, L.rec0, nodes, h0.w);
+  __syncthreads();
+  R f[7] = {0, 0, 0, 0, 0, 0, 0};
+  if (active) {
+    const R *A = sn + (loc & 0xfffu) * SB_S, *B = sn + ((loc >> 12) & 0xfffu) * SB_S;
+    const int kind = loc >> 24;
+    if (kind == 0) {
+      if constexpr (HLLC) {
+        side_flux<R, R, 1, SA, 2>(P, (const R *)nullptr, (const R *)nullptr, (const R *)nullptr, (const R *)nullptr, A,
+                                  B, wx, wy, wz, f);
+      } else {
+        const R UA[5] = {A[0], A[0] * A[1], A[0] * A[2], A[0] * A[3], A[4]};
+        const R UB[5] = {B[0], B[0] * B[1], B[0] * B[2], B[0] * B[3], B[4]};
+        simple_flux(P, P.ftype, UA, A[5], UB, B[5], wx, wy, wz, R(0), f);
+        f[5] = SA ? sa_side_convection(A, B, wx, wy, wz) : R(0);
+      }
+      if constexpr (STEP) {  // each end's own speed through the side
+        const R al = wx * wx + wy * wy + wz * wz;
+        f[5] = TimeStepPart<R>::speed(P, A, wx, wy, wz, al);
+        f[6] = TimeStepPart<R>::speed(P, B, wx, wy, wz, al);
+      }
+    } else {
+      const int ind = kind - 1;
+      const R al = wx * wx + wy * wy + wz * wz, rnorm = sqrt(al);
+      if (rnorm > R(1e-10) && (ind <= 4 || ind == 9)) {
+        const R irn = R(1) / rnorm;
+        R f1[5], f2[5];
+        bside_state_flux(P, ind, A, wx * irn, wy * irn, wz * irn, f1);
+        bside_state_flux(P, ind, B, wx * irn, wy * irn, wz * irn, f2);
+#pragma unroll
+        for (int c = 0; c < 5; ++c)
+          f[c] = P.bterm == 1 ? rnorm * (R(3) * f1[c] + f2[c]) : rnorm * R(4) * f1[c];
+      }
+      if constexpr (STEP)
+        f[5] = R(2) * TimeStepPart<R>::speed(P, A, wx, wy, wz, al) + TimeStepPart<R>::speed(P, B, wx, wy, wz, al);
+    }
+  }
+  __syncthreads();  // the records are no longer needed: the results take their place
+  if (active) {
+#pragma unroll
+    for (int c = 0; c < SB_S; ++c) sn[SB_S * t + c] = f[c];
+  }
+  __syncthreads();
+  if (me >= h0.y) return;
+  R r[6] = {0, 0, 0, 0, 0, 0}, lam = 0;
+  for (int q = q0 + sub; q < q1; q += SB_SUB) {
+    const unsigned v = sinc[q];
+    const R *o = sn + SB_S * (v >> 1);
+    const bool second = v & 1u;
+#pragma unroll
+    for (int c = 0; c < (SA ? 6 : 5); ++c) r[c] += second ? -o[c] : o[c];
+    if constexpr (STEP) lam += second ? o[6] : o[5];
+  }
+#pragma unroll
+  for (int c = 0; c < (SA ? 6 : 5); ++c) r[c] = lsum<SB_SUB>(r[c]);
+  if constexpr (STEP) lam = lsum<SB_SUB>(lam);
+  if (sub) return;
+  if constexpr (STEP) L.dt[i] = R(0.5) / (lam / L.vol[i]);
+  stage_node<R, MODE, SA>(L, P, S, i, r, L.rec1);
 }
 
 // ---------------------------------------------------------------------------

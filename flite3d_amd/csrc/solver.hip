@@ -159,6 +159,7 @@ struct Level {
   void *w, *wb, *vol, *xyz, *wd, *nrm, *warea;
   void *u, *uprev, *rhs, *diss, *src, *p, *dt, *dtt, *mu, *vort, *divg, *tdiff;
   void *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;
+  void *rec1 = nullptr;  // second record buffer of the one-launch stages (levels that use them)
   void *jst = nullptr;  // JST node records (fluxType 1-3 only)
   void *uold = nullptr, *uold2 = nullptr;  // unsteady only
   void *gcl = nullptr, *bgcl = nullptr, *volp = nullptr, *volp2 = nullptr, *cmv = nullptr;  // moving mesh only
@@ -177,11 +178,18 @@ struct Level {
   } sb[FB_NSHAPES];
   int fb_shape = 0;
   void *pbuf = nullptr;  // sized for the largest nent of the shapes
-  bool flux_partials = false;  // the last interior fluxes went to pbuf (k_flux_blk), not fbuf
+  int flux_src = FLUX_SIDES;  // where the last interior fluxes are: fbuf, pbuf (k_flux_blk) or the stage's own blocks
   // node blocks of the LDS-staged gathers (ngb = 0: the per-node kernels)
   int ngb = 0;
   int *gb_first = nullptr, *gb_nptr = nullptr, *gb_node = nullptr;
   unsigned short *ell_loc = nullptr;
+  // node blocks of the one-launch stages (nsb = 0: none)
+  int nsb = 0;
+  long long sb_ntask = 0;
+  int *sb_head = nullptr, *sb_node = nullptr, *sb_iptr = nullptr;
+  unsigned *sb_loc = nullptr;
+  unsigned short *sb_inc = nullptr;
+  void *sb_w = nullptr;
   // transfer from the next finer level (coarse levels)
   int *f2c = nullptr, *cptr = nullptr, *clist = nullptr;
   double *rw = nullptr;
@@ -210,11 +218,13 @@ struct Level {
     v.nent = B.nent; v.fb_iptr = B.iptr; v.fb_inc = B.inc; v.pn_ptr = B.pn_ptr; v.pn_ent = B.pn_ent;
     v.pbuf = (R *)pbuf;
     v.ngb = ngb; v.gb_first = gb_first; v.gb_nptr = gb_nptr; v.gb_node = gb_node; v.ell_loc = ell_loc;
+    v.nsb = nsb; v.sb_ntask = sb_ntask; v.sb_head = sb_head; v.sb_node = sb_node; v.sb_iptr = sb_iptr;
+    v.sb_loc = sb_loc; v.sb_inc = sb_inc; v.sb_w = (const R *)sb_w;
     v.vol = (const R *)vol; v.xyz = has_coords ? (const R *)xyz : nullptr;
     v.wd = (const R *)wd; v.nrm = (const R *)nrm; v.ncls = ncls;
     v.u = (R *)u; v.uprev = (R *)uprev; v.rhs = (R *)rhs; v.diss = (R *)diss; v.src = (R *)src;
     v.p = (R *)p; v.dt = (R *)dt; v.dtt = (R *)dtt; v.mu = (R *)mu; v.vort = (R *)vort;
-    v.divg = (R *)divg; v.tdiff = (R *)tdiff; v.rec0 = (R *)rec0; v.grec = (R *)grec;
+    v.divg = (R *)divg; v.tdiff = (R *)tdiff; v.rec0 = (R *)rec0; v.rec1 = (R *)rec1; v.grec = (R *)grec;
     v.tau = (R *)tau; v.dnu = (R *)dnu; v.fbuf = (R *)fbuf; v.bbuf = (R *)bbuf; v.ws = (R *)ws;
     v.jst = (R *)jst;
     v.uold = (R *)uold;
@@ -234,6 +244,7 @@ struct flite_ctx {
   int lanes_override = 0;  // FLITE_GATHER_LANES: 1, 4 or 16 on every level (0 = by size)
   int shape_override = -1;  // FLITE_SIDE_BLOCK: side-block shape by sides per block (-1: shape 0)
   bool flux_per_side = false;  // FLITE_FLUX_KERNEL=side: one lane per side with direct record loads
+  bool flux_apart = false;     // FLITE_FLUX_KERNEL=block or side: fluxes and stage in launches of their own on every level
   bool gather_per_node = false;  // FLITE_GATHER_KERNEL=node: no LDS-staged node blocks
   bool grad_direct = false;      // FLITE_GRAD_STORE=direct: per-thread record stores in the gradient
   // One cycle's launches form the same sequence with the same arguments
@@ -680,6 +691,132 @@ int build_side_blocks(Level &L, int shape, const std::vector<int> &ea, const std
   return 0;
 }
 
+// Node blocks of the one-launch stages (LevelDev::sb_*): consecutive nodes,
+// at most SB_NODES of them with at most SB_TASKS sides and (boundary side,
+// own end) pairs, SB_CAP staged nodes and SB_INC incidences.  No blocks if a
+// single node exceeds a limit.
+struct StageTables {
+  std::vector<int> head, node, iptr;
+  std::vector<unsigned> loc;
+  std::vector<unsigned short> inc;
+  std::vector<double> w;
+};
+
+StageTables build_stage_blocks(int n, const std::vector<int> &ell_ptr, const std::vector<int> &ell_k,
+                               const std::vector<int> &ell_e, const std::vector<int> &ell_nbr,
+                               const std::vector<double> &ellw, size_t nslot, const std::vector<int> &bs_ptr,
+                               const std::vector<int> &bs_list, const std::vector<int> &ba, const std::vector<int> &bb,
+                               const std::vector<int> &bind, const std::vector<double> &wb) {
+  StageTables T;
+  T.iptr.push_back(0);
+  struct Side {
+    int e, a, b;  // device side, its ends
+    double w[3];
+  };
+  std::vector<double> wv[3];
+  std::vector<int> own_stamp(n, -1), local(n, 0), halo;
+  std::vector<Side> sides;
+  // sides of node i not seen from an earlier node of the block start..i-1
+  auto new_sides = [&](int start, int i, std::vector<Side> *out) {
+    int cnt = 0;
+    const int s = i / SLICE, lane = i % SLICE;
+    for (int k = 0; k < ell_k[s]; ++k) {
+      const size_t slot = ell_ptr[s] + (size_t)k * SLICE + lane;
+      const int v = ell_e[slot], j = ell_nbr[slot];
+      if (v < 0 || (j >= start && j < i)) continue;
+      ++cnt;
+      if (!out) continue;
+      Side d{v >> 1, (v & 1) ? j : i, (v & 1) ? i : j, {0, 0, 0}};
+      for (int q = 0; q < 3; ++q) d.w[q] = (v & 1) ? -ellw[q * nslot + slot] : ellw[q * nslot + slot];
+      out->push_back(d);
+    }
+    return cnt;
+  };
+  auto degree = [&](int i) {
+    const int s = i / SLICE, lane = i % SLICE;
+    int d = bs_ptr[i + 1] - bs_ptr[i];
+    for (int k = 0; k < ell_k[s]; ++k) d += ell_e[ell_ptr[s] + (size_t)k * SLICE + lane] >= 0;
+    return d;
+  };
+  // neighbours of node i that block `blk` has not staged, stamped as they are counted
+  auto new_staged = [&](int blk, int i, std::vector<int> *out) {
+    int cnt = 0;
+    auto see = [&](int j) {
+      if (own_stamp[j] == blk) return;
+      own_stamp[j] = blk;
+      ++cnt;
+      if (out) out->push_back(j);
+    };
+    see(i);
+    const int s = i / SLICE, lane = i % SLICE;
+    for (int k = 0; k < ell_k[s]; ++k) {
+      const size_t slot = ell_ptr[s] + (size_t)k * SLICE + lane;
+      if (ell_e[slot] >= 0) see(ell_nbr[slot]);
+    }
+    for (int k = bs_ptr[i]; k < bs_ptr[i + 1]; ++k) {
+      const int v = bs_list[k], b = v >> 1;
+      see((v & 1) ? ba[b] : bb[b]);
+    }
+    return cnt;
+  };
+  for (int start = 0, blk = 0; start < n; ++blk) {
+    int end = start, tasks = 0, staged = 0, inc = 0;
+    for (; end < n && end - start < SB_NODES; ++end) {
+      const int nt = new_sides(start, end, nullptr) + (bs_ptr[end + 1] - bs_ptr[end]), ni = degree(end);
+      const int ns = new_staged(blk, end, nullptr);
+      if (tasks + nt > SB_TASKS || staged + ns > SB_CAP || inc + ni > SB_INC) break;
+      tasks += nt;
+      staged += ns;
+      inc += ni;
+    }
+    if (end == start) return StageTables{};  // one node alone exceeds a limit
+    // staged positions: the block's nodes, then the others ascending
+    sides.clear();
+    halo.clear();
+    const int mark = n + blk;  // a stamp of its own: the loop above also stamped the rejected node's neighbours
+    for (int i = start; i < end; ++i) {
+      local[i] = i - start;
+      own_stamp[i] = mark;
+    }
+    for (int i = start; i < end; ++i) {
+      new_sides(start, i, &sides);
+      new_staged(mark, i, &halo);
+    }
+    std::sort(halo.begin(), halo.end());
+    for (size_t q = 0; q < halo.size(); ++q) local[halo[q]] = end - start + (int)q;
+    std::sort(sides.begin(), sides.end(), [](const Side &x, const Side &y) { return x.e < y.e; });
+    const int task0 = (int)T.loc.size(), inc0 = (int)T.inc.size(), node0 = (int)T.node.size();
+    std::vector<std::vector<unsigned short>> list(end - start);
+    for (const Side &d : sides) {
+      const unsigned t = (unsigned)T.loc.size() - task0;
+      T.loc.push_back((unsigned)local[d.a] | (unsigned)local[d.b] << 12);
+      for (int q = 0; q < 3; ++q) wv[q].push_back(d.w[q]);
+      if (d.a >= start && d.a < end) list[d.a - start].push_back((unsigned short)(t << 1));
+      if (d.b >= start && d.b < end) list[d.b - start].push_back((unsigned short)(t << 1 | 1));
+    }
+    for (int i = start; i < end; ++i)
+      for (int k = bs_ptr[i]; k < bs_ptr[i + 1]; ++k) {
+        const int v = bs_list[k], b = v >> 1, o = (v & 1) ? ba[b] : bb[b];
+        const unsigned t = (unsigned)T.loc.size() - task0;
+        T.loc.push_back((unsigned)local[i] | (unsigned)local[o] << 12 | (unsigned)(std::max(bind[b], 0) + 1) << 24);
+        for (int q = 0; q < 3; ++q) wv[q].push_back(wb[3 * (size_t)b + q]);
+        list[i - start].push_back((unsigned short)(t << 1));
+      }
+    for (const auto &l : list) {
+      T.inc.insert(T.inc.end(), l.begin(), l.end());
+      T.iptr.push_back((int)T.inc.size());
+    }
+    for (int i = start; i < end; ++i) T.node.push_back(i);
+    T.node.insert(T.node.end(), halo.begin(), halo.end());
+    for (int v : {start, end - start, node0, (int)T.node.size() - node0, task0, (int)T.loc.size() - task0, inc0,
+                  (int)T.inc.size() - inc0})
+      T.head.push_back(v);
+    start = end;
+  }
+  for (int q = 0; q < 3; ++q) T.w.insert(T.w.end(), wv[q].begin(), wv[q].end());
+  return T;
+}
+
 int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int> &h2d, bool coarse_fp32,
                 std::unique_ptr<Level> &out) {
   auto Lp = std::make_unique<Level>();
@@ -928,6 +1065,21 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
   TRY(al_real(&L.tdiff, (size_t)(n) * NB));
   TRY(al_real(&L.rec0, (size_t)(8 * (size_t)n) * NB));
   bool need_grad = L.has_coords && c->hp.hllc_flux_order > 1;
+  const bool second = need_grad && c->hp.flux_type == 4;
+  if (!second && S.gcl.empty() && S.bgcl.empty() && ne > 0) {
+    StageTables T = build_stage_blocks(n, ell_ptr, ell_k, ell_e, ell_nbr, ellw, nslot, bs_ptr, bs_list, ba, bb, S.bi, wb);
+    L.nsb = T.head.empty() ? 0 : (int)(T.head.size() / 8);
+    if (L.nsb > 0) {
+      L.sb_ntask = (long long)T.loc.size();
+      TRY(P.upload(&L.sb_head, T.head));
+      TRY(P.upload(&L.sb_node, T.node));
+      TRY(P.upload(&L.sb_iptr, T.iptr));
+      TRY(P.upload(&L.sb_loc, T.loc));
+      TRY(P.upload(&L.sb_inc, T.inc));
+      TRY(up_real(&L.sb_w, T.w));
+      TRY(al_real(&L.rec1, (size_t)(8 * (size_t)n) * NB));
+    }
+  }
   L.gstride = need_grad ? GREC * (long long)n : 0;
   TRY(al_real(&L.grec, need_grad ? GREC * (size_t)n * NB : 1));
   TRY(al_real(&L.tau, (size_t)(VREC * (size_t)n) * NB));  // tau and dnu share the record
@@ -1089,17 +1241,39 @@ int op_grad(flite_ctx *c, Level &L) {
   });
 }
 
+bool jst_active(const flite_ctx *c, const Level &L) {
+  const flite_params &hp = c->hp;
+  if (hp.flux_type == 4 && L.gnum == 1) return false;  // DEF:11506
+  return !(hp.fourth_order_dissipation_factor == 0.0 && hp.second_order_dissipation_factor == 0.0);  // DEF:11508
+}
+
+bool viscous(const flite_ctx *c) { return c->hp.reynolds_number > 0.0; }
+
+// Stages that evaluate their own fluxes (k_stage_blk): levels without
+// second-order sides and without a moving mesh's side terms.
+bool stage_blocks(const flite_ctx *c, const Level &L) { return L.nsb > 0 && !c->flux_apart; }
+
+// ... whose first stage also forms the time steps: nothing else of the step
+// reads them before
+bool stage_steps(const flite_ctx *c, const Level &L) {
+  return stage_blocks(c, L) && !viscous(c) && !jst_active(c, L);
+}
+
 int op_flux(flite_ctx *c, Level &L) {
   DevParams P = c->P;
   bool o2 = L.has_coords && c->hp.hllc_flux_order > 1;
   if (L.gnum <= (int)c->evals.size()) c->evals[L.gnum - 1] += 1;
+  if (stage_blocks(c, L)) {
+    L.flux_src = FLUX_BLOCK;
+    return 0;
+  }
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
     if (L.ne > 0 && P.ftype != 4) {
       // central / LLF / Roe: one flux per side into fbuf
       Timed tm(c, "flux", L.gnum);
       dim3 g(nblk(L.ne) * L.nbatch), b(NTHR);
-      L.flux_partials = false;
+      L.flux_src = FLUX_SIDES;
 #define LAUNCH_SIMPLE(FT)                                                                        \
   if (P.sa) hipLaunchKernelGGL((k_flux_simple<R, FT, true>), g, b, 0, c->stream, V, P);          \
   else hipLaunchKernelGGL((k_flux_simple<R, FT, false>), g, b, 0, c->stream, V, P);
@@ -1115,8 +1289,8 @@ int op_flux(flite_ctx *c, Level &L) {
       Timed tm(c, "flux", L.gnum);
       dim3 g(nblk(L.ne) * L.nbatch), b(NTHR);
       bool n4 = P.nsig == 4;  // LED exponent: 4 inviscid, 2 viscous
-      L.flux_partials = !c->flux_per_side;
-      if (L.flux_partials) {
+      L.flux_src = c->flux_per_side ? FLUX_SIDES : FLUX_PARTIALS;
+      if (L.flux_src == FLUX_PARTIALS) {
         auto blk = [&](auto shape) {
           constexpr int SH = decltype(shape)::value;
           dim3 gb((unsigned)L.sb[SH].nfb * L.nbatch), bb(FB_SHAPE_THR[SH]);
@@ -1154,29 +1328,59 @@ int op_flux(flite_ctx *c, Level &L) {
   });
 }
 
-int op_stage(flite_ctx *c, Level &L, int mode, const StageArgs &S0) {
+// step: the stage also forms the level's time steps (stage_steps)
+int op_stage(flite_ctx *c, Level &L, int mode, const StageArgs &S0, bool step = false) {
   DevParams P = c->P;
   StageArgs S = S0;
-  S.partials = L.flux_partials;
+  S.partials = L.flux_src == FLUX_PARTIALS;
   Timed tm(c, "stage", L.gnum);
-  return with_level(L, [&](auto V) {
-    using R = std::remove_pointer_t<decltype(V.u)>;
-    return with_lanes(L.lanes, [&](auto sc) {
-      constexpr int SUB = decltype(sc)::value;
-      dim3 g(nblk((long long)L.n * SUB) * L.nbatch), t(NTHR);
-#define LAUNCH_STAGE(M)                                                                       \
-  if (P.sa) hipLaunchKernelGGL((k_stage<R, M, true, SUB>), g, t, 0, c->stream, V, P, S);      \
-  else hipLaunchKernelGGL((k_stage<R, M, false, SUB>), g, t, 0, c->stream, V, P, S);
-      switch (mode) {
-        case MODE_RHS: LAUNCH_STAGE(MODE_RHS); break;
-        case MODE_STAGE: LAUNCH_STAGE(MODE_STAGE); break;
-        case MODE_COARSE: LAUNCH_STAGE(MODE_COARSE); break;
-        default: LAUNCH_STAGE(MODE_FINE); break;
-      }
-#undef LAUNCH_STAGE
-      return check_launch();
+  // f(mode, with SA) as constants
+  auto dispatch = [&](auto f) {
+    auto by_sa = [&](auto mc) {
+      if (P.sa) f(mc, std::true_type{});
+      else f(mc, std::false_type{});
+    };
+    switch (mode) {
+      case MODE_RHS: by_sa(std::integral_constant<int, MODE_RHS>{}); break;
+      case MODE_STAGE: by_sa(std::integral_constant<int, MODE_STAGE>{}); break;
+      case MODE_COARSE: by_sa(std::integral_constant<int, MODE_COARSE>{}); break;
+      default: by_sa(std::integral_constant<int, MODE_FINE>{}); break;
+    }
+    return check_launch();
+  };
+  if (L.flux_src != FLUX_BLOCK)
+    return with_level(L, [&](auto V) {
+      using R = std::remove_pointer_t<decltype(V.u)>;
+      return with_lanes(L.lanes, [&](auto sc) {
+        constexpr int SUB = decltype(sc)::value;
+        dim3 g(nblk((long long)L.n * SUB) * L.nbatch), t(NTHR);
+        return dispatch([&](auto mc, auto sac) {
+          hipLaunchKernelGGL((k_stage<R, decltype(mc)::value, decltype(sac)::value, SUB>), g, t, 0, c->stream, V, P, S);
+        });
+      });
     });
-  });
+  TRY(with_level(L, [&](auto V) {
+    using R = std::remove_pointer_t<decltype(V.u)>;
+    dim3 g((unsigned)L.nsb * L.nbatch), t(NTHR);
+    return dispatch([&](auto mc, auto sac) {
+      constexpr int M = decltype(mc)::value;
+      constexpr bool SA = decltype(sac)::value;
+      auto go = [&](auto hc) {
+        constexpr bool H = decltype(hc)::value;
+        if constexpr (!SA && (M == MODE_STAGE || M == MODE_COARSE)) {
+          if (step) {
+            hipLaunchKernelGGL((k_stage_blk<R, M, SA, H, true>), g, t, 0, c->stream, V, P, S);
+            return;
+          }
+        }
+        hipLaunchKernelGGL((k_stage_blk<R, M, SA, H, false>), g, t, 0, c->stream, V, P, S);
+      };
+      if (P.ftype == 4) go(std::true_type{});
+      else go(std::false_type{});
+    });
+  }));
+  if (mode == MODE_STAGE && S.next_record) std::swap(L.rec0, L.rec1);
+  return 0;
 }
 
 int op_timesteps(flite_ctx *c, Level &L) {
@@ -1205,14 +1409,6 @@ int op_zero_diss(flite_ctx *c, Level &L) {
 // adds its node totals: -viscous + JST is the reference's JST - viscous, each
 // a single addition.  Without a viscous term the JST totals overwrite the
 // array; with neither, the step's start zeroes it (zero_dissipation).
-bool jst_active(const flite_ctx *c, const Level &L) {
-  const flite_params &hp = c->hp;
-  if (hp.flux_type == 4 && L.gnum == 1) return false;  // DEF:11506
-  return !(hp.fourth_order_dissipation_factor == 0.0 && hp.second_order_dissipation_factor == 0.0);  // DEF:11508
-}
-
-bool viscous(const flite_ctx *c) { return c->hp.reynolds_number > 0.0; }
-
 // no kernel of the step writes the level's dissipation: its start must
 bool zero_dissipation(const flite_ctx *c, const Level &L) {
   return !viscous(c) && !(jst_active(c, L) && L.ne > 0);
@@ -1361,7 +1557,7 @@ int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss, bool begun, bool
     if (viscous(c)) {
       // makeTimeSteps, makeViscosityTerm, makeTurbulentTimeSteps, makeSADiffusion
       TRY(op_step_terms(c, L, true, true));
-    } else {
+    } else if (!stage_steps(c, L)) {
       TRY(op_timesteps(c, L));
     }
     TRY(op_jst(c, L, viscous(c)));
@@ -1379,7 +1575,7 @@ int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss, bool begun, bool
     S.fas = L.gnum > 1;
     S.has_src = L.gnum > 1;
     S.next_record = k < hp.rk_stages || record_last;
-    TRY(op_stage(c, L, MODE_STAGE, S));
+    TRY(op_stage(c, L, MODE_STAGE, S, k == 1 && calc_diss && stage_steps(c, L)));
   }
   return 0;
 }
@@ -1411,7 +1607,7 @@ int do_restrict(flite_ctx *c, int fine_level, bool recorded = false, bool begin 
   }));
   if (visc) {
     TRY(op_step_terms(c, K, true, true));
-  } else {
+  } else if (!stage_steps(c, K)) {
     TRY(op_timesteps(c, K));
   }
   TRY(op_jst(c, K, visc));
@@ -1423,7 +1619,7 @@ int do_restrict(flite_ctx *c, int fine_level, bool recorded = false, bool begin 
   S.calc_turb = 1;
   S.fas = 0;
   S.has_src = 1;
-  TRY(op_stage(c, K, MODE_COARSE, S));
+  TRY(op_stage(c, K, MODE_COARSE, S, stage_steps(c, K)));
   // fine part (DEF:12236-12361)
   if (!recorded) TRY(op_prep(c, F, true, 0, zero_dissipation(c, F)));
   if (visc) TRY(op_step_terms(c, F, false, false));
@@ -1680,6 +1876,7 @@ int flite_ctx_create(const flite_params *p, int n_levels, int n_batch, flite_ctx
     std::string v(e);
     if (v != "side" && v != "block") return fail(FLITE_E_ARG, "FLITE_FLUX_KERNEL must be side or block");
     c->flux_per_side = v == "side";
+    c->flux_apart = true;
   }
   if (const char *e = std::getenv("FLITE_CYCLE_GRAPH")) {
     std::string v(e);
@@ -2329,7 +2526,7 @@ int tangent_core(flite_ctx *c) {
     if (P.sa) hipLaunchKernelGGL(k_flux_tangent<true>, dim3(nblk(L.ne)), dim3(NTHR), 0, c->stream, V, P, V.src);
     else hipLaunchKernelGGL(k_flux_tangent<false>, dim3(nblk(L.ne)), dim3(NTHR), 0, c->stream, V, P, V.src);
   }
-  L.flux_partials = false;  // the tangent fluxes are per-side records
+  L.flux_src = FLUX_SIDES;  // the tangent fluxes are per-side records
   if (L.nbs > 0) hipLaunchKernelGGL(k_bflux_tangent, dim3(nblk(L.nbs)), dim3(NTHR), 0, c->stream, V, P, V.src);
   TRY(check_launch());
   StageArgs S{};
@@ -2883,7 +3080,7 @@ int flite_autotune(flite_ctx *c, int repeats, int *lanes_out) {
     L.lanes = best;
     lanes_out[l] = best;
     // the flux kernel's side-block shape (levels that use side blocks)
-    if (rc == 0 && L.ne > 0 && !c->flux_per_side && c->P.ftype == 4) {
+    if (rc == 0 && L.ne > 0 && !c->flux_per_side && c->P.ftype == 4 && !stage_blocks(c, L)) {
       int bs = L.fb_shape;
       float bms = 1e30f;
       rc = op_prep(c, L, true);
