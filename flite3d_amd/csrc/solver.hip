@@ -824,10 +824,15 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
   L.gnum = level;
   L.fp32 = coarse_fp32 && level > 1;
   L.n = S.n;
-  // enough lanes to give the chip >= ~1M threads on mid-size levels, and
-  // short per-lane gather chains on the small coarse ones
+  // lanes per node of the gather walks: as few as still keep the chip busy,
+  // since every doubling adds a butterfly step over all of a walk's sums.
+  // Measured, us for 1 / 4 / 16 lanes: gradient at 36k nodes 24 / 17 / 31, at
+  // 275k 71 / 82 / 163, at 2.1M 434 / 596 / 1214; the SA pass A at 1.3k 50 /
+  // 17 / 11, 30k 75 / 28 / 31, 255k 100 / 109 / 179.  The count is the
+  // level's own, not times the batch: a condition of a batch keeps the order
+  // of its sums, and with it the bits, of its single run.
   L.nbatch = c->nbatch;
-  L.lanes = c->lanes_override ? c->lanes_override : (S.n >= (1 << 20) ? 1 : S.n >= (1 << 16) ? 4 : 16);
+  L.lanes = c->lanes_override ? c->lanes_override : (S.n >= (1 << 17) ? 1 : S.n >= (1 << 14) ? 4 : 16);
   L.fb_shape = c->shape_override >= 0 ? c->shape_override : 0;
   L.ne = S.ne;
   L.nbs = S.nbs;
