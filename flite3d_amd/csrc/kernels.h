@@ -4162,7 +4162,7 @@ __global__ void k_prolong(LevelDev<RF> F, LevelDev<RC> K, DevParams P, Transfer 
 // DEF:14710-14806), all on the device: up to MON_BLOCKS blocks stride over
 // the nodes and the wall nodes, each thread accumulating its share in stride
 // order; wavefront butterflies and one LDS step reduce the block to a record
-// of MON_REC doubles; the last block reduces the records.  The order of
+// of MON_REC doubles; k_monitor_final reduces the records.  The order of
 // every sum is fixed, so the results are reproducible bit for bit.  Record:
 // sum (u - uprev)^2 [7], max |u - uprev| [7], host index of that maximum [7]
 // (smallest index on ties), force integrals [8] (lift, drag, latF,
@@ -4240,26 +4240,21 @@ __device__ __forceinline__ void wave_maxloc(double &m, int &k) {
   for (int s = 1; s < 64; s <<= 1) maxloc(m, k, __shfl_xor(m, s, 64), __shfl_xor(k, s, 64));
 }
 
-// One launch: every block reduces its share to a record (block b's quantity
-// q at part[MON_BLOCKS q + b]), and the block that finishes last reduces the
-// records, each quantity by one wavefront, to `out` (MON_REC doubles in host
-// memory the device can write).  `ticket` counts the finished blocks and
-// wraps back to zero with the last one.  The records pass between the XCDs'
-// L2 caches through agent-scope stores and loads on both sides of the
-// ticket.  A launch this small is latency alone, so the quantities share one
-// barrier.  A barrier pair for each (16 us), a second launch of one block for
-// the records (28 us) and the copy of the result made the call 66 us on 729
-// nodes; it is 33 us now, most of it the launch and the wait.
+// Every block reduces its share to a record (block b's quantity q at
+// part[MON_BLOCKS q + b]); k_monitor_final reduces the records, each quantity
+// by one wavefront, to MON_REC doubles in host memory the device can write.
+// Launches this small are latency alone, so the quantities share one barrier.
+// (One launch whose last block reduces the records needs a device-wide fence
+// in every block, which writes back its XCD's L2: it took 18 us on 9k nodes
+// and 57 on 275k, where the two launches take 16 and 27.)
 template <typename R>
 __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParams P, ForceFrame F, int nres,
                                                          const int *host_index, const int *wall_nodes, int nw,
-                                                         const R *warea, double *part, unsigned *ticket, double *out,
-                                                         int bsel) {
+                                                         const R *warea, double *part, int bsel) {
   L.to_batch(bsel);
   P.to_batch(bsel);
   constexpr int NW = NTHR / 64;
   __shared__ double lds[MON_REC][NW];
-  __shared__ bool last;
   const int n = L.n, stride = gridDim.x * NTHR;
   double sum[7], mx[7];
   int mi[7];
@@ -4315,31 +4310,46 @@ __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParam
     } else {
       for (int w = 0; w < NW; ++w) v += lds[q][w];
     }
-    __hip_atomic_store(part + (size_t)MON_BLOCKS * q + blockIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    part[(size_t)MON_BLOCKS * q + blockIdx.x] = v;
   }
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) last = atomicInc(ticket, gridDim.x - 1) == gridDim.x - 1;
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
-  const int nrec = gridDim.x;
-  auto rec = [&](int r, int b) {
-    return __hip_atomic_load(part + (size_t)MON_BLOCKS * r + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  for (int r = wave; r < MON_REC; r += NW) {
-    if (r >= 14 && r < 21) continue;
-    double v = 0;
-    int k = 0x7fffffff;
-    for (int b = lane; b < nrec; b += 64) {
-      if (r >= 7 && r < 14) maxloc(v, k, rec(r, b), (int)rec(r + 7, b));
-      else v += rec(r, b);
+}
+
+// wavefront w of one block takes quantities w, w + FIN_NW, ..; all of a
+// stride's records are requested before the first is used
+constexpr int FIN_THR = 512, FIN_NW = FIN_THR / 64;
+__global__ __launch_bounds__(FIN_THR) void k_monitor_final(const double *part, int nrec, double *out) {
+  constexpr int PER = (MON_REC + FIN_NW - 1) / FIN_NW;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double v[PER];
+  int kx[PER];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    v[p] = 0;
+    kx[p] = 0x7fffffff;
+  }
+  for (int b = lane; b < nrec; b += 64) {
+    double x[PER], y[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int r = wave + p * FIN_NW;
+      x[p] = r < MON_REC ? part[(size_t)MON_BLOCKS * r + b] : 0.0;
+      y[p] = r >= 7 && r < 14 ? part[(size_t)MON_BLOCKS * (r + 7) + b] : 0.0;
     }
-    if (r >= 7 && r < 14) wave_maxloc(v, k);
-    else v = wave_sum(v);
-    if (lane == 0) {
-      out[r] = v;
-      if (r >= 7 && r < 14) out[r + 7] = double(k);
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int r = wave + p * FIN_NW;
+      if (r >= 7 && r < 14) maxloc(v[p], kx[p], x[p], (int)y[p]);
+      else v[p] += x[p];
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int r = wave + p * FIN_NW;
+    if (r >= 7 && r < 14) wave_maxloc(v[p], kx[p]);
+    else v[p] = wave_sum(v[p]);
+    if (lane == 0 && r < MON_REC && !(r >= 14 && r < 21)) {
+      out[r] = v[p];
+      if (r >= 7 && r < 14) out[r + 7] = double(kx[p]);
     }
   }
 }

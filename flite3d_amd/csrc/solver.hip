@@ -193,9 +193,8 @@ struct Level {
   // transfer from the next finer level (coarse levels)
   int *f2c = nullptr, *cptr = nullptr, *clist = nullptr;
   double *rw = nullptr;
-  // monitor records: MON_BLOCKS block records (MON_REC doubles each), and the count of finished blocks
+  // monitor records: MON_BLOCKS block records, MON_REC doubles each
   double *m_part = nullptr;
-  unsigned *m_ticket = nullptr;
   double *abuf = nullptr;  // adjoint side shares, 10 per side (allocated on first use)
   double *vmesh = nullptr;  // viscous mesh-adjoint shares, 3 per side and boundary side (first use)
   // second-order linearisation (allocated on first use): per-side adjoint
@@ -1101,7 +1100,6 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
   TRY(al_real(&L.uold, c->hp.flow_type != 0 ? (size_t)(6 * (size_t)n) * NB : 1));
   TRY(al_real(&L.uold2, c->hp.flow_type != 0 ? (size_t)(6 * (size_t)n) * NB : 1));
   TRY(P.alloc(&L.m_part, (size_t)MON_REC * MON_BLOCKS));
-  TRY(P.alloc(&L.m_ticket, 1));
   // transfer operators from the finer level
   if (level > 1) {
     Level &F = *c->lev[level - 2];
@@ -2237,8 +2235,10 @@ int monitor_into(flite_ctx *c, double *part, double res[7], double maxres[7], in
   int nw = (int)L.wall_dev.size();
   TRY(with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
-    hipLaunchKernelGGL(k_monitor_reduce<R>, dim3(std::min(MON_BLOCKS, nblk(L.n))), dim3(NTHR), 0, c->stream, V, P, F,
-                       nres, L.host_index, L.wall_nodes, nw, (const R *)L.warea, part, L.m_ticket, c->mon_host, bsel);
+    const int nrec = std::min(MON_BLOCKS, nblk(L.n));
+    hipLaunchKernelGGL(k_monitor_reduce<R>, dim3(nrec), dim3(NTHR), 0, c->stream, V, P, F, nres, L.host_index,
+                       L.wall_nodes, nw, (const R *)L.warea, part, bsel);
+    hipLaunchKernelGGL(k_monitor_final, dim3(1), dim3(FIN_THR), 0, c->stream, (const double *)part, nrec, c->mon_host);
     return check_launch();
   }));
   TRY(sync(c));
