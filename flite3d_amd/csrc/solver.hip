@@ -256,6 +256,10 @@ struct flite_ctx {
   std::vector<flite_params> hp_b;  // per condition (batched contexts)
   double *cond_dev = nullptr;      // per-condition Mach and inflow state on the device
   int sel = 0;                     // condition that field/state/monitor calls act on
+  // columns of a field in host numbering on their way in or out (grown to the
+  // largest field asked for, released with the context)
+  double *xfer = nullptr;
+  size_t xfer_cap = 0;
   double *mon_host = nullptr;      // the monitor's MON_REC results, in pinned host memory the kernel writes
   std::vector<std::unique_ptr<Level>> lev;
   // coarse levels of the other precision (flite_set_coarse_precision),
@@ -1777,6 +1781,31 @@ void *field_ptr(Level &L, int field, int *ncomp, size_t *stride_nodes) {
   }
 }
 
+int need_xfer(flite_ctx *c, size_t count) {
+  if (c->xfer_cap >= count) return 0;
+  if (c->xfer) (void)hipFree(c->xfer);
+  c->xfer = nullptr;
+  c->xfer_cap = 0;
+  HIPTRY(hipMalloc((void **)&c->xfer, count * sizeof(double)));
+  c->xfer_cap = count;
+  return 0;
+}
+
+// nc columns of n doubles, the host's at leading dimension ld
+int copy_columns(flite_ctx *c, double *dst, const double *src, int n, int ld, int nc, bool to_host) {
+  const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
+  if (ld == n) {
+    HIPTRY(hipMemcpyAsync(dst, src, (size_t)nc * n * sizeof(double), kind, c->stream));
+    return 0;
+  }
+  for (int k = 0; k < nc; ++k) {
+    double *d = dst + (size_t)k * (to_host ? ld : n);
+    const double *s = src + (size_t)k * (to_host ? n : ld);
+    HIPTRY(hipMemcpyAsync(d, s, (size_t)n * sizeof(double), kind, c->stream));
+  }
+  return 0;
+}
+
 }  // namespace
 
 // ===========================================================================
@@ -1923,6 +1952,7 @@ void flite_ctx_destroy(flite_ctx *c) {
   c->lev_alt.clear();
   if (c->cond_dev) (void)hipFree(c->cond_dev);
   if (c->mon_host) (void)hipHostFree(c->mon_host);
+  if (c->xfer) (void)hipFree(c->xfer);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -1962,51 +1992,33 @@ int flite_field_get(flite_ctx *c, int level, int field, double *out, int ld) {
   TRY(check_level(c, level));
   Level &L = *c->lev[level - 1];
   if (!out || ld < L.n) return fail(FLITE_E_ARG, "bad output buffer");
-  TRY(sync(c));
-  const size_t es = L.fp32 ? 4 : 8;
-  auto to_host = [&](const void *dptr, size_t count, std::vector<double> &h) -> int {
-    h.resize(count);
-    if (L.fp32) {
-      std::vector<float> t(count);
-      HIPTRY(hipMemcpy(t.data(), dptr, count * es, hipMemcpyDeviceToHost));
-      for (size_t k = 0; k < count; ++k) h[k] = t[k];
-    } else {
-      HIPTRY(hipMemcpy(h.data(), dptr, count * es, hipMemcpyDeviceToHost));
-    }
-    return 0;
-  };
-  std::vector<double> h;
   const size_t sb = (size_t)c->sel;  // selected condition
+  const long long n = L.n;
+  // nc components, component k of device node d at p + base + sk k + si d
+  auto fetch = [&](const void *p, size_t base, long long sk, long long si, int nc, int inv) -> int {
+    TRY(need_xfer(c, (size_t)nc * L.n));
+    auto go = [&](auto zero) -> int {
+      using R = decltype(zero);
+      hipLaunchKernelGGL(k_field_out<R>, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, (const R *)p + base, sk, si,
+                         (const int *)L.host_index, L.n, nc, inv, c->xfer);
+      return check_launch();
+    };
+    TRY(L.fp32 ? go(0.0f) : go(0.0));
+    TRY(copy_columns(c, out, c->xfer, L.n, ld, nc, true));
+    return sync(c);
+  };
   if (field == FLITE_FIELD_GRADIENT) {
     if (!(L.has_coords && c->hp.hllc_flux_order > 1)) return fail(FLITE_E_STATE, "no gradient on this level");
-    TRY(to_host((char *)L.grec + sb * (size_t)L.gstride * es, GREC * (size_t)L.n, h));
-    for (int hh = 0; hh < L.n; ++hh) {
-      const double *g = &h[GREC * (size_t)L.h2d[hh]];
-      for (int k = 0; k < 15; ++k) out[(size_t)k * ld + hh] = g[k];
-      for (int k = 0; k < 5; ++k) {  // limits from their stored reciprocals
-        out[(size_t)(15 + k) * ld + hh] = g[15 + k] != 0.0 ? 1.0 / g[15 + k] : 0.0;
-        out[(size_t)(20 + k) * ld + hh] = g[20 + k] != 0.0 ? 1.0 / g[20 + k] : 0.0;
-      }
-    }
-    return 0;
+    return fetch(L.grec, sb * (size_t)L.gstride, 1, GREC, 25, 15);  // limits from their stored reciprocals
   }
-  if (field == FLITE_FIELD_WALL_STRESS) {
-    TRY(to_host((char *)L.ws + sb * 3 * (size_t)L.n * es, 3 * (size_t)L.n, h));
-    for (int hh = 0; hh < L.n; ++hh)
-      for (int k = 0; k < 3; ++k) out[(size_t)k * ld + hh] = h[3 * (size_t)L.h2d[hh] + k];
-    return 0;
-  }
+  if (field == FLITE_FIELD_WALL_STRESS) return fetch(L.ws, sb * 3 * (size_t)n, 1, 3, 3, 3);
   int nc;
   size_t stride;
   if ((field == FLITE_FIELD_UOLD || field == FLITE_FIELD_UOLD2) && c->hp.flow_type == 0)
     return fail(FLITE_E_STATE, "no solutions of earlier physical times in a steady run");
   void *p = field_ptr(L, field, &nc, &stride);
   if (!p) return fail(FLITE_E_ARG, "bad field");
-  p = (char *)p + sb * nc * stride * es;
-  TRY(to_host(p, nc * stride, h));
-  for (int k = 0; k < nc; ++k)
-    for (int hh = 0; hh < L.n; ++hh) out[(size_t)k * ld + hh] = h[(size_t)k * stride + L.h2d[hh]];
-  return 0;
+  return fetch(p, sb * nc * stride, (long long)stride, 1, nc, nc);
 }
 
 int flite_field_set(flite_ctx *c, int level, int field, const double *in, int ld) {
@@ -2020,17 +2032,16 @@ int flite_field_set(flite_ctx *c, int level, int field, const double *in, int ld
   void *p = field_ptr(L, field, &nc, &stride);
   if (!p) return fail(FLITE_E_ARG, "field cannot be set");
   p = (char *)p + (size_t)c->sel * nc * stride * (L.fp32 ? 4 : 8);
-  TRY(sync(c));
-  std::vector<double> h(nc * stride);
-  for (int k = 0; k < nc; ++k)
-    for (int hh = 0; hh < L.n; ++hh) h[(size_t)k * stride + L.h2d[hh]] = in[(size_t)k * ld + hh];
-  if (L.fp32) {
-    std::vector<float> t(h.begin(), h.end());
-    HIPTRY(hipMemcpy(p, t.data(), t.size() * 4, hipMemcpyHostToDevice));
-  } else {
-    HIPTRY(hipMemcpy(p, h.data(), h.size() * 8, hipMemcpyHostToDevice));
-  }
-  return 0;
+  TRY(need_xfer(c, (size_t)nc * L.n));
+  TRY(copy_columns(c, c->xfer, in, L.n, ld, nc, false));
+  auto go = [&](auto zero) -> int {
+    using R = decltype(zero);
+    hipLaunchKernelGGL(k_field_in<R>, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, (const double *)c->xfer,
+                       (const int *)L.host_index, L.n, nc, (R *)p);
+    return check_launch();
+  };
+  TRY(L.fp32 ? go(0.0f) : go(0.0));
+  return sync(c);
 }
 
 int flite_state_set(flite_ctx *c, int level, const double *u, int ld, int ncomp, int batch) {
