@@ -133,7 +133,7 @@ struct LevelDev {
   R *u, *uprev, *rhs, *diss, *src, *p, *dt, *dtt, *mu, *vort, *divg, *tdiff;
   R *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;  // tau, dnu: VREC-strided, one shared record
   R *rec1;  // the next state's gather records while a walking stage reads rec0 (null: no such stage)
-  R *jst;  // JST node record (8 per node): L(U) 5, pressure switch, side count, pad
+  R *jst;  // JST node record (8 per node): L(U) 5, pressure switch, side count, volume / time step
   R *uold, *uold2;  // solutions at the last two physical times (6 per node, unsteady only)
   // moving meshes (null on a fixed mesh): GCL weight per side and 2 per
   // boundary side, previous volumes and movement (3 per node AoS) on level 1
@@ -1312,140 +1312,6 @@ __global__ void k_flux_simple(LevelDev<R> L, DevParams P) {
   } else {
     o[5] = 0;
   }
-}
-
-// JST passes 1, 2 and the node step of makeArtificialDissipation2
-// (DEF:11531-11563, 11659-11672, 11746-11751), gathered per node over its
-// sides in their stored orientation (d = U_a - U_b as the side loop forms
-// it, taken with - at a and + at b):
-//   L_i = (1/conn_i) sum (U_j - U_i), energy on E + p;
-//   nu_i = 12 |sum (p_j - p_i) / sum (p_i + p_j)|;  conn_i = sides at i.
-template <typename R>
-__global__ void k_jst_sums(LevelDev<R> L, DevParams P) {
-  int bb_;
-  int i = btid(L.nb, bb_);
-  L.to_batch(bb_);
-  P.to_batch(bb_);
-  if (i >= L.n) return;
-  const size_t n = L.n;
-  R h[5] = {0, 0, 0, 0, 0}, h7 = 0, h8 = 0, conn = 0;
-  for_edges<1>(L, i, 0, [&](int e, int role) {
-    int a = L.ea[e], b = L.eb[e];
-    R d[5];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) d[c] = L.u[c * n + a] - L.u[c * n + b];
-    d[4] = d[4] + L.p[a] - L.p[b];
-    R dp = L.p[a] - L.p[b], sp = L.p[a] + L.p[b];
-    if (role == 0) {
-#pragma unroll
-      for (int c = 0; c < 5; ++c) h[c] = h[c] - d[c];
-      h7 = h7 - dp;
-    } else {
-#pragma unroll
-      for (int c = 0; c < 5; ++c) h[c] = h[c] + d[c];
-      h7 = h7 + dp;
-    }
-    h8 = h8 + sp;
-    conn += R(1);
-  });
-  R fact = R(1) / conn;
-  R *o = L.jst + 8 * (size_t)i;
-#pragma unroll
-  for (int c = 0; c < 5; ++c) o[c] = fact * h[c];
-  o[5] = R(12) * fabs(h7 / h8);
-  o[6] = conn;
-  o[7] = 0;
-}
-
-// JST pass 3 (DEF:11788-11939): per side (a, b) with dr4 = L_a - L_b and
-// dr2 = U_a - U_b,
-//   scalar: d0 = min(V_a/dt_a, V_b/dt_b) / (conn_a + conn_b),
-//           d2 = d0 k2 max(nu_a, nu_b), d4 = dim(d0 k4, d2);
-//   matrix: dr4, dr2 <- |w| |A| dr4, |w| |A| dr2 (Roe matrix along w in
-//           Turkel's form, Harten's fix), d2 = k2 max(nu), d4 = dim(k4, d2);
-// D_a += -dr4 d4 + dr2 d2 and D_b += dr4 d4 - dr2 d2, gathered per node into
-// the dissipation array (`add`: on top of the viscous term there; k4:
-// coarse-grid factor below grid 1).
-template <typename R, bool MATRIX>
-__global__ void k_jst_flux(LevelDev<R> L, DevParams P, int add) {
-  int bb_;
-  int i = btid(L.nb, bb_);
-  L.to_batch(bb_);
-  P.to_batch(bb_);
-  if (i >= L.n) return;
-  const size_t n = L.n;
-  const R k2 = R(P.k2), k4 = R(L.gnum == 1 ? P.k4 : P.k4c);
-  R acc[5] = {0, 0, 0, 0, 0};
-  for_edges<1>(L, i, 0, [&](int e, int role) {
-    int a = L.ea[e], b = L.eb[e];
-    const R *ja = L.jst + 8 * (size_t)a, *jb = L.jst + 8 * (size_t)b;
-    R d4v[5], d2v[5];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      d4v[c] = ja[c] - jb[c];
-      d2v[c] = L.u[c * n + a] - L.u[c * n + b];
-    }
-    R nu = ja[5] > jb[5] ? ja[5] : jb[5];
-    R d2, d4;
-    if constexpr (!MATRIX) {
-      R va = L.vol[a] / L.dt[a], vb = L.vol[b] / L.dt[b];
-      R d0 = (va < vb ? va : vb) / (ja[6] + jb[6]);
-      d2 = d0 * k2 * nu;
-      d4 = d0 * k4;
-    } else {
-      const R hcf = R(P.hcf), gam1 = R(P.gamma - 1.0);
-      const R eps1 = R(1) / (hcf > R(1.e-5) ? hcf : R(1.e-5));
-      R rnx = L.w[3 * e], rny = L.w[3 * e + 1], rnz = L.w[3 * e + 2];
-      R al = sqrt(rnx * rnx + rny * rny + rnz * rnz), vmo1 = R(1) / al;
-      rnx *= vmo1;
-      rny *= vmo1;
-      rnz *= vmo1;
-      R rhol = L.u[a], ra = R(1) / rhol;
-      R uxl = L.u[n + a] * ra, vyl = L.u[2 * n + a] * ra, wzl = L.u[3 * n + a] * ra;
-      R hl = (L.u[4 * n + a] + L.p[a]) * ra;
-      R rhor = L.u[b], rb = R(1) / rhor;
-      R uxr = L.u[n + b] * rb, vyr = L.u[2 * n + b] * rb, wzr = L.u[3 * n + b] * rb;
-      R hr = (L.u[4 * n + b] + L.p[b]) * rb;
-      R di = sqrt(rhor / rhol), d1 = R(1) / (di + R(1));
-      R ui = (di * uxr + uxl) * d1, vi = (di * vyr + vyl) * d1, wi = (di * wzr + wzl) * d1;
-      R hi = (di * hr + hl) * d1;
-      R ci2 = gam1 * (hi - R(0.5) * (ui * ui + vi * vi + wi * wi)), ci = sqrt(ci2);
-      R af = R(0.5) * (ui * ui + vi * vi + wi * wi), ucp = ui * rnx + vi * rny + wi * rnz;
-      R l1 = fabs(ucp + ci), l2 = fabs(ucp - ci), l3 = fabs(ucp);
-      if (l1 < hcf) l1 = R(0.5) * (l1 * l1 * eps1 + hcf);
-      if (l2 < hcf) l2 = R(0.5) * (l2 * l2 * eps1 + hcf);
-      if (l3 < hcf) l3 = R(0.5) * (l3 * l3 * eps1 + hcf);
-      R s1 = R(0.5) * (l1 + l2), s2 = R(0.5) * (l1 - l2);
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        R *q = k == 0 ? d4v : d2v;
-        R a1 = gam1 * (af * q[0] - ui * q[1] - vi * q[2] - wi * q[3] + q[4]);
-        R a2 = -ucp * q[0] + q[1] * rnx + q[2] * rny + q[3] * rnz;
-        R cc1 = ((s1 - l3) * a1 / ci2) + (s2 * a2 / ci);
-        R cc2 = (s2 * a1 / ci) + (s1 - l3) * a2;
-        R t0 = al * (l3 * q[0] + cc1), t1 = al * (l3 * q[1] + cc1 * ui + cc2 * rnx);
-        R t2 = al * (l3 * q[2] + cc1 * vi + cc2 * rny), t3 = al * (l3 * q[3] + cc1 * wi + cc2 * rnz);
-        R t4 = al * (l3 * q[4] + cc1 * hi + cc2 * ucp);
-        q[0] = t0;
-        q[1] = t1;
-        q[2] = t2;
-        q[3] = t3;
-        q[4] = t4;
-      }
-      d2 = k2 * nu;
-      d4 = k4;
-    }
-    d4 = d4 > d2 ? d4 - d2 : R(0);
-    if (role == 0) {
-#pragma unroll
-      for (int c = 0; c < 5; ++c) acc[c] = acc[c] - d4v[c] * d4 + d2v[c] * d2;
-    } else {
-#pragma unroll
-      for (int c = 0; c < 5; ++c) acc[c] = acc[c] + d4v[c] * d4 - d2v[c] * d2;
-    }
-  });
-#pragma unroll
-  for (int c = 0; c < 5; ++c) L.diss[c * n + i] = (add ? L.diss[c * n + i] : R(0)) + acc[c];
 }
 
 // makeSASourceTerm (DEF:9285-9370) of one node on any arithmetic type: the
@@ -3491,6 +3357,60 @@ struct SADiff2Part {
   __device__ void finish(const LevelDev<R> &L, const DevParams &, int i, const R *) { L.tdiff[i] = acc + d3; }
 };
 
+// JST passes 1, 2 and the node step of makeArtificialDissipation2
+// (DEF:11531-11563, 11659-11672, 11746-11751):
+//   L_i = (1/conn_i) sum (U_j - U_i), energy on E + p;
+//   nu_i = 12 |sum (p_j - p_i) / sum (p_i + p_j)|;  conn_i = sides at i,
+// with the node's volume over its time step (the one in L.dt, or that of
+// makeTimeSteps earlier in the same walk) for the scalar form's scale.
+template <typename R>
+struct JstSumsPart {
+  static constexpr bool AUX = false;
+  R U[5], p, h[5], h7, h8, conn;
+  static __device__ __forceinline__ void state(const R *q, R *u) {
+    u[0] = q[0];
+    u[1] = q[0] * q[1];
+    u[2] = q[0] * q[2];
+    u[3] = q[0] * q[3];
+    u[4] = q[4];
+  }
+  __device__ void init(const LevelDev<R> &, const DevParams &, int, const R *qi) {
+    state(qi, U);
+    p = qi[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) h[c] = 0;
+    h7 = h8 = conn = 0;
+  }
+  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *, const R *qj, R, R, R) {
+    R V[5];
+    state(qj, V);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) h[c] += V[c] - U[c];
+    h[4] += (V[4] - U[4]) + (qj[5] - p);
+    h7 += qj[5] - p;
+    h8 += p + qj[5];
+    conn += R(1);
+  }
+  __device__ void bside(const LevelDev<R> &, const DevParams &, const R *, int, int, int, const R *, R, R, R) {}
+  template <int SUB>
+  __device__ void reduce() {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) h[c] = lsum<SUB>(h[c]);
+    h7 = lsum<SUB>(h7);
+    h8 = lsum<SUB>(h8);
+    conn = lsum<SUB>(conn);
+  }
+  __device__ void finish(const LevelDev<R> &L, const DevParams &, int i, const R *) {
+    R fact = R(1) / conn;
+    R *o = L.jst + 8 * (size_t)i;
+#pragma unroll
+    for (int c = 0; c < 5; ++c) o[c] = fact * h[c];
+    o[5] = R(12) * fabs(h7 / h8);
+    o[6] = conn;
+    o[7] = L.vol[i] / L.dt[i];
+  }
+};
+
 // one walk of node i's interior and boundary sides feeding up to three parts
 template <typename R, int SUB, typename A, typename B, typename C, typename Walk>
 __device__ __forceinline__ void gather_body(LevelDev<R> &L, const DevParams &P, int i, int sub, Walk walk) {
@@ -3553,6 +3473,117 @@ __global__ __launch_bounds__(NTHR) void k_gather_blk(LevelDev<R> L, DevParams P)
   int i = L.gb_first[blk] + (int)threadIdx.x / GB_SUB, sub = (int)threadIdx.x % GB_SUB;
   if (i >= L.gb_first[blk + 1]) return;
   gather_body<R, GB_SUB, A, B, C>(L, P, i, sub, [&](auto f) { walk_staged<GB_SUB, S>(L, sn, i, sub, f); });
+}
+
+// JST pass 3 (DEF:11788-11939): per side (a, b) with dr4 = L_a - L_b and
+// dr2 = U_a - U_b,
+//   scalar: d0 = min(V_a/dt_a, V_b/dt_b) / (conn_a + conn_b),
+//           d2 = d0 k2 max(nu_a, nu_b), d4 = dim(d0 k4, d2);
+//   matrix: dr4, dr2 <- |w| |A| dr4, |w| |A| dr2 (Roe matrix along w in
+//           Turkel's form, Harten's fix), d2 = k2 max(nu), d4 = dim(k4, d2).
+// D_a += -dr4 d4 + dr2 d2 and D_b += dr4 d4 - dr2 d2: at either end the
+// differences taken from the node itself enter with the same signs.  Walked
+// per node into the dissipation array (`add`: on top of the viscous term
+// there; k4: coarse-grid factor below grid 1); the Roe averages take the
+// side's stored orientation, so both ends form the same matrix.
+// Both passes read the 64-byte records of the neighbours with the level's
+// lanes per node; with one lane per node and the conserved state's seven
+// scattered words per neighbour they took 19 + 27 us on 9k nodes and 23 + 40
+// us on 160, now 8.5 + 6.6 and 6.6 + 5.8 (the first with the time steps).
+template <typename R, bool MATRIX, int SUB>
+__global__ void k_jst_flux(LevelDev<R> L, DevParams P, int add) {
+  int i, sub;
+  int bb_;
+  node_lanes<SUB>(L.nb, bb_, i, sub);
+  L.to_batch(bb_);
+  P.to_batch(bb_);
+  if (i >= L.n) return;
+  const size_t n = L.n;
+  const R k2 = R(P.k2), k4 = R(L.gnum == 1 ? P.k4 : P.k4c);
+  R qi[8], ji[8], Ui[5], acc[5] = {0, 0, 0, 0, 0};
+  ldrec<8>(L.rec0 + 8 * (size_t)i, qi);
+  ldrec<8>(L.jst + 8 * (size_t)i, ji);
+  JstSumsPart<R>::state(qi, Ui);
+  const int s = i / SLICE, lane = i % SLICE;
+  const int base = L.ell_ptr[s], K = L.ell_k[s];
+  const long long ns = L.nslot;
+  for (int k = sub; k < K; k += SUB) {
+    const int slot = base + k * SLICE + lane;
+    const int e = L.ell_e[slot];
+    if (e < 0) continue;
+    const size_t j = L.ell_nbr[slot];
+    R qj[8], jj[8], Uj[5];
+    ldrec<8>(L.rec0 + 8 * j, qj);
+    ldrec<8>(L.jst + 8 * j, jj);
+    JstSumsPart<R>::state(qj, Uj);
+    R d4v[5], d2v[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      d4v[c] = ji[c] - jj[c];
+      d2v[c] = Ui[c] - Uj[c];
+    }
+    R nu = ji[5] > jj[5] ? ji[5] : jj[5];
+    R d2, d4;
+    if constexpr (!MATRIX) {
+      R d0 = (ji[7] < jj[7] ? ji[7] : jj[7]) / (ji[6] + jj[6]);
+      d2 = d0 * k2 * nu;
+      d4 = d0 * k4;
+    } else {
+      const R hcf = R(P.hcf), gam1 = R(P.gamma - 1.0);
+      const R eps1 = R(1) / (hcf > R(1.e-5) ? hcf : R(1.e-5));
+      R rnx = L.ellw[slot], rny = L.ellw[ns + slot], rnz = L.ellw[2 * ns + slot];
+      R al = sqrt(rnx * rnx + rny * rny + rnz * rnz), vmo1 = R(1) / al;
+      rnx *= vmo1;
+      rny *= vmo1;
+      rnz *= vmo1;
+      const bool second = e & 1;
+      R A[6], B[6];  // first and second end: rho, u, v, w, rhoE, p
+#pragma unroll
+      for (int c = 0; c < 6; ++c) {
+        A[c] = second ? qj[c] : qi[c];
+        B[c] = second ? qi[c] : qj[c];
+      }
+      R hl = (A[4] + A[5]) * (R(1) / A[0]), hr = (B[4] + B[5]) * (R(1) / B[0]);
+      R di = sqrt(B[0] / A[0]), d1 = R(1) / (di + R(1));
+      R ui = (di * B[1] + A[1]) * d1, vi = (di * B[2] + A[2]) * d1, wi = (di * B[3] + A[3]) * d1;
+      R hi = (di * hr + hl) * d1;
+      R ci2 = gam1 * (hi - R(0.5) * (ui * ui + vi * vi + wi * wi)), ci = sqrt(ci2);
+      R af = R(0.5) * (ui * ui + vi * vi + wi * wi), ucp = ui * rnx + vi * rny + wi * rnz;
+      R l1 = fabs(ucp + ci), l2 = fabs(ucp - ci), l3 = fabs(ucp);
+      if (l1 < hcf) l1 = R(0.5) * (l1 * l1 * eps1 + hcf);
+      if (l2 < hcf) l2 = R(0.5) * (l2 * l2 * eps1 + hcf);
+      if (l3 < hcf) l3 = R(0.5) * (l3 * l3 * eps1 + hcf);
+      R s1 = R(0.5) * (l1 + l2), s2 = R(0.5) * (l1 - l2);
+#pragma unroll
+      for (int k_ = 0; k_ < 2; ++k_) {
+        R *q = k_ == 0 ? d4v : d2v;
+        R a1 = gam1 * (af * q[0] - ui * q[1] - vi * q[2] - wi * q[3] + q[4]);
+        R a2 = -ucp * q[0] + q[1] * rnx + q[2] * rny + q[3] * rnz;
+        R cc1 = ((s1 - l3) * a1 / ci2) + (s2 * a2 / ci);
+        R cc2 = (s2 * a1 / ci) + (s1 - l3) * a2;
+        R t0 = al * (l3 * q[0] + cc1), t1 = al * (l3 * q[1] + cc1 * ui + cc2 * rnx);
+        R t2 = al * (l3 * q[2] + cc1 * vi + cc2 * rny), t3 = al * (l3 * q[3] + cc1 * wi + cc2 * rnz);
+        R t4 = al * (l3 * q[4] + cc1 * hi + cc2 * ucp);
+        q[0] = t0;
+        q[1] = t1;
+        q[2] = t2;
+        q[3] = t3;
+        q[4] = t4;
+      }
+      d2 = k2 * nu;
+      d4 = k4;
+    }
+    d4 = d4 > d2 ? d4 - d2 : R(0);
+#pragma unroll
+    for (int c = 0; c < 5; ++c) acc[c] = acc[c] - d4v[c] * d4 + d2v[c] * d2;
+  }
+  if (SUB > 1) {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) acc[c] = lsum<SUB>(acc[c]);
+    if (sub) return;
+  }
+#pragma unroll
+  for (int c = 0; c < 5; ++c) L.diss[c * n + i] = (add ? L.diss[c * n + i] : R(0)) + acc[c];
 }
 
 // new laminar viscosity into the gather records after a fused pass

@@ -160,7 +160,7 @@ struct Level {
   void *u, *uprev, *rhs, *diss, *src, *p, *dt, *dtt, *mu, *vort, *divg, *tdiff;
   void *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;
   void *rec1 = nullptr;  // second record buffer of the one-launch stages (levels that use them)
-  void *jst = nullptr;  // JST node records (fluxType 1-3 only)
+  void *jst = nullptr;  // JST node records (levels with the JST dissipation)
   void *uold = nullptr, *uold2 = nullptr;  // unsteady only
   void *gcl = nullptr, *bgcl = nullptr, *volp = nullptr, *volp2 = nullptr, *cmv = nullptr;  // moving mesh only
   int *ea, *eb, *ba, *bb, *bind, *ell_ptr, *ell_k, *bs_ptr, *bs_list, *ncls, *host_index, *wall_nodes;
@@ -694,6 +694,12 @@ int build_side_blocks(Level &L, int shape, const std::vector<int> &ea, const std
   return 0;
 }
 
+bool jst_active(const flite_ctx *c, const Level &L) {
+  const flite_params &hp = c->hp;
+  if (hp.flux_type == 4 && L.gnum == 1) return false;  // DEF:11506
+  return !(hp.fourth_order_dissipation_factor == 0.0 && hp.second_order_dissipation_factor == 0.0);  // DEF:11508
+}
+
 // Node blocks of the one-launch stages (LevelDev::sb_*): consecutive nodes,
 // at most SB_NODES of them with at most SB_TASKS sides and (boundary side,
 // own end) pairs, SB_CAP staged nodes and SB_INC incidences.  No blocks if a
@@ -1100,7 +1106,7 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
   }
   TRY(al_real(&L.bbuf, (size_t)(10 * (size_t)nbs) * NB));
   TRY(al_real(&L.ws, (size_t)(3 * (size_t)n) * NB));
-  TRY(al_real(&L.jst, c->hp.flux_type != 4 ? (size_t)(8 * (size_t)n) * NB : 1));
+  TRY(al_real(&L.jst, jst_active(c, L) ? (size_t)(8 * (size_t)n) * NB : 1));
   TRY(al_real(&L.uold, c->hp.flow_type != 0 ? (size_t)(6 * (size_t)n) * NB : 1));
   TRY(al_real(&L.uold2, c->hp.flow_type != 0 ? (size_t)(6 * (size_t)n) * NB : 1));
   TRY(P.alloc(&L.m_part, (size_t)MON_REC * MON_BLOCKS));
@@ -1246,12 +1252,6 @@ int op_grad(flite_ctx *c, Level &L) {
       return check_launch();
     });
   });
-}
-
-bool jst_active(const flite_ctx *c, const Level &L) {
-  const flite_params &hp = c->hp;
-  if (hp.flux_type == 4 && L.gnum == 1) return false;  // DEF:11506
-  return !(hp.fourth_order_dissipation_factor == 0.0 && hp.second_order_dissipation_factor == 0.0);  // DEF:11508
 }
 
 bool viscous(const flite_ctx *c) { return c->hp.reynolds_number > 0.0; }
@@ -1421,17 +1421,22 @@ bool zero_dissipation(const flite_ctx *c, const Level &L) {
   return !viscous(c) && !(jst_active(c, L) && L.ne > 0);
 }
 
-int op_jst(flite_ctx *c, Level &L, bool add) {
-  if (!jst_active(c, L) || L.ne == 0) return 0;
+// steps: the first pass's walk forms the time steps too
+int op_jst(flite_ctx *c, Level &L, bool add, bool steps = false) {
+  if (!jst_active(c, L) || L.ne == 0) return steps ? op_timesteps(c, L) : 0;
   DevParams P = c->P;
   Timed tm(c, "dissipation", L.gnum);
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
-    dim3 g(nblk(L.n) * L.nbatch), b(NTHR);
-    hipLaunchKernelGGL(k_jst_sums<R>, g, b, 0, c->stream, V, P);
-    if (P.matdiss) hipLaunchKernelGGL((k_jst_flux<R, true>), g, b, 0, c->stream, V, P, int(add));
-    else hipLaunchKernelGGL((k_jst_flux<R, false>), g, b, 0, c->stream, V, P, int(add));
-    return check_launch();
+    if (steps) launch_gather<TimeStepPart<R>, JstSumsPart<R>, NoPart<R>>(c, L, V, P);
+    else launch_gather<JstSumsPart<R>, NoPart<R>, NoPart<R>>(c, L, V, P);
+    return with_lanes(L.lanes, [&](auto sc) {
+      constexpr int SUB = decltype(sc)::value;
+      dim3 g(nblk((long long)L.n * SUB) * L.nbatch), b(NTHR);
+      if (P.matdiss) hipLaunchKernelGGL((k_jst_flux<R, true, SUB>), g, b, 0, c->stream, V, P, int(add));
+      else hipLaunchKernelGGL((k_jst_flux<R, false, SUB>), g, b, 0, c->stream, V, P, int(add));
+      return check_launch();
+    });
   });
 }
 
@@ -1567,10 +1572,10 @@ int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss, bool begun, bool
     if (viscous(c)) {
       // makeTimeSteps, makeViscosityTerm, makeTurbulentTimeSteps, makeSADiffusion
       TRY(op_step_terms(c, L, true, true));
+      TRY(op_jst(c, L, true));
     } else if (!stage_steps(c, L)) {
-      TRY(op_timesteps(c, L));
+      TRY(op_jst(c, L, false, true));
     }
-    TRY(op_jst(c, L, viscous(c)));
   }
   for (int k = 1; k <= hp.rk_stages; ++k) {
     // stage k > 1 starts from the pressure and records the previous stage
@@ -1617,10 +1622,10 @@ int do_restrict(flite_ctx *c, int fine_level, bool recorded = false, bool begin 
   }));
   if (visc) {
     TRY(op_step_terms(c, K, true, true));
+    TRY(op_jst(c, K, true));
   } else if (!stage_steps(c, K)) {
-    TRY(op_timesteps(c, K));
+    TRY(op_jst(c, K, false, true));
   }
-  TRY(op_jst(c, K, visc));
   TRY(op_flux(c, K));
   StageArgs S;
   S.alpha = 1.0;
@@ -2187,7 +2192,7 @@ int flite_apply(flite_ctx *c, int level, int op) {
     case FLITE_OP_PRESSURE:
     case FLITE_OP_PRESSURE_ABS: TRY(op_prep(c, L, true)); break;
     case FLITE_OP_TIMESTEPS: TRY(op_prep(c, L, false)); TRY(op_timesteps(c, L)); break;
-    case FLITE_OP_DISSIPATION: TRY(op_zero_diss(c, L)); TRY(op_jst(c, L, false)); break;
+    case FLITE_OP_DISSIPATION: TRY(op_prep(c, L, false)); TRY(op_zero_diss(c, L)); TRY(op_jst(c, L, false)); break;
     case FLITE_OP_VISCOUS:
       if (!(c->hp.reynolds_number > 0.0)) return fail(FLITE_E_ARG, "viscous term needs ReynoldsNumber > 0");
       TRY(op_prep(c, L, false));
