@@ -76,6 +76,10 @@ enum : int { NC_NONE = 0, NC_WALL = 1, NC_SYM = 2, NC_FAR1 = 3, NC_FAR2 = 4, NC_
 constexpr int NC_MASK = 15;
 constexpr int NC_BFIRST = 16;
 
+// node blocks of the one-launch stages: nodes, tasks (one a thread), staged
+// nodes, incidences, lanes summing a node
+constexpr int SB_NODES = 32, SB_TASKS = NTHR, SB_CAP = 224, SB_INC = 512, SB_SUB = NTHR / SB_NODES;
+
 template <typename R>
 struct LevelDev {
   int n, ne, nbs, gnum;
@@ -113,20 +117,20 @@ struct LevelDev {
   int ngb;
   const int *gb_first, *gb_nptr, *gb_node;
   const unsigned short *ell_loc;
-  // node blocks of the one-launch stages (k_stage_blk): block k's header is
-  // sb_head[8 k ..] = {first node, nodes, first staged entry, staged nodes,
-  // first task, tasks, first incidence, incidences}.  Staged nodes: the
-  // block's own, then their other neighbours.  Task t: sb_loc[t] = both ends'
-  // staged positions (12 bits each) | kind << 24 (0: an interior side, k + 1:
-  // a boundary side of indicator k (k <= 0 as 0: they are walls alike), seen
-  // from its first listed end), sb_w[3]
-  // (SoA, stride sb_ntask) its weight; sb_inc[sb_iptr[i] ..] = node i's tasks
-  // within the block (task << 1 | 1 when the node is the side's second end)
+  // node blocks of the one-launch stages (k_stage_blk), block k's tables at
+  // fixed places: sb_node[SB_CAP k ..] = the staged nodes, the block's own
+  // (consecutive) first and then their other neighbours, -1 beyond;
+  // sb_loc[SB_TASKS k + t] = task t: both ends' staged positions (12 bits
+  // each) | kind << 24 (0: an interior side, k + 1: a boundary side of
+  // indicator k (k <= 0 as 0: they are walls alike), seen from its first
+  // listed end, 255: none), sb_w[3] (SoA, stride SB_TASKS nsb) its weight;
+  // sb_inc[SB_INC k + ..] = the tasks of the block's nodes (task << 1 | 1
+  // when the node is the side's second end), node m's from sb_iptr[(SB_NODES
+  // + 1) k + m] (the block's nodes end where the list does)
   int nsb;
-  long long sb_ntask;
-  const int *sb_head, *sb_node, *sb_iptr;
+  const int *sb_node;
   const unsigned *sb_loc;
-  const unsigned short *sb_inc;
+  const unsigned short *sb_inc, *sb_iptr;
   const R *sb_w;
   const R *vol, *xyz, *wd, *nrm;  // nrm: 3 per node AoS
   const int *ncls;
@@ -959,6 +963,128 @@ __global__ void k_flux(LevelDev<R> L, DevParams P) {
   side_flux<R, R, ORDER, SA, NSIG>(P, G1, G2, X1, X2, A, B, wx, wy, wz, L.fbuf + 6 * (size_t)e, wg);
 }
 
+// physical flux of one state through unit normal
+template <typename R>
+__device__ __forceinline__ void phys_flux(const R *q, R rnx, R rny, R rnz, R *f) {
+  R rho = q[0], u = q[1], v = q[2], w = q[3], pr = q[5], rh = q[4] + q[5];
+  R nv = u * rnx + v * rny + w * rnz;
+  f[0] = rho * nv;
+  f[1] = pr * rnx + rho * u * nv;
+  f[2] = pr * rny + rho * v * nv;
+  f[3] = pr * rnz + rho * w * nv;
+  f[4] = rh * nv;
+}
+
+// farfield Roe flux of one state against the inflow state (DEF:2258-2446)
+template <typename R>
+__device__ __forceinline__ void farfield_roe(const double *inf, const R *q, R gm1, R rnx, R rny, R rnz, R *f) {
+  R ro = R(inf[0]), uo = R(inf[1]), vo = R(inf[2]), wo = R(inf[3]), eo = R(inf[4]), po = R(inf[5]);
+  R rho = q[0], uu = q[1], vv = q[2], ww = q[3], eps = q[4], pr = q[5];
+  R rh = eps + pr, h = rh / rho;
+  R nv = uu * rnx + vv * rny + ww * rnz;
+  R fl1 = rho * nv, fl2 = pr * rnx + rho * uu * nv, fl3 = pr * rny + rho * vv * nv;
+  R fl4 = pr * rnz + rho * ww * nv, fl5 = rh * nv;
+  R epsr = eo * ro, hr = eo + po / ro;
+  R unr = uo * rnx + vo * rny + wo * rnz;
+  R fr1 = ro * unr, fr2 = rnx * po + ro * uo * unr, fr3 = rny * po + ro * vo * unr;
+  R fr4 = rnz * po + ro * wo * unr, fr5 = (epsr + po) * unr;
+  R di = sqrt(ro / rho), d1 = R(1) / (di + R(1));
+  R ui = (di * uo + uu) * d1, vi = (di * vo + vv) * d1, wi = (di * wo + ww) * d1, hi = (di * hr + h) * d1;
+  R af = R(0.5) * (ui * ui + vi * vi + wi * wi);
+  R ci2 = gm1 * (hi - af);
+  ci2 = ci2 > R(1e-5) ? ci2 : R(1e-5);
+  R ci = sqrt(ci2), ici = R(1) / ci;
+  R ucp = ui * rnx + vi * rny + wi * rnz;
+  R du1 = ro - rho, du2 = ro * uo - rho * uu, du3 = ro * vo - rho * vv;
+  R du4 = ro * wo - rho * ww, du5 = epsr - eps;
+  R rl1 = fabs(ucp + ci), rl2 = fabs(ucp - ci), rl3 = fabs(ucp);
+  R s1 = R(0.5) * (rl1 + rl2), s2 = R(0.5) * (rl1 - rl2);
+  R al1x = gm1 * (af * du1 - ui * du2 - vi * du3 - wi * du4 + du5);
+  R al2x = -ucp * du1 + du2 * rnx + du3 * rny + du4 * rnz;
+  R cc1 = ((s1 - rl3) * al1x / ci2) + (s2 * al2x * ici);
+  R cc2 = (s2 * al1x * ici) + (s1 - rl3) * al2x;
+  f[0] = R(0.5) * (fr1 + fl1) - R(0.5) * (rl3 * du1 + cc1);
+  f[1] = R(0.5) * (fr2 + fl2) - R(0.5) * (rl3 * du2 + cc1 * ui + cc2 * rnx);
+  f[2] = R(0.5) * (fr3 + fl3) - R(0.5) * (rl3 * du3 + cc1 * vi + cc2 * rny);
+  f[3] = R(0.5) * (fr4 + fl4) - R(0.5) * (rl3 * du4 + cc1 * wi + cc2 * rnz);
+  f[4] = R(0.5) * (fr5 + fl5) - R(0.5) * (rl3 * du5 + cc1 * hi + cc2 * ucp);
+}
+
+// the boundary flux of one end's state along the side's unit normal
+template <typename R>
+__device__ __forceinline__ void bside_state_flux(const DevParams &P, int ind, const R *q, R rnx, R rny, R rnz, R *f) {
+  if (ind <= 2 || ind == 9) {
+    phys_flux(q, rnx, rny, rnz, f);
+  } else {
+    double inf[6];
+    P.inflow_row(ind - 3, inf);
+    farfield_roe(inf, q, R(P.gamma - 1.0), rnx, rny, rnz, f);
+  }
+}
+
+// boundary-side loop of makeRHS (DEF:2116-2446): contributions to both ends,
+// bbuf[10*s + 5*end + c]
+template <typename R>
+__device__ __forceinline__ void bflux_side(const LevelDev<R> &L, const DevParams &P, int s) {
+  int ia = L.ba[s], ib = L.bb[s], ind = L.bind[s];
+  R wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
+  R *o = L.bbuf + 10 * (size_t)s;
+  // moving mesh: -(3 U_1 + U_2) g_1 / dt to the first end, -(U_1 + 3 U_2)
+  // g_2 / dt to the second (boundaryTerm 1), -4 U_k g_k / dt otherwise, on
+  // every boundary side (DEF:2124-2179)
+  R gc[10];
+#pragma unroll
+  for (int c = 0; c < 10; ++c) gc[c] = 0;
+  if (L.bgcl) {
+    const size_t n = L.n;
+    R g1 = L.bgcl[2 * (size_t)s] / R(P.dtp), g2 = L.bgcl[2 * (size_t)s + 1] / R(P.dtp);
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      R a = L.u[c * n + ia], b = L.u[c * n + ib];
+      if (P.bterm == 1) {
+        gc[c] = -(R(3) * a + b) * g1;
+        gc[5 + c] = -(a + R(3) * b) * g2;
+      } else {
+        gc[c] = -a * (R(4) * g1);
+        gc[5 + c] = -b * (R(4) * g2);
+      }
+    }
+  }
+  R rnorm = sqrt(wx * wx + wy * wy + wz * wz);
+  if (!(rnorm > R(1e-10)) || !(ind <= 4 || ind == 9)) {
+#pragma unroll
+    for (int c = 0; c < 10; ++c) o[c] = gc[c];
+    return;
+  }
+  R irn = R(1) / rnorm;
+  R rnx = wx * irn, rny = wy * irn, rnz = wz * irn;
+  const R *A = L.rec0 + 8 * (size_t)ia;
+  const R *B = L.rec0 + 8 * (size_t)ib;
+  R f1[5], f2[5];
+  bside_state_flux(P, ind, A, rnx, rny, rnz, f1);
+  bside_state_flux(P, ind, B, rnx, rny, rnz, f2);
+#pragma unroll
+  for (int c = 0; c < 5; ++c) {
+    if (P.bterm == 1) {
+      o[c] = gc[c] + rnorm * (R(3) * f1[c] + f2[c]);
+      o[5 + c] = gc[5 + c] + rnorm * (f1[c] + R(3) * f2[c]);
+    } else {
+      o[c] = gc[c] + rnorm * R(4) * f1[c];
+      o[5 + c] = gc[5 + c] + rnorm * R(4) * f2[c];
+    }
+  }
+}
+
+template <typename R>
+__global__ __launch_bounds__(NTHR) void k_bflux(LevelDev<R> L, DevParams P) {
+  int bb_;
+  int s = btid(L.nb, bb_);
+  L.to_batch(bb_);
+  P.to_batch(bb_);
+  if (s >= L.nbs) return;
+  bflux_side(L, P, s);
+}
+
 // The same flux with the two ends' records staged in LDS per block of
 // sides, and the sides' fluxes summed per node inside the block.  A block
 // serves up to FB_SIDES consecutive sides that touch at most FB_NODES
@@ -978,6 +1104,11 @@ __global__ void k_flux(LevelDev<R> L, DevParams P) {
 // Every load of a block depends on its header or on nothing: the node list
 // sits at a fixed place per block, so the records are two loads away from
 // the start, and the sides' own words are requested before the staging.
+// BND: blocks spread evenly among the side blocks evaluate the boundary sides,
+// one a thread, instead of a launch of their own (k_bflux).  That saves the
+// launch where it is the cost: us merged / apart, 13.4 / 18 with 19k boundary
+// sides, 114 / 120 with 74k, but 72 / 68 with 89k, 230 / 227 with 115k and
+// 914 / 907 with 295k (the longer code takes registers from the sides).
 // side-block shapes: FB_SHAPE_THR[k] sides per block (one thread each)
 // touching at most FB_SHAPE_NODES[k] distinct nodes; the autotuner picks
 // one per level (shape 0 unless it finds another faster)
@@ -992,7 +1123,7 @@ template <int ORDER>
 constexpr int fb_stride() {  // LDS words per node: record 7 | grad + bounds 25 | coordinates 3
   return ORDER > 1 ? FB_REC + GREC - 1 + 3 : FB_REC;  // odd: lanes reading different nodes spread over banks
 }
-template <typename R, int ORDER, bool SA, int NSIG, int SHAPE>
+template <typename R, int ORDER, bool SA, int NSIG, int SHAPE, bool BND>
 __global__ __launch_bounds__(FB_SHAPE_THR[SHAPE]) void k_flux_blk(LevelDev<R> L, DevParams P) {
   constexpr int FB_THR = FB_SHAPE_THR[SHAPE], FB_SIDES = FB_THR, FB_NODES = FB_SHAPE_NODES[SHAPE];
   constexpr int S = fb_stride<ORDER>();
@@ -1003,7 +1134,18 @@ __global__ __launch_bounds__(FB_SHAPE_THR[SHAPE]) void k_flux_blk(LevelDev<R> L,
   int bb_ = lb % L.nb, blk = lb / L.nb;
   L.to_batch(bb_);
   P.to_batch(bb_);
-  if (blk >= L.nfb) return;
+  if constexpr (BND) {
+    const int nbb = (L.nbs + FB_THR - 1) / FB_THR, all = L.nfb + nbb;
+    const int before = (int)((long long)blk * nbb / all);  // boundary blocks before this one
+    if ((int)((long long)(blk + 1) * nbb / all) > before) {
+      const int s = before * FB_THR + (int)threadIdx.x;
+      if (s < L.nbs) bflux_side(L, P, s);
+      return;
+    }
+    blk -= before;
+  } else if (blk >= L.nfb) {
+    return;
+  }
   const int4 h0 = reinterpret_cast<const int4 *>(L.fb_head)[blk];
   const int4 h1 = reinterpret_cast<const int4 *>(L.fb_head)[blk + 1];
   const int n0 = h0.y, nn = h1.y - h0.y, ibase = h0.z;
@@ -1084,123 +1226,6 @@ __global__ __launch_bounds__(FB_SHAPE_THR[SHAPE]) void k_flux_blk(LevelDev<R> L,
     o[0] = half ? r[3] : r[0];
     o[1] = half ? r[4] : r[1];
     o[2] = half ? r[5] : r[2];
-  }
-}
-
-// physical flux of one state through unit normal
-template <typename R>
-__device__ __forceinline__ void phys_flux(const R *q, R rnx, R rny, R rnz, R *f) {
-  R rho = q[0], u = q[1], v = q[2], w = q[3], pr = q[5], rh = q[4] + q[5];
-  R nv = u * rnx + v * rny + w * rnz;
-  f[0] = rho * nv;
-  f[1] = pr * rnx + rho * u * nv;
-  f[2] = pr * rny + rho * v * nv;
-  f[3] = pr * rnz + rho * w * nv;
-  f[4] = rh * nv;
-}
-
-// farfield Roe flux of one state against the inflow state (DEF:2258-2446)
-template <typename R>
-__device__ __forceinline__ void farfield_roe(const double *inf, const R *q, R gm1, R rnx, R rny, R rnz, R *f) {
-  R ro = R(inf[0]), uo = R(inf[1]), vo = R(inf[2]), wo = R(inf[3]), eo = R(inf[4]), po = R(inf[5]);
-  R rho = q[0], uu = q[1], vv = q[2], ww = q[3], eps = q[4], pr = q[5];
-  R rh = eps + pr, h = rh / rho;
-  R nv = uu * rnx + vv * rny + ww * rnz;
-  R fl1 = rho * nv, fl2 = pr * rnx + rho * uu * nv, fl3 = pr * rny + rho * vv * nv;
-  R fl4 = pr * rnz + rho * ww * nv, fl5 = rh * nv;
-  R epsr = eo * ro, hr = eo + po / ro;
-  R unr = uo * rnx + vo * rny + wo * rnz;
-  R fr1 = ro * unr, fr2 = rnx * po + ro * uo * unr, fr3 = rny * po + ro * vo * unr;
-  R fr4 = rnz * po + ro * wo * unr, fr5 = (epsr + po) * unr;
-  R di = sqrt(ro / rho), d1 = R(1) / (di + R(1));
-  R ui = (di * uo + uu) * d1, vi = (di * vo + vv) * d1, wi = (di * wo + ww) * d1, hi = (di * hr + h) * d1;
-  R af = R(0.5) * (ui * ui + vi * vi + wi * wi);
-  R ci2 = gm1 * (hi - af);
-  ci2 = ci2 > R(1e-5) ? ci2 : R(1e-5);
-  R ci = sqrt(ci2), ici = R(1) / ci;
-  R ucp = ui * rnx + vi * rny + wi * rnz;
-  R du1 = ro - rho, du2 = ro * uo - rho * uu, du3 = ro * vo - rho * vv;
-  R du4 = ro * wo - rho * ww, du5 = epsr - eps;
-  R rl1 = fabs(ucp + ci), rl2 = fabs(ucp - ci), rl3 = fabs(ucp);
-  R s1 = R(0.5) * (rl1 + rl2), s2 = R(0.5) * (rl1 - rl2);
-  R al1x = gm1 * (af * du1 - ui * du2 - vi * du3 - wi * du4 + du5);
-  R al2x = -ucp * du1 + du2 * rnx + du3 * rny + du4 * rnz;
-  R cc1 = ((s1 - rl3) * al1x / ci2) + (s2 * al2x * ici);
-  R cc2 = (s2 * al1x * ici) + (s1 - rl3) * al2x;
-  f[0] = R(0.5) * (fr1 + fl1) - R(0.5) * (rl3 * du1 + cc1);
-  f[1] = R(0.5) * (fr2 + fl2) - R(0.5) * (rl3 * du2 + cc1 * ui + cc2 * rnx);
-  f[2] = R(0.5) * (fr3 + fl3) - R(0.5) * (rl3 * du3 + cc1 * vi + cc2 * rny);
-  f[3] = R(0.5) * (fr4 + fl4) - R(0.5) * (rl3 * du4 + cc1 * wi + cc2 * rnz);
-  f[4] = R(0.5) * (fr5 + fl5) - R(0.5) * (rl3 * du5 + cc1 * hi + cc2 * ucp);
-}
-
-// the boundary flux of one end's state along the side's unit normal
-template <typename R>
-__device__ __forceinline__ void bside_state_flux(const DevParams &P, int ind, const R *q, R rnx, R rny, R rnz, R *f) {
-  if (ind <= 2 || ind == 9) {
-    phys_flux(q, rnx, rny, rnz, f);
-  } else {
-    double inf[6];
-    P.inflow_row(ind - 3, inf);
-    farfield_roe(inf, q, R(P.gamma - 1.0), rnx, rny, rnz, f);
-  }
-}
-
-// boundary-side loop of makeRHS (DEF:2116-2446): contributions to both ends,
-// bbuf[10*s + 5*end + c]
-template <typename R>
-__global__ void k_bflux(LevelDev<R> L, DevParams P) {
-  int bb_;
-  int s = btid(L.nb, bb_);
-  L.to_batch(bb_);
-  P.to_batch(bb_);
-  if (s >= L.nbs) return;
-  int ia = L.ba[s], ib = L.bb[s], ind = L.bind[s];
-  R wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
-  R *o = L.bbuf + 10 * (size_t)s;
-  // moving mesh: -(3 U_1 + U_2) g_1 / dt to the first end, -(U_1 + 3 U_2)
-  // g_2 / dt to the second (boundaryTerm 1), -4 U_k g_k / dt otherwise, on
-  // every boundary side (DEF:2124-2179)
-  R gc[10];
-#pragma unroll
-  for (int c = 0; c < 10; ++c) gc[c] = 0;
-  if (L.bgcl) {
-    const size_t n = L.n;
-    R g1 = L.bgcl[2 * (size_t)s] / R(P.dtp), g2 = L.bgcl[2 * (size_t)s + 1] / R(P.dtp);
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      R a = L.u[c * n + ia], b = L.u[c * n + ib];
-      if (P.bterm == 1) {
-        gc[c] = -(R(3) * a + b) * g1;
-        gc[5 + c] = -(a + R(3) * b) * g2;
-      } else {
-        gc[c] = -a * (R(4) * g1);
-        gc[5 + c] = -b * (R(4) * g2);
-      }
-    }
-  }
-  R rnorm = sqrt(wx * wx + wy * wy + wz * wz);
-  if (!(rnorm > R(1e-10)) || !(ind <= 4 || ind == 9)) {
-#pragma unroll
-    for (int c = 0; c < 10; ++c) o[c] = gc[c];
-    return;
-  }
-  R irn = R(1) / rnorm;
-  R rnx = wx * irn, rny = wy * irn, rnz = wz * irn;
-  const R *A = L.rec0 + 8 * (size_t)ia;
-  const R *B = L.rec0 + 8 * (size_t)ib;
-  R f1[5], f2[5];
-  bside_state_flux(P, ind, A, rnx, rny, rnz, f1);
-  bside_state_flux(P, ind, B, rnx, rny, rnz, f2);
-#pragma unroll
-  for (int c = 0; c < 5; ++c) {
-    if (P.bterm == 1) {
-      o[c] = gc[c] + rnorm * (R(3) * f1[c] + f2[c]);
-      o[5 + c] = gc[5 + c] + rnorm * (f1[c] + R(3) * f2[c]);
-    } else {
-      o[c] = gc[c] + rnorm * R(4) * f1[c];
-      o[5 + c] = gc[5 + c] + rnorm * R(4) * f2[c];
-    }
   }
 }
 
@@ -3600,25 +3625,26 @@ __global__ void k_mu_record(LevelDev<R> L) {
 // node-local pieces shared by the stage kernels
 // ---------------------------------------------------------------------------
 
-// makeSASourceTerm (DEF:9285-9370) for node i; returns the rhs(:,6) increment
+// what the boundary conditions read of a node: its class and unit normal
 template <typename R>
-__device__ __forceinline__ double sa_source(const LevelDev<R> &L, const DevParams &P, int i) {
-  const int n = L.n;
-  double mu = L.mu[i];
-  if (mu < 0.1 / P.Re) {
-    mu = 0.1 * P.Re;
-    L.mu[i] = R(mu);
-  }
-  return sa_source_t<double>(P, double(L.u[i]), double(L.u[5 * n + i]), mu, double(L.vort[i]), double(L.divg[i]),
-                             double(L.wd[i]), double(L.vol[i]));
+struct NodeBc {
+  int cls;
+  R n[3];
+};
+template <typename R>
+__device__ __forceinline__ NodeBc<R> node_bc(const LevelDev<R> &L, int i) {
+  NodeBc<R> b{L.ncls[i] & NC_MASK, {0, 0, 0}};
+  if (b.cls != NC_NONE)
+    for (int k = 0; k < 3; ++k) b.n[k] = L.nrm[3 * (size_t)i + k];
+  return b;
 }
 
 // setBCsOnIncrementField (DEF:4978-5140) for node i on r[0..5]
 template <typename R>
-__device__ __forceinline__ void bc_increment(const LevelDev<R> &L, const DevParams &P, int i, R *r) {
-  int cls = L.ncls[i] & NC_MASK;
+__device__ __forceinline__ void bc_increment(const DevParams &P, const NodeBc<R> &b, R *r) {
+  const int cls = b.cls;
   if (cls == NC_NONE || cls == NC_FAR1 || cls == NC_FAR2) return;
-  R nx = L.nrm[3 * (size_t)i], ny = L.nrm[3 * (size_t)i + 1], nz = L.nrm[3 * (size_t)i + 2];
+  const R nx = b.n[0], ny = b.n[1], nz = b.n[2];
   if (cls == NC_WALL && P.Re > 0.0) {
     r[1] = r[2] = r[3] = 0;
     if (!P.isentropic) r[4] = 0;
@@ -3639,10 +3665,11 @@ __device__ __forceinline__ void bc_increment(const LevelDev<R> &L, const DevPara
 // mesh; coarse levels carry none (the reference reads an array it never
 // allocates there) and take zero.
 template <typename R>
-__device__ __forceinline__ void bc_solution(const LevelDev<R> &L, const DevParams &P, int i, R *q, R rho_g) {
-  int cls = L.ncls[i] & NC_MASK;
+__device__ __forceinline__ void bc_solution(const LevelDev<R> &L, const DevParams &P, int i, const NodeBc<R> &b, R *q,
+                                            R rho_g) {
+  const int cls = b.cls;
   if (cls == NC_NONE || cls == NC_FAR1 || cls == NC_FAR2) return;
-  R nx = L.nrm[3 * (size_t)i], ny = L.nrm[3 * (size_t)i + 1], nz = L.nrm[3 * (size_t)i + 2];
+  const R nx = b.n[0], ny = b.n[1], nz = b.n[2];
   const bool moving = L.cmv && L.gnum == 1 && cls == NC_WALL;
   if (cls == NC_WALL && P.Re > 0.0) {
     if (moving) {  // u(2:4) = u(1) * coordinateMovement / dt (DEF:4408)
@@ -3677,12 +3704,12 @@ __device__ __forceinline__ void bc_solution(const LevelDev<R> &L, const DevParam
 
 // setOuterBoundaryConditions (DEF:4018-4251) for node i
 template <typename R>
-__device__ __forceinline__ void outer_bc(const LevelDev<R> &L, const DevParams &P, int i, R *q, R p) {
-  int cls = L.ncls[i] & NC_MASK;
+__device__ __forceinline__ void outer_bc(const DevParams &P, const NodeBc<R> &b, R *q, R p) {
+  const int cls = b.cls;
   if (cls != NC_FAR1 && cls != NC_FAR2) return;
   double inf[6];
   P.inflow_row(cls - NC_FAR1, inf);
-  R nx = L.nrm[3 * (size_t)i], ny = L.nrm[3 * (size_t)i + 1], nz = L.nrm[3 * (size_t)i + 2];
+  const R nx = b.n[0], ny = b.n[1], nz = b.n[2];
   R rho0 = R(inf[0]), U1 = R(inf[1]), U2 = R(inf[2]), U3 = R(inf[3]);
   R gm1 = R(P.gamma - 1.0);
   R nv = U1 * nx + U2 * ny + U3 * nz;
@@ -3757,24 +3784,67 @@ struct StageArgs {
                              // reference's makePressureField leaves it)
 };
 
+// what a stage reads of its own node, beside its convective residual
+template <typename R>
+struct NodeIn {
+  R up[6], vol, dt, diss[5], p, u0, u5, src[6], mu, vort, divg, wd, dtt, tdiff;
+  NodeBc<R> bc;
+};
+template <typename R, bool SA>
+__device__ __forceinline__ NodeIn<R> node_in(const LevelDev<R> &L, const StageArgs &S, int i) {
+  const size_t n = L.n;
+  NodeIn<R> in;
+  for (int c = 0; c < 6; ++c) in.up[c] = L.uprev[c * n + i];
+  for (int c = 0; c < 5; ++c) in.diss[c] = L.diss[c * n + i];
+  in.vol = L.vol[i];
+  in.dt = L.dt[i];
+  in.p = L.p[i];
+  in.u0 = L.u[i];
+  in.u5 = L.u[5 * n + i];
+  if (S.fas || S.has_src)
+    for (int c = 0; c < 6; ++c) in.src[c] = L.src[c * n + i];
+  in.mu = L.mu[i];
+  if constexpr (SA) {
+    in.vort = L.vort[i];
+    in.divg = L.divg[i];
+    in.wd = L.wd[i];
+    in.dtt = L.dtt[i];
+    in.tdiff = L.tdiff[i];
+  }
+  in.bc = node_bc(L, i);
+  return in;
+}
+
+// makeSASourceTerm (DEF:9285-9370) for node i: the rhs(:,6) increment
+template <typename R>
+__device__ __forceinline__ double sa_source(const LevelDev<R> &L, const DevParams &P, int i, NodeIn<R> &in) {
+  double mu = in.mu;
+  if (mu < 0.1 / P.Re) {
+    mu = 0.1 * P.Re;
+    L.mu[i] = in.mu = R(mu);
+  }
+  return sa_source_t<double>(P, double(in.u0), double(in.u5), mu, double(in.vort), double(in.divg), double(in.wd),
+                             double(in.vol));
+}
+
 // the stage at node i from its convective residual r[6]; rec: where the
 // next state's gather record goes
 template <typename R, int MODE, bool SA>
-__device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams &P, const StageArgs &S, int i, R *r,
-                                           R *rec) {
+__device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams &P, const StageArgs &S, int i,
+                                           NodeIn<R> &in, R *r, R *rec) {
   const int n = L.n;
   bool sa_on = SA && S.calc_turb;
-  if (sa_on) r[5] += R(sa_source(L, P, i));
+  if (sa_on) r[5] += R(sa_source(L, P, i, in));
   if (MODE == MODE_RHS) {
     for (int c = 0; c < 6; ++c) L.rhs[(size_t)c * n + i] = r[c];
     return;
   }
-  if (MODE != MODE_RHS && P.unsteady && P.add_time) {
+  if (P.unsteady && P.add_time) {
     // addTimeDifferences (DEF:1184-1241): BDF2 on grid 1 with the volumes
     // of the last two physical times (equal to V on a fixed mesh), BDF1
     // elsewhere, over components 1:5 (1:6 with SA).  restrictGrid adds it
     // on both grids (DEF:12208 on the restricted state, DEF:12285)
-    const R V = L.vol[i], dtp = R(P.dtp);
+    const R V = in.vol, dtp = R(P.dtp);
     const R VP = L.volp ? L.volp[i] : V, VP2 = L.volp2 ? L.volp2[i] : V;
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
@@ -3786,19 +3856,19 @@ __device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams
         r[c] = r[c] + V * (L.u[k] - L.uold[k]) / dtp;
     }
   }
-  for (int c = 0; c < 5; ++c) r[c] += L.diss[(size_t)c * n + i];
-  if (SA) r[5] += L.tdiff[i];
+  for (int c = 0; c < 5; ++c) r[c] += in.diss[c];
+  if (SA) r[5] += in.tdiff;
   if (!SA) r[5] = 0;
   // solveSystem (DEF:1407-1479); unsteady: dt / (1 + 1.5 dt / dtp) for the
   // mean flow (DEF:1427-1436)
-  R V = L.vol[i], dt = L.dt[i];
+  R V = in.vol, dt = in.dt;
   if (P.unsteady) dt = dt / (R(1.0) + R(1.5) * dt / R(P.dtp));
   for (int c = 0; c < 5; ++c) r[c] = dt * r[c] / V;
-  if (SA) r[5] = L.dtt[i] * r[5] / V;
-  bc_increment(L, P, i, r);
+  if (SA) r[5] = in.dtt * r[5] / V;
+  bc_increment(P, in.bc, r);
   // updateSolutionVector (DEF:1292-1405)
-  R up[6], q[6];
-  for (int c = 0; c < 6; ++c) up[c] = L.uprev[(size_t)c * n + i];
+  R q[6];
+  const R *up = in.up;
   R dtj = R(S.dtj);
   for (int c = 0; c < 5; ++c) r[c] = dtj * r[c];
   if (SA) r[5] = R(S.dtj_t) * r[5];
@@ -3814,10 +3884,10 @@ __device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams
     R t = up[5] - r[5];
     q[5] = t > R(0) ? t : R(0);
   } else {
-    q[5] = L.u[5 * (size_t)n + i];
+    q[5] = in.u5;
   }
   // density check on the grid's own u (DEF:1398-1403)
-  R ug0 = L.u[i];
+  R ug0 = in.u0;
   if (MODE == MODE_FINE) {
     if (ug0 < R(P.min_rho)) L.u[i] = R(P.min_rho);
   } else if (q[0] < R(P.min_rho)) {
@@ -3825,42 +3895,40 @@ __device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams
   }
   // restrictGrid applies the state conditions to the updated state it
   // holds in rhs (DEF:12333-12336) while grp%u keeps the grid's own state
-  bc_solution(L, P, i, q, MODE == MODE_FINE ? (ug0 < R(P.min_rho) ? R(P.min_rho) : ug0) : q[0]);
-  R pi = L.p[i];
+  bc_solution(L, P, i, in.bc, q, MODE == MODE_FINE ? (ug0 < R(P.min_rho) ? R(P.min_rho) : ug0) : q[0]);
   if (MODE == MODE_STAGE) {
     if (S.fas) {
       R a = R(S.alpha);
-      for (int c = 0; c < 5; ++c) q[c] -= a * L.src[(size_t)c * n + i];
-      if (sa_on) q[5] -= a * L.src[5 * (size_t)n + i];
+      for (int c = 0; c < 5; ++c) q[c] -= a * in.src[c];
+      if (sa_on) q[5] -= a * in.src[5];
     }
     q[0] = q[0] > R(P.min_rho) ? q[0] : R(P.min_rho);
     if (sa_on) {
       q[5] = q[5] > R(0) ? q[5] : R(0);
       if (q[5] > R(P.max_turb)) q[5] = R(P.max_turb);
     }
-    outer_bc(L, P, i, q, pi);
+    outer_bc(P, in.bc, q, in.p);
     for (int c = 0; c < 6; ++c) L.u[(size_t)c * n + i] = q[c];
     if (!S.next_record) return;
     // pressure and gather record of the new state, as k_prep forms them, so
     // the next stage starts without a separate pass
-    write_record(L, P, i, q, L.mu[i], rec);
+    write_record(L, P, i, q, in.mu, rec);
   } else if (MODE == MODE_COARSE) {
-    outer_bc(L, P, i, q, pi);
+    outer_bc(P, in.bc, q, in.p);
     for (int c = 0; c < 6; ++c) {
       L.src[(size_t)c * n + i] = q[c] - up[c];
       L.u[(size_t)c * n + i] = up[c];
     }
   } else {  // MODE_FINE
     if (S.has_src) {
-      for (int c = 0; c < 5; ++c) q[c] -= L.src[(size_t)c * n + i];
-      if (SA) q[5] -= L.src[5 * (size_t)n + i];
+      for (int c = 0; c < 5; ++c) q[c] -= in.src[c];
+      if (SA) q[5] -= in.src[5];
     }
     if (SA) {
       q[5] = q[5] > R(0) ? q[5] : R(0);
-      R ug5 = L.u[5 * (size_t)n + i];
-      if (ug5 > R(P.max_turb)) L.u[5 * (size_t)n + i] = R(P.max_turb);
+      if (in.u5 > R(P.max_turb)) L.u[5 * (size_t)n + i] = R(P.max_turb);
     }
-    outer_bc(L, P, i, q, pi);
+    outer_bc(P, in.bc, q, in.p);
     for (int c = 0; c < 5; ++c) L.rhs[(size_t)c * n + i] = q[c] - up[c];
     L.rhs[5 * (size_t)n + i] = SA ? q[5] - up[5] : R(0);
   }
@@ -3877,7 +3945,8 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
   R r[6];
   gather_rhs<R, SA, SUB>(L, i, sub, S.partials, r);
   if (sub) return;
-  stage_node<R, MODE, SA>(L, P, S, i, r, L.rec0);
+  NodeIn<R> in = node_in<R, SA>(L, S, i);
+  stage_node<R, MODE, SA>(L, P, S, i, in, r, L.rec0);
 }
 
 // One launch per stage: the residual of a block of consecutive nodes and
@@ -3891,8 +3960,10 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
 // the sides, for two launches less (side fluxes, boundary fluxes) and no
 // partial sums through memory.  The neighbours' records are read while other
 // blocks write theirs, so the next state's go to rec1 and the host swaps the
-// two.  Latency bounds it (a launch and a chain of four loads), so one task
-// a thread and blocks as large as that allows.  Per stage, FP64 without SA,
+// two.  Latency bounds it, so one task a thread and blocks as large as that
+// allows, tables at fixed places (the chain is node ids, records, result),
+// and what the update reads of the block's own nodes staged beside the
+// records.  Per stage, FP64 without SA,
 // against the three launches: 8.8 us for 18 on 1.3k nodes, 23.5 for 27 on
 // 33k.  (A walk of each node's own sides, every flux at both ends, measured
 // 14 and 40 us.)  Second-order sides stay with k_flux_blk: their records are
@@ -3900,46 +3971,68 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
 // more than the launches.
 // STEP: the nodes' local time steps (makeTimeSteps, inviscid) from the same
 // tasks.
-constexpr int SB_NODES = 32, SB_TASKS = NTHR, SB_CAP = 224, SB_INC = 512, SB_SUB = NTHR / SB_NODES;
 constexpr int SB_S = 7;  // LDS stride of a record (not mu) and of a task's result, odd
+
+constexpr int SB_IN = 32;  // rows of the update's inputs
 
 template <typename R, int MODE, bool SA, bool HLLC, bool STEP>
 __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, StageArgs S) {
   static_assert(SB_CAP <= SB_TASKS && !(SA && STEP), "one LDS area serves the records and the results");
   __shared__ R sn[SB_TASKS * SB_S];
+  __shared__ R own[SB_IN * SB_NODES];
   __shared__ unsigned short sinc[SB_INC];
   const int lb = xcd_block(), bb_ = lb % L.nb, blk = lb / L.nb, t = threadIdx.x;
   L.to_batch(bb_);
   P.to_batch(bb_);
   if (blk >= L.nsb) return;
-  const int4 h0 = reinterpret_cast<const int4 *>(L.sb_head)[2 * blk];
-  const int4 h1 = reinterpret_cast<const int4 *>(L.sb_head)[2 * blk + 1];
-  const int *nodes = L.sb_node + h0.z;
-  // this thread's task and node: their words are requested before the staging
-  const bool active = t < h1.y;
-  unsigned loc = 0;
-  R wx = 0, wy = 0, wz = 0;
-  if (active) {
-    loc = L.sb_loc[h1.x + t];
-    wx = L.sb_w[h1.x + t];
-    wy = L.sb_w[L.sb_ntask + h1.x + t];
-    wz = L.sb_w[2 * L.sb_ntask + h1.x + t];
-  }
-  const int me = t / SB_SUB, sub = t % SB_SUB, i = h0.x + me;
-  int q0 = 0, q1 = 0;
-  if (me < h0.y) {
-    q0 = L.sb_iptr[i] - h1.z;
-    q1 = L.sb_iptr[i + 1] - h1.z;
-  }
+  const int *nodes = L.sb_node + (size_t)SB_CAP * blk;
+  const size_t task = (size_t)SB_TASKS * blk + t, nt = (size_t)SB_TASKS * L.nsb, n = L.n;
+  // this thread's task, the node it sums for and the block's incidences
+  const unsigned loc = L.sb_loc[task];
+  const R wx = L.sb_w[task], wy = L.sb_w[nt + task], wz = L.sb_w[2 * nt + task];
+  const int me = t / SB_SUB, sub = t % SB_SUB, i = nodes[0] + me;
+  const unsigned short *ip = L.sb_iptr + (SB_NODES + 1) * (size_t)blk + me;
+  const int q0 = ip[0], q1 = ip[1];
 #pragma unroll
-  for (int q = 0; q < SB_INC / NTHR; ++q)
-    if (t + q * NTHR < h1.w) sinc[t + q * NTHR] = L.sb_inc[h1.z + t + q * NTHR];
-  fb_stage<SB_CAP, 8, 8, 0, SB_S, R, SB_S>(sn, L.rec0, nodes, h0.w);
+  for (int q = 0; q < SB_INC / NTHR; ++q) sinc[t + q * NTHR] = L.sb_inc[(size_t)SB_INC * blk + t + q * NTHR];
+  // the nodes' records, two words a load
+  {
+    constexpr int PER = (SB_CAP * 4 + NTHR - 1) / NTHR;
+    using P2 = typename Pair<R>::type;
+    int g[PER];
+    P2 v[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int k = (t + q * NTHR) / 4;
+      g[q] = k < SB_CAP ? nodes[k] : -1;
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+      if (g[q] >= 0) v[q] = reinterpret_cast<const P2 *>(L.rec0 + 8 * (size_t)g[q])[t % 4];
+    // and the own nodes' inputs of the update: row r of thread group r
+    const int m = t % SB_NODES, r8 = t / SB_NODES, oi = nodes[0] + m < (int)n ? nodes[0] + m : (int)n - 1;
+    R x0 = r8 < 6 ? L.uprev[r8 * n + oi] : r8 == 6 ? L.vol[oi] : L.dt[oi];
+    R x1 = r8 < 5 ? L.diss[r8 * n + oi] : r8 == 5 ? L.p[oi] : L.u[(r8 == 6 ? 0 : 5) * n + oi];
+    R x2 = r8 < 6 ? L.src[r8 * n + oi] : L.nrm[3 * (size_t)oi + r8 - 6];
+    R x3 = r8 == 0 ? L.nrm[3 * (size_t)oi + 2] : r8 == 1 ? R(L.ncls[oi]) : r8 == 2 ? L.mu[oi] : r8 == 3 ? L.vort[oi]
+           : r8 == 4 ? L.divg[oi] : r8 == 5 ? L.wd[oi] : r8 == 6 ? L.dtt[oi] : L.tdiff[oi];
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+      if (g[q] >= 0) {
+        R *o = sn + SB_S * ((t + q * NTHR) / 4) + 2 * (t % 4);
+        o[0] = v[q].x;
+        if (t % 4 < 3) o[1] = v[q].y;  // not mu
+      }
+    own[t] = x0;
+    own[NTHR + t] = x1;
+    own[2 * NTHR + t] = x2;
+    own[3 * NTHR + t] = x3;
+  }
   __syncthreads();
+  const int kind = loc >> 24;
   R f[7] = {0, 0, 0, 0, 0, 0, 0};
-  if (active) {
+  if (kind != 255) {
     const R *A = sn + (loc & 0xfffu) * SB_S, *B = sn + ((loc >> 12) & 0xfffu) * SB_S;
-    const int kind = loc >> 24;
     if (kind == 0) {
       if constexpr (HLLC) {
         side_flux<R, R, 1, SA, 2>(P, (const R *)nullptr, (const R *)nullptr, (const R *)nullptr, (const R *)nullptr, A,
@@ -3972,12 +4065,12 @@ __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, 
     }
   }
   __syncthreads();  // the records are no longer needed: the results take their place
-  if (active) {
+  if (kind != 255) {
 #pragma unroll
     for (int c = 0; c < SB_S; ++c) sn[SB_S * t + c] = f[c];
   }
   __syncthreads();
-  if (me >= h0.y) return;
+  if (q0 == q1) return;  // beyond the block's nodes (each has a side)
   R r[6] = {0, 0, 0, 0, 0, 0}, lam = 0;
   for (int q = q0 + sub; q < q1; q += SB_SUB) {
     const unsigned v = sinc[q];
@@ -3991,8 +4084,26 @@ __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, 
   for (int c = 0; c < (SA ? 6 : 5); ++c) r[c] = lsum<SB_SUB>(r[c]);
   if constexpr (STEP) lam = lsum<SB_SUB>(lam);
   if (sub) return;
-  if constexpr (STEP) L.dt[i] = R(0.5) / (lam / L.vol[i]);
-  stage_node<R, MODE, SA>(L, P, S, i, r, L.rec1);
+  auto row = [&](int x) { return own[SB_NODES * x + me]; };
+  NodeIn<R> in;
+  for (int c = 0; c < 6; ++c) in.up[c] = row(c);
+  in.vol = row(6);
+  in.dt = row(7);
+  for (int c = 0; c < 5; ++c) in.diss[c] = row(8 + c);
+  in.p = row(13);
+  in.u0 = row(14);
+  in.u5 = row(15);
+  for (int c = 0; c < 6; ++c) in.src[c] = row(16 + c);
+  for (int c = 0; c < 3; ++c) in.bc.n[c] = row(22 + c);
+  in.bc.cls = int(row(25)) & NC_MASK;
+  in.mu = row(26);
+  in.vort = row(27);
+  in.divg = row(28);
+  in.wd = row(29);
+  in.dtt = row(30);
+  in.tdiff = row(31);
+  if constexpr (STEP) L.dt[i] = in.dt = R(0.5) / (lam / in.vol);
+  stage_node<R, MODE, SA>(L, P, S, i, in, r, L.rec1);
 }
 
 // ---------------------------------------------------------------------------
@@ -4026,8 +4137,9 @@ __global__ void k_bc_state(LevelDev<R> L, DevParams P, R *a, int outer) {
   int n = L.n;
   R q[6];
   for (int c = 0; c < 6; ++c) q[c] = a[(size_t)c * n + i];
-  bc_solution(L, P, i, q, a == L.u ? q[0] : L.u[i]);
-  if (outer) outer_bc(L, P, i, q, L.p[i]);
+  const NodeBc<R> b = node_bc(L, i);
+  bc_solution(L, P, i, b, q, a == L.u ? q[0] : L.u[i]);
+  if (outer) outer_bc(P, b, q, L.p[i]);
   for (int c = 0; c < 6; ++c) a[(size_t)c * n + i] = q[c];
 }
 
@@ -4118,8 +4230,9 @@ __global__ void k_restrict_state(LevelDev<RC> K, DevParams P, Transfer T, const 
   for (int c = 0; c < 6; ++c) q[c] = RC(acc[c]);
   K.mu[k] = mu;
   RC pp = state_pressure(P, q);
-  bc_solution(K, P, k, q, q[0]);
-  outer_bc(K, P, k, q, pp);
+  const NodeBc<RC> b = node_bc(K, k);
+  bc_solution(K, P, k, b, q, q[0]);
+  outer_bc(P, b, q, pp);
 #pragma unroll
   for (int c = 0; c < 6; ++c) K.u[(size_t)c * K.n + k] = q[c];
   begin_step(K, P, k, q, mu, 6, zero);
@@ -4142,7 +4255,7 @@ __global__ void k_restrict_forcing(LevelDev<RC> K, DevParams P, Transfer T, cons
   RC r[6], q[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) r[c] = RC(acc[c]);
-  bc_increment(K, P, k, r);
+  bc_increment(P, node_bc(K, k), r);
   const int nc = P.sa ? 6 : 5;
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
@@ -4175,12 +4288,13 @@ __global__ void k_prolong(LevelDev<RF> F, LevelDev<RC> K, DevParams P, Transfer 
   RC q[6], r[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) q[c] = RC(acc[c]);
-  bc_solution(K, P, k, q, K.u[k]);
-  outer_bc(K, P, k, q, K.p[k]);
+  const NodeBc<RC> kb = node_bc(K, k);
+  bc_solution(K, P, k, kb, q, K.u[k]);
+  outer_bc(P, kb, q, K.p[k]);
 #pragma unroll
   for (int c = 0; c < 6; ++c) r[c] = K.u[c * nc + k] - q[c];
   if (!P.sa) r[5] = 0;
-  bc_increment(K, P, k, r);
+  bc_increment(P, kb, r);
   if (sub == 0) {
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
@@ -4195,6 +4309,7 @@ __global__ void k_prolong(LevelDev<RF> F, LevelDev<RC> K, DevParams P, Transfer 
 #pragma unroll
     for (int c = 0; c < 5; ++c) d[c] = RF(P.prolong_relax) * d[c];
     d[5] = RF(P.turb_prolong_relax) * d[5];
+    const NodeBc<RF> fb = node_bc(F, i);
     if (F.ncls[i] & NC_BFIRST)
 #pragma unroll
       for (int c = 0; c < 5; ++c) d[c] = RF(P.mg_bc_relax) * d[c];
@@ -4204,8 +4319,8 @@ __global__ void k_prolong(LevelDev<RF> F, LevelDev<RC> K, DevParams P, Transfer 
       v[c] = F.u[c * n + i];
       if (c < ncomp_add) v[c] = v[c] + d[c];
     }
-    bc_solution(F, P, i, v, v[0]);
-    outer_bc(F, P, i, v, F.p[i]);
+    bc_solution(F, P, i, fb, v, v[0]);
+    outer_bc(P, fb, v, F.p[i]);
     if (P.sa) v[5] = v[5] > RF(0) ? v[5] : RF(0);
     v[0] = v[0] > RF(P.min_rho) ? v[0] : RF(P.min_rho);
 #pragma unroll

@@ -185,10 +185,9 @@ struct Level {
   unsigned short *ell_loc = nullptr;
   // node blocks of the one-launch stages (nsb = 0: none)
   int nsb = 0;
-  long long sb_ntask = 0;
-  int *sb_head = nullptr, *sb_node = nullptr, *sb_iptr = nullptr;
+  int *sb_node = nullptr;
   unsigned *sb_loc = nullptr;
-  unsigned short *sb_inc = nullptr;
+  unsigned short *sb_inc = nullptr, *sb_iptr = nullptr;
   void *sb_w = nullptr;
   // transfer from the next finer level (coarse levels)
   int *f2c = nullptr, *cptr = nullptr, *clist = nullptr;
@@ -217,8 +216,8 @@ struct Level {
     v.nent = B.nent; v.fb_iptr = B.iptr; v.fb_inc = B.inc; v.pn_ptr = B.pn_ptr; v.pn_ent = B.pn_ent;
     v.pbuf = (R *)pbuf;
     v.ngb = ngb; v.gb_first = gb_first; v.gb_nptr = gb_nptr; v.gb_node = gb_node; v.ell_loc = ell_loc;
-    v.nsb = nsb; v.sb_ntask = sb_ntask; v.sb_head = sb_head; v.sb_node = sb_node; v.sb_iptr = sb_iptr;
-    v.sb_loc = sb_loc; v.sb_inc = sb_inc; v.sb_w = (const R *)sb_w;
+    v.nsb = nsb; v.sb_node = sb_node; v.sb_loc = sb_loc; v.sb_inc = sb_inc; v.sb_iptr = sb_iptr;
+    v.sb_w = (const R *)sb_w;
     v.vol = (const R *)vol; v.xyz = has_coords ? (const R *)xyz : nullptr;
     v.wd = (const R *)wd; v.nrm = (const R *)nrm; v.ncls = ncls;
     v.u = (R *)u; v.uprev = (R *)uprev; v.rhs = (R *)rhs; v.diss = (R *)diss; v.src = (R *)src;
@@ -703,11 +702,11 @@ bool jst_active(const flite_ctx *c, const Level &L) {
 // Node blocks of the one-launch stages (LevelDev::sb_*): consecutive nodes,
 // at most SB_NODES of them with at most SB_TASKS sides and (boundary side,
 // own end) pairs, SB_CAP staged nodes and SB_INC incidences.  No blocks if a
-// single node exceeds a limit.
+// single node exceeds a limit or has no side.
 struct StageTables {
-  std::vector<int> head, node, iptr;
+  std::vector<int> node;
   std::vector<unsigned> loc;
-  std::vector<unsigned short> inc;
+  std::vector<unsigned short> inc, iptr;
   std::vector<double> w;
 };
 
@@ -717,7 +716,6 @@ StageTables build_stage_blocks(int n, const std::vector<int> &ell_ptr, const std
                                const std::vector<int> &bs_list, const std::vector<int> &ba, const std::vector<int> &bb,
                                const std::vector<int> &bind, const std::vector<double> &wb) {
   StageTables T;
-  T.iptr.push_back(0);
   struct Side {
     int e, a, b;  // device side, its ends
     double w[3];
@@ -773,6 +771,7 @@ StageTables build_stage_blocks(int n, const std::vector<int> &ell_ptr, const std
     for (; end < n && end - start < SB_NODES; ++end) {
       const int nt = new_sides(start, end, nullptr) + (bs_ptr[end + 1] - bs_ptr[end]), ni = degree(end);
       const int ns = new_staged(blk, end, nullptr);
+      if (ni == 0) return StageTables{};  // the kernel tells a block's end by it
       if (tasks + nt > SB_TASKS || staged + ns > SB_CAP || inc + ni > SB_INC) break;
       tasks += nt;
       staged += ns;
@@ -794,32 +793,36 @@ StageTables build_stage_blocks(int n, const std::vector<int> &ell_ptr, const std
     std::sort(halo.begin(), halo.end());
     for (size_t q = 0; q < halo.size(); ++q) local[halo[q]] = end - start + (int)q;
     std::sort(sides.begin(), sides.end(), [](const Side &x, const Side &y) { return x.e < y.e; });
-    const int task0 = (int)T.loc.size(), inc0 = (int)T.inc.size(), node0 = (int)T.node.size();
+    const size_t task0 = (size_t)SB_TASKS * blk;
+    unsigned t = 0;
+    auto add_task = [&](unsigned word, const double *w) {
+      T.loc.push_back(word);
+      for (int q = 0; q < 3; ++q) wv[q].push_back(w[q]);
+      return t++;
+    };
     std::vector<std::vector<unsigned short>> list(end - start);
     for (const Side &d : sides) {
-      const unsigned t = (unsigned)T.loc.size() - task0;
-      T.loc.push_back((unsigned)local[d.a] | (unsigned)local[d.b] << 12);
-      for (int q = 0; q < 3; ++q) wv[q].push_back(d.w[q]);
-      if (d.a >= start && d.a < end) list[d.a - start].push_back((unsigned short)(t << 1));
-      if (d.b >= start && d.b < end) list[d.b - start].push_back((unsigned short)(t << 1 | 1));
+      const unsigned k = add_task((unsigned)local[d.a] | (unsigned)local[d.b] << 12, d.w);
+      if (d.a >= start && d.a < end) list[d.a - start].push_back((unsigned short)(k << 1));
+      if (d.b >= start && d.b < end) list[d.b - start].push_back((unsigned short)(k << 1 | 1));
     }
     for (int i = start; i < end; ++i)
       for (int k = bs_ptr[i]; k < bs_ptr[i + 1]; ++k) {
         const int v = bs_list[k], b = v >> 1, o = (v & 1) ? ba[b] : bb[b];
-        const unsigned t = (unsigned)T.loc.size() - task0;
-        T.loc.push_back((unsigned)local[i] | (unsigned)local[o] << 12 | (unsigned)(std::max(bind[b], 0) + 1) << 24);
-        for (int q = 0; q < 3; ++q) wv[q].push_back(wb[3 * (size_t)b + q]);
-        list[i - start].push_back((unsigned short)(t << 1));
+        const unsigned word = (unsigned)local[i] | (unsigned)local[o] << 12 | (unsigned)(std::max(bind[b], 0) + 1) << 24;
+        list[i - start].push_back((unsigned short)(add_task(word, &wb[3 * (size_t)b]) << 1));
       }
-    for (const auto &l : list) {
-      T.inc.insert(T.inc.end(), l.begin(), l.end());
-      T.iptr.push_back((int)T.inc.size());
+    T.loc.resize(task0 + SB_TASKS, 255u << 24);
+    for (int q = 0; q < 3; ++q) wv[q].resize(task0 + SB_TASKS, 0.0);
+    const size_t inc0 = T.inc.size();
+    for (int m = 0; m <= SB_NODES; ++m) {
+      T.iptr.push_back((unsigned short)(T.inc.size() - inc0));
+      if (m < end - start) T.inc.insert(T.inc.end(), list[m].begin(), list[m].end());
     }
+    T.inc.resize(inc0 + SB_INC, 0);
     for (int i = start; i < end; ++i) T.node.push_back(i);
     T.node.insert(T.node.end(), halo.begin(), halo.end());
-    for (int v : {start, end - start, node0, (int)T.node.size() - node0, task0, (int)T.loc.size() - task0, inc0,
-                  (int)T.inc.size() - inc0})
-      T.head.push_back(v);
+    T.node.resize((size_t)SB_CAP * (blk + 1), -1);
     start = end;
   }
   for (int q = 0; q < 3; ++q) T.w.insert(T.w.end(), wv[q].begin(), wv[q].end());
@@ -1080,12 +1083,11 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
   TRY(al_real(&L.rec0, (size_t)(8 * (size_t)n) * NB));
   bool need_grad = L.has_coords && c->hp.hllc_flux_order > 1;
   const bool second = need_grad && c->hp.flux_type == 4;
-  if (!second && S.gcl.empty() && S.bgcl.empty() && ne > 0) {
+  if (!second && S.gcl.empty() && S.bgcl.empty() && ne > 0 &&
+      n <= (c->P.sa ? 1 << 14 : 1 << 16)) {
     StageTables T = build_stage_blocks(n, ell_ptr, ell_k, ell_e, ell_nbr, ellw, nslot, bs_ptr, bs_list, ba, bb, S.bi, wb);
-    L.nsb = T.head.empty() ? 0 : (int)(T.head.size() / 8);
+    L.nsb = (int)(T.loc.size() / SB_TASKS);
     if (L.nsb > 0) {
-      L.sb_ntask = (long long)T.loc.size();
-      TRY(P.upload(&L.sb_head, T.head));
       TRY(P.upload(&L.sb_node, T.node));
       TRY(P.upload(&L.sb_iptr, T.iptr));
       TRY(P.upload(&L.sb_loc, T.loc));
@@ -1257,7 +1259,11 @@ int op_grad(flite_ctx *c, Level &L) {
 bool viscous(const flite_ctx *c) { return c->hp.reynolds_number > 0.0; }
 
 // Stages that evaluate their own fluxes (k_stage_blk): levels without
-// second-order sides and without a moving mesh's side terms.
+// second-order sides and without a moving mesh's side terms, up to 16k nodes
+// with SA and 64k without (build_level): the repeated sides cost little where
+// latency is the time.  Per stage, us in one launch / as fluxes and stage: SA
+// 14 / 20 at 5k nodes, 33 / 26 at 31k, 193 / 103 at 255k; inviscid 8 / 14 at
+// 1.3k, 10 / 15 at 9k, 23 / 26 at 33k.
 bool stage_blocks(const flite_ctx *c, const Level &L) { return L.nsb > 0 && !c->flux_apart; }
 
 // ... whose first stage also forms the time steps: nothing else of the step
@@ -1265,6 +1271,9 @@ bool stage_blocks(const flite_ctx *c, const Level &L) { return L.nsb > 0 && !c->
 bool stage_steps(const flite_ctx *c, const Level &L) {
   return stage_blocks(c, L) && !viscous(c) && !jst_active(c, L);
 }
+
+// boundary sides up to which k_flux_blk evaluates them too (its BND)
+constexpr int BND_MERGED = 80000;
 
 int op_flux(flite_ctx *c, Level &L) {
   DevParams P = c->P;
@@ -1274,6 +1283,7 @@ int op_flux(flite_ctx *c, Level &L) {
     L.flux_src = FLUX_BLOCK;
     return 0;
   }
+  bool bflux_done = false;
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
     if (L.ne > 0 && P.ftype != 4) {
@@ -1298,23 +1308,30 @@ int op_flux(flite_ctx *c, Level &L) {
       bool n4 = P.nsig == 4;  // LED exponent: 4 inviscid, 2 viscous
       L.flux_src = c->flux_per_side ? FLUX_SIDES : FLUX_PARTIALS;
       if (L.flux_src == FLUX_PARTIALS) {
-        auto blk = [&](auto shape) {
+        auto blk = [&](auto shape, auto bnd) {
           constexpr int SH = decltype(shape)::value;
-          dim3 gb((unsigned)L.sb[SH].nfb * L.nbatch), bb(FB_SHAPE_THR[SH]);
+          constexpr bool BND = decltype(bnd)::value;
+          const int nb_blocks = BND ? nblk(L.nbs, FB_SHAPE_THR[SH]) : 0;
+          dim3 gb((unsigned)(L.sb[SH].nfb + nb_blocks) * L.nbatch), bb(FB_SHAPE_THR[SH]);
           if (o2 && P.sa) {
-            if (n4) hipLaunchKernelGGL((k_flux_blk<R, 2, true, 4, SH>), gb, bb, 0, c->stream, V, P);
-            else hipLaunchKernelGGL((k_flux_blk<R, 2, true, 2, SH>), gb, bb, 0, c->stream, V, P);
+            if (n4) hipLaunchKernelGGL((k_flux_blk<R, 2, true, 4, SH, BND>), gb, bb, 0, c->stream, V, P);
+            else hipLaunchKernelGGL((k_flux_blk<R, 2, true, 2, SH, BND>), gb, bb, 0, c->stream, V, P);
           } else if (o2) {
-            if (n4) hipLaunchKernelGGL((k_flux_blk<R, 2, false, 4, SH>), gb, bb, 0, c->stream, V, P);
-            else hipLaunchKernelGGL((k_flux_blk<R, 2, false, 2, SH>), gb, bb, 0, c->stream, V, P);
+            if (n4) hipLaunchKernelGGL((k_flux_blk<R, 2, false, 4, SH, BND>), gb, bb, 0, c->stream, V, P);
+            else hipLaunchKernelGGL((k_flux_blk<R, 2, false, 2, SH, BND>), gb, bb, 0, c->stream, V, P);
           } else if (P.sa) {
-            hipLaunchKernelGGL((k_flux_blk<R, 1, true, 2, SH>), gb, bb, 0, c->stream, V, P);
+            hipLaunchKernelGGL((k_flux_blk<R, 1, true, 2, SH, BND>), gb, bb, 0, c->stream, V, P);
           } else {
-            hipLaunchKernelGGL((k_flux_blk<R, 1, false, 2, SH>), gb, bb, 0, c->stream, V, P);
+            hipLaunchKernelGGL((k_flux_blk<R, 1, false, 2, SH, BND>), gb, bb, 0, c->stream, V, P);
           }
         };
-        if (L.fb_shape == 0) blk(std::integral_constant<int, 0>{});
-        else blk(std::integral_constant<int, 1>{});
+        auto by_shape = [&](auto bnd) {
+          if (L.fb_shape == 0) blk(std::integral_constant<int, 0>{}, bnd);
+          else blk(std::integral_constant<int, 1>{}, bnd);
+        };
+        bflux_done = L.nbs <= BND_MERGED;
+        if (bflux_done) by_shape(std::true_type{});
+        else by_shape(std::false_type{});
       } else if (o2 && P.sa) {
         if (n4) hipLaunchKernelGGL((k_flux<R, 2, true, 4>), g, b, 0, c->stream, V, P);
         else hipLaunchKernelGGL((k_flux<R, 2, true, 2>), g, b, 0, c->stream, V, P);
@@ -1327,7 +1344,7 @@ int op_flux(flite_ctx *c, Level &L) {
         hipLaunchKernelGGL((k_flux<R, 1, false, 2>), g, b, 0, c->stream, V, P);
       }
     }
-    if (L.nbs > 0) {
+    if (L.nbs > 0 && !bflux_done) {
       Timed tm(c, "bflux", L.gnum);
       hipLaunchKernelGGL(k_bflux<R>, dim3(nblk(L.nbs) * L.nbatch), dim3(NTHR), 0, c->stream, V, P);
     }
