@@ -1418,7 +1418,7 @@ __device__ __forceinline__ void bside_end_flux(const DevParams &P, int ind, cons
 // tangent: fbuf/bbuf <- d(fluxes)/dU along du; the stage gather (MODE_RHS)
 // then sums them into rhs = (dR/dU) du
 template <bool SA>
-__global__ void k_flux_tangent(LevelDev<double> L, DevParams P, const double *du) {
+__global__ __launch_bounds__(NTHR) void k_flux_tangent(LevelDev<double> L, DevParams P, const double *du) {
   using ad::Dual;
   int e = gtid_x();
   if (e >= L.ne) return;
@@ -1444,7 +1444,7 @@ __global__ void k_flux_tangent(LevelDev<double> L, DevParams P, const double *du
   f[5] = SA ? o[5].d : 0.0;
 }
 
-__global__ void k_bflux_tangent(LevelDev<double> L, DevParams P, const double *du) {
+__global__ __launch_bounds__(NTHR) void k_bflux_tangent(LevelDev<double> L, DevParams P, const double *du) {
   using ad::Dual;
   int s = gtid_x();
   if (s >= L.nbs) return;
@@ -1482,7 +1482,7 @@ __global__ void k_bflux_tangent(LevelDev<double> L, DevParams P, const double *d
 // adjoint, interior sides: side e adds +f to R(ea) and -f to R(eb), so its
 // share of (dR/dU)^T lam is (df/dU_ea)^T d and (df/dU_eb)^T d with
 // d = lam(ea) - lam(eb).  abuf[10*e + k]: k < 5 for U_ea, k >= 5 for U_eb.
-__global__ void k_flux_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *abuf) {
+__global__ __launch_bounds__(NTHR) void k_flux_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *abuf) {
   using ad::Dual;
   int e = gtid_x();
   if (e >= L.ne) return;
@@ -1518,7 +1518,7 @@ __global__ void k_flux_adjoint(LevelDev<double> L, DevParams P, const double *la
 // (boundaryTerm 1; 4F_a and 4F_b for 2), so U_a receives
 // |w| (dF_a/dU_a)^T (3 lam_a + lam_b), and alike for U_b.  bbuf layout as
 // the residual's: [10*s + 5*end + k].
-__global__ void k_bflux_adjoint(LevelDev<double> L, DevParams P, const double *lam) {
+__global__ __launch_bounds__(NTHR) void k_bflux_adjoint(LevelDev<double> L, DevParams P, const double *lam) {
   using ad::Dual;
   int s = gtid_x();
   if (s >= L.nbs) return;
@@ -1558,7 +1558,7 @@ __global__ void k_bflux_adjoint(LevelDev<double> L, DevParams P, const double *l
 }
 
 // adjoint gather: out(i) = sum of node i's shares over its sides
-__global__ void k_adjoint_gather(LevelDev<double> L, const double *abuf, double *out) {
+__global__ __launch_bounds__(NTHR) void k_adjoint_gather(LevelDev<double> L, const double *abuf, double *out) {
   int i = gtid_x();
   if (i >= L.n) return;
   double r[5] = {0, 0, 0, 0, 0};
@@ -1583,7 +1583,7 @@ __global__ void k_adjoint_gather(LevelDev<double> L, const double *abuf, double 
 // DEF:6873-6880, first order at both orders: the node values of nu~ and
 // the velocities): node i's share of sum over sides of (lam6_ea - lam6_eb) f6
 // from six dual passes per side seeded on its own (U, nu~), added to out
-__global__ void k_sa_conv_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *out) {
+__global__ __launch_bounds__(NTHR) void k_sa_conv_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *out) {
   using ad::Dual;
   int i = gtid_x();
   if (i >= L.n) return;
@@ -1625,7 +1625,7 @@ __global__ void k_sa_conv_adjoint(LevelDev<double> L, DevParams P, const double 
 // three dual passes per side, seeded on the weight components, give the
 // three components of the derivative.  Side e adds +f to R(ea) and -f to
 // R(eb), so its share is (lam_a - lam_b) . df/dw.
-__global__ void k_flux_metric_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *gw) {
+__global__ __launch_bounds__(NTHR) void k_flux_metric_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *gw) {
   using ad::Dual;
   int e = gtid_x();
   if (e >= L.ne) return;
@@ -1656,7 +1656,7 @@ __global__ void k_flux_metric_adjoint(LevelDev<double> L, DevParams P, const dou
 
 // boundary sides: R(a) += |w|(3F_a + F_b), R(b) += |w|(F_a + 3F_b)
 // (boundaryTerm 1; 4F_a and 4F_b for 2) with F evaluated along w/|w|
-__global__ void k_bflux_metric_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *gwb) {
+__global__ __launch_bounds__(NTHR) void k_bflux_metric_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *gwb) {
   using ad::Dual;
   int s = gtid_x();
   if (s >= L.nbs) return;
@@ -1721,7 +1721,7 @@ constexpr int LIN_SIDE = 10 + 2 * LIN_G;    // adjoint shares per side: U_a 5, U
 // the gather record's tangent dq[DQ i ..] = (rho, u, v, w, E, p, nu~, 0)
 // along du (nu~ = u(:,6) with Spalart-Allmaras, else 0)
 constexpr int DQ = 8;
-__global__ void k_record_tangent(LevelDev<double> L, DevParams P, const double *du, double *dq) {
+__global__ __launch_bounds__(NTHR) void k_record_tangent(LevelDev<double> L, DevParams P, const double *du, double *dq) {
   using ad::Dual;
   int i = gtid_x();
   if (i >= L.n) return;
@@ -1742,7 +1742,7 @@ __global__ void k_record_tangent(LevelDev<double> L, DevParams P, const double *
 // branch of the side flux is taken as in the residual and the adjoint; the
 // tangents follow the same walk in slot order, the bounds' with the extremal
 // neighbour that k_minmax_arg names.
-__global__ void k_grad_tangent(LevelDev<double> L, const double *dq, ad::Dual *gd) {
+__global__ __launch_bounds__(NTHR) void k_grad_tangent(LevelDev<double> L, const double *dq, ad::Dual *gd) {
   using ad::Dual;
   int i = gtid_x();
   if (i >= L.n) return;
@@ -1798,7 +1798,7 @@ __global__ void k_grad_tangent(LevelDev<double> L, const double *dq, ad::Dual *g
 // second-order side fluxes along (du, dG, dB): fbuf[6 e + c] = d f_c
 // (component 5: the SA convection along d nu~)
 template <int NSIG, bool SA>
-__global__ void k_flux_tangent2(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *gd) {
+__global__ __launch_bounds__(NTHR) void k_flux_tangent2(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *gd) {
   using ad::Dual;
   int e = gtid_x();
   if (e >= L.ne) return;
@@ -1821,7 +1821,7 @@ __global__ void k_flux_tangent2(LevelDev<double> L, DevParams P, const double *d
 // node i's extremal neighbours: amin[10 i + c] = the node whose q_c sets
 // the lower bound of component c (-1 if none: the bound is 0), amin[10 i +
 // 5 + c] the upper one, with grad_minmax_body's comparisons in slot order
-__global__ void k_minmax_arg(LevelDev<double> L, int *amin) {
+__global__ __launch_bounds__(NTHR) void k_minmax_arg(LevelDev<double> L, int *amin) {
   int i = gtid_x();
   if (i >= L.n) return;
   double q0[5], mn[5], mx[5];
@@ -1936,7 +1936,7 @@ __global__ __launch_bounds__(NTHR) void k_flux_adjoint2(LevelDev<double> L, DevP
 
 // per node: ub = its conserved-state shares (sides and boundary sides),
 // gbn = its gradient and bound shares
-__global__ void k_adjoint_gather2(LevelDev<double> L, const double *abuf2, double *ub, double *gbn) {
+__global__ __launch_bounds__(NTHR) void k_adjoint_gather2(LevelDev<double> L, const double *abuf2, double *ub, double *gbn) {
   int i = gtid_x();
   if (i >= L.n) return;
   double r[5] = {0, 0, 0, 0, 0}, g[LIN_G];
@@ -1963,7 +1963,7 @@ __global__ void k_adjoint_gather2(LevelDev<double> L, const double *abuf2, doubl
 
 // transpose of the gradient and bounds: qb[5 j + c] = sum over the G and B
 // that q_j(c) enters of their shares times d(G, B)/dq_j(c)
-__global__ void k_grad_adjoint(LevelDev<double> L, const double *gbn, const int *amin, double *qb) {
+__global__ __launch_bounds__(NTHR) void k_grad_adjoint(LevelDev<double> L, const double *gbn, const int *amin, double *qb) {
   int j = gtid_x();
   if (j >= L.n) return;
   double r[5] = {0, 0, 0, 0, 0}, sw[3] = {0, 0, 0};
@@ -2009,7 +2009,7 @@ __global__ void k_grad_adjoint(LevelDev<double> L, const double *gbn, const int 
 }
 
 // out(i) = ub(i) + (dq/dU)^T qb(i): the record's dependence on the state
-__global__ void k_record_adjoint(LevelDev<double> L, DevParams P, const double *ub, const double *qb, double *out) {
+__global__ __launch_bounds__(NTHR) void k_record_adjoint(LevelDev<double> L, DevParams P, const double *ub, const double *qb, double *out) {
   using ad::Dual;
   int i = gtid_x();
   if (i >= L.n) return;
@@ -2043,7 +2043,7 @@ __global__ void k_record_adjoint(LevelDev<double> L, DevParams P, const double *
 // per side: gw[3 e + k] (direct and through both ends' gradients) and
 // gdx[3 e + k] = d(lam^T R)/d dx_k
 template <int NSIG>
-__global__ void k_flux_mesh_adjoint2(LevelDev<double> L, DevParams P, const double *lam, const double *gbn,
+__global__ __launch_bounds__(NTHR) void k_flux_mesh_adjoint2(LevelDev<double> L, DevParams P, const double *lam, const double *gbn,
                                      double *gw, double *gdx) {
   using ad::Dual;
   int e = gtid_x();
@@ -2098,7 +2098,7 @@ __global__ void k_flux_mesh_adjoint2(LevelDev<double> L, DevParams P, const doub
 // per boundary side: adds the gradients' share to gwb (the direct share of
 // the first-order boundary flux is k_bflux_metric_adjoint's): G_a holds
 // (3 q_a + q_b) w_b / V_a and G_b holds (3 q_b + q_a) w_b / V_b
-__global__ void k_bgrad_mesh_adjoint(LevelDev<double> L, const double *gbn, double *gwb) {
+__global__ __launch_bounds__(NTHR) void k_bgrad_mesh_adjoint(LevelDev<double> L, const double *gbn, double *gwb) {
   int s = gtid_x();
   if (s >= L.nbs) return;
   int ia = L.ba[s], ib = L.bb[s];
@@ -2116,7 +2116,7 @@ __global__ void k_bgrad_mesh_adjoint(LevelDev<double> L, const double *gbn, doub
 }
 
 // per node: d(lam^T R)/dV_i = -sum gbn_i . G_i / V_i (G is a sum over V)
-__global__ void k_vol_mesh_adjoint(LevelDev<double> L, const double *gbn, double *gvol) {
+__global__ __launch_bounds__(NTHR) void k_vol_mesh_adjoint(LevelDev<double> L, const double *gbn, double *gvol) {
   int i = gtid_x();
   if (i >= L.n) return;
   const double *g = L.grec + GREC * (size_t)i, *s = gbn + LIN_G * (size_t)i;
@@ -2289,7 +2289,7 @@ __device__ __forceinline__ void visc_grad_sums(const LevelDev<double> &L, const 
 // With Spalart-Allmaras also aux[3 i ..] = (laminar viscosity, vorticity,
 // divergence) on dual numbers, for the SA source and diffusion (aux may be
 // null otherwise)
-__global__ void k_visc_tangent_node(LevelDev<double> L, DevParams P, const double *dq, ad::Dual *taud,
+__global__ __launch_bounds__(NTHR) void k_visc_tangent_node(LevelDev<double> L, DevParams P, const double *dq, ad::Dual *taud,
                                     ad::Dual *aux) {
   using ad::Dual;
   int i = gtid_x();
@@ -2310,7 +2310,7 @@ __global__ void k_visc_tangent_node(LevelDev<double> L, DevParams P, const doubl
 }
 
 // tangent pass 2: dvis(c, i) = -dA (c = 1..4), 0 for c = 0
-__global__ void k_visc_tangent_flux(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *taud,
+__global__ __launch_bounds__(NTHR) void k_visc_tangent_flux(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *taud,
                                     double *dvis) {
   using ad::Dual;
   int i = gtid_x();
@@ -2349,7 +2349,7 @@ __global__ void k_visc_tangent_flux(LevelDev<double> L, DevParams P, const doubl
 // duals aux = (laminar viscosity, vorticity, divergence) of
 // k_visc_tangent_node.
 // pass 1: dnud[4 i ..] = the grad nu~ record (grad 3, nodal cb2 term)
-__global__ void k_sa_diff1_tangent(LevelDev<double> L, DevParams P, const double *dq, ad::Dual *dnud) {
+__global__ __launch_bounds__(NTHR) void k_sa_diff1_tangent(LevelDev<double> L, DevParams P, const double *dq, ad::Dual *dnud) {
   using ad::Dual;
   int i = gtid_x();
   if (i >= L.n) return;
@@ -2390,7 +2390,7 @@ __device__ __forceinline__ ad::Dual sa_diff_coef(const LevelDev<double> &L, cons
 }
 
 // pass 2 and the source: dsa[i] = d(tdiff + source) at node i
-__global__ void k_sa_tangent(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *aux,
+__global__ __launch_bounds__(NTHR) void k_sa_tangent(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *aux,
                              const ad::Dual *dnud, double *dsa) {
   using ad::Dual;
   int i = gtid_x();
@@ -2429,7 +2429,7 @@ __global__ void k_sa_tangent(LevelDev<double> L, DevParams P, const double *dq, 
 // adjoint pass 1: shares of lam^T(-A) on node i's stress record (taub 9)
 // and velocities through the energy flux (ub 3), from its own terms and its
 // neighbours' terms; tau values in taud (pass 1 without tangents)
-__global__ void k_visc_adjoint_tau(LevelDev<double> L, DevParams P, const double *lam, const ad::Dual *taud,
+__global__ __launch_bounds__(NTHR) void k_visc_adjoint_tau(LevelDev<double> L, DevParams P, const double *lam, const ad::Dual *taud,
                                    double *taub, double *ubv) {
   using ad::Dual;
   int i = gtid_x();
@@ -2527,7 +2527,7 @@ __global__ void k_visc_adjoint_tau(LevelDev<double> L, DevParams P, const double
 // node) also the shares on the mesh quantities the node reads: its volume,
 // its wall normal (wall nodes, the adiabatic projection) and, with
 // Spalart-Allmaras, its wall distance (the source).
-__global__ void k_visc_adjoint_node(LevelDev<double> L, DevParams P, const double *lam, const double *taub,
+__global__ __launch_bounds__(NTHR) void k_visc_adjoint_node(LevelDev<double> L, DevParams P, const double *lam, const double *taub,
                                     double *gbar, double *tbar, double *rnbar, double *mbar) {
   using ad::Dual;
   int i = gtid_x();
@@ -2583,7 +2583,7 @@ __global__ void k_visc_adjoint_node(LevelDev<double> L, DevParams P, const doubl
 // adjoint pass 3: the Green-Gauss sums transposed, abar[4 j + q] on node j's
 // record (u, v, w, T), plus its direct shares (T through the viscosity, the
 // velocities through the energy flux)
-__global__ void k_visc_adjoint_grad(LevelDev<double> L, const double *gbar, const double *tbar, const double *ubv,
+__global__ __launch_bounds__(NTHR) void k_visc_adjoint_grad(LevelDev<double> L, const double *gbar, const double *tbar, const double *ubv,
                                     double *abar) {
   int j = gtid_x();
   if (j >= L.n) return;
@@ -2626,7 +2626,7 @@ __global__ void k_visc_adjoint_grad(LevelDev<double> L, const double *gbar, cons
 
 // adjoint pass 4: out(c, i) += (da/dU)^T abar (the record's dependence on
 // the conserved state)
-__global__ void k_visc_adjoint_record(LevelDev<double> L, DevParams P, const double *abar, double *out) {
+__global__ __launch_bounds__(NTHR) void k_visc_adjoint_record(LevelDev<double> L, DevParams P, const double *abar, double *out) {
   using ad::Dual;
   int i = gtid_x();
   if (i >= L.n) return;
@@ -2657,7 +2657,7 @@ __global__ void k_visc_adjoint_record(LevelDev<double> L, DevParams P, const dou
 // With mbar it also adds the share on node k's volume (through d_k and the
 // nodal term) to mbar[5 k] and keeps (d_k, v_k) in sad[4 k ..] for the side
 // weights' shares (k_visc_mesh_side / k_visc_mesh_bside).
-__global__ void k_sa_diff_adjoint1(LevelDev<double> L, DevParams P, const double *lam, double *gnbar, double *tbar,
+__global__ __launch_bounds__(NTHR) void k_sa_diff_adjoint1(LevelDev<double> L, DevParams P, const double *lam, double *gnbar, double *tbar,
                                    double *rnbar, double *mbar, double *sad) {
   using ad::Dual;
   int k = gtid_x();
@@ -2716,7 +2716,7 @@ __global__ void k_sa_diff_adjoint1(LevelDev<double> L, DevParams P, const double
 // g with sum_j w_mj + 3 (or 4) sum_b w_b, its neighbours' g with w_jm =
 // -w_mj and, boundaryTerm 1, its boundary partners' g with w_b), plus the
 // (rho, nu~) shares; added to out
-__global__ void k_sa_diff_adjoint2(LevelDev<double> L, DevParams P, const double *gnbar, const double *rnbar,
+__global__ __launch_bounds__(NTHR) void k_sa_diff_adjoint2(LevelDev<double> L, DevParams P, const double *gnbar, const double *rnbar,
                                    double *out) {
   int m = gtid_x();
   if (m >= L.n) return;
@@ -2755,7 +2755,7 @@ __device__ __forceinline__ void visc_rec_v(const LevelDev<double> &L, const DevP
 // and the SA diffusion's side terms -f2 (v_a d_a + v_b d_b).w of node a
 // (node b: the negative).  gbar / gnbar are the shares on the sums; lam
 // null: the sums of the viscous records only (the drag's friction).
-__global__ void k_visc_mesh_side(LevelDev<double> L, DevParams P, const double *lam, const ad::Dual *taud,
+__global__ __launch_bounds__(NTHR) void k_visc_mesh_side(LevelDev<double> L, DevParams P, const double *lam, const ad::Dual *taud,
                                  const double *gbar, const double *gnbar, const double *sad, double *dgw) {
   int e = gtid_x();
   if (e >= L.ne) return;
@@ -2809,7 +2809,7 @@ __global__ void k_visc_mesh_side(LevelDev<double> L, DevParams P, const double *
 // of each end (indicators other than 2 and 9) and the SA diffusion's
 // boundary terms (boundaryTerm 1: -f2 (3 v_i d_i + v_o d_o).w_b, 2:
 // -4 f2 v_i d_i.w_b); added to dgwb[3 s ..]
-__global__ void k_visc_mesh_bside(LevelDev<double> L, DevParams P, const double *lam, const ad::Dual *taud,
+__global__ __launch_bounds__(NTHR) void k_visc_mesh_bside(LevelDev<double> L, DevParams P, const double *lam, const ad::Dual *taud,
                                   const double *gbar, const double *gnbar, const double *sad, double *dgwb) {
   int s = gtid_x();
   if (s >= L.nbs) return;
@@ -2873,7 +2873,7 @@ __global__ void k_visc_mesh_bside(LevelDev<double> L, DevParams P, const double 
 // shares on the stress record (taub[9 i ..], the heat-flux slots 0), on the
 // wall area (gaf[i]) and on the normal (gnf[3 i ..]: fct A_i tau_i t); the
 // caller clears the arrays elsewhere.
-__global__ void k_friction_shares(LevelDev<double> L, const int *wall_nodes, int nw, const double *warea,
+__global__ __launch_bounds__(NTHR) void k_friction_shares(LevelDev<double> L, const int *wall_nodes, int nw, const double *warea,
                                   double fct, double t0, double t1, double t2, double groundplane,
                                   const ad::Dual *taud, double *taub, double *gaf, double *gnf) {
   int k = gtid();
@@ -2906,7 +2906,7 @@ __global__ void k_friction_shares(LevelDev<double> L, const int *wall_nodes, int
 // mesh adjoint of the SA convection (first order at both HLLC orders):
 // side e's share on its weight w, (lam6_a - lam6_b) df6/dw from three dual
 // passes; added to dgw[3 e ..]
-__global__ void k_sa_conv_mesh_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *dgw) {
+__global__ __launch_bounds__(NTHR) void k_sa_conv_mesh_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *dgw) {
   using ad::Dual;
   int e = gtid_x();
   if (e >= L.ne) return;
