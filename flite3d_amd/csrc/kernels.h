@@ -453,6 +453,7 @@ __device__ __forceinline__ bool gb_stage(const LevelDev<R> &L, R *sn, int blk) {
 // ---------------------------------------------------------------------------
 template <typename R>
 __device__ __forceinline__ R state_pressure(const DevParams &P, const R *q) {
+#pragma clang fp contract(off)
   R pp = R(P.gamma - 1.0) * (q[4] - R(0.5) * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0]);
   return pp > R(0.1) ? pp : R(0.1);
 }
@@ -4353,6 +4354,7 @@ struct ForceFrame {
 template <typename R>
 __device__ __forceinline__ void force_terms(const LevelDev<R> &L, const DevParams &P, const ForceFrame &F, int ip,
                                             const R *warea, double *o) {
+#pragma clang fp contract(off)
   for (int c = 0; c < 8; ++c) o[c] = 0;
   double z = L.xyz ? double(L.xyz[3 * (size_t)ip + 2]) : 0.0;
   if (!(z > F.groundplane + 0.01)) return;
@@ -4446,12 +4448,20 @@ __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParam
       maxloc(mx[j], mi[j], fabs(d), hi);
     }
   }
+  // force integrals; walls of up to NTHR nodes are summed in the register's
+  // order, as the loop this stands for, and without contraction, so that an
+  // inviscid drag has the bits of a serial program's whatever the state
   double f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  const bool serial = nw <= NTHR;
+  __shared__ double terms[8][NTHR];
   for (int k = blockIdx.x * NTHR + threadIdx.x; k < nw; k += stride) {
     double o[8];
     force_terms(L, P, F, wall_nodes[k], warea, o);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) f[c] += o[c];
+    for (int c = 0; c < 8; ++c) {
+      if (serial) terms[c][threadIdx.x] = o[c];
+      else f[c] += o[c];
+    }
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
@@ -4481,6 +4491,8 @@ __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParam
       v = q < 14 ? m : double(k);
     } else {
       for (int w = 0; w < NW; ++w) v += lds[q][w];
+      if (serial && blockIdx.x == 0 && q >= 21)
+        for (int k = 0; k < nw; ++k) v += terms[q - 21][k];
     }
     part[(size_t)MON_BLOCKS * q + blockIdx.x] = v;
   }
