@@ -1416,6 +1416,247 @@ __device__ __forceinline__ void bside_end_flux(const DevParams &P, int ind, cons
   }
 }
 
+// (dA/dU)^T of the gather record's (rho, u, v, w, rhoE): shares b[5] on the
+// record to shares on the conserved state
+__device__ __forceinline__ void record_share(const double *A, const double *b, double *out) {
+  const double ir = 1.0 / A[0];
+  out[0] = b[0] - (b[1] * A[1] + b[2] * A[2] + b[3] * A[3]) * ir;
+  out[1] = b[1] * ir;
+  out[2] = b[2] * ir;
+  out[3] = b[3] * ir;
+  out[4] = b[4];
+}
+// the pressure's share bp of a record, on its primitive entries b[5]
+// (p = (gamma - 1)(E - rho |v|^2 / 2), no share where it is clipped)
+__device__ __forceinline__ void pressure_share(double gm1, double r, const double *v, double p_raw, double bp, double &br,
+                                               double *bv, double &be) {
+  if (!(p_raw > 0.1)) return;
+  be += gm1 * bp;
+  br -= 0.5 * gm1 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) * bp;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) bv[k] -= gm1 * r * v[k] * bp;
+}
+
+// Reverse sweep of side_flux_d (components 0..4): with multipliers dl on the
+// flux, the shares sa, sb on the two ends' (rho, u, v, w, rhoE) and, second
+// order (d non-null), sd on the slopes.  The pressures of the records are
+// those of their states (state_record).  One forward and one backward pass
+// over the branch the values take; seeding dual numbers on each of the 15
+// inputs evaluated the whole flux 15 times at one wavefront a SIMD.
+template <bool SECOND>
+__device__ __forceinline__ void side_flux_reverse(const DevParams &P, const double *A, const double *B,
+                                                  const double *d, double wx, double wy, double wz, const double *dl,
+                                                  double *sa, double *sb, double *sd) {
+  const double gm1 = P.gamma - 1.0, beta = P.beta0;
+  const double nx = 2.0 * wx, ny = 2.0 * wy, nz = 2.0 * wz, n2 = nx * nx + ny * ny + nz * nz;
+  const double inv = n2 > 0.0 ? 1.0 / ::sqrt(n2) : 0.0, size = n2 * inv;
+  const double n[3] = {nx * inv, ny * inv, nz * inv};
+  // forward: the two faces' states
+  struct Face {
+    double r, v[3], e, p, p_raw, rinv, h, nv, q, x, c;
+    double br, bv[3], be, bp, bh, bnv, bc;
+    bool fr, fe;
+  } f[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    Face &F = f[k];
+    const double *R = k ? B : A;
+    const double sg = k ? -1.0 : 1.0;
+    F.r = R[0];
+    F.e = R[4];
+    F.fr = F.fe = false;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) F.v[q] = R[1 + q];
+    if constexpr (SECOND) {
+      F.fr = R[0] + sg * d[0] > 0.1;
+      F.fe = R[4] + sg * d[4] > 0.0001;
+      if (F.fr) F.r = R[0] + sg * d[0];
+      if (F.fe) F.e = R[4] + sg * d[4];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) F.v[q] = R[1 + q] + sg * d[1 + q];
+    }
+    F.q = F.v[0] * F.v[0] + F.v[1] * F.v[1] + F.v[2] * F.v[2];
+    F.p_raw = gm1 * (F.e - 0.5 * F.q * F.r);
+    F.p = F.p_raw > 0.1 ? F.p_raw : 0.1;
+    F.rinv = 1.0 / F.r;
+    F.h = (F.e + F.p) * F.rinv;
+    F.nv = F.v[0] * n[0] + F.v[1] * n[1] + F.v[2] * n[2];
+    F.x = F.h - 0.5 * F.q;
+    F.c = ::sqrt(gm1 * ::fabs(F.x));
+    F.br = F.be = F.bp = F.bh = F.bnv = F.bc = 0.0;
+    F.bv[0] = F.bv[1] = F.bv[2] = 0.0;
+  }
+  const double rr = ::sqrt(f[1].r * f[0].rinv), iro = 1.0 / (1.0 + rr);
+  double ut[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) ut[q] = (f[0].v[q] + f[1].v[q] * rr) * iro;
+  const double ht = (f[0].h + f[1].h * rr) * iro, qt = ut[0] * n[0] + ut[1] * n[1] + ut[2] * n[2];
+  const double y = gm1 * (ht - 0.5 * (ut[0] * ut[0] + ut[1] * ut[1] + ut[2] * ut[2])), ct = ::sqrt(::fabs(y));
+  // the wave speeds and which of the three candidates each is
+  int kl = 0, kr = 0;
+  double sl = f[0].nv - beta * f[0].c, sr = f[1].nv + beta * f[1].c;
+  if (qt - ct < sl) { sl = qt - ct; kl = 1; }
+  if (f[1].nv - beta * f[1].c < sl) { sl = f[1].nv - beta * f[1].c; kl = 2; }
+  if (qt + ct > sr) { sr = qt + ct; kr = 1; }
+  if (f[0].nv + beta * f[0].c > sr) { sr = f[0].nv + beta * f[0].c; kr = 2; }
+  const double num = f[1].r * f[1].nv * (sr - f[1].nv) - f[0].r * f[0].nv * (sl - f[0].nv) + f[0].p - f[1].p;
+  const double den = f[1].r * (sr - f[1].nv) - f[0].r * (sl - f[0].nv), fact = den != 0.0 ? 1.0 / den : 0.0;
+  const double sm = fact * num;
+  const bool lft = sl > 0.0 || (sl <= 0.0 && sm > 0.0), rgt = (sm <= 0.0 && sr >= 0.0) || sr < 0.0;
+  if (!lft && !rgt) {
+    // the central flux of the nodes' states (NaN wave speeds)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const double *R = k ? B : A;
+      double *o = k ? sb : sa;
+      const double wn = wx * R[1] + wy * R[2] + wz * R[3], ww[3] = {wx, wy, wz};
+      const double m = dl[0] + dl[1] * R[1] + dl[2] * R[2] + dl[3] * R[3], h = R[4] + R[5];
+      double bv[3];
+      o[0] = wn * m;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) bv[q] = R[0] * (ww[q] * m + wn * dl[1 + q]) + h * ww[q] * dl[4];
+      o[4] = wn * dl[4];
+      const double p_raw = gm1 * (R[4] - 0.5 * (R[1] * R[1] + R[2] * R[2] + R[3] * R[3]) * R[0]);
+      pressure_share(gm1, R[0], R + 1, p_raw, dl[1] * wx + dl[2] * wy + dl[3] * wz + wn * dl[4], o[0], bv, o[4]);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) o[1 + q] = bv[q];
+    }
+    if constexpr (SECOND)
+#pragma unroll
+      for (int c = 0; c < 5; ++c) sd[c] = 0.0;
+    return;
+  }
+  // backward: the upwind side K, on selected copies
+  double g[5];
+#pragma unroll
+  for (int c = 0; c < 5; ++c) g[c] = dl[c] * size;
+  const double r = lft ? f[0].r : f[1].r, e = lft ? f[0].e : f[1].e, p = lft ? f[0].p : f[1].p;
+  const double nv = lft ? f[0].nv : f[1].nv, sk = lft ? sl : sr;
+  double v[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) v[q] = lft ? f[0].v[q] : f[1].v[q];
+  double br, bv[3], be, bp, bnv, bsk = 0.0, bsm = 0.0;
+  {
+    const double S = g[0] + g[1] * v[0] + g[2] * v[1] + g[3] * v[2];
+    br = nv * S;
+    bnv = r * S + (e + p) * g[4];
+    be = nv * g[4];
+    bp = g[1] * n[0] + g[2] * n[1] + g[3] * n[2] + nv * g[4];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) bv[q] = r * nv * g[1 + q];
+  }
+  const bool star = lft ? !(sl > 0.0) : !(sr < 0.0);
+  if (star && sk - sm != 0.0) {
+    const double k = 1.0 / (sk - sm), a = sk - nv;
+    const double pks = r * (nv - sk) * (nv - sm) + p, ps = pks - p;
+    double s[5], b[5];
+    s[0] = r * a * k;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) s[1 + q] = (a * r * v[q] + ps * n[q]) * k;
+    s[4] = (a * e - p * nv + pks * sm) * k;
+    bsk += g[0] * (s[0] - r) + g[4] * (s[4] - e);
+    br -= g[0] * sk;
+    be -= g[4] * sk;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      bsk += g[1 + q] * (s[1 + q] - r * v[q]);
+      br -= g[1 + q] * sk * v[q];
+      bv[q] -= g[1 + q] * sk * r;
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c) b[c] = g[c] * sk;
+    const double bden = -k * (b[0] * s[0] + b[1] * s[1] + b[2] * s[2] + b[3] * s[3] + b[4] * s[4]);
+    const double bw = b[0] + b[1] * v[0] + b[2] * v[1] + b[3] * v[2];
+    const double ba = k * (r * bw + b[4] * e);
+    const double bps = k * (b[1] * n[0] + b[2] * n[1] + b[3] * n[2]), bpks = k * sm * b[4] + bps;
+    br += k * a * bw;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) bv[q] += k * a * r * b[1 + q];
+    be += k * a * b[4];
+    bp += bpks - bps - k * nv * b[4];
+    bnv -= k * p * b[4];
+    bsm += k * pks * b[4];
+    br += bpks * (nv - sk) * (nv - sm);
+    bnv += bpks * r * ((nv - sm) + (nv - sk));
+    bsk -= bpks * r * (nv - sm);
+    bsm -= bpks * r * (nv - sk);
+    bsk += ba + bden;
+    bnv -= ba;
+    bsm -= bden;
+  }
+  double bsl = lft ? bsk : 0.0, bsr = lft ? 0.0 : bsk;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const bool mine = lft == (k == 0);
+    Face &F = f[k];
+    F.br = mine ? br : 0.0;
+    F.be = mine ? be : 0.0;
+    F.bp = mine ? bp : 0.0;
+    F.bnv = mine ? bnv : 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) F.bv[q] = mine ? bv[q] : 0.0;
+  }
+  {  // the contact speed
+    const double bnum = bsm * fact, bden = -bsm * num * fact * fact;
+    f[1].br += bnum * f[1].nv * (sr - f[1].nv) + bden * (sr - f[1].nv);
+    f[1].bnv += bnum * f[1].r * (sr - 2.0 * f[1].nv) - bden * f[1].r;
+    bsr += bnum * f[1].r * f[1].nv + bden * f[1].r;
+    f[0].br -= bnum * f[0].nv * (sl - f[0].nv) + bden * (sl - f[0].nv);
+    f[0].bnv += -bnum * f[0].r * (sl - 2.0 * f[0].nv) + bden * f[0].r;
+    bsl -= bnum * f[0].r * f[0].nv + bden * f[0].r;
+    f[0].bp += bnum;
+    f[1].bp -= bnum;
+  }
+  // the outer wave speeds
+  f[0].bnv += (kl == 0 ? bsl : 0.0) + (kr == 2 ? bsr : 0.0);
+  f[0].bc = beta * ((kr == 2 ? bsr : 0.0) - (kl == 0 ? bsl : 0.0));
+  f[1].bnv += (kl == 2 ? bsl : 0.0) + (kr == 0 ? bsr : 0.0);
+  f[1].bc = beta * ((kr == 0 ? bsr : 0.0) - (kl == 2 ? bsl : 0.0));
+  const double bqt = (kl == 1 ? bsl : 0.0) + (kr == 1 ? bsr : 0.0);
+  const double bct = (kr == 1 ? bsr : 0.0) - (kl == 1 ? bsl : 0.0);
+  const double by = ct > 0.0 ? bct * (y < 0.0 ? -0.5 : 0.5) / ct : 0.0, bht = gm1 * by;
+  double brr = 0.0, biro = bht * (f[0].h + f[1].h * rr);
+  f[0].bh += bht * iro;
+  f[1].bh += bht * iro * rr;
+  brr += bht * iro * f[1].h;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const double but = bqt * n[q] - gm1 * by * ut[q];
+    f[0].bv[q] += but * iro;
+    f[1].bv[q] += but * iro * rr;
+    brr += but * iro * f[1].v[q];
+    biro += but * (f[0].v[q] + f[1].v[q] * rr);
+  }
+  brr -= biro * iro * iro;
+  const double brat = rr > 0.0 ? 0.5 * brr / rr : 0.0;
+  f[1].br += brat * f[0].rinv;
+  f[0].br -= brat * rr * rr * f[0].rinv;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    Face &F = f[k];
+    const double bx = F.c > 0.0 ? F.bc * gm1 * (F.x < 0.0 ? -0.5 : 0.5) / F.c : 0.0;
+    F.bh += bx;
+    F.be += F.bh * F.rinv;
+    F.bp += F.bh * F.rinv;
+    F.br -= F.bh * F.h * F.rinv;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) F.bv[q] += F.bnv * n[q] - bx * F.v[q];
+    pressure_share(gm1, F.r, F.v, F.p_raw, F.bp, F.br, F.bv, F.be);
+    double *o = k ? sb : sa;
+    o[0] = F.br;
+    o[1] = F.bv[0];
+    o[2] = F.bv[1];
+    o[3] = F.bv[2];
+    o[4] = F.be;
+  }
+  if constexpr (SECOND) {
+    sd[0] = (f[0].fr ? f[0].br : 0.0) - (f[1].fr ? f[1].br : 0.0);
+    sd[4] = (f[0].fe ? f[0].be : 0.0) - (f[1].fe ? f[1].be : 0.0);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sd[1 + q] = f[0].bv[q] - f[1].bv[q];
+  }
+}
+
 // tangent: fbuf/bbuf <- d(fluxes)/dU along du; the stage gather (MODE_RHS)
 // then sums them into rhs = (dR/dU) du
 template <bool SA>
@@ -1484,7 +1725,6 @@ __global__ __launch_bounds__(NTHR) void k_bflux_tangent(LevelDev<double> L, DevP
 // share of (dR/dU)^T lam is (df/dU_ea)^T d and (df/dU_eb)^T d with
 // d = lam(ea) - lam(eb).  abuf[10*e + k]: k < 5 for U_ea, k >= 5 for U_eb.
 __global__ __launch_bounds__(NTHR) void k_flux_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *abuf) {
-  using ad::Dual;
   int e = gtid_x();
   if (e >= L.ne) return;
   size_t n = L.n;
@@ -1496,23 +1736,13 @@ __global__ __launch_bounds__(NTHR) void k_flux_adjoint(LevelDev<double> L, DevPa
     ub[c] = L.u[c * n + ib];
     d[c] = lam[c * n + ia] - lam[c * n + ib];
   }
-  Dual wx(L.w[3 * e]), wy(L.w[3 * e + 1]), wz(L.w[3 * e + 2]);
-#pragma unroll 1
-  for (int k = 0; k < 10; ++k) {
-    Dual Ua[5], Ub[5], A[8], B[8], o[6];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      Ua[c] = Dual(ua[c], k == c ? 1.0 : 0.0);
-      Ub[c] = Dual(ub[c], k == c + 5 ? 1.0 : 0.0);
-    }
-    state_record(Ua, P.gamma, A);
-    state_record(Ub, P.gamma, B);
-    side_flux<Dual, double, 1, false, 2, double, double>(P, nullptr, nullptr, nullptr, nullptr, A, B, wx, wy, wz, o);
-    double acc = 0;
-#pragma unroll
-    for (int c = 0; c < 5; ++c) acc += d[c] * o[c].d;
-    abuf[10 * (size_t)e + k] = acc;
-  }
+  double A[8], B[8], sa[5], sb[5], sd[5];
+  state_record(ua, P.gamma, A);
+  state_record(ub, P.gamma, B);
+  side_flux_reverse<false>(P, A, B, nullptr, L.w[3 * e], L.w[3 * e + 1], L.w[3 * e + 2], d, sa, sb, sd);
+  double *o = abuf + 10 * (size_t)e;
+  record_share(A, sa, o);
+  record_share(B, sb, o + 5);
 }
 
 // adjoint, boundary sides: R(a) += |w|(3F_a + F_b), R(b) += |w|(F_a + 3F_b)
@@ -1559,21 +1789,26 @@ __global__ __launch_bounds__(NTHR) void k_bflux_adjoint(LevelDev<double> L, DevP
 }
 
 // adjoint gather: out(i) = sum of node i's shares over its sides
+template <int SUB>
 __global__ __launch_bounds__(NTHR) void k_adjoint_gather(LevelDev<double> L, const double *abuf, double *out) {
-  int i = gtid_x();
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
   if (i >= L.n) return;
   double r[5] = {0, 0, 0, 0, 0};
-  for_edges<1>(L, i, 0, [&](int e, int role) {
+  for_edges<SUB>(L, i, sub, [&](int e, int role) {
     const double *a = abuf + 10 * (size_t)e + 5 * role;
 #pragma unroll
     for (int c = 0; c < 5; ++c) r[c] += a[c];
   });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
+  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
     int v = L.bs_list[k];
     const double *b = L.bbuf + 10 * (size_t)(v >> 1) + 5 * (v & 1);
 #pragma unroll
     for (int c = 0; c < 5; ++c) r[c] += b[c];
   }
+#pragma unroll
+  for (int c = 0; c < 5; ++c) r[c] = lsum<SUB>(r[c]);
+  if (sub) return;
   size_t n = L.n;
 #pragma unroll
   for (int c = 0; c < 5; ++c) out[c * n + i] = r[c];
@@ -1582,41 +1817,44 @@ __global__ __launch_bounds__(NTHR) void k_adjoint_gather(LevelDev<double> L, con
 
 // adjoint of the SA convection (the side flux's component 6, makeSARHS
 // DEF:6873-6880, first order at both orders: the node values of nu~ and
-// the velocities): node i's share of sum over sides of (lam6_ea - lam6_eb) f6
-// from six dual passes per side seeded on its own (U, nu~), added to out
+// the velocities): node i's share of sum over sides of (lam6_ea - lam6_eb) f6,
+// added to out.  With m = nu~ v, X = w.(m_b - m_a) and s the sign of X / (nu~_a
+// - nu~_b), f6 = w.(m_a + m_b) + s X, so with the node-signed weight node i's
+// own m enters a side's term as (lam_i - lam_j)(1 - s) w.m_i: the walk sums
+// that one vector, and its shares on v and nu~ follow at the end.  (Six dual
+// passes of every side took 168 us at 275k nodes, 73 now.)
+template <int SUB>
 __global__ __launch_bounds__(NTHR) void k_sa_conv_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *out) {
-  using ad::Dual;
-  int i = gtid_x();
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
   if (i >= L.n) return;
   const size_t n = L.n;
-  double ui[6], acc[6] = {0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int c = 0; c < 6; ++c) ui[c] = L.u[c * n + i];
-  for_edges<1>(L, i, 0, [&](int e, int role) {
-    const int o = role ? L.ea[e] : L.eb[e];
-    const double dl = lam[5 * n + L.ea[e]] - lam[5 * n + L.eb[e]];
-    double uo[6];
-#pragma unroll
-    for (int c = 0; c < 6; ++c) uo[c] = L.u[c * n + o];
-    const Dual wx(L.w[3 * e]), wy(L.w[3 * e + 1]), wz(L.w[3 * e + 2]);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      Dual Ui[5], Uo[5], S[8], O[8];
-#pragma unroll
-      for (int c = 0; c < 5; ++c) {
-        Ui[c] = Dual(ui[c], k == c ? 1.0 : 0.0);
-        Uo[c] = Dual(uo[c]);
-      }
-      state_record(Ui, P.gamma, S);
-      state_record(Uo, P.gamma, O);
-      S[6] = Dual(ui[5], k == 5 ? 1.0 : 0.0);
-      O[6] = Dual(uo[5]);
-      const Dual f = role ? sa_side_convection(O, S, wx, wy, wz) : sa_side_convection(S, O, wx, wy, wz);
-      acc[k] += dl * f.d;
+  double qi[8], z[3] = {0, 0, 0};
+  ldrec<8>(L.rec0 + 8 * (size_t)i, qi);
+  const double li = lam[5 * n + i];
+  for_edges_w<SUB>(L, i, sub, [&](int j, double wx, double wy, double wz) {
+    double qj[8];
+    ldrec<8>(L.rec0 + 8 * (size_t)j, qj);
+    const double dt = qi[6] - qj[6];
+    double c = li - lam[5 * n + j];
+    if (::fabs(dt) > 1e-20) {
+      const double x = wx * (qj[1] * qj[6] - qi[1] * qi[6]) + wy * (qj[2] * qj[6] - qi[2] * qi[6]) +
+                       wz * (qj[3] * qj[6] - qi[3] * qi[6]);
+      c *= x / dt < 0.0 ? 2.0 : 0.0;
     }
+    z[0] += c * wx;
+    z[1] += c * wy;
+    z[2] += c * wz;
   });
 #pragma unroll
-  for (int c = 0; c < 6; ++c) out[c * n + i] += acc[c];
+  for (int k = 0; k < 3; ++k) z[k] = lsum<SUB>(z[k]);
+  if (sub) return;
+  const double b[5] = {0.0, z[0] * qi[6], z[1] * qi[6], z[2] * qi[6], 0.0};
+  double o[5];
+  record_share(qi, b, o);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) out[c * n + i] += o[c];
+  out[5 * n + i] += z[0] * qi[1] + z[1] * qi[2] + z[2] * qi[3];
 }
 
 // Metric adjoint: the derivative of lam^T R with respect to the side
@@ -1716,7 +1954,9 @@ __global__ __launch_bounds__(NTHR) void k_bflux_metric_adjoint(LevelDev<double> 
 // extremum and with the node itself).
 // ---------------------------------------------------------------------------
 constexpr int LIN_G = 25;                   // gradient 15 | 1/lo 5 | 1/hi 5
-constexpr int LIN_SIDE = 10 + 2 * LIN_G;    // adjoint shares per side: U_a 5, U_b 5, (G,B)_a 25, (G,B)_b 25
+// adjoint shares per side: U_a 5 | slope projection 5, bound 5, side vector
+// 3, code | U_b 5 (an end reads 19 consecutive words)
+constexpr int LIN_SIDE = 24;
 
 // tangent of the gather record (rho, u, v, w, rhoE, p) along du
 // the gather record's tangent dq[DQ i ..] = (rho, u, v, w, E, p, nu~, 0)
@@ -1854,157 +2094,219 @@ __global__ __launch_bounds__(NTHR) void k_minmax_arg(LevelDev<double> L, int *am
   }
 }
 
+// LED-limited projection (led) with its derivatives: da along the projection,
+// div along the reciprocal bound its sign selects
+template <int NSIG>
+__device__ __forceinline__ double led_slopes(double a, double ilo, double ihi, double &da, double &div, bool &hi) {
+  hi = a > 0.0;
+  const double iv = hi ? ihi : ilo;
+  da = div = 0.0;
+  if (!(a > 0.0 || a < 0.0)) {
+    da = 1.0;
+    return a;
+  }
+  if (iv == 0.0) return 0.0;
+  const double t = 2.0 * a * iv, t2 = t * t;
+  if (NSIG == 4) {
+    const double den = 1.0 + t2 * t2, iden = 1.0 / ::sqrt(::sqrt(den));
+    da = iden / den;
+    div = -2.0 * a * a * t * t2 * da;
+    return a * iden;
+  }
+  const double den = 1.0 + t2, iden = 1.0 / ::sqrt(den);
+  da = iden / den;
+  div = -2.0 * a * a * t * da;
+  return a * iden;
+}
+
 // adjoint shares of side e: dl = lam_a - lam_b against df/d(U_a, U_b,
 // G_a, B_a, G_b, B_b).  The gradients and bounds reach the flux only through
-// the five MUSCL slopes d_j, so one dual pass per state component and per
-// slope gives dl^T df/d(U_a, U_b, d), and the slopes' own derivatives (a few
-// scalar dual passes of muscl_slope per component) carry the d shares to
-// the gradients (d a_j / d G = half the side vector) and the bounds.
+// the five MUSCL slopes d_j: the reverse sweep of the flux gives the shares
+// on U_a, U_b and d, and a slope is one end's limited projection (minmod), so
+// its share goes to one end's gradient (along half the side vector) and one
+// of that end's bounds.  Per component: the share on the projection, on the
+// bound, and 3 bits of the code: 1 (first end) or 2 (second) or 0 (none), + 4
+// for the upper bound.  (15 dual passes of the flux and 60 stored words took
+// 1.9 ms and the gather 0.57 ms at 64^3; 0.31 and 0.37 now.)
 template <int NSIG>
 __global__ __launch_bounds__(NTHR) void k_flux_adjoint2(LevelDev<double> L, DevParams P, const double *lam,
                                                         double *abuf2) {
-  using ad::Dual;
   int e = gtid_x();
   if (e >= L.ne) return;
   size_t n = L.n;
   int ia = L.ea[e], ib = L.eb[e];
-  double ua[5], ub[5], dl[5];
+  double A[8], B[8], dl[5], d[5], da[5], db[5], iva[5], ivb[5];
+  ldrec<8>(L.rec0 + 8 * (size_t)ia, A);
+  ldrec<8>(L.rec0 + 8 * (size_t)ib, B);
 #pragma unroll
-  for (int c = 0; c < 5; ++c) {
-    ua[c] = L.u[c * n + ia];
-    ub[c] = L.u[c * n + ib];
-    dl[c] = lam[c * n + ia] - lam[c * n + ib];
-  }
+  for (int c = 0; c < 5; ++c) dl[c] = lam[c * n + ia] - lam[c * n + ib];
   const double *ga = L.grec + GREC * (size_t)ia, *gb = L.grec + GREC * (size_t)ib;
   const double *xa = L.xyz + 3 * (size_t)ia, *xb = L.xyz + 3 * (size_t)ib;
-  const double w0 = L.w[3 * e], w1 = L.w[3 * e + 1], w2 = L.w[3 * e + 2];
-  double pa[5], pb[5], d[5];
-  const double hl = muscl_projections<double>(P, ga, gb, xa, xb, pa, pb);
-#pragma unroll
-  for (int j = 0; j < 5; ++j)
-    d[j] = muscl_slope<NSIG, double>(P, pa[j], pb[j], ga[15 + j], ga[20 + j], gb[15 + j], gb[20 + j], hl);
-  double *out = abuf2 + LIN_SIDE * (size_t)e;
-  double sd[5] = {0, 0, 0, 0, 0};
-#pragma unroll 1
-  for (int k = 0; k < 15; ++k) {
-    Dual Ua[5], Ub[5], A[8], B[8], D[5], o[6];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      Ua[c] = Dual(ua[c], k == c ? 1.0 : 0.0);
-      Ub[c] = Dual(ub[c], k == 5 + c ? 1.0 : 0.0);
-      D[c] = Dual(d[c], k == 10 + c ? 1.0 : 0.0);
-    }
-    state_record(Ua, P.gamma, A);
-    state_record(Ub, P.gamma, B);
-    side_flux_d<Dual, double, false>(P, A, B, D, Dual(w0), Dual(w1), Dual(w2), o, 0.0);
-    double acc = 0;
-#pragma unroll
-    for (int c = 0; c < 5; ++c) acc += dl[c] * o[c].d;
-    if (k < 10) out[k] = acc;
-#pragma unroll
-    for (int c = 0; c < 5; ++c)
-      if (k == 10 + c) sd[c] = acc;  // selects, not an indexed private array
-  }
   const double dx = xb[0] - xa[0], dy = xb[1] - xa[1], dz = xb[2] - xa[2];
-  const double hx = 0.5 * dx, hy = 0.5 * dy, hz = 0.5 * dz;
-  double *oa = out + 10, *ob = out + 10 + LIN_G;
-#pragma unroll 1
-  for (int j = 0; j < 5; ++j) {
-    const double aj = muscl_projection<double>(ga, dx, dy, dz, j), bj = muscl_projection<double>(gb, dx, dy, dz, j);
-    const double s = j == 0 ? sd[0] : j == 1 ? sd[1] : j == 2 ? sd[2] : j == 3 ? sd[3] : sd[4];
-    // d_j's derivatives along (a_j, b_j, ilo_a, ihi_a, ilo_b, ihi_b)
-    double dd[6];
+  const double hl = 0.5 * P.clip * ::sqrt(dx * dx + dy * dy + dz * dz);
+  int code = 0;
 #pragma unroll
-    for (int q = 0; q < 6; ++q) {
-      Dual c = muscl_slope<NSIG, Dual>(P, Dual(aj, q == 0 ? 1.0 : 0.0), Dual(bj, q == 1 ? 1.0 : 0.0),
-                                       Dual(ga[15 + j], q == 2 ? 1.0 : 0.0), Dual(ga[20 + j], q == 3 ? 1.0 : 0.0),
-                                       Dual(gb[15 + j], q == 4 ? 1.0 : 0.0), Dual(gb[20 + j], q == 5 ? 1.0 : 0.0),
-                                       Dual(hl));
-      dd[q] = s * c.d;
+  for (int j = 0; j < 5; ++j) {
+    double a = muscl_projection<double>(ga, dx, dy, dz, j), b = muscl_projection<double>(gb, dx, dy, dz, j);
+    bool ha = false, hb = false;
+    da[j] = db[j] = 1.0;
+    iva[j] = ivb[j] = 0.0;
+    if (P.autoclip == 1) {
+      a = led_slopes<NSIG>(a, ga[15 + j], ga[20 + j], da[j], iva[j], ha);
+      b = -led_slopes<NSIG>(-b, gb[15 + j], gb[20 + j], db[j], ivb[j], hb);
+      ivb[j] = -ivb[j];
     }
-    oa[j] = dd[0] * hx;
-    oa[j + 5] = dd[0] * hy;
-    oa[j + 10] = dd[0] * hz;
-    oa[15 + j] = dd[2];
-    oa[20 + j] = dd[3];
-    ob[j] = dd[1] * hx;
-    ob[j + 5] = dd[1] * hy;
-    ob[j + 10] = dd[1] * hz;
-    ob[15 + j] = dd[4];
-    ob[20 + j] = dd[5];
+    double c = 0.0;
+    int who = 0;
+    if (!(a * b <= 0.0)) {
+      const bool first = ::fabs(a) <= ::fabs(b);
+      c = first ? a : b;
+      who = first ? 1 : 2;
+      if (::fabs(c) > hl && hl > 0.0) {
+        c = c > 0.0 ? hl : -hl;
+        who = 0;
+      }
+    }
+    d[j] = c;
+    // the chosen end's derivatives, in da and iva
+    da[j] = who == 1 ? da[j] : who == 2 ? db[j] : 0.0;
+    iva[j] = who == 1 ? iva[j] : who == 2 ? ivb[j] : 0.0;
+    code |= (who | ((who == 1 ? ha : hb) ? 4 : 0)) << (3 * j);
   }
+  double sa[5], sb[5], sd[5], o[5];
+  side_flux_reverse<true>(P, A, B, d, L.w[3 * e], L.w[3 * e + 1], L.w[3 * e + 2], dl, sa, sb, sd);
+  double2 *out = reinterpret_cast<double2 *>(abuf2 + LIN_SIDE * (size_t)e);
+  double w[LIN_SIDE];
+  record_share(A, sa, o);
+#pragma unroll
+  for (int c = 0; c < 5; ++c) w[c] = o[c];
+  record_share(B, sb, o);
+#pragma unroll
+  for (int c = 0; c < 5; ++c) {
+    w[19 + c] = o[c];
+    w[5 + c] = sd[c] * da[c];
+    w[10 + c] = sd[c] * iva[c];
+  }
+  w[15] = dx;
+  w[16] = dy;
+  w[17] = dz;
+  w[18] = double(code);
+#pragma unroll
+  for (int c = 0; c < LIN_SIDE / 2; ++c) out[c] = make_double2(w[2 * c], w[2 * c + 1]);
 }
 
 // per node: ub = its conserved-state shares (sides and boundary sides),
-// gbn = its gradient and bound shares
+// gbn = its gradient and bound shares.  SCALED: the gradients' divided by the
+// node's volume and the bounds' times their squares, GREC words a node, as
+// k_grad_adjoint reads its neighbours'.
+template <bool SCALED, int SUB>
 __global__ __launch_bounds__(NTHR) void k_adjoint_gather2(LevelDev<double> L, const double *abuf2, double *ub, double *gbn) {
-  int i = gtid_x();
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
   if (i >= L.n) return;
   double r[5] = {0, 0, 0, 0, 0}, g[LIN_G];
 #pragma unroll
   for (int c = 0; c < LIN_G; ++c) g[c] = 0;
-  for_edges<1>(L, i, 0, [&](int e, int role) {
-    const double *a = abuf2 + LIN_SIDE * (size_t)e;
+  for_edges<SUB>(L, i, sub, [&](int e, int role) {
+    const double *a = abuf2 + LIN_SIDE * (size_t)e, *u = a + 19 * role;
+    const double hx = 0.5 * a[15], hy = 0.5 * a[16], hz = 0.5 * a[17];
+    const int code = int(a[18]);
 #pragma unroll
-    for (int c = 0; c < 5; ++c) r[c] += a[5 * role + c];
-#pragma unroll
-    for (int c = 0; c < LIN_G; ++c) g[c] += a[10 + LIN_G * role + c];
+    for (int c = 0; c < 5; ++c) {
+      r[c] += u[c];
+      const int k = code >> (3 * c);
+      const bool mine = (k & 3) == role + 1;
+      const double v = mine ? a[5 + c] : 0.0, b = mine ? a[10 + c] : 0.0;
+      g[c] += v * hx;
+      g[5 + c] += v * hy;
+      g[10 + c] += v * hz;
+      g[15 + c] += k & 4 ? 0.0 : b;
+      g[20 + c] += k & 4 ? b : 0.0;
+    }
   });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
+  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
     int v = L.bs_list[k];
     const double *b = L.bbuf + 10 * (size_t)(v >> 1) + 5 * (v & 1);
 #pragma unroll
     for (int c = 0; c < 5; ++c) r[c] += b[c];
   }
 #pragma unroll
-  for (int c = 0; c < 5; ++c) ub[5 * (size_t)i + c] = r[c];
+  for (int c = 0; c < 5; ++c) r[c] = lsum<SUB>(r[c]);
 #pragma unroll
-  for (int c = 0; c < LIN_G; ++c) gbn[LIN_G * (size_t)i + c] = g[c];
+  for (int c = 0; c < LIN_G; ++c) g[c] = lsum<SUB>(g[c]);
+  if (sub) return;
+#pragma unroll
+  for (int c = 0; c < 5; ++c) ub[5 * (size_t)i + c] = r[c];
+  if constexpr (SCALED) {
+    const double iv = 1.0 / L.vol[i], *B = L.grec + GREC * (size_t)i;
+    double *o = gbn + GREC * (size_t)i;
+#pragma unroll
+    for (int c = 0; c < 15; ++c) o[c] = g[c] * iv;
+#pragma unroll
+    for (int c = 15; c < LIN_G; ++c) o[c] = g[c] * B[c] * B[c];
+  } else {
+#pragma unroll
+    for (int c = 0; c < LIN_G; ++c) gbn[LIN_G * (size_t)i + c] = g[c];
+  }
 }
 
 // transpose of the gradient and bounds: qb[5 j + c] = sum over the G and B
-// that q_j(c) enters of their shares times d(G, B)/dq_j(c)
+// that q_j(c) enters of their shares times d(G, B)/dq_j(c); gbn as
+// k_adjoint_gather2<true> scales it, so a neighbour costs its 15 gradient
+// shares, its ten extremal-neighbour indices and a bound's share only where
+// node j attains it (with the raw shares, the volumes and the bounds read per
+// neighbour it took 462 us at 64^3, 161 now).
+template <int SUB>
 __global__ __launch_bounds__(NTHR) void k_grad_adjoint(LevelDev<double> L, const double *gbn, const int *amin, double *qb) {
-  int j = gtid_x();
+  int j, sub, bb_;
+  node_lanes<SUB>(1, bb_, j, sub);
   if (j >= L.n) return;
-  double r[5] = {0, 0, 0, 0, 0}, sw[3] = {0, 0, 0};
-  const double *gj = gbn + LIN_G * (size_t)j;
+  double r[5] = {0, 0, 0, 0, 0}, s[3] = {0, 0, 0};
+  const double *gj = gbn + GREC * (size_t)j;
   // neighbours i: G_i holds (q_i + q_j) w_s(i -> j) / V_i with w_s(i -> j) = -w_s(j -> i)
-  for_edges_w<1>(L, j, 0, [&](int i, double wx, double wy, double wz) {
-    sw[0] += wx;
-    sw[1] += wy;
-    sw[2] += wz;
-    const double *gi = gbn + LIN_G * (size_t)i;
-    const double *Bi = L.grec + GREC * (size_t)i;
-    double iv = 1.0 / L.vol[i];
+  for_edges_w<SUB>(L, j, sub, [&](int i, double wx, double wy, double wz) {
+    s[0] += wx;
+    s[1] += wy;
+    s[2] += wz;
+    const double *gi = gbn + GREC * (size_t)i;
+    double g[16];
+    ldrec<16>(gi, g);
+    const int2 *am = reinterpret_cast<const int2 *>(amin + 10 * (size_t)i);
+    int k[10];
 #pragma unroll
     for (int c = 0; c < 5; ++c) {
-      r[c] -= (gi[c] * wx + gi[5 + c] * wy + gi[10 + c] * wz) * iv;
-      if (amin[10 * (size_t)i + c] == j) r[c] -= gi[15 + c] * Bi[15 + c] * Bi[15 + c];
-      if (amin[10 * (size_t)i + 5 + c] == j) r[c] -= gi[20 + c] * Bi[20 + c] * Bi[20 + c];
+      int2 t = am[c];
+      k[2 * c] = t.x;
+      k[2 * c + 1] = t.y;
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      r[c] -= g[c] * wx + g[5 + c] * wy + g[10 + c] * wz;
+      if (k[c] == j) r[c] -= gi[15 + c];
+      if (k[5 + c] == j) r[c] -= gi[20 + c];
     }
   });
   // boundary sides: G_j holds (3 q_j + q_o) w_b / V_j and G_o (3 q_o + q_j) w_b / V_o
-  double sb[3] = {0, 0, 0};
-  for (int k = L.bs_ptr[j]; k < L.bs_ptr[j + 1]; ++k) {
-    int v = L.bs_list[k], s = v >> 1;
-    int o = (v & 1) ? L.ba[s] : L.bb[s];
-    double wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
-    sb[0] += wx;
-    sb[1] += wy;
-    sb[2] += wz;
-    const double *go = gbn + LIN_G * (size_t)o;
-    double iv = 1.0 / L.vol[o];
+  for (int k = L.bs_ptr[j] + sub; k < L.bs_ptr[j + 1]; k += SUB) {
+    int v = L.bs_list[k], b = v >> 1;
+    int o = (v & 1) ? L.ba[b] : L.bb[b];
+    double wx = L.wb[3 * b], wy = L.wb[3 * b + 1], wz = L.wb[3 * b + 2];
+    s[0] += 3.0 * wx;
+    s[1] += 3.0 * wy;
+    s[2] += 3.0 * wz;
+    const double *go = gbn + GREC * (size_t)o;
 #pragma unroll
-    for (int c = 0; c < 5; ++c) r[c] += (go[c] * wx + go[5 + c] * wy + go[10 + c] * wz) * iv;
+    for (int c = 0; c < 5; ++c) r[c] += go[c] * wx + go[5 + c] * wy + go[10 + c] * wz;
   }
-  const double *Bj = L.grec + GREC * (size_t)j;
-  double iv = 1.0 / L.vol[j];
-  double s0 = sw[0] + 3.0 * sb[0], s1 = sw[1] + 3.0 * sb[1], s2 = sw[2] + 3.0 * sb[2];
+#pragma unroll
+  for (int c = 0; c < 5; ++c) r[c] = lsum<SUB>(r[c]);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) s[c] = lsum<SUB>(s[c]);
+  if (sub) return;
 #pragma unroll
   for (int c = 0; c < 5; ++c) {
-    r[c] += (gj[c] * s0 + gj[5 + c] * s1 + gj[10 + c] * s2) * iv;
-    r[c] += gj[15 + c] * Bj[15 + c] * Bj[15 + c] + gj[20 + c] * Bj[20 + c] * Bj[20 + c];
+    r[c] += gj[c] * s[0] + gj[5 + c] * s[1] + gj[10 + c] * s[2];
+    r[c] += gj[15 + c] + gj[20 + c];
     qb[5 * (size_t)j + c] = r[c];
   }
 }
@@ -2428,94 +2730,71 @@ __global__ __launch_bounds__(NTHR) void k_sa_tangent(LevelDev<double> L, DevPara
 }
 
 // adjoint pass 1: shares of lam^T(-A) on node i's stress record (taub 9)
-// and velocities through the energy flux (ub 3), from its own terms and its
-// neighbours' terms; tau values in taud (pass 1 without tangents)
+// and velocities through the energy flux (ub 3); tau values in taud (pass 1
+// without tangents).  A side's flux is the sum of its ends' own parts, each
+// linear in the weight, so node i's part meets -(lam_i - lam_j) w over its
+// sides and -(3 lam_i + lam_o) w_b over its boundary sides: the walk sums
+// those 4 x 3 numbers, and the shares follow from the node's own stress and
+// velocity.  (Twelve dual passes of each side's flux at both ends took 489 us
+// at 275k nodes, 73 now.)
+template <int SUB>
 __global__ __launch_bounds__(NTHR) void k_visc_adjoint_tau(LevelDev<double> L, DevParams P, const double *lam, const ad::Dual *taud,
                                    double *taub, double *ubv) {
-  using ad::Dual;
-  int i = gtid_x();
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
   if (i >= L.n) return;
   const size_t n = L.n;
-  double ti[9], qi[3], mi[4];
+  double li[4], M[4][3];
 #pragma unroll
-  for (int c = 0; c < 9; ++c) ti[c] = taud[9 * (size_t)i + c].v;
-  {
-    const double *q = L.rec0 + 8 * (size_t)i;
-    qi[0] = q[1];
-    qi[1] = q[2];
-    qi[2] = q[3];
+  for (int c = 0; c < 4; ++c) {
+    li[c] = lam[(c + 1) * n + i];
+    M[c][0] = M[c][1] = M[c][2] = 0.0;
   }
+  for_edges_w<SUB>(L, i, sub, [&](int j, double wx, double wy, double wz) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) mi[c] = -lam[(c + 1) * n + i];
-  double tb[9], ub[3];
-#pragma unroll
-  for (int c = 0; c < 9; ++c) tb[c] = 0;
-  ub[0] = ub[1] = ub[2] = 0;
-  // one term's shares on node i's inputs: term = m . F(self first or second)
-  auto shares = [&](const double *to, const double *qo, double wx, double wy, double wz, const double *m,
-                    bool self_first, bool bside) {
-#pragma unroll 1
-    for (int k = 0; k < 12; ++k) {
-      Dual ts[9], tt[9], qs[3], qt[3], a[4] = {Dual(0.0), Dual(0.0), Dual(0.0), Dual(0.0)};
-#pragma unroll
-      for (int c = 0; c < 9; ++c) {
-        ts[c] = Dual(ti[c], k == c ? 1.0 : 0.0);
-        tt[c] = Dual(to[c]);
-      }
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        qs[c] = Dual(qi[c], k == 9 + c ? 1.0 : 0.0);
-        qt[c] = Dual(qo[c]);
-      }
-      if (self_first) {
-        if (bside) visc_bside(ts, tt, qs, qt, wx, wy, wz, a);
-        else visc_edge(ts, tt, qs, qt, wx, wy, wz, a);
-      } else {
-        if (bside) visc_bside(tt, ts, qt, qs, wx, wy, wz, a);
-        else visc_edge(tt, ts, qt, qs, wx, wy, wz, a);
-      }
-      double acc = 0;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) acc += m[c] * a[c].d;
-      if (k < 9) tb[k] += acc;
-      else ub[k - 9] += acc;
+    for (int c = 0; c < 4; ++c) {
+      const double m = lam[(c + 1) * n + j] - li[c];
+      M[c][0] += m * wx;
+      M[c][1] += m * wy;
+      M[c][2] += m * wz;
     }
-  };
-  for_edges_w<1>(L, i, 0, [&](int j, double wx, double wy, double wz) {
-    double tj[9], qj[3], mj[4];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) tj[c] = taud[9 * (size_t)j + c].v;
-    const double *q = L.rec0 + 8 * (size_t)j;
-    qj[0] = q[1];
-    qj[1] = q[2];
-    qj[2] = q[3];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) mj[c] = -lam[(c + 1) * n + j];
-    shares(tj, qj, wx, wy, wz, mi, true, false);     // node i's term, weight w_ij
-    shares(tj, qj, -wx, -wy, -wz, mj, false, false);  // node j's term, weight w_ji = -w_ij
   });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
+  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
     int v = L.bs_list[k], s = v >> 1;
     int ind = L.bind[s];
     if (ind == 2 || ind == 9) continue;
     int o = (v & 1) ? L.ba[s] : L.bb[s];
-    double to[9], qo[3], mo[4];
 #pragma unroll
-    for (int c = 0; c < 9; ++c) to[c] = taud[9 * (size_t)o + c].v;
-    const double *q = L.rec0 + 8 * (size_t)o;
-    qo[0] = q[1];
-    qo[1] = q[2];
-    qo[2] = q[3];
+    for (int c = 0; c < 4; ++c) {
+      const double m = -(3.0 * li[c] + lam[(c + 1) * n + o]);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) mo[c] = -lam[(c + 1) * n + o];
-    const double wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
-    shares(to, qo, wx, wy, wz, mi, true, true);   // node i's boundary term
-    shares(to, qo, wx, wy, wz, mo, false, true);  // the partner's boundary term
+      for (int d = 0; d < 3; ++d) M[c][d] += m * L.wb[3 * s + d];
+    }
   }
 #pragma unroll
-  for (int c = 0; c < 9; ++c) taub[9 * (size_t)i + c] = tb[c];
+  for (int c = 0; c < 4; ++c)
 #pragma unroll
-  for (int c = 0; c < 3; ++c) ubv[3 * (size_t)i + c] = ub[c];
+    for (int d = 0; d < 3; ++d) M[c][d] = lsum<SUB>(M[c][d]);
+  if (sub) return;
+  double t[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) t[c] = taud[9 * (size_t)i + c].v;
+  const double *q = L.rec0 + 8 * (size_t)i;
+  const double u = q[1], v = q[2], w = q[3];
+  const double *E = M[3];  // the energy flux: k grad T + tau . v
+  double *tb = taub + 9 * (size_t)i, *ub = ubv + 3 * (size_t)i;
+  tb[0] = M[0][0] + u * E[0];
+  tb[1] = M[0][1] + M[1][0] + v * E[0] + u * E[1];
+  tb[2] = M[0][2] + M[2][0] + w * E[0] + u * E[2];
+  tb[3] = M[1][1] + v * E[1];
+  tb[4] = M[1][2] + M[2][1] + w * E[1] + v * E[2];
+  tb[5] = M[2][2] + w * E[2];
+  tb[6] = E[0];
+  tb[7] = E[1];
+  tb[8] = E[2];
+  ub[0] = t[0] * E[0] + t[1] * E[1] + t[2] * E[2];
+  ub[1] = t[1] * E[0] + t[3] * E[1] + t[4] * E[2];
+  ub[2] = t[2] * E[0] + t[4] * E[1] + t[5] * E[2];
 }
 
 // adjoint pass 2: the stress law transposed at each node, gbar[12] on the

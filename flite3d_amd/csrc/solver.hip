@@ -304,6 +304,15 @@ int with_lanes(int lanes, F f) {
   }
 }
 
+// f(lanes per node as a constant, grid) with the level's lanes
+template <typename F>
+void launch_nodes(const Level &L, F f) {
+  with_lanes(L.lanes, [&](auto sc) {
+    f(sc, dim3(nblk((long long)L.n * decltype(sc)::value)));
+    return 0;
+  });
+}
+
 int check_launch() {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(FLITE_E_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
@@ -2413,7 +2422,10 @@ int visc_adjoint(flite_ctx *c, Level &L) {
   Vlin S(L);
   dim3 g(nblk(L.n)), b(NTHR);
   hipLaunchKernelGGL(k_visc_tangent_node, g, b, 0, c->stream, V, P, (const double *)nullptr, S.taud, (ad::Dual *)nullptr);
-  hipLaunchKernelGGL(k_visc_adjoint_tau, g, b, 0, c->stream, V, P, V.src, (const ad::Dual *)S.taud, S.taub, S.ubv);
+  launch_nodes(L, [&](auto sc, dim3 gl) {
+    hipLaunchKernelGGL(k_visc_adjoint_tau<decltype(sc)::value>, gl, b, 0, c->stream, V, P, V.src,
+                       (const ad::Dual *)S.taud, S.taub, S.ubv);
+  });
   hipLaunchKernelGGL(k_visc_adjoint_node, g, b, 0, c->stream, V, P, V.src, (const double *)S.taub, S.gbar, S.tbar,
                      S.rnbar, (double *)nullptr);
   if (P.sa)
@@ -2449,7 +2461,10 @@ int visc_mesh_adjoint(flite_ctx *c, Level &L) {
   const size_t ns = 3 * ((size_t)std::max(1, L.ne) + (size_t)std::max(1, L.nbs));
   hipLaunchKernelGGL(k_fill<double>, dim3(nblk((long long)ns)), dim3(NTHR), 0, c->stream, L.vmesh, 0.0, ns);
   hipLaunchKernelGGL(k_visc_tangent_node, g, b, 0, c->stream, V, P, (const double *)nullptr, S.taud, (ad::Dual *)nullptr);
-  hipLaunchKernelGGL(k_visc_adjoint_tau, g, b, 0, c->stream, V, P, V.src, (const ad::Dual *)S.taud, S.taub, S.ubv);
+  launch_nodes(L, [&](auto sc, dim3 gl) {
+    hipLaunchKernelGGL(k_visc_adjoint_tau<decltype(sc)::value>, gl, b, 0, c->stream, V, P, V.src,
+                       (const ad::Dual *)S.taud, S.taub, S.ubv);
+  });
   hipLaunchKernelGGL(k_visc_adjoint_node, g, b, 0, c->stream, V, P, V.src, (const double *)S.taub, S.gbar, S.tbar,
                      S.rnbar, S.mbar);
   if (P.sa)
@@ -2591,7 +2606,7 @@ int adjoint_core(flite_ctx *c) {
     if (!L.abuf2) TRY(L.pool.alloc(&L.abuf2, (size_t)LIN_SIDE * std::max(1, L.ne)));
     DevParams P = c->P;
     LevelDev<double> V = L.view<double>();
-    double *ub = L.lin, *gbn = L.lin + 5 * (size_t)L.n, *qb = L.lin + 30 * (size_t)L.n;
+    double *gbn = L.lin, *ub = L.lin + GREC * (size_t)L.n, *qb = L.lin + (GREC + 5) * (size_t)L.n;
     hipLaunchKernelGGL(k_minmax_arg, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, L.amin);
     if (L.ne > 0) {
       if (P.nsig == 4)
@@ -2600,12 +2615,16 @@ int adjoint_core(flite_ctx *c) {
         hipLaunchKernelGGL(k_flux_adjoint2<2>, dim3(nblk(L.ne)), dim3(NTHR), 0, c->stream, V, P, V.src, L.abuf2);
     }
     if (L.nbs > 0) hipLaunchKernelGGL(k_bflux_adjoint, dim3(nblk(L.nbs)), dim3(NTHR), 0, c->stream, V, P, V.src);
-    hipLaunchKernelGGL(k_adjoint_gather2, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, (const double *)L.abuf2, ub, gbn);
-    hipLaunchKernelGGL(k_grad_adjoint, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, (const double *)gbn,
-                       (const int *)L.amin, qb);
-    hipLaunchKernelGGL(k_record_adjoint, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, P, (const double *)ub,
-                       (const double *)qb, V.rhs);
-    if (P.sa) hipLaunchKernelGGL(k_sa_conv_adjoint, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, P, V.src, V.rhs);
+    launch_nodes(L, [&](auto sc, dim3 gl) {
+      constexpr int SUB = decltype(sc)::value;
+      hipLaunchKernelGGL((k_adjoint_gather2<true, SUB>), gl, dim3(NTHR), 0, c->stream, V, (const double *)L.abuf2, ub,
+                         gbn);
+      hipLaunchKernelGGL(k_grad_adjoint<SUB>, gl, dim3(NTHR), 0, c->stream, V, (const double *)gbn,
+                         (const int *)L.amin, qb);
+      hipLaunchKernelGGL(k_record_adjoint, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, P, (const double *)ub,
+                         (const double *)qb, V.rhs);
+      if (P.sa) hipLaunchKernelGGL(k_sa_conv_adjoint<SUB>, gl, dim3(NTHR), 0, c->stream, V, P, V.src, V.rhs);
+    });
     TRY(check_launch());
     if (laminar(c)) TRY(visc_adjoint(c, L));
     return 0;
@@ -2615,11 +2634,15 @@ int adjoint_core(flite_ctx *c) {
   LevelDev<double> V = L.view<double>();
   if (L.ne > 0) hipLaunchKernelGGL(k_flux_adjoint, dim3(nblk(L.ne)), dim3(NTHR), 0, c->stream, V, P, V.src, L.abuf);
   if (L.nbs > 0) hipLaunchKernelGGL(k_bflux_adjoint, dim3(nblk(L.nbs)), dim3(NTHR), 0, c->stream, V, P, V.src);
-  hipLaunchKernelGGL(k_adjoint_gather, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, L.abuf, V.rhs);
-  if (P.sa) hipLaunchKernelGGL(k_sa_conv_adjoint, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, P, V.src, V.rhs);
+  if (P.sa) TRY(op_prep(c, L, true));  // the SA convection reads the records
+  launch_nodes(L, [&](auto sc, dim3 gl) {
+    constexpr int SUB = decltype(sc)::value;
+    hipLaunchKernelGGL(k_adjoint_gather<SUB>, gl, dim3(NTHR), 0, c->stream, V, (const double *)L.abuf, V.rhs);
+    if (P.sa) hipLaunchKernelGGL(k_sa_conv_adjoint<SUB>, gl, dim3(NTHR), 0, c->stream, V, P, V.src, V.rhs);
+  });
   TRY(check_launch());
   if (laminar(c)) {
-    TRY(op_prep(c, L, true));
+    if (!P.sa) TRY(op_prep(c, L, true));
     TRY(visc_adjoint(c, L));
   }
   return 0;
@@ -2863,7 +2886,10 @@ int flite_mesh_adjoint(flite_ctx *c, const double *lam, int ld_lam, double *gw, 
       hipLaunchKernelGGL(k_flux_adjoint2<2>, dim3(nblk(ne)), dim3(NTHR), 0, c->stream, V, P, V.src, L.abuf2);
   }
   if (nbs > 0) hipLaunchKernelGGL(k_bflux_adjoint, dim3(nblk(nbs)), dim3(NTHR), 0, c->stream, V, P, V.src);
-  hipLaunchKernelGGL(k_adjoint_gather2, dim3(nblk(n)), dim3(NTHR), 0, c->stream, V, (const double *)L.abuf2, ub, gbn);
+  launch_nodes(L, [&](auto sc, dim3 gl) {
+    hipLaunchKernelGGL((k_adjoint_gather2<false, decltype(sc)::value>), gl, dim3(NTHR), 0, c->stream, V,
+                       (const double *)L.abuf2, ub, gbn);
+  });
   if (ne > 0) {
     if (P.nsig == 4)
       hipLaunchKernelGGL(k_flux_mesh_adjoint2<4>, dim3(nblk(ne)), dim3(NTHR), 0, c->stream, V, P, V.src,
