@@ -28,9 +28,14 @@ namespace fk {
 
 constexpr int SLICE = 64;
 constexpr int GREC = 26;
-// viscous record per node: stress 6 + k grad T 3 | grad nu~ 3 + cb2 term | pad,
-// 16 values = one 128-byte line, so a neighbour's tau and grad nu~ come in
-// one cache line (tau at offset 0, dnu at offset 9)
+// viscous record per node: a side's viscous and SA-diffusion fluxes are
+// w.(node's own part + the other's), so the record holds those parts, all that
+// a neighbour reads, in one 128-byte line: stress 6 | energy flux k grad T +
+// tau.v 3 | diffusion flux (Re mu/rho + nu~) grad nu~ 3 | the SA time step's
+// viscosity | nodal cb2 term | pad.  (Stress, velocity, grad nu~ and the
+// diffusion coefficient's three factors took this line and the neighbour's
+// gather record: the second pass, staged, took 838 us with the SA time steps
+// and 767 without on 2.1M nodes, 601 and 441 now.)
 constexpr int VREC = 16;
 constexpr int NTHR = 256;
 
@@ -135,7 +140,7 @@ struct LevelDev {
   const R *vol, *xyz, *wd, *nrm;  // nrm: 3 per node AoS
   const int *ncls;
   R *u, *uprev, *rhs, *diss, *src, *p, *dt, *dtt, *mu, *vort, *divg, *tdiff;
-  R *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;  // tau, dnu: VREC-strided, one shared record
+  R *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;  // tau, dnu = tau + 9: VREC-strided, one shared record
   R *rec1;  // the next state's gather records while a walking stage reads rec0 (null: no such stage)
   R *jst;  // JST node record (8 per node): L(U) 5, pressure switch, side count, volume / time step
   R *uold, *uold2;  // solutions at the last two physical times (6 per node, unsteady only)
@@ -397,17 +402,23 @@ __device__ __forceinline__ void fb_stage(R *sn, const R *src, const int *nodes, 
   }
 }
 
-// Neighbour walks of node i: f(qj, tj, wx, wy, wz) per interior side with
-// qj the neighbour's gather record (8 words, in registers), tj its viscous
-// record and w the node-signed side weights.  walk_global reads the
-// neighbours' records from memory; walk_staged from the LDS slots a node
-// block staged (words 0..7 gather record, 8.. viscous record).
-template <int SUB, typename R, typename F>
+// Neighbour walks of node i: f(qj, tj, wx, wy, wz) per interior side with w
+// the node-signed side weights and either qj the neighbour's gather record
+// (AUXW = 0) or tj the first AUXW words of its viscous record, in registers.
+// walk_global reads the neighbours' records from memory; walk_staged the
+// viscous records from the LDS slots a node block staged.
+template <int SUB, int AUXW = 0, typename R, typename F>
 __device__ __forceinline__ void walk_global(const LevelDev<R> &L, int i, int sub, F f) {
   for_edges_w<SUB>(L, i, sub, [&](int j, R wx, R wy, R wz) {
-    R qj[8];
-    ldrec<8>(L.rec0 + 8 * (size_t)j, qj);
-    f(qj, L.tau + VREC * (size_t)j, wx, wy, wz);
+    if constexpr (AUXW == 0) {
+      R qj[8];
+      ldrec<8>(L.rec0 + 8 * (size_t)j, qj);
+      f(qj, (const R *)nullptr, wx, wy, wz);
+    } else {
+      R tj[AUXW];
+      ldrec<AUXW>(L.tau + VREC * (size_t)j, tj);
+      f((const R *)nullptr, tj, wx, wy, wz);
+    }
   });
 }
 template <int SUB, int S, typename R, typename F>
@@ -419,11 +430,7 @@ __device__ __forceinline__ void walk_staged(const LevelDev<R> &L, const R *sn, i
     int slot = base + k * SLICE + lane;
     unsigned loc = ldnt(L.ell_loc + slot);
     if (loc == 0xffffu) continue;
-    const R *q = sn + loc * S;
-    R qj[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) qj[c] = q[c];
-    f(qj, q + 8, ldnt(L.ellw + slot), ldnt(L.ellw + ns + slot), ldnt(L.ellw + 2 * ns + slot));
+    f((const R *)nullptr, sn + loc * S, ldnt(L.ellw + slot), ldnt(L.ellw + ns + slot), ldnt(L.ellw + 2 * ns + slot));
   }
 }
 
@@ -437,18 +444,8 @@ __device__ __forceinline__ void walk_staged(const LevelDev<R> &L, const R *sn, i
 constexpr int GB_SUB = 4;
 constexpr int GB_NODES = NTHR / GB_SUB;
 constexpr int GB_CAP = 288;
-constexpr int GB_AUX = 12;  // viscous-record words staged: stress 6 + k grad T 3 + grad nu~ 3
 
-template <typename R, int S, bool AUX>
-__device__ __forceinline__ bool gb_stage(const LevelDev<R> &L, R *sn, int blk) {
-  if (blk >= L.ngb) return false;
-  const int n0 = L.gb_nptr[blk], nn = L.gb_nptr[blk + 1] - n0;
-  const int *nodes = L.gb_node + n0;
-  fb_stage<GB_CAP, 8, 8, 0, S>(sn, L.rec0, nodes, nn);
-  if constexpr (AUX) fb_stage<GB_CAP, GB_AUX, VREC, 8, S>(sn, L.tau, nodes, nn);
-  return true;
-}
-
+// ---------------------------------------------------------------------------
 // node preparation: makePressureField (DEF:13612-13630) + gather records
 // ---------------------------------------------------------------------------
 template <typename R>
@@ -537,7 +534,7 @@ __global__ void k_pack(LevelDev<R> L, DevParams P) {
 // kernels walk it alone.
 template <typename R>
 struct GradPart {
-  static constexpr bool AUX = false;
+  static constexpr int AUXW = 0;
   R q0[5], g[15], mn[5], mx[5];
   __device__ void init(const LevelDev<R> &, const DevParams &, int, const R *qi) {
 #pragma unroll
@@ -3307,7 +3304,7 @@ __global__ void k_drag_state_gradient(LevelDev<double> L, DevParams P, const int
 // ---------------------------------------------------------------------------
 template <typename R>
 struct NoPart {
-  static constexpr bool AUX = false;  // reads the neighbours' viscous records
+  static constexpr int AUXW = 0;  // words read of the neighbours' viscous records (0: reads the gather records)
   __device__ void init(const LevelDev<R> &, const DevParams &, int, const R *) {}
   __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *, const R *, R, R, R) {}
   __device__ void bside(const LevelDev<R> &, const DevParams &, const R *, int, int, int, const R *, R, R, R) {}
@@ -3319,7 +3316,7 @@ struct NoPart {
 // makeTimeSteps (DEF:13335-13610)
 template <typename R>
 struct TimeStepPart {
-  static constexpr bool AUX = false;
+  static constexpr int AUXW = 0;
   R lam, lamv, cc, am, gam;
   bool visc;
   // a state's convective speed through a face: |w.v| + |w| c
@@ -3379,13 +3376,12 @@ struct TimeStepPart {
 
 // makeViscosityTerm (DEF:5198-5893), pass 1: gradients of (u,v,w,T) and the
 // node loop (Sutherland, SA eddy viscosity, stress, heat flux, vorticity,
-// divergence, adiabatic wall, wall stress).  tau: stress 6 + k grad T 3.
-// WRITE_REC also stores the new laminar viscosity in the gather record;
-// when fused with makeTimeSteps (which reads the neighbours' previous one)
-// that store is left to k_mu_record after the pass.
-template <typename R, bool WRITE_REC>
+// divergence, adiabatic wall, wall stress).  tau: stress 6 + energy flux 3.
+// The gather records keep the previous laminar viscosity, which makeTimeSteps
+// reads of the neighbours in the same walk.
+template <typename R>
 struct ViscNodePart {
-  static constexpr bool AUX = false;
+  static constexpr int AUXW = 0;
   R gog1, ai[4], g[12];
   __device__ void init(const LevelDev<R> &, const DevParams &P, int, const R *qi) {
     gog1 = R(P.gamma / (P.gamma - 1.0));
@@ -3430,7 +3426,6 @@ struct ViscNodePart {
     R mu = R(1.0 / P.Re) * ((tct * sqrt(tct)) * ((Tin + R(198.6)) / (tc * Tin * T + R(198.6))));
     R k = R(1.0 / P.Pr) * mu;
     L.mu[i] = mu;
-    if (WRITE_REC) L.rec0[8 * (size_t)i + 7] = mu;
     L.vort[i] = sqrt((dudy - dvdx) * (dudy - dvdx) + (dvdz - dwdy) * (dvdz - dwdy) + (dwdx - dudz) * (dwdx - dudz));
     L.divg[i] = dudx + dvdy + dwdz;
     if (P.sa) {
@@ -3465,6 +3460,9 @@ struct ViscNodePart {
       L.ws[3 * (size_t)i + 1] = t[1] * nx + t[3] * ny + t[4] * nz;
       L.ws[3 * (size_t)i + 2] = t[2] * nx + t[4] * ny + t[5] * nz;
     }
+    t[6] += ai[0] * t[0] + ai[1] * t[1] + ai[2] * t[2];
+    t[7] += ai[0] * t[1] + ai[1] * t[3] + ai[2] * t[4];
+    t[8] += ai[0] * t[2] + ai[1] * t[4] + ai[2] * t[5];
     R *o = L.tau + VREC * (size_t)i;
 #pragma unroll
     for (int c = 0; c < 9; ++c) o[c] = t[c];
@@ -3474,49 +3472,35 @@ struct ViscNodePart {
 // makeViscosityTerm pass 2 (DEF:5640-5893): dissipation(:,2:5) = -sum
 template <typename R>
 struct ViscFluxPart {
-  static constexpr bool AUX = true;
-  R t1[9], u1, v1, w1, a[4];
-  __device__ void init(const LevelDev<R> &L, const DevParams &, int i, const R *qi) {
+  static constexpr int AUXW = 10;
+  R t1[9], a[4];
+  __device__ void init(const LevelDev<R> &L, const DevParams &, int i, const R *) {
     const R *ti = L.tau + VREC * (size_t)i;
 #pragma unroll
     for (int c = 0; c < 9; ++c) t1[c] = ti[c];
-    u1 = qi[1];
-    v1 = qi[2];
-    w1 = qi[3];
 #pragma unroll
     for (int c = 0; c < 4; ++c) a[c] = 0;
   }
-  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *tj, const R *qj, R wx, R wy,
-                       R wz) {
-    R u2 = qj[1], v2 = qj[2], w2 = qj[3];
-    R d[9];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) d[c] = t1[c] + tj[c];
-    R dut1 = u1 * t1[0] + u2 * tj[0] + v1 * t1[1] + v2 * tj[1] + w1 * t1[2] + w2 * tj[2];
-    R dut2 = u1 * t1[1] + u2 * tj[1] + v1 * t1[3] + v2 * tj[3] + w1 * t1[4] + w2 * tj[4];
-    R dut3 = u1 * t1[2] + u2 * tj[2] + v1 * t1[4] + v2 * tj[4] + w1 * t1[5] + w2 * tj[5];
+  __device__ __forceinline__ void add(const R *d, R wx, R wy, R wz) {
     a[0] += wx * d[0] + wy * d[1] + wz * d[2];
     a[1] += wx * d[1] + wy * d[3] + wz * d[4];
     a[2] += wx * d[2] + wy * d[4] + wz * d[5];
-    a[3] += wx * (d[6] + dut1) + wy * (d[7] + dut2) + wz * (d[8] + dut3);
+    a[3] += wx * d[6] + wy * d[7] + wz * d[8];
   }
-  __device__ void bside(const LevelDev<R> &L, const DevParams &, const R *, int, int o, int ind, const R *qo, R wx,
-                        R wy, R wz) {
-    if (ind == 2 || ind == 9) return;  // symmetry / inviscid wall carry no viscous flux
-    const R *to = L.tau + VREC * (size_t)o;
-    R u2 = qo[1], v2 = qo[2], w2 = qo[3];
+  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *tj, const R *, R wx, R wy, R wz) {
     R d[9];
 #pragma unroll
-    for (int c = 0; c < 9; ++c) d[c] = t1[c] + to[c];
-    R du11 = u1 * t1[0] + v1 * t1[1] + w1 * t1[2], du12 = u2 * to[0] + v2 * to[1] + w2 * to[2];
-    R du21 = u1 * t1[1] + v1 * t1[3] + w1 * t1[4], du22 = u2 * to[1] + v2 * to[3] + w2 * to[4];
-    R du31 = u1 * t1[2] + v1 * t1[4] + w1 * t1[5], du32 = u2 * to[2] + v2 * to[4] + w2 * to[5];
-    R dut1 = du11 + du12, dut2 = du21 + du22, dut3 = du31 + du32;
-    a[0] += (wx * d[0] + wy * d[1] + wz * d[2]) + R(2) * (wx * t1[0] + wy * t1[1] + wz * t1[2]);
-    a[1] += (wx * d[1] + wy * d[3] + wz * d[4]) + R(2) * (wx * t1[1] + wy * t1[3] + wz * t1[4]);
-    a[2] += (wx * d[2] + wy * d[4] + wz * d[5]) + R(2) * (wx * t1[2] + wy * t1[4] + wz * t1[5]);
-    a[3] += (wx * (d[6] + dut1) + wy * (d[7] + dut2) + wz * (d[8] + dut3)) +
-            R(2) * (wx * (t1[6] + du11) + wy * (t1[7] + du21) + wz * (t1[8] + du31));
+    for (int c = 0; c < 9; ++c) d[c] = t1[c] + tj[c];
+    add(d, wx, wy, wz);
+  }
+  __device__ void bside(const LevelDev<R> &L, const DevParams &, const R *, int, int o, int ind, const R *, R wx, R wy,
+                        R wz) {
+    if (ind == 2 || ind == 9) return;  // symmetry / inviscid wall carry no viscous flux
+    const R *to = L.tau + VREC * (size_t)o;
+    R d[9];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) d[c] = (t1[c] + to[c]) + R(2) * t1[c];
+    add(d, wx, wy, wz);
   }
   template <int SUB>
   __device__ void reduce() {
@@ -3534,34 +3518,36 @@ struct ViscFluxPart {
 };
 
 // makeTurbulentTimeSteps (DEF:12878-13099)
+// its viscosity 1.5 (mu + 3 cb2 nu~ / Re) comes from the viscous records
+// (sa_step_viscosity, SADiff1Part)
+template <typename R>
+__device__ __forceinline__ R sa_step_viscosity(const DevParams &P, R mu, R nu) {
+  return R(1.5) * (mu + R(3) * R(0.622) * nu * R(1.0 / P.Re));
+}
 template <typename R>
 struct SATimeStepPart {
-  static constexpr bool AUX = false;
-  R ioRe, oos, cb2, tk, lam, lamv;
-  __device__ void init(const LevelDev<R> &, const DevParams &P, int, const R *) {
-    ioRe = R(1.0 / P.Re);
-    oos = R(1.5);
-    cb2 = R(0.622);
+  static constexpr int AUXW = 14;
+  R tk, lam, lamv, self;
+  __device__ void init(const LevelDev<R> &L, const DevParams &P, int i, const R *) {
     tk = R(P.turb_k);
+    self = L.tau[VREC * (size_t)i + 12];
     lam = 0;
     lamv = 0;
   }
-  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *qi, const R *, const R *qj, R wx, R wy,
-                       R wz) {
+  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *qi, const R *tj, const R *, R wx, R wy, R wz) {
     R al = wx * wx + wy * wy + wz * wz;
     R vn = wx * qi[1] + wy * qi[2] + wz * qi[3];
     lam += tk * sqrt(al) + fabs(vn);
-    R vis = oos * (qj[7] + R(3) * cb2 * qj[6] * ioRe);
-    lamv += R(2) * vis * al;
+    lamv += R(2) * tj[12] * al;
   }
-  __device__ void bside(const LevelDev<R> &, const DevParams &, const R *qi, int, int, int, const R *qo, R wx, R wy,
+  __device__ void bside(const LevelDev<R> &L, const DevParams &P, const R *qi, int, int o, int, const R *, R wx, R wy,
                         R wz) {
+    const R *qo = L.rec0 + 8 * (size_t)o;
     R al = wx * wx + wy * wy + wz * wz;
     R vn1 = tk * sqrt(al) + fabs(wx * qi[1] + wy * qi[2] + wz * qi[3]);
     R vn2 = tk * sqrt(al) + fabs(wx * qo[1] + wy * qo[2] + wz * qo[3]);
     lam += vn1 + (vn1 + vn2);
-    R dv1 = R(2) * (oos * (qi[7] + R(3) * cb2 * qi[6] * ioRe)) * al;
-    R dv2 = R(2) * (oos * (qo[7] + R(3) * cb2 * qo[6] * ioRe)) * al;
+    R dv1 = R(2) * self * al, dv2 = R(2) * L.tau[VREC * (size_t)o + 12] * al;
     lamv += dv1 + (dv1 + dv2);
   }
   template <int SUB>
@@ -3569,25 +3555,38 @@ struct SATimeStepPart {
     lam = lsum<SUB>(lam);
     lamv = lsum<SUB>(lamv);
   }
-  __device__ void finish(const LevelDev<R> &L, const DevParams &, int i, const R *qi) {
+  __device__ void finish(const LevelDev<R> &L, const DevParams &P, int i, const R *qi) {
     R V = L.vol[i];
     R dt = R(0.5) / (lam / V + lamv / (V * V));
     R wd = L.wd[i];
     R di = wd > R(1e-10) ? R(1) / wd : R(1e10);
     di = di * di;
-    R ik2 = R(1.0 / (0.41 * 0.41)), cb1 = R(0.1355), ct3 = R(1.1);
-    R cw1 = cb1 * ik2 + (R(1) + cb2) * oos;
+    R ioRe = R(1.0 / P.Re), ik2 = R(1.0 / (0.41 * 0.41)), cb1 = R(0.1355), ct3 = R(1.1);
+    R cw1 = cb1 * ik2 + (R(1) + R(0.622)) * R(1.5);
     R nu = qi[6];
     R S = fabs(L.divg[i]) + cb1 * (L.vort[i] + (R(1) + ct3) * nu * ik2 * di * ioRe) + cw1 * nu * di * ioRe;
     L.dtt[i] = dt / (R(1) + R(0.5) * S * dt);
   }
 };
 
-// makeSADiffusion (DEF:7436-7808), pass 1: grad nu~ (dnu: 3 + nodal cb2
-// term).  nu~ = u(:,6) is read from the gather records.
+// the SA time step's viscosity alone into the viscous records (parity op)
+template <typename R>
+__global__ void k_sa_step_viscosity(LevelDev<R> L, DevParams P) {
+  int bb_;
+  int i = btid(L.nb, bb_);
+  L.to_batch(bb_);
+  P.to_batch(bb_);
+  if (i >= L.n) return;
+  L.tau[VREC * (size_t)i + 12] = sa_step_viscosity(P, L.mu[i], L.rec0[8 * (size_t)i + 6]);
+}
+
+// makeSADiffusion (DEF:7436-7808), pass 1: grad nu~, into the viscous record
+// as the node's part of the diffusion flux (with the laminar viscosity that
+// pass 1 of the viscous term has just stored), the SA time step's viscosity
+// and the nodal cb2 term.  nu~ = u(:,6) is read from the gather records.
 template <typename R>
 struct SADiff1Part {
-  static constexpr bool AUX = false;
+  static constexpr int AUXW = 0;
   R ti, g[3];
   __device__ void init(const LevelDev<R> &, const DevParams &, int, const R *qi) {
     ti = qi[6];
@@ -3612,54 +3611,49 @@ struct SADiff1Part {
 #pragma unroll
     for (int c = 0; c < 3; ++c) g[c] = lsum<SUB>(g[c]);
   }
-  __device__ void finish(const LevelDev<R> &L, const DevParams &P, int i, const R *) {
+  __device__ void finish(const LevelDev<R> &L, const DevParams &P, int i, const R *qi) {
     R vt = R(1) / L.vol[i];
     R dx = g[0] * vt, dy = g[1] * vt, dz = g[2] * vt;
     R fact = R(1.0 / P.Re * 0.622 / (2.0 / 3.0));
+    R mu = L.mu[i], v = R(P.Re) * mu / qi[0] + ti;
     R *o = L.dnu + VREC * (size_t)i;
-    o[0] = dx;
-    o[1] = dy;
-    o[2] = dz;
-    o[3] = -(fact * (g[0] * dx + g[1] * dy + g[2] * dz));
+    o[0] = v * dx;
+    o[1] = v * dy;
+    o[2] = v * dz;
+    o[3] = sa_step_viscosity(P, mu, ti);
+    o[4] = -(fact * (g[0] * dx + g[1] * dy + g[2] * dz));
   }
 };
 
 // makeSADiffusion pass 2
 template <typename R>
 struct SADiff2Part {
-  static constexpr bool AUX = true;
-  R Re, fact, v1, acc, d0, d1, d2, d3;
-  __device__ void init(const LevelDev<R> &L, const DevParams &P, int i, const R *qi) {
+  static constexpr int AUXW = 12;
+  R fact, acc, d0, d1, d2, d3;
+  __device__ void init(const LevelDev<R> &L, const DevParams &P, int i, const R *) {
     const R *di = L.dnu + VREC * (size_t)i;
     d0 = di[0];
     d1 = di[1];
     d2 = di[2];
-    d3 = di[3];
-    Re = R(P.Re);
+    d3 = di[4];
     fact = R(1.0 / P.Re / (2.0 / 3.0));
-    v1 = Re * qi[7] / qi[0] + qi[6];
     acc = 0;
   }
-  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *tj, const R *qj, R wx, R wy,
-                       R wz) {
-    const R *dj = tj + 9;  // grad nu~ follows the 9 stress words in the viscous record
-    R v2 = Re * qj[7] / qj[0] + qj[6];
-    R fd = v1 * (wx * d0 + wy * d1 + wz * d2) + v2 * (wx * dj[0] + wy * dj[1] + wz * dj[2]);
-    acc -= fact * fd;
+  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *tj, const R *, R wx, R wy, R wz) {
+    acc += wx * (d0 + tj[9]) + wy * (d1 + tj[10]) + wz * (d2 + tj[11]);
   }
-  __device__ void bside(const LevelDev<R> &L, const DevParams &P, const R *, int, int o, int, const R *qo, R wx, R wy,
+  __device__ void bside(const LevelDev<R> &L, const DevParams &P, const R *, int, int o, int, const R *, R wx, R wy,
                         R wz) {
     const R *dq = L.dnu + VREC * (size_t)o;
-    R vo = Re * qo[7] / qo[0] + qo[6];
-    R fd1 = v1 * (wx * d0 + wy * d1 + wz * d2);
-    R fd2 = vo * (wx * dq[0] + wy * dq[1] + wz * dq[2]);
-    acc -= P.bterm == 1 ? fact * (R(3) * fd1 + fd2) : fact * R(4) * fd1;
+    R fd1 = wx * d0 + wy * d1 + wz * d2;
+    R fd2 = wx * dq[0] + wy * dq[1] + wz * dq[2];
+    acc += P.bterm == 1 ? R(3) * fd1 + fd2 : R(4) * fd1;
   }
   template <int SUB>
   __device__ void reduce() {
     acc = lsum<SUB>(acc);
   }
-  __device__ void finish(const LevelDev<R> &L, const DevParams &, int i, const R *) { L.tdiff[i] = acc + d3; }
+  __device__ void finish(const LevelDev<R> &L, const DevParams &, int i, const R *) { L.tdiff[i] = d3 - fact * acc; }
 };
 
 // JST passes 1, 2 and the node step of makeArtificialDissipation2
@@ -3670,7 +3664,7 @@ struct SADiff2Part {
 // makeTimeSteps earlier in the same walk) for the scalar form's scale.
 template <typename R>
 struct JstSumsPart {
-  static constexpr bool AUX = false;
+  static constexpr int AUXW = 0;
   R U[5], p, h[5], h7, h8, conn;
   static __device__ __forceinline__ void state(const R *q, R *u) {
     u[0] = q[0];
@@ -3716,6 +3710,8 @@ struct JstSumsPart {
   }
 };
 
+constexpr int max3(int a, int b, int c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
+
 // one walk of node i's interior and boundary sides feeding up to three parts
 template <typename R, int SUB, typename A, typename B, typename C, typename Walk>
 __device__ __forceinline__ void gather_body(LevelDev<R> &L, const DevParams &P, int i, int sub, Walk walk) {
@@ -3736,7 +3732,7 @@ __device__ __forceinline__ void gather_body(LevelDev<R> &L, const DevParams &P, 
     int o = (v & 1) ? L.ba[s] : L.bb[s];
     int ind = L.bind[s];
     R qo[8];
-    ldrec<8>(L.rec0 + 8 * (size_t)o, qo);
+    if constexpr (max3(A::AUXW, B::AUXW, C::AUXW) == 0) ldrec<8>(L.rec0 + 8 * (size_t)o, qo);
     R wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
     a.bside(L, P, qi, s, o, ind, qo, wx, wy, wz);
     b.bside(L, P, qi, s, o, ind, qo, wx, wy, wz);
@@ -3754,26 +3750,30 @@ __device__ __forceinline__ void gather_body(LevelDev<R> &L, const DevParams &P, 
 }
 
 template <typename R, int SUB, typename A, typename B, typename C>
-__global__ void k_gather(LevelDev<R> L, DevParams P) {
+__global__ __launch_bounds__(NTHR) void k_gather(LevelDev<R> L, DevParams P) {
+  constexpr int W = max3(A::AUXW, B::AUXW, C::AUXW);
   int i, sub;
   int bb_;
   node_lanes<SUB>(L.nb, bb_, i, sub);
   L.to_batch(bb_);
   P.to_batch(bb_);
   if (i >= L.n) return;
-  gather_body<R, SUB, A, B, C>(L, P, i, sub, [&](auto f) { walk_global<SUB>(L, i, sub, f); });
+  gather_body<R, SUB, A, B, C>(L, P, i, sub, [&](auto f) { walk_global<SUB, W>(L, i, sub, f); });
 }
 
 template <typename R, typename A, typename B, typename C>
 __global__ __launch_bounds__(NTHR) void k_gather_blk(LevelDev<R> L, DevParams P) {
-  constexpr bool AUX = A::AUX || B::AUX || C::AUX;
-  constexpr int S = AUX ? 8 + GB_AUX + 1 : 9;  // odd LDS stride in words
+  constexpr int W = max3(A::AUXW, B::AUXW, C::AUXW);
+  static_assert(W > 0, "only viscous records are staged");
+  constexpr int NS = W == 12 ? 12 : W - 1, S = NS | 1;  // words used, an odd LDS stride
   __shared__ R sn[GB_CAP * S];
   int lb = xcd_block();
   int bb_ = lb % L.nb, blk = lb / L.nb;
   L.to_batch(bb_);
   P.to_batch(bb_);
-  if (!gb_stage<R, S, AUX>(L, sn, blk)) return;
+  if (blk >= L.ngb) return;
+  const int n0 = L.gb_nptr[blk], nn = L.gb_nptr[blk + 1] - n0;
+  fb_stage<GB_CAP, W, VREC, 0, S, R, NS>(sn, L.tau, L.gb_node + n0, nn);
   __syncthreads();
   int i = L.gb_first[blk] + (int)threadIdx.x / GB_SUB, sub = (int)threadIdx.x % GB_SUB;
   if (i >= L.gb_first[blk + 1]) return;
@@ -3889,16 +3889,6 @@ __global__ void k_jst_flux(LevelDev<R> L, DevParams P, int add) {
   }
 #pragma unroll
   for (int c = 0; c < 5; ++c) L.diss[c * n + i] = (add ? L.diss[c * n + i] : R(0)) + acc[c];
-}
-
-// new laminar viscosity into the gather records after a fused pass
-template <typename R>
-__global__ void k_mu_record(LevelDev<R> L) {
-  int bb_;
-  int i = btid(L.nb, bb_);
-  L.to_batch(bb_);
-  if (i >= L.n) return;
-  L.rec0[8 * (size_t)i + 7] = L.mu[i];
 }
 
 // ---------------------------------------------------------------------------

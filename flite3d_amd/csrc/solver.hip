@@ -350,9 +350,11 @@ int scratch_setup(int dev) {
 template <typename A, typename B, typename C, typename V>
 void launch_gather(flite_ctx *c, const Level &L, const V &v, const DevParams &P) {
   using R = std::remove_pointer_t<decltype(v.u)>;
-  if (L.ngb > 0 && L.lanes <= 4 && (A::AUX || B::AUX || C::AUX)) {
-    hipLaunchKernelGGL((k_gather_blk<R, A, B, C>), dim3((unsigned)L.ngb * L.nbatch), dim3(NTHR), 0, c->stream, v, P);
-    return;
+  if constexpr (max3(A::AUXW, B::AUXW, C::AUXW) > 0) {
+    if (L.ngb > 0 && L.lanes <= 4) {
+      hipLaunchKernelGGL((k_gather_blk<R, A, B, C>), dim3((unsigned)L.ngb * L.nbatch), dim3(NTHR), 0, c->stream, v, P);
+      return;
+    }
   }
   with_lanes(L.lanes, [&](auto sc) {
     constexpr int SUB = decltype(sc)::value;
@@ -1471,7 +1473,7 @@ int op_viscous(flite_ctx *c, Level &L) {
   Timed tm(c, "viscous", L.gnum);
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
-    launch_gather<ViscNodePart<R, true>, NoPart<R>, NoPart<R>>(c, L, V, P);
+    launch_gather<ViscNodePart<R>, NoPart<R>, NoPart<R>>(c, L, V, P);
     launch_gather<ViscFluxPart<R>, NoPart<R>, NoPart<R>>(c, L, V, P);
     return check_launch();
   });
@@ -1481,6 +1483,7 @@ int op_sa_timesteps(flite_ctx *c, Level &L) {
   DevParams P = c->P;
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
+    hipLaunchKernelGGL(k_sa_step_viscosity<R>, dim3(nblk(L.n) * L.nbatch), dim3(NTHR), 0, c->stream, V, P);
     launch_gather<SATimeStepPart<R>, NoPart<R>, NoPart<R>>(c, L, V, P);
     return check_launch();
   });
@@ -1501,9 +1504,10 @@ int op_sa_diffusion(flite_ctx *c, Level &L) {
 //   pass A: [makeTimeSteps] + makeViscosityTerm pass 1 + [makeSADiffusion pass 1]
 //   pass B: makeViscosityTerm pass 2 + [makeTurbulentTimeSteps] + [makeSADiffusion pass 2]
 // Pass B only needs pass A's node results (mu, tau, vorticity, divergence,
-// grad nu~), which is the dependency order of the separate routines.  With
-// time steps in pass A they read the previous laminar viscosity, so the new
-// one reaches the gather records after the pass (k_mu_record).
+// grad nu~), which is the dependency order of the separate routines, and of a
+// neighbour only its viscous record.  Time steps in pass A read the previous
+// laminar viscosity of the gather records; the new one goes to the viscous
+// records and to L.mu.
 int op_step_terms(flite_ctx *c, Level &L, bool timesteps, bool sa_timesteps) {
   DevParams P = c->P;
   bool sa = P.sa;
@@ -1511,16 +1515,14 @@ int op_step_terms(flite_ctx *c, Level &L, bool timesteps, bool sa_timesteps) {
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
     if (timesteps && sa) {
-      launch_gather<TimeStepPart<R>, ViscNodePart<R, false>, SADiff1Part<R>>(c, L, V, P);
+      launch_gather<TimeStepPart<R>, ViscNodePart<R>, SADiff1Part<R>>(c, L, V, P);
     } else if (timesteps) {
-      launch_gather<TimeStepPart<R>, ViscNodePart<R, false>, NoPart<R>>(c, L, V, P);
+      launch_gather<TimeStepPart<R>, ViscNodePart<R>, NoPart<R>>(c, L, V, P);
     } else if (sa) {
-      launch_gather<ViscNodePart<R, true>, SADiff1Part<R>, NoPart<R>>(c, L, V, P);
+      launch_gather<ViscNodePart<R>, SADiff1Part<R>, NoPart<R>>(c, L, V, P);
     } else {
-      launch_gather<ViscNodePart<R, true>, NoPart<R>, NoPart<R>>(c, L, V, P);
+      launch_gather<ViscNodePart<R>, NoPart<R>, NoPart<R>>(c, L, V, P);
     }
-    if (timesteps)
-      hipLaunchKernelGGL(k_mu_record<R>, dim3(nblk(L.n) * L.nbatch), dim3(NTHR), 0, c->stream, V);
     if (sa && sa_timesteps) {
     launch_gather<ViscFluxPart<R>, SATimeStepPart<R>, SADiff2Part<R>>(c, L, V, P);
     } else if (sa) {
@@ -2511,7 +2513,7 @@ int visc_friction_reverse(flite_ctx *c, Level &L, bool mesh) {
 int wall_stress(flite_ctx *c, Level &L) {
   DevParams P = c->P;
   LevelDev<double> V = L.view<double>();
-  launch_gather<ViscNodePart<double, true>, NoPart<double>, NoPart<double>>(c, L, V, P);
+  launch_gather<ViscNodePart<double>, NoPart<double>, NoPart<double>>(c, L, V, P);
   return check_launch();
 }
 
