@@ -1101,7 +1101,11 @@ __global__ __launch_bounds__(NTHR) void k_bflux(LevelDev<R> L, DevParams P) {
 // sums per node.
 // Every load of a block depends on its header or on nothing: the node list
 // sits at a fixed place per block, so the records are two loads away from
-// the start, and the sides' own words are requested before the staging.
+// the start, and the sides' own words are requested before the staging.  The
+// list goes through LDS, and all three records' loads are requested before
+// the first is stored: reading the list beside every record load and waiting
+// for each record in turn kept 24 reads in flight a CU and took 884 us on
+// 14.8M sides (second order, SA), 656 now; 219 and 165 on 3.6M.
 // BND: blocks spread evenly among the side blocks evaluate the boundary sides,
 // one a thread, instead of a launch of their own (k_bflux).  That saves the
 // launch where it is the cost: us merged / apart, 13.4 / 18 with 19k boundary
@@ -1127,6 +1131,7 @@ __global__ __launch_bounds__(FB_SHAPE_THR[SHAPE]) void k_flux_blk(LevelDev<R> L,
   constexpr int S = fb_stride<ORDER>();
   constexpr int SN = FB_NODES * S > FB_SIDES * FB_SF ? FB_NODES * S : FB_SIDES * FB_SF;
   __shared__ R sn[SN];
+  __shared__ int sid[FB_NODES];
   __shared__ unsigned short sinc[2 * FB_SIDES];
   int lb = xcd_block();
   int bb_ = lb % L.nb, blk = lb / L.nb;
@@ -1147,7 +1152,7 @@ __global__ __launch_bounds__(FB_SHAPE_THR[SHAPE]) void k_flux_blk(LevelDev<R> L,
   const int4 h0 = reinterpret_cast<const int4 *>(L.fb_head)[blk];
   const int4 h1 = reinterpret_cast<const int4 *>(L.fb_head)[blk + 1];
   const int n0 = h0.y, nn = h1.y - h0.y, ibase = h0.z;
-  const int *nodes = L.fb_node + (size_t)blk * FB_NODES;
+  if (threadIdx.x < FB_NODES) sid[threadIdx.x] = L.fb_node[(size_t)blk * FB_NODES + threadIdx.x];
   // this thread's side: its words are requested before the staging
   const int e = h0.x + (int)threadIdx.x;
   const bool active = e < h1.x;
@@ -1176,10 +1181,53 @@ __global__ __launch_bounds__(FB_SHAPE_THR[SHAPE]) void k_flux_blk(LevelDev<R> L,
       if (t < ni) sinc[t] = L.fb_inc[ibase + t];
     }
   }
-  fb_stage<FB_NODES, 8, 8, 0, S, R, FB_REC, FB_THR>(sn, L.rec0, nodes, nn);
-  if constexpr (ORDER > 1) {
-    fb_stage<FB_NODES, GREC, GREC, FB_REC, S, R, GREC - 1, FB_THR>(sn, L.grec, nodes, nn);
-    fb_stage<FB_NODES, 3, 3, FB_REC + GREC - 1, S, R, 3, FB_THR>(sn, L.xyz, nodes, nn);
+  // the nodes' records, all loads in flight before the first goes to LDS
+  __syncthreads();
+  {
+    using P2 = typename Pair<R>::type;
+    const int t = threadIdx.x;
+    constexpr int U0 = 4, U1 = GREC / 2;  // two-word units of the two records
+    constexpr int N0 = (FB_NODES * U0 + FB_THR - 1) / FB_THR;
+    constexpr int N1 = ORDER > 1 ? (FB_NODES * U1 + FB_THR - 1) / FB_THR : 0;
+    constexpr int N2 = ORDER > 1 ? (FB_NODES * 3 + FB_THR - 1) / FB_THR : 0;
+    P2 v0[N0], v1[N1 ? N1 : 1];
+    R v2[N2 ? N2 : 1];
+#pragma unroll
+    for (int q = 0; q < N0; ++q) {
+      const int x = t + q * FB_THR, k = x / U0;
+      if (k < nn) v0[q] = reinterpret_cast<const P2 *>(L.rec0 + 8 * (size_t)sid[k])[x - k * U0];
+    }
+#pragma unroll
+    for (int q = 0; q < N1; ++q) {
+      const int x = t + q * FB_THR, k = x / U1;
+      if (k < nn) v1[q] = reinterpret_cast<const P2 *>(L.grec + GREC * (size_t)sid[k])[x - k * U1];
+    }
+#pragma unroll
+    for (int q = 0; q < N2; ++q) {
+      const int x = t + q * FB_THR, k = x / 3;
+      if (k < nn) v2[q] = L.xyz[3 * (size_t)sid[k] + (x - 3 * k)];
+    }
+#pragma unroll
+    for (int q = 0; q < N0; ++q) {
+      const int x = t + q * FB_THR, k = x / U0, j = x - k * U0;
+      if (k < nn) {
+        sn[k * S + 2 * j] = v0[q].x;
+        if (2 * j + 1 < FB_REC) sn[k * S + 2 * j + 1] = v0[q].y;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < N1; ++q) {
+      const int x = t + q * FB_THR, k = x / U1, j = x - k * U1;
+      if (k < nn) {
+        sn[k * S + FB_REC + 2 * j] = v1[q].x;
+        if (2 * j + 1 < GREC - 1) sn[k * S + FB_REC + 2 * j + 1] = v1[q].y;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < N2; ++q) {
+      const int x = t + q * FB_THR, k = x / 3;
+      if (k < nn) sn[k * S + FB_REC + GREC - 1 + (x - 3 * k)] = v2[q];
+    }
   }
   __syncthreads();
   R fo[6];
