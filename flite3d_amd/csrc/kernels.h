@@ -368,39 +368,6 @@ __device__ __forceinline__ void for_edges_w(const LevelDev<R> &L, int i, int sub
 template <typename R> struct Pair;
 template <> struct Pair<double> { using type = double2; };
 template <> struct Pair<float> { using type = float2; };
-// one staging pass: the first NS (default NW) of the NW words at src +
-// STRIDE*g of each of the nn (<= CAP) listed nodes g, loaded in pairs when
-// the record allows it, into LDS words OFF.. of the node's S-word slot
-template <int CAP, int NW, int STRIDE, int OFF, int S, typename R, int NS = NW, int THR = NTHR>
-__device__ __forceinline__ void fb_stage(R *sn, const R *src, const int *nodes, int nn) {
-  constexpr bool PAIRS = NW % 2 == 0 && STRIDE % 2 == 0;
-  constexpr int U = PAIRS ? NW / 2 : NW;  // load units per node
-  constexpr int PER = (CAP * U + THR - 1) / THR;
-  using P2 = typename Pair<R>::type;
-  P2 pv[PAIRS ? PER : 1];
-  R sv[PAIRS ? 1 : PER];
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    int t = threadIdx.x + q * THR, k = t / U, j = t - k * U;
-    if (k < nn) {
-      size_t g = (size_t)nodes[k];
-      if constexpr (PAIRS) pv[q] = reinterpret_cast<const P2 *>(src + STRIDE * g)[j];
-      else sv[q] = src[STRIDE * g + j];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    int t = threadIdx.x + q * THR, k = t / U, j = t - k * U;
-    if (k < nn) {
-      if constexpr (PAIRS) {
-        sn[k * S + OFF + 2 * j] = pv[q].x;
-        if (NS == NW || 2 * j + 1 < NS) sn[k * S + OFF + 2 * j + 1] = pv[q].y;
-      } else if (NS == NW || j < NS) {
-        sn[k * S + OFF + j] = sv[q];
-      }
-    }
-  }
-}
 
 // Neighbour walks of node i: f(qj, tj, wx, wy, wz) per interior side with w
 // the node-signed side weights and either qj the neighbour's gather record
@@ -3820,8 +3787,28 @@ __global__ __launch_bounds__(NTHR) void k_gather_blk(LevelDev<R> L, DevParams P)
   L.to_batch(bb_);
   P.to_batch(bb_);
   if (blk >= L.ngb) return;
-  const int n0 = L.gb_nptr[blk], nn = L.gb_nptr[blk + 1] - n0;
-  fb_stage<GB_CAP, W, VREC, 0, S, R, NS>(sn, L.tau, L.gb_node + n0, nn);
+  __shared__ int sid[GB_CAP];
+  const int n0 = L.gb_nptr[blk], nn = L.gb_nptr[blk + 1] - n0, t = threadIdx.x;
+  for (int k = t; k < nn; k += NTHR) sid[k] = L.gb_node[n0 + k];
+  __syncthreads();
+  {
+    using P2 = typename Pair<R>::type;
+    constexpr int U = W / 2, PER = (GB_CAP * U + NTHR - 1) / NTHR;
+    P2 v[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int x = t + q * NTHR, k = x / U;
+      if (k < nn) v[q] = reinterpret_cast<const P2 *>(L.tau + VREC * (size_t)sid[k])[x - k * U];
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int x = t + q * NTHR, k = x / U, j = x - k * U;
+      if (k < nn) {
+        sn[k * S + 2 * j] = v[q].x;
+        if (2 * j + 1 < NS) sn[k * S + 2 * j + 1] = v[q].y;
+      }
+    }
+  }
   __syncthreads();
   int i = L.gb_first[blk] + (int)threadIdx.x / GB_SUB, sub = (int)threadIdx.x % GB_SUB;
   if (i >= L.gb_first[blk + 1]) return;
