@@ -1249,8 +1249,12 @@ int op_prep(flite_ctx *c, Level &L, bool compute_p, int ncopy = 0, bool zero = f
   });
 }
 
+bool has_gradients(const flite_ctx *c, const Level &L) {
+  return L.has_coords && c->hp.hllc_flux_order > 1 && c->hp.flux_type == 4;
+}
+
 int op_grad(flite_ctx *c, Level &L) {
-  if (!(L.has_coords && c->hp.hllc_flux_order > 1 && c->hp.flux_type == 4)) return 0;
+  if (!has_gradients(c, L)) return 0;
   DevParams P = c->P;
   Timed tm(c, "grad", L.gnum);
   return with_level(L, [&](auto V) {
@@ -1508,21 +1512,23 @@ int op_sa_diffusion(flite_ctx *c, Level &L) {
 // neighbour only its viscous record.  Time steps in pass A read the previous
 // laminar viscosity of the gather records; the new one goes to the viscous
 // records and to L.mu.
-int op_step_terms(flite_ctx *c, Level &L, bool timesteps, bool sa_timesteps) {
+// gradients: pass A forms the gradient records of the state too (the caller
+// then skips op_grad).
+int op_step_terms(flite_ctx *c, Level &L, bool timesteps, bool sa_timesteps, bool gradients = false) {
   DevParams P = c->P;
   bool sa = P.sa;
   Timed tm(c, "viscous", L.gnum);
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
-    if (timesteps && sa) {
-      launch_gather<TimeStepPart<R>, ViscNodePart<R>, SADiff1Part<R>>(c, L, V, P);
-    } else if (timesteps) {
-      launch_gather<TimeStepPart<R>, ViscNodePart<R>, NoPart<R>>(c, L, V, P);
-    } else if (sa) {
-      launch_gather<ViscNodePart<R>, SADiff1Part<R>, NoPart<R>>(c, L, V, P);
-    } else {
-      launch_gather<ViscNodePart<R>, NoPart<R>, NoPart<R>>(c, L, V, P);
-    }
+    auto pass_a = [&](auto node) {
+      using N = decltype(node);
+      if (timesteps && sa) launch_gather<TimeStepPart<R>, N, SADiff1Part<R>>(c, L, V, P);
+      else if (timesteps) launch_gather<TimeStepPart<R>, N, NoPart<R>>(c, L, V, P);
+      else if (sa) launch_gather<N, SADiff1Part<R>, NoPart<R>>(c, L, V, P);
+      else launch_gather<N, NoPart<R>, NoPart<R>>(c, L, V, P);
+    };
+    if (gradients) pass_a(GradViscPart<R>{});
+    else pass_a(ViscNodePart<R>{});
     if (sa && sa_timesteps) {
     launch_gather<ViscFluxPart<R>, SATimeStepPart<R>, SADiff2Part<R>>(c, L, V, P);
     } else if (sa) {
@@ -1599,7 +1605,7 @@ int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss, bool begun, bool
   if (calc_diss) {
     if (viscous(c)) {
       // makeTimeSteps, makeViscosityTerm, makeTurbulentTimeSteps, makeSADiffusion
-      TRY(op_step_terms(c, L, true, true));
+      TRY(op_step_terms(c, L, true, true, has_gradients(c, L)));
       TRY(op_jst(c, L, true));
     } else if (!stage_steps(c, L)) {
       TRY(op_jst(c, L, false, true));
@@ -1608,7 +1614,7 @@ int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss, bool begun, bool
   for (int k = 1; k <= hp.rk_stages; ++k) {
     // stage k > 1 starts from the pressure and records the previous stage
     // kernel wrote with the new state
-    TRY(op_grad(c, L));
+    if (!(k == 1 && calc_diss && viscous(c))) TRY(op_grad(c, L));  // else pass A formed them
     TRY(op_flux(c, L));
     StageArgs S;
     S.alpha = hp.rk_coefficients[k - 1];
@@ -1665,9 +1671,9 @@ int do_restrict(flite_ctx *c, int fine_level, bool recorded = false, bool begin 
   TRY(op_stage(c, K, MODE_COARSE, S, stage_steps(c, K)));
   // fine part (DEF:12236-12361)
   if (!recorded) TRY(op_prep(c, F, true, 0, zero_dissipation(c, F)));
-  if (visc) TRY(op_step_terms(c, F, false, false));
+  if (visc) TRY(op_step_terms(c, F, false, false, has_gradients(c, F)));
   TRY(op_jst(c, F, visc));  // with the time steps of the last smoothing step
-  TRY(op_grad(c, F));
+  if (!visc) TRY(op_grad(c, F));
   TRY(op_flux(c, F));
   S.has_src = F.gnum > 1;
   TRY(op_stage(c, F, MODE_FINE, S));
