@@ -599,23 +599,13 @@ __device__ __forceinline__ void grad_minmax_body(LevelDev<R> &L, const DevParams
   for (int c = 0; c < GREC; ++c) out[c] = v[c];
 }
 
-// one node per thread, the block's records stored through LDS in two
-// halves of 13 words: a thread's record lands in LDS at a 13-word stride
+// the block's records stored through LDS in two halves of 13 words (one node
+// per thread): a thread's record lands in LDS at a 13-word stride
 // (conflict-free for 64-bit words), then consecutive lanes store
 // consecutive words of the block's contiguous record range, instead of
 // every store instruction touching one cache line per lane
 template <typename R>
-__global__ void __launch_bounds__(NTHR) k_grad_minmax_st(LevelDev<R> L, DevParams P) {
-  __shared__ R st[NTHR * (GREC / 2)];
-  int bb_;
-  int i = btid(L.nb, bb_);
-  L.to_batch(bb_);
-  P.to_batch(bb_);
-  const int i0 = i - (int)threadIdx.x;
-  R v[GREC];
-  bool ok = i < L.n && grad_minmax_vals<R, 1>(L, P, i, 0, [&](auto f) { walk_global<1>(L, i, 0, f); }, v);
-  const int cnt = L.n - i0 < NTHR ? L.n - i0 : NTHR;
-  R *base = L.grec + GREC * (size_t)i0;
+__device__ __forceinline__ void store_grec(R *st, const R *v, bool ok, R *base, int cnt) {
   constexpr int HW = GREC / 2;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -632,6 +622,19 @@ __global__ void __launch_bounds__(NTHR) k_grad_minmax_st(LevelDev<R> L, DevParam
     }
     __syncthreads();
   }
+}
+
+template <typename R>
+__global__ void __launch_bounds__(NTHR) k_grad_minmax_st(LevelDev<R> L, DevParams P) {
+  __shared__ R st[NTHR * (GREC / 2)];
+  int bb_;
+  int i = btid(L.nb, bb_);
+  L.to_batch(bb_);
+  P.to_batch(bb_);
+  const int i0 = i - (int)threadIdx.x;
+  R v[GREC];
+  bool ok = i < L.n && grad_minmax_vals<R, 1>(L, P, i, 0, [&](auto f) { walk_global<1>(L, i, 0, f); }, v);
+  store_grec(st, v, ok, L.grec + GREC * (size_t)i0, L.n - i0 < NTHR ? L.n - i0 : NTHR);
 }
 
 template <typename R, int SUB>
@@ -1971,8 +1974,9 @@ constexpr int LIN_G = 25;                   // gradient 15 | 1/lo 5 | 1/hi 5
 constexpr int LIN_SIDE = 24;
 
 // tangent of the gather record (rho, u, v, w, rhoE, p) along du
-// the gather record's tangent dq[DQ i ..] = (rho, u, v, w, E, p, nu~, 0)
-// along du (nu~ = u(:,6) with Spalart-Allmaras, else 0)
+// the gather record's tangent dq[DQ i ..] = (rho, u, v, w, E, p, nu~, T)
+// along du (nu~ = u(:,6) with Spalart-Allmaras, else 0; T of the viscous
+// record)
 constexpr int DQ = 8;
 __global__ __launch_bounds__(NTHR) void k_record_tangent(LevelDev<double> L, DevParams P, const double *du, double *dq) {
   using ad::Dual;
@@ -1987,88 +1991,88 @@ __global__ __launch_bounds__(NTHR) void k_record_tangent(LevelDev<double> L, Dev
 #pragma unroll
   for (int c = 0; c < 6; ++c) o[c] = A[c].d;
   o[6] = P.sa ? du[5 * n + i] : 0.0;
-  o[7] = 0.0;
+  o[7] = (Dual(P.gamma / (P.gamma - 1.0)) * A[5] / A[0]).d;
 }
 
-// gradient and bounds of grad_minmax_body on dual numbers: gd[26 i + k].
-// The values are the level's own gradient records (grec), so that every
-// branch of the side flux is taken as in the residual and the adjoint; the
-// tangents follow the same walk in slot order, the bounds' with the extremal
-// neighbour that k_minmax_arg names.
-__global__ __launch_bounds__(NTHR) void k_grad_tangent(LevelDev<double> L, const double *dq, ad::Dual *gd) {
-  using ad::Dual;
-  int i = gtid_x();
-  if (i >= L.n) return;
-  Dual q0[5], g[15], mn[5], mx[5];
+// tangents of the gradient records along dq: gt[GREC i + k] (gradients 15,
+// reciprocal bounds 10).  The bounds move with the extremal neighbours that
+// k_minmax_arg names; B = 1 / (q_k - q_i), so dB = -B^2 (dq_k - dq_i).  The
+// values are the level's own records, so that every branch of the side flux
+// is taken as in the residual and the adjoint.  275k nodes: 253 us on dual
+// records with the bounds compared in the walk; 198 with the named neighbours'
+// ten words read behind a branch each and 216 following their indices in the
+// walk; 174 with the records stored through LDS; 107 with the ten reads in
+// flight together.
+template <int SUB>
+__device__ __forceinline__ bool grad_tangent_vals(const LevelDev<double> &L, int i, int sub, const double *dq, const int *amin,
+                                                  double *out) {
+  double q0[8], g[15];
+  ldrec<8>(dq + DQ * (size_t)i, q0);
 #pragma unroll
-  for (int c = 0; c < 5; ++c) {
-    q0[c] = Dual(L.rec0[8 * (size_t)i + c], dq[DQ * (size_t)i + c]);
-    mn[c] = Dual(1e15);
-    mx[c] = Dual(1e15);
-  }
-#pragma unroll
-  for (int c = 0; c < 15; ++c) g[c] = Dual(0.0);
-  for_edges_w<1>(L, i, 0, [&](int j, double wx, double wy, double wz) {
+  for (int c = 0; c < 15; ++c) g[c] = 0.0;
+  for_edges_w<SUB>(L, i, sub, [&](int j, double wx, double wy, double wz) {
+    double qj[6];
+    ldrec<6>(dq + DQ * (size_t)j, qj);
 #pragma unroll
     for (int c = 0; c < 5; ++c) {
-      Dual qj(L.rec0[8 * (size_t)j + c], dq[DQ * (size_t)j + c]);
-      Dual sq = q0[c] + qj;
-      g[c] += sq * Dual(wx);
-      g[5 + c] += sq * Dual(wy);
-      g[10 + c] += sq * Dual(wz);
-      mn[c] = rmin(mn[c], rmin(q0[c], qj));
-      mx[c] = rmin(mx[c], rmin(-q0[c], -qj));
+      const double s = q0[c] + qj[c];
+      g[c] += s * wx;
+      g[5 + c] += s * wy;
+      g[10 + c] += s * wz;
     }
   });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
+  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
     int v = L.bs_list[k], s = v >> 1;
     int o = (v & 1) ? L.ba[s] : L.bb[s];
-    double wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
+    const double wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
 #pragma unroll
     for (int c = 0; c < 5; ++c) {
-      Dual qo(L.rec0[8 * (size_t)o + c], dq[DQ * (size_t)o + c]);
-      Dual t = Dual(2.0) * q0[c] + (q0[c] + qo);
-      g[c] += t * Dual(wx);
-      g[5 + c] += t * Dual(wy);
-      g[10 + c] += t * Dual(wz);
+      const double t = 3.0 * q0[c] + dq[DQ * (size_t)o + c];
+      g[c] += t * wx;
+      g[5 + c] += t * wy;
+      g[10 + c] += t * wz;
     }
   }
-  Dual vt = Dual(1.0) / Dual(L.vol[i]);
-  const double *gv = L.grec + GREC * (size_t)i;
-  Dual *out = gd + 26 * (size_t)i;
 #pragma unroll
-  for (int c = 0; c < 15; ++c) out[c] = Dual(gv[c], (g[c] * vt).d);
+  for (int c = 0; c < 15; ++c) g[c] = lsum<SUB>(g[c]);
+  if (sub) return false;
+  const double vt = 1.0 / L.vol[i];
+  double B[12], dm[10];  // B: words 14 .. 25 of the record, in aligned pairs
+  int km[10];
+  const int2 *ap = reinterpret_cast<const int2 *>(amin + 10 * (size_t)i);
 #pragma unroll
   for (int c = 0; c < 5; ++c) {
-    Dual lo = mn[c] - q0[c];
-    Dual hi = -mx[c] - q0[c];
-    out[15 + c] = Dual(gv[15 + c], lo < Dual(0.0) ? (Dual(1.0) / lo).d : 0.0);
-    out[20 + c] = Dual(gv[20 + c], hi > Dual(0.0) ? (Dual(1.0) / hi).d : 0.0);
+    const int2 k2 = ap[c];
+    km[2 * c] = k2.x;
+    km[2 * c + 1] = k2.y;
   }
-  out[25] = Dual(0.0);
+  ldrec<12>(L.grec + GREC * (size_t)i + 14, B);
+  // the ten reads in flight together: no branch on the index
+#pragma unroll
+  for (int c = 0; c < 10; ++c) dm[c] = dq[DQ * (size_t)(km[c] < 0 ? i : km[c]) + (c < 5 ? c : c - 5)];
+#pragma unroll
+  for (int c = 0; c < 15; ++c) out[c] = g[c] * vt;
+#pragma unroll
+  for (int c = 0; c < 10; ++c) out[15 + c] = km[c] < 0 ? 0.0 : -B[1 + c] * B[1 + c] * (dm[c] - q0[c < 5 ? c : c - 5]);
+  out[25] = 0.0;
+  return true;
 }
 
-// second-order side fluxes along (du, dG, dB): fbuf[6 e + c] = d f_c
-// (component 5: the SA convection along d nu~)
-template <int NSIG, bool SA>
-__global__ __launch_bounds__(NTHR) void k_flux_tangent2(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *gd) {
-  using ad::Dual;
-  int e = gtid_x();
-  if (e >= L.ne) return;
-  int ia = L.ea[e], ib = L.eb[e];
-  Dual A[8], B[8], o[6];
+template <int SUB>
+__global__ __launch_bounds__(NTHR) void k_grad_tangent(LevelDev<double> L, const double *dq, const int *amin, double *gt) {
+  __shared__ double st[SUB == 1 ? NTHR * (GREC / 2) : 1];
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
+  double v[GREC];
+  const bool ok = i < L.n && grad_tangent_vals<SUB>(L, i, sub, dq, amin, v);
+  if (SUB == 1) {
+    const int i0 = i - (int)threadIdx.x;
+    store_grec(st, v, ok, gt + GREC * (size_t)i0, L.n - i0 < NTHR ? L.n - i0 : NTHR);
+  } else if (ok) {
+    double *out = gt + GREC * (size_t)i;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    A[c] = Dual(L.rec0[8 * (size_t)ia + c], c < 7 ? dq[DQ * (size_t)ia + c] : 0.0);
-    B[c] = Dual(L.rec0[8 * (size_t)ib + c], c < 7 ? dq[DQ * (size_t)ib + c] : 0.0);
+    for (int c = 0; c < GREC; ++c) out[c] = v[c];
   }
-  side_flux<Dual, double, 2, SA, NSIG, Dual>(P, gd + 26 * (size_t)ia, gd + 26 * (size_t)ib, L.xyz + 3 * (size_t)ia,
-                                             L.xyz + 3 * (size_t)ib, A, B, Dual(L.w[3 * e]), Dual(L.w[3 * e + 1]),
-                                             Dual(L.w[3 * e + 2]), o);
-  double *f = L.fbuf + 6 * (size_t)e;
-#pragma unroll
-  for (int c = 0; c < 5; ++c) f[c] = o[c].d;
-  f[5] = SA ? o[5].d : 0.0;
 }
 
 // node i's extremal neighbours: amin[10 i + c] = the node whose q_c sets
@@ -2129,6 +2133,81 @@ __device__ __forceinline__ double led_slopes(double a, double ilo, double ihi, d
   da = iden / den;
   div = -2.0 * a * a * t * da;
   return a * iden;
+}
+
+// One end's projected gradients on half the side vector and the bounds their
+// signs select (SG -1: the second end, whose slope is -led(-b)), values from
+// the gradient record G and tangents from T, limited: v the limited
+// projections, t their tangents
+template <int NSIG>
+__device__ __forceinline__ void limited_tangents(const DevParams &P, const double *G, const double *T, double dx, double dy,
+                                                 double dz, double sg, double *v, double *t) {
+  double g[GREC], r[GREC];
+  ldrec<GREC>(G, g);
+  ldrec<GREC>(T, r);
+#pragma unroll
+  for (int j = 0; j < 5; ++j) {
+    const double a = 0.5 * (g[j] * dx + g[j + 5] * dy + g[j + 10] * dz);
+    const double ta = 0.5 * (r[j] * dx + r[j + 5] * dy + r[j + 10] * dz);
+    v[j] = a;
+    t[j] = ta;
+    if (P.autoclip == 1) {
+      double da, div;
+      bool hi;
+      v[j] = sg * led_slopes<NSIG>(sg * a, g[15 + j], g[20 + j], da, div, hi);
+      t[j] = da * ta + sg * div * (hi ? r[20 + j] : r[15 + j]);
+    }
+  }
+}
+
+// second-order side fluxes along (dq, dG, dB): fbuf[6 e + c] = d f_c
+// (component 5: the SA convection along d nu~); the slopes' tangents in closed
+// form, the HLLC flux of the states and slopes on dual numbers (275k nodes,
+// 1.87M sides: 259 us with the limiter on dual numbers too, 235 now, bound by
+// the two ends' records: 1.1 KB a side through L2)
+template <int NSIG, bool SA>
+__global__ __launch_bounds__(NTHR) void k_flux_tangent2(LevelDev<double> L, DevParams P, const double *dq, const double *gt) {
+  using ad::Dual;
+  int e = gtid_x();
+  if (e >= L.ne) return;
+  int ia = L.ea[e], ib = L.eb[e];
+  const double *xa = L.xyz + 3 * (size_t)ia, *xb = L.xyz + 3 * (size_t)ib;
+  const double dx = xb[0] - xa[0], dy = xb[1] - xa[1], dz = xb[2] - xa[2];
+  const double hl = 0.5 * P.clip * ::sqrt(dx * dx + dy * dy + dz * dz);
+  double va[5], ta[5], vb[5], tb[5];
+  limited_tangents<NSIG>(P, L.grec + GREC * (size_t)ia, gt + GREC * (size_t)ia, dx, dy, dz, 1.0, va, ta);
+  limited_tangents<NSIG>(P, L.grec + GREC * (size_t)ib, gt + GREC * (size_t)ib, dx, dy, dz, -1.0, vb, tb);
+  Dual A[8], B[8], D[5], o[6];
+#pragma unroll
+  for (int j = 0; j < 5; ++j) {
+    double c = 0.0, t = 0.0;
+    if (!(va[j] * vb[j] <= 0.0)) {
+      const bool first = ::fabs(va[j]) <= ::fabs(vb[j]);
+      c = first ? va[j] : vb[j];
+      t = first ? ta[j] : tb[j];
+      if (::fabs(c) > hl && hl > 0.0) {
+        c = c > 0.0 ? hl : -hl;
+        t = 0.0;
+      }
+    }
+    D[j] = Dual(c, t);
+  }
+  {
+    double v[8], t[8];
+    ldrec<8>(L.rec0 + 8 * (size_t)ia, v);
+    ldrec<8>(dq + DQ * (size_t)ia, t);
+#pragma unroll
+    for (int c = 0; c < 7; ++c) A[c] = Dual(v[c], t[c]);
+    ldrec<8>(L.rec0 + 8 * (size_t)ib, v);
+    ldrec<8>(dq + DQ * (size_t)ib, t);
+#pragma unroll
+    for (int c = 0; c < 7; ++c) B[c] = Dual(v[c], t[c]);
+  }
+  side_flux_d<Dual, double, SA>(P, A, B, D, Dual(L.w[3 * e]), Dual(L.w[3 * e + 1]), Dual(L.w[3 * e + 2]), o, 0.0);
+  double *f = L.fbuf + 6 * (size_t)e;
+#pragma unroll
+  for (int c = 0; c < 5; ++c) f[c] = o[c].d;
+  f[5] = SA ? o[5].d : 0.0;
 }
 
 // adjoint shares of side e: dl = lam_a - lam_b against df/d(U_a, U_b,
@@ -2550,195 +2629,200 @@ __device__ __forceinline__ void visc_bside(const T *t1, const T *to, const T *q1
           T(2) * (wx * (t1[6] + du11) + wy * (t1[7] + du21) + wz * (t1[8] + du31));
 }
 
-// node record (u, v, w, T) as dual numbers from the gather record and its
-// tangent dq (null: no tangent)
-__device__ __forceinline__ void visc_rec(const LevelDev<double> &L, const DevParams &P, const double *dq, int i,
-                                         ad::Dual *a, ad::Dual *rho_out = nullptr, ad::Dual *nu_out = nullptr) {
-  using ad::Dual;
-  const double *q = L.rec0 + 8 * (size_t)i;
-  const double *t = dq ? dq + DQ * (size_t)i : nullptr;
-  Dual rho(q[0], t ? t[0] : 0.0), p(q[5], t ? t[5] : 0.0);
-  a[0] = Dual(q[1], t ? t[1] : 0.0);
-  a[1] = Dual(q[2], t ? t[2] : 0.0);
-  a[2] = Dual(q[3], t ? t[3] : 0.0);
-  a[3] = Dual(P.gamma / (P.gamma - 1.0)) * p / rho;
-  if (rho_out) *rho_out = rho;
-  if (nu_out) *nu_out = Dual(q[6], t ? t[6] : 0.0);
-}
-
 __device__ __forceinline__ bool visc_wall(const LevelDev<double> &L, int i) {
   return L.gnum == 1 && (L.ncls[i] & NC_MASK) == NC_WALL;
 }
 
-// Green-Gauss sums g[12] of the node records (dual; tangents from dq)
-__device__ __forceinline__ void visc_grad_sums(const LevelDev<double> &L, const DevParams &P, const double *dq, int i,
-                                               const ad::Dual *ai, ad::Dual *g) {
-  using ad::Dual;
+// Green-Gauss sums g[12] of the node records (values)
+template <int SUB>
+__device__ __forceinline__ void visc_sums(const LevelDev<double> &L, const DevParams &P, int i, int sub, double *g) {
+  const double gog1 = P.gamma / (P.gamma - 1.0);
+  double q[8];
+  ldrec<8>(L.rec0 + 8 * (size_t)i, q);
+  const double ai[4] = {q[1], q[2], q[3], gog1 * q[5] / q[0]};
 #pragma unroll
-  for (int c = 0; c < 12; ++c) g[c] = Dual(0.0);
-  for_edges_w<1>(L, i, 0, [&](int j, double wx, double wy, double wz) {
-    Dual aj[4];
-    visc_rec(L, P, dq, j, aj);
+  for (int c = 0; c < 12; ++c) g[c] = 0.0;
+  for_edges_w<SUB>(L, i, sub, [&](int j, double wx, double wy, double wz) {
+    double r[8];
+    ldrec<8>(L.rec0 + 8 * (size_t)j, r);
+    const double aj[4] = {r[1], r[2], r[3], gog1 * r[5] / r[0]}, ww[3] = {wx, wy, wz};
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) g[4 * d + c] += (ai[c] + aj[c]) * ww[d];
+  });
+  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
+    int v = L.bs_list[k], s = v >> 1;
+    int o = (v & 1) ? L.ba[s] : L.bb[s];
+    double r[8];
+    ldrec<8>(L.rec0 + 8 * (size_t)o, r);
+    const double ao[4] = {r[1], r[2], r[3], gog1 * r[5] / r[0]};
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) g[4 * d + c] += (2.0 * ai[c] + (ai[c] + ao[c])) * L.wb[3 * s + d];
+  }
+#pragma unroll
+  for (int c = 0; c < 12; ++c) g[c] = lsum<SUB>(g[c]);
+}
+
+// the stress and heat-flux record of each node (values, for the adjoint and
+// mesh kernels), taud[9 i + c]
+template <int SUB>
+__global__ __launch_bounds__(NTHR) void k_visc_stress(LevelDev<double> L, DevParams P, ad::Dual *taud) {
+  using ad::Dual;
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
+  if (i >= L.n) return;
+  double g[12], t[9];
+  visc_sums<SUB>(L, P, i, sub, g);
+  if (sub) return;
+  const double *q = L.rec0 + 8 * (size_t)i;
+  visc_tau(P, g, L.vol[i], P.gamma / (P.gamma - 1.0) * q[5] / q[0], visc_wall(L, i), L.nrm + 3 * (size_t)i, t, q[0], q[6]);
+#pragma unroll
+  for (int c = 0; c < 9; ++c) taud[9 * (size_t)i + c] = Dual(t[c]);
+}
+
+// Tangent of the viscous term and, with Spalart-Allmaras, of its diffusion
+// (makeSADiffusion, DEF:7436-7808) and source (makeSASourceTerm,
+// DEF:9285-9370) along the record tangent dq.  Pass 1, one walk: the sums of
+// (u, v, w, T) and nu~ and their tangents; from them on dual numbers the
+// node's parts of the side fluxes, whose tangents vt[12 i ..] = stress 6 |
+// energy flux 3 | diffusion flux 3 are all that pass 2 reads of a neighbour;
+// dnode[i] = the tangent of the nodal cb2 term and the source.  (Two walks per
+// pass, on dual records with both ends' factors, took 542 us at 275k nodes;
+// 204 now, 131 + 73.)
+template <int SUB>
+__global__ __launch_bounds__(NTHR) void k_visc_tangent1(LevelDev<double> L, DevParams P, const double *dq, double *vt,
+                                                        double *dnode) {
+  using ad::Dual;
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
+  if (i >= L.n) return;
+  const double gog1 = P.gamma / (P.gamma - 1.0);
+  double qi[8], di[8];
+  ldrec<8>(L.rec0 + 8 * (size_t)i, qi);
+  ldrec<8>(dq + DQ * (size_t)i, di);
+  // (u, v, w, T, nu~) and tangents
+  const double a0[5] = {qi[1], qi[2], qi[3], gog1 * qi[5] / qi[0], qi[6]}, t0[5] = {di[1], di[2], di[3], di[7], di[6]};
+  double g[15], h[15];
+#pragma unroll
+  for (int c = 0; c < 15; ++c) g[c] = h[c] = 0.0;
+  for_edges_w<SUB>(L, i, sub, [&](int j, double wx, double wy, double wz) {
+    double q[8], d[8];
+    ldrec<8>(L.rec0 + 8 * (size_t)j, q);
+    ldrec<8>(dq + DQ * (size_t)j, d);
+    const double aj[5] = {q[1], q[2], q[3], gog1 * q[5] / q[0], q[6]}, tj[5] = {d[1], d[2], d[3], d[7], d[6]};
     const double ww[3] = {wx, wy, wz};
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int k = 0; k < 3; ++k)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) g[4 * d + q] += (ai[q] + aj[q]) * Dual(ww[d]);
+      for (int c = 0; c < 5; ++c) {
+        g[5 * k + c] += (a0[c] + aj[c]) * ww[k];
+        h[5 * k + c] += (t0[c] + tj[c]) * ww[k];
+      }
   });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
+  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
     int v = L.bs_list[k], s = v >> 1;
     int o = (v & 1) ? L.ba[s] : L.bb[s];
-    Dual ao[4];
-    visc_rec(L, P, dq, o, ao);
-    const double ww[3] = {L.wb[3 * s], L.wb[3 * s + 1], L.wb[3 * s + 2]};
+    double q[8], d[8];
+    ldrec<8>(L.rec0 + 8 * (size_t)o, q);
+    ldrec<8>(dq + DQ * (size_t)o, d);
+    const double ao[5] = {q[1], q[2], q[3], gog1 * q[5] / q[0], q[6]}, to[5] = {d[1], d[2], d[3], d[7], d[6]};
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int x = 0; x < 3; ++x) {
+      const double w = L.wb[3 * s + x];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) g[4 * d + q] += (Dual(2.0) * ai[q] + (ai[q] + ao[q])) * Dual(ww[d]);
+      for (int c = 0; c < 5; ++c) {
+        const bool four = c == 4 && P.bterm != 1;  // nu~ with boundaryTerm 2
+        g[5 * x + c] += (four ? 4.0 * a0[c] : 3.0 * a0[c] + ao[c]) * w;
+        h[5 * x + c] += (four ? 4.0 * t0[c] : 3.0 * t0[c] + to[c]) * w;
+      }
+    }
   }
+#pragma unroll
+  for (int c = 0; c < 15; ++c) {
+    g[c] = lsum<SUB>(g[c]);
+    h[c] = lsum<SUB>(h[c]);
+  }
+  if (sub) return;
+  Dual G[12], t[9];
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) G[4 * k + c] = Dual(g[5 * k + c], h[5 * k + c]);
+  const Dual u(a0[0], t0[0]), v(a0[1], t0[1]), w(a0[2], t0[2]), T(a0[3], t0[3]);
+  const Dual rho(qi[0], di[0]), nu(qi[6], di[6]);
+  const double V = L.vol[i];
+  visc_tau(P, G, V, T, visc_wall(L, i), L.nrm + 3 * (size_t)i, t, rho, nu);
+  double *out = vt + 12 * (size_t)i;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) out[c] = t[c].d;
+  out[6] = (t[6] + u * t[0] + v * t[1] + w * t[2]).d;
+  out[7] = (t[7] + u * t[1] + v * t[3] + w * t[4]).d;
+  out[8] = (t[8] + u * t[2] + v * t[4] + w * t[5]).d;
+  if (!P.sa) {
+    out[9] = out[10] = out[11] = 0.0;
+    return;
+  }
+  Dual mu = sutherland(P, T);
+  const Dual coef = Dual(P.Re) * mu / rho + nu;
+  const double iv = 1.0 / V, f1 = 1.0 / P.Re * 0.622 / (2.0 / 3.0);
+  double gg = 0.0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const Dual d(g[5 * k + 4] * iv, h[5 * k + 4] * iv);
+    out[9 + k] = (coef * d).d;
+    gg += 2.0 * g[5 * k + 4] * d.d;
+  }
+  Dual vort, divg;
+  visc_vort_divg(G, V, vort, divg);
+  if (mu < Dual(0.1 / P.Re)) mu = Dual(0.1 * P.Re);  // sa_source's guard
+  dnode[i] = -f1 * gg + sa_source_t<Dual>(P, rho, nu, mu, vort, divg, L.wd[i], V).d;
 }
 
-// tangent pass 1: the stress and heat-flux record of each node on dual
-// numbers, taud[18 i + 2 c] = value, [18 i + 2 c + 1] = tangent (dq null:
-// values only, for the adjoint)
-// With Spalart-Allmaras also aux[3 i ..] = (laminar viscosity, vorticity,
-// divergence) on dual numbers, for the SA source and diffusion (aux may be
-// null otherwise)
-__global__ __launch_bounds__(NTHR) void k_visc_tangent_node(LevelDev<double> L, DevParams P, const double *dq, ad::Dual *taud,
-                                    ad::Dual *aux) {
-  using ad::Dual;
-  int i = gtid_x();
-  if (i >= L.n) return;
-  Dual ai[4], g[12], t[9], rho, nu;
-  visc_rec(L, P, dq, i, ai, &rho, &nu);
-  visc_grad_sums(L, P, dq, i, ai, g);
-  visc_tau(P, g, L.vol[i], ai[3], visc_wall(L, i), L.nrm + 3 * (size_t)i, t, rho, nu);
-#pragma unroll
-  for (int c = 0; c < 9; ++c) taud[9 * (size_t)i + c] = t[c];
-  if (P.sa && aux) {
-    Dual vort, divg;
-    visc_vort_divg(g, L.vol[i], vort, divg);
-    aux[3 * (size_t)i] = sutherland(P, ai[3]);
-    aux[3 * (size_t)i + 1] = vort;
-    aux[3 * (size_t)i + 2] = divg;
-  }
-}
-
-// tangent pass 2: dvis(c, i) = -dA (c = 1..4), 0 for c = 0
-__global__ __launch_bounds__(NTHR) void k_visc_tangent_flux(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *taud,
-                                    double *dvis) {
-  using ad::Dual;
-  int i = gtid_x();
+// pass 2: the side fluxes' tangents from both ends' parts, added to out
+template <int SUB>
+__global__ __launch_bounds__(NTHR) void k_visc_tangent2(LevelDev<double> L, DevParams P, const double *vt,
+                                                        const double *dnode, double *out) {
+  int i, sub, bb_;
+  node_lanes<SUB>(1, bb_, i, sub);
   if (i >= L.n) return;
   const size_t n = L.n;
-  Dual t1[9], q1[4], a[4] = {Dual(0.0), Dual(0.0), Dual(0.0), Dual(0.0)};
+  double ti[12], a[5] = {0, 0, 0, 0, 0};
+  ldrec<12>(vt + 12 * (size_t)i, ti);
+  auto add = [&](const double *d, double wx, double wy, double wz) {
+    a[0] += wx * d[0] + wy * d[1] + wz * d[2];
+    a[1] += wx * d[1] + wy * d[3] + wz * d[4];
+    a[2] += wx * d[2] + wy * d[4] + wz * d[5];
+    a[3] += wx * d[6] + wy * d[7] + wz * d[8];
+  };
+  for_edges_w<SUB>(L, i, sub, [&](int j, double wx, double wy, double wz) {
+    double d[12];
+    ldrec<12>(vt + 12 * (size_t)j, d);
 #pragma unroll
-  for (int c = 0; c < 9; ++c) t1[c] = taud[9 * (size_t)i + c];
-  visc_rec(L, P, dq, i, q1);
-  for_edges_w<1>(L, i, 0, [&](int j, double wx, double wy, double wz) {
-    Dual tj[9], qj[4];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) tj[c] = taud[9 * (size_t)j + c];
-    visc_rec(L, P, dq, j, qj);
-    visc_edge(t1, tj, q1, qj, wx, wy, wz, a);
+    for (int c = 0; c < 12; ++c) d[c] += ti[c];
+    add(d, wx, wy, wz);
+    a[4] += wx * d[9] + wy * d[10] + wz * d[11];
   });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
-    int v = L.bs_list[k], s = v >> 1;
-    int ind = L.bind[s];
-    if (ind == 2 || ind == 9) continue;
+  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
+    int v = L.bs_list[k], s = v >> 1, ind = L.bind[s];
     int o = (v & 1) ? L.ba[s] : L.bb[s];
-    Dual to[9], qo[4];
+    const double wx = L.wb[3 * s], wy = L.wb[3 * s + 1], wz = L.wb[3 * s + 2];
+    double d[12], e[12];
+    ldrec<12>(vt + 12 * (size_t)o, d);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) to[c] = taud[9 * (size_t)o + c];
-    visc_rec(L, P, dq, o, qo);
-    visc_bside(t1, to, q1, qo, L.wb[3 * s], L.wb[3 * s + 1], L.wb[3 * s + 2], a);
+    for (int c = 0; c < 12; ++c) e[c] = 3.0 * ti[c] + d[c];
+    if (ind != 2 && ind != 9) add(e, wx, wy, wz);
+    if (P.bterm == 1) a[4] += wx * e[9] + wy * e[10] + wz * e[11];
+    else a[4] += 4.0 * (wx * ti[9] + wy * ti[10] + wz * ti[11]);
   }
-  dvis[i] = 0.0;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) dvis[(c + 1) * n + i] = -a[c].d;
-}
-
-// Spalart-Allmaras tangent (makeSADiffusion, DEF:7436-7808, and
-// makeSASourceTerm, DEF:9285-9370, as SADiff1Part / SADiff2Part / sa_source
-// compute them), on dual numbers from the record tangent dq and the node
-// duals aux = (laminar viscosity, vorticity, divergence) of
-// k_visc_tangent_node.
-// pass 1: dnud[4 i ..] = the grad nu~ record (grad 3, nodal cb2 term)
-__global__ __launch_bounds__(NTHR) void k_sa_diff1_tangent(LevelDev<double> L, DevParams P, const double *dq, ad::Dual *dnud) {
-  using ad::Dual;
-  int i = gtid_x();
-  if (i >= L.n) return;
-  Dual ti(L.rec0[8 * (size_t)i + 6], dq[DQ * (size_t)i + 6]);
-  Dual g[3] = {Dual(0.0), Dual(0.0), Dual(0.0)};
-  for_edges_w<1>(L, i, 0, [&](int j, double wx, double wy, double wz) {
-    Dual sj = ti + Dual(L.rec0[8 * (size_t)j + 6], dq[DQ * (size_t)j + 6]);
-    g[0] += Dual(wx) * sj;
-    g[1] += Dual(wy) * sj;
-    g[2] += Dual(wz) * sj;
-  });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
-    int v = L.bs_list[k], s = v >> 1;
-    int o = (v & 1) ? L.ba[s] : L.bb[s];
-    Dual to(L.rec0[8 * (size_t)o + 6], dq[DQ * (size_t)o + 6]);
-    Dual c = P.bterm == 1 ? (Dual(3.0) * ti + to) : Dual(4.0) * ti;
-    g[0] += c * Dual(L.wb[3 * s]);
-    g[1] += c * Dual(L.wb[3 * s + 1]);
-    g[2] += c * Dual(L.wb[3 * s + 2]);
-  }
-  Dual vt = Dual(1.0) / Dual(L.vol[i]);
-  Dual dx = g[0] * vt, dy = g[1] * vt, dz = g[2] * vt;
-  Dual fact = Dual(1.0 / P.Re * 0.622 / (2.0 / 3.0));
-  Dual *o = dnud + 4 * (size_t)i;
-  o[0] = dx;
-  o[1] = dy;
-  o[2] = dz;
-  o[3] = -(fact * (g[0] * dx + g[1] * dy + g[2] * dz));
-}
-
-// the diffusion coefficient Re mu / rho + nu~ of node j on dual numbers
-__device__ __forceinline__ ad::Dual sa_diff_coef(const LevelDev<double> &L, const DevParams &P, const double *dq,
-                                                 const ad::Dual *aux, int j) {
-  using ad::Dual;
-  Dual rho(L.rec0[8 * (size_t)j], dq[DQ * (size_t)j]);
-  Dual nu(L.rec0[8 * (size_t)j + 6], dq[DQ * (size_t)j + 6]);
-  return Dual(P.Re) * aux[3 * (size_t)j] / rho + nu;
-}
-
-// pass 2 and the source: dsa[i] = d(tdiff + source) at node i
-__global__ __launch_bounds__(NTHR) void k_sa_tangent(LevelDev<double> L, DevParams P, const double *dq, const ad::Dual *aux,
-                             const ad::Dual *dnud, double *dsa) {
-  using ad::Dual;
-  int i = gtid_x();
-  if (i >= L.n) return;
-  const Dual *di = dnud + 4 * (size_t)i;
-  Dual fact = Dual(1.0 / P.Re / (2.0 / 3.0));
-  Dual v1 = sa_diff_coef(L, P, dq, aux, i);
-  Dual acc(0.0);
-  for_edges_w<1>(L, i, 0, [&](int j, double wx, double wy, double wz) {
-    const Dual *dj = dnud + 4 * (size_t)j;
-    Dual v2 = sa_diff_coef(L, P, dq, aux, j);
-    Dual w0(wx), w1(wy), w2(wz);
-    Dual fd = v1 * (w0 * di[0] + w1 * di[1] + w2 * di[2]) + v2 * (w0 * dj[0] + w1 * dj[1] + w2 * dj[2]);
-    acc -= fact * fd;
-  });
-  for (int k = L.bs_ptr[i]; k < L.bs_ptr[i + 1]; ++k) {
-    int v = L.bs_list[k], s = v >> 1;
-    int o = (v & 1) ? L.ba[s] : L.bb[s];
-    const Dual *dd = dnud + 4 * (size_t)o;
-    Dual vo = sa_diff_coef(L, P, dq, aux, o);
-    Dual w0(L.wb[3 * s]), w1(L.wb[3 * s + 1]), w2(L.wb[3 * s + 2]);
-    Dual fd1 = v1 * (w0 * di[0] + w1 * di[1] + w2 * di[2]);
-    Dual fd2 = vo * (w0 * dd[0] + w1 * dd[1] + w2 * dd[2]);
-    acc -= P.bterm == 1 ? fact * (Dual(3.0) * fd1 + fd2) : fact * Dual(4.0) * fd1;
-  }
-  Dual tdiff = acc + di[3];
-  // the source, with the laminar viscosity guard of sa_source
-  Dual mu = aux[3 * (size_t)i];
-  if (mu < Dual(0.1 / P.Re)) mu = Dual(0.1 * P.Re);
-  Dual rho(L.rec0[8 * (size_t)i], dq[DQ * (size_t)i]);
-  Dual nu(L.rec0[8 * (size_t)i + 6], dq[DQ * (size_t)i + 6]);
-  Dual src = sa_source_t<Dual>(P, rho, nu, mu, aux[3 * (size_t)i + 1], aux[3 * (size_t)i + 2], L.wd[i], L.vol[i]);
-  dsa[i] = tdiff.d + src.d;
+  for (int c = 0; c < 5; ++c) a[c] = lsum<SUB>(a[c]);
+  if (sub) return;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) out[(c + 1) * n + i] -= a[c];
+  if (P.sa) out[5 * n + i] += dnode[i] - 1.0 / P.Re / (2.0 / 3.0) * a[4];
 }
 
 // adjoint pass 1: shares of lam^T(-A) on node i's stress record (taub 9)
@@ -2824,9 +2908,10 @@ __global__ __launch_bounds__(NTHR) void k_visc_adjoint_node(LevelDev<double> L, 
   using ad::Dual;
   int i = gtid_x();
   if (i >= L.n) return;
-  Dual ai[4], g[12], rho, nu;
-  visc_rec(L, P, nullptr, i, ai, &rho, &nu);
-  visc_grad_sums(L, P, nullptr, i, ai, g);
+  double gv[12];
+  visc_sums<1>(L, P, i, 0, gv);
+  const double *qi = L.rec0 + 8 * (size_t)i;
+  const double Tv = P.gamma / (P.gamma - 1.0) * qi[5] / qi[0];
   const double *tb = taub + 9 * (size_t)i;
   const bool wall = visc_wall(L, i);
   const double l6 = (P.sa && lam) ? lam[5 * (size_t)L.n + i] : 0.0;
@@ -2841,8 +2926,8 @@ __global__ __launch_bounds__(NTHR) void k_visc_adjoint_node(LevelDev<double> L, 
     if (k >= 16 && k <= 18 && !wall) continue;
     Dual gs[12], t[9];
 #pragma unroll
-    for (int c = 0; c < 12; ++c) gs[c] = Dual(g[c].v, k == c ? 1.0 : 0.0);
-    const Dual T(ai[3].v, k == 12 ? 1.0 : 0.0), R(rho.v, k == 13 ? 1.0 : 0.0), N(nu.v, k == 14 ? 1.0 : 0.0);
+    for (int c = 0; c < 12; ++c) gs[c] = Dual(gv[c], k == c ? 1.0 : 0.0);
+    const Dual T(Tv, k == 12 ? 1.0 : 0.0), R(qi[0], k == 13 ? 1.0 : 0.0), N(qi[6], k == 14 ? 1.0 : 0.0);
     const Dual Vd(L.vol[i], k == 15 ? 1.0 : 0.0), Wd(L.wd[i], k == 19 ? 1.0 : 0.0);
     const Dual nd[3] = {Dual(nr[0], k == 16 ? 1.0 : 0.0), Dual(nr[1], k == 17 ? 1.0 : 0.0),
                         Dual(nr[2], k == 18 ? 1.0 : 0.0)};
@@ -3031,7 +3116,7 @@ __global__ __launch_bounds__(NTHR) void k_sa_diff_adjoint2(LevelDev<double> L, D
   out[5 * n + m] += r;
 }
 
-// (u, v, w, T) of node i's record, as visc_rec forms it
+// (u, v, w, T) of node i's record
 __device__ __forceinline__ void visc_rec_v(const LevelDev<double> &L, const DevParams &P, int i, double *a) {
   const double *q = L.rec0 + 8 * (size_t)i;
   a[0] = q[1];
@@ -3270,13 +3355,6 @@ __global__ void k_add_rho_nu(const double *rnbar, int n, double *out) {
   if (i >= n) return;
   out[i] += rnbar[2 * (size_t)i];
   out[5 * (size_t)n + i] += rnbar[2 * (size_t)i + 1];
-}
-
-// tangent: out += dvis
-__global__ void k_add_vector(double *out, const double *add, int n, int ncomp) {
-  int i = gtid_x();
-  if (i >= n) return;
-  for (int c = 0; c < ncomp; ++c) out[(size_t)c * n + i] += add[(size_t)c * n + i];
 }
 
 // partial derivative of the pressure drag (calculateLiftAndDrag,

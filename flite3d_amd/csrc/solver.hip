@@ -2370,28 +2370,25 @@ int alloc_vlin(Level &L) {
 
 // tangent of the viscous term along the direction in V.src, added to V.rhs
 // With Spalart-Allmaras it also adds the tangent of the SA diffusion and
-// source to component 6 (the eddy viscosity is in the stress already).
-// Scratch per node: dq 8 | tau duals 18 | aux duals 6 | grad nu~ duals 8 |
-// out 6
-int visc_tangent(flite_ctx *c, Level &L) {
+// source to component 6 (the eddy viscosity is in the stress already).  dq:
+// the records' tangents if the caller has formed them.  Scratch per node: the
+// flux parts' tangents 12 | the node's own terms 1, pad 1 | dq 8
+int visc_tangent(flite_ctx *c, Level &L, const double *dq) {
   TRY(alloc_vlin(L));
   DevParams P = c->P;
   LevelDev<double> V = L.view<double>();
   const size_t n = L.n;
-  double *dq = L.vlin, *dvis = L.vlin + 40 * n;
-  ad::Dual *taud = reinterpret_cast<ad::Dual *>(L.vlin + 8 * n);
-  ad::Dual *aux = reinterpret_cast<ad::Dual *>(L.vlin + 26 * n);
-  ad::Dual *dnud = reinterpret_cast<ad::Dual *>(L.vlin + 32 * n);
-  dim3 g(nblk(L.n)), b(NTHR);
-  hipLaunchKernelGGL(k_record_tangent, g, b, 0, c->stream, V, P, V.src, dq);
-  hipLaunchKernelGGL(k_visc_tangent_node, g, b, 0, c->stream, V, P, (const double *)dq, taud, aux);
-  hipLaunchKernelGGL(k_visc_tangent_flux, g, b, 0, c->stream, V, P, (const double *)dq, (const ad::Dual *)taud, dvis);
-  if (P.sa) {
-    hipLaunchKernelGGL(k_sa_diff1_tangent, g, b, 0, c->stream, V, P, (const double *)dq, dnud);
-    hipLaunchKernelGGL(k_sa_tangent, g, b, 0, c->stream, V, P, (const double *)dq, (const ad::Dual *)aux,
-                       (const ad::Dual *)dnud, dvis + 5 * n);
+  double *vt = L.vlin, *dnode = L.vlin + 12 * n;
+  dim3 b(NTHR);
+  if (!dq) {
+    hipLaunchKernelGGL(k_record_tangent, dim3(nblk(L.n)), b, 0, c->stream, V, P, V.src, L.vlin + 14 * n);
+    dq = L.vlin + 14 * n;
   }
-  hipLaunchKernelGGL(k_add_vector, g, b, 0, c->stream, V.rhs, (const double *)dvis, L.n, P.sa ? 6 : 5);
+  launch_nodes(L, [&](auto sc, dim3 g) {
+    constexpr int SUB = decltype(sc)::value;
+    hipLaunchKernelGGL(k_visc_tangent1<SUB>, g, b, 0, c->stream, V, P, dq, vt, dnode);
+    hipLaunchKernelGGL(k_visc_tangent2<SUB>, g, b, 0, c->stream, V, P, (const double *)vt, (const double *)dnode, V.rhs);
+  });
   return check_launch();
 }
 
@@ -2429,7 +2426,9 @@ int visc_adjoint(flite_ctx *c, Level &L) {
   LevelDev<double> V = L.view<double>();
   Vlin S(L);
   dim3 g(nblk(L.n)), b(NTHR);
-  hipLaunchKernelGGL(k_visc_tangent_node, g, b, 0, c->stream, V, P, (const double *)nullptr, S.taud, (ad::Dual *)nullptr);
+  launch_nodes(L, [&](auto sc, dim3 gl) {
+    hipLaunchKernelGGL(k_visc_stress<decltype(sc)::value>, gl, b, 0, c->stream, V, P, S.taud);
+  });
   launch_nodes(L, [&](auto sc, dim3 gl) {
     hipLaunchKernelGGL(k_visc_adjoint_tau<decltype(sc)::value>, gl, b, 0, c->stream, V, P, V.src,
                        (const ad::Dual *)S.taud, S.taub, S.ubv);
@@ -2468,7 +2467,9 @@ int visc_mesh_adjoint(flite_ctx *c, Level &L) {
   dim3 g(nblk(L.n)), b(NTHR);
   const size_t ns = 3 * ((size_t)std::max(1, L.ne) + (size_t)std::max(1, L.nbs));
   hipLaunchKernelGGL(k_fill<double>, dim3(nblk((long long)ns)), dim3(NTHR), 0, c->stream, L.vmesh, 0.0, ns);
-  hipLaunchKernelGGL(k_visc_tangent_node, g, b, 0, c->stream, V, P, (const double *)nullptr, S.taud, (ad::Dual *)nullptr);
+  launch_nodes(L, [&](auto sc, dim3 gl) {
+    hipLaunchKernelGGL(k_visc_stress<decltype(sc)::value>, gl, b, 0, c->stream, V, P, S.taud);
+  });
   launch_nodes(L, [&](auto sc, dim3 gl) {
     hipLaunchKernelGGL(k_visc_adjoint_tau<decltype(sc)::value>, gl, b, 0, c->stream, V, P, V.src,
                        (const ad::Dual *)S.taud, S.taub, S.ubv);
@@ -2501,7 +2502,9 @@ int visc_friction_reverse(flite_ctx *c, Level &L, bool mesh) {
   double PI = 4.0 * std::atan(1.0);
   double ar = hp.alpha * PI / 180., br = hp.beta * PI / 180.;
   double t0 = std::cos(ar) * std::cos(br), t1 = std::sin(br), t2 = std::sin(ar);
-  hipLaunchKernelGGL(k_visc_tangent_node, g, b, 0, c->stream, V, P, (const double *)nullptr, S.taud, (ad::Dual *)nullptr);
+  launch_nodes(L, [&](auto sc, dim3 gl) {
+    hipLaunchKernelGGL(k_visc_stress<decltype(sc)::value>, gl, b, 0, c->stream, V, P, S.taud);
+  });
   hipLaunchKernelGGL(k_fill<double>, dim3(nblk((long long)(9 * n))), b, 0, c->stream, S.taub, 0.0, 9 * n);
   hipLaunchKernelGGL(k_fill<double>, dim3(nblk((long long)(4 * n))), b, 0, c->stream, S.gaf, 0.0, 4 * n);
   const int nw = (int)L.wall_dev.size();
@@ -2573,18 +2576,20 @@ int tangent_core(flite_ctx *c) {
     TRY(op_prep(c, L, true));
     TRY(op_grad(c, L));
     TRY(alloc_lin(L));
-    double *dq = L.lin;
-    ad::Dual *gd = reinterpret_cast<ad::Dual *>(L.lin + DQ * (size_t)L.n);
+    double *dq = L.lin, *gt = L.lin + DQ * (size_t)L.n;
     hipLaunchKernelGGL(k_record_tangent, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, P, V.src, dq);
-    hipLaunchKernelGGL(k_grad_tangent, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, (const double *)dq, gd);
+    hipLaunchKernelGGL(k_minmax_arg, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, V, L.amin);
+    launch_nodes(L, [&](auto sc, dim3 gl) {
+      hipLaunchKernelGGL(k_grad_tangent<decltype(sc)::value>, gl, dim3(NTHR), 0, c->stream, V, (const double *)dq,
+                         (const int *)L.amin, gt);
+    });
     if (L.ne > 0) {
       dim3 ge(nblk(L.ne)), be(NTHR);
-      const double *dqc = dq;
-      const ad::Dual *gdc = gd;
-      if (P.nsig == 4 && P.sa) hipLaunchKernelGGL((k_flux_tangent2<4, true>), ge, be, 0, c->stream, V, P, dqc, gdc);
-      else if (P.nsig == 4) hipLaunchKernelGGL((k_flux_tangent2<4, false>), ge, be, 0, c->stream, V, P, dqc, gdc);
-      else if (P.sa) hipLaunchKernelGGL((k_flux_tangent2<2, true>), ge, be, 0, c->stream, V, P, dqc, gdc);
-      else hipLaunchKernelGGL((k_flux_tangent2<2, false>), ge, be, 0, c->stream, V, P, dqc, gdc);
+      const double *dqc = dq, *gtc = gt;
+      if (P.nsig == 4 && P.sa) hipLaunchKernelGGL((k_flux_tangent2<4, true>), ge, be, 0, c->stream, V, P, dqc, gtc);
+      else if (P.nsig == 4) hipLaunchKernelGGL((k_flux_tangent2<4, false>), ge, be, 0, c->stream, V, P, dqc, gtc);
+      else if (P.sa) hipLaunchKernelGGL((k_flux_tangent2<2, true>), ge, be, 0, c->stream, V, P, dqc, gtc);
+      else hipLaunchKernelGGL((k_flux_tangent2<2, false>), ge, be, 0, c->stream, V, P, dqc, gtc);
     }
   } else if (L.ne > 0) {
     if (P.sa) hipLaunchKernelGGL(k_flux_tangent<true>, dim3(nblk(L.ne)), dim3(NTHR), 0, c->stream, V, P, V.src);
@@ -2596,8 +2601,9 @@ int tangent_core(flite_ctx *c) {
   StageArgs S{};
   TRY(op_stage(c, L, MODE_RHS, S));
   if (laminar(c)) {
-    if (!second_order(c, L)) TRY(op_prep(c, L, true));
-    TRY(visc_tangent(c, L));
+    const bool second = second_order(c, L);
+    if (!second) TRY(op_prep(c, L, true));
+    TRY(visc_tangent(c, L, second ? L.lin : nullptr));
   }
   return 0;
 }
