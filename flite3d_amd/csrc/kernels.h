@@ -2218,7 +2218,8 @@ __global__ __launch_bounds__(NTHR) void k_flux_tangent2(LevelDev<double> L, DevP
 // of that end's bounds.  Per component: the share on the projection, on the
 // bound, and 3 bits of the code: 1 (first end) or 2 (second) or 0 (none), + 4
 // for the upper bound.  (15 dual passes of the flux and 60 stored words took
-// 1.9 ms and the gather 0.57 ms at 64^3; 0.31 and 0.37 now.)
+// 1.9 ms and the gather 0.57 ms at 64^3; 0.25 and 0.23 now, 0.33 of the first
+// before the two gradient records were read as whole aligned pairs.)
 template <int NSIG>
 __global__ __launch_bounds__(NTHR) void k_flux_adjoint2(LevelDev<double> L, DevParams P, const double *lam,
                                                         double *abuf2) {
@@ -2231,7 +2232,9 @@ __global__ __launch_bounds__(NTHR) void k_flux_adjoint2(LevelDev<double> L, DevP
   ldrec<8>(L.rec0 + 8 * (size_t)ib, B);
 #pragma unroll
   for (int c = 0; c < 5; ++c) dl[c] = lam[c * n + ia] - lam[c * n + ib];
-  const double *ga = L.grec + GREC * (size_t)ia, *gb = L.grec + GREC * (size_t)ib;
+  double ga[GREC], gb[GREC];
+  ldrec<GREC>(L.grec + GREC * (size_t)ia, ga);
+  ldrec<GREC>(L.grec + GREC * (size_t)ib, gb);
   const double *xa = L.xyz + 3 * (size_t)ia, *xb = L.xyz + 3 * (size_t)ib;
   const double dx = xb[0] - xa[0], dy = xb[1] - xa[1], dz = xb[2] - xa[2];
   const double hl = 0.5 * P.clip * ::sqrt(dx * dx + dy * dy + dz * dz);
@@ -2290,54 +2293,72 @@ __global__ __launch_bounds__(NTHR) void k_flux_adjoint2(LevelDev<double> L, DevP
 // gbn = its gradient and bound shares.  SCALED: the gradients' divided by the
 // node's volume and the bounds' times their squares, GREC words a node, as
 // k_grad_adjoint reads its neighbours'.
+// A side's words are read as aligned pairs, whole, and masked afterwards (a
+// load behind each mask waits for the one before), and the scaled records are
+// stored through LDS: 360 -> 226 us on 275k nodes with 1.87M sides.
 template <bool SCALED, int SUB>
 __global__ __launch_bounds__(NTHR) void k_adjoint_gather2(LevelDev<double> L, const double *abuf2, double *ub, double *gbn) {
+  constexpr bool STORE = SCALED && SUB == 1;
+  __shared__ double st[STORE ? NTHR * (GREC / 2) : 1];
   int i, sub, bb_;
   node_lanes<SUB>(1, bb_, i, sub);
-  if (i >= L.n) return;
-  double r[5] = {0, 0, 0, 0, 0}, g[LIN_G];
+  if (!STORE && i >= L.n) return;
+  double r[5] = {0, 0, 0, 0, 0}, g[GREC];
 #pragma unroll
-  for (int c = 0; c < LIN_G; ++c) g[c] = 0;
-  for_edges<SUB>(L, i, sub, [&](int e, int role) {
-    const double *a = abuf2 + LIN_SIDE * (size_t)e, *u = a + 19 * role;
-    const double hx = 0.5 * a[15], hy = 0.5 * a[16], hz = 0.5 * a[17];
-    const int code = int(a[18]);
+  for (int c = 0; c < GREC; ++c) g[c] = 0;
+  if (i < L.n) {
+    for_edges<SUB>(L, i, sub, [&](int e, int role) {
+      const double *a = abuf2 + LIN_SIDE * (size_t)e;
+      double u[6], w[16];  // words 0 .. 5 or 18 .. 23, and 4 .. 19
+      ldrec<6>(a + 18 * role, u);
+      ldrec<16>(a + 4, w);
+      const double hx = 0.5 * w[11], hy = 0.5 * w[12], hz = 0.5 * w[13];
+      const int code = int(w[14]);
 #pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      r[c] += u[c];
-      const int k = code >> (3 * c);
-      const bool mine = (k & 3) == role + 1;
-      const double v = mine ? a[5 + c] : 0.0, b = mine ? a[10 + c] : 0.0;
-      g[c] += v * hx;
-      g[5 + c] += v * hy;
-      g[10 + c] += v * hz;
-      g[15 + c] += k & 4 ? 0.0 : b;
-      g[20 + c] += k & 4 ? b : 0.0;
+      for (int c = 0; c < 5; ++c) {
+        r[c] += role ? u[c + 1] : u[c];
+        const int k = code >> (3 * c);
+        const bool mine = (k & 3) == role + 1;
+        const double v = mine ? w[1 + c] : 0.0, b = mine ? w[6 + c] : 0.0;
+        g[c] += v * hx;
+        g[5 + c] += v * hy;
+        g[10 + c] += v * hz;
+        g[15 + c] += k & 4 ? 0.0 : b;
+        g[20 + c] += k & 4 ? b : 0.0;
+      }
+    });
+    for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
+      int v = L.bs_list[k];
+      const double *b = L.bbuf + 10 * (size_t)(v >> 1) + 5 * (v & 1);
+#pragma unroll
+      for (int c = 0; c < 5; ++c) r[c] += b[c];
     }
-  });
-  for (int k = L.bs_ptr[i] + sub; k < L.bs_ptr[i + 1]; k += SUB) {
-    int v = L.bs_list[k];
-    const double *b = L.bbuf + 10 * (size_t)(v >> 1) + 5 * (v & 1);
-#pragma unroll
-    for (int c = 0; c < 5; ++c) r[c] += b[c];
   }
 #pragma unroll
   for (int c = 0; c < 5; ++c) r[c] = lsum<SUB>(r[c]);
 #pragma unroll
   for (int c = 0; c < LIN_G; ++c) g[c] = lsum<SUB>(g[c]);
-  if (sub) return;
+  const bool ok = i < L.n && !sub;
+  if (ok) {
 #pragma unroll
-  for (int c = 0; c < 5; ++c) ub[5 * (size_t)i + c] = r[c];
-  if constexpr (SCALED) {
-    const double iv = 1.0 / L.vol[i], *B = L.grec + GREC * (size_t)i;
-    double *o = gbn + GREC * (size_t)i;
+    for (int c = 0; c < 5; ++c) ub[5 * (size_t)i + c] = r[c];
+    if constexpr (SCALED) {
+      const double iv = 1.0 / L.vol[i];
+      double B[12];  // words 14 .. 25 of the gradient record
+      ldrec<12>(L.grec + GREC * (size_t)i + 14, B);
 #pragma unroll
-    for (int c = 0; c < 15; ++c) o[c] = g[c] * iv;
+      for (int c = 0; c < 15; ++c) g[c] *= iv;
 #pragma unroll
-    for (int c = 15; c < LIN_G; ++c) o[c] = g[c] * B[c] * B[c];
-  } else {
+      for (int c = 15; c < LIN_G; ++c) g[c] = g[c] * B[c - 14] * B[c - 14];
+    }
+  }
+  if constexpr (STORE) {
+    const int i0 = i - (int)threadIdx.x;
+    store_grec(st, g, ok, gbn + GREC * (size_t)i0, L.n - i0 < NTHR ? L.n - i0 : NTHR);
+  } else if (ok) {
+    constexpr int NW = SCALED ? GREC : LIN_G;
 #pragma unroll
-    for (int c = 0; c < LIN_G; ++c) gbn[LIN_G * (size_t)i + c] = g[c];
+    for (int c = 0; c < NW; ++c) gbn[NW * (size_t)i + c] = g[c];
   }
 }
 
@@ -2346,7 +2367,8 @@ __global__ __launch_bounds__(NTHR) void k_adjoint_gather2(LevelDev<double> L, co
 // k_adjoint_gather2<true> scales it, so a neighbour costs its 15 gradient
 // shares, its ten extremal-neighbour indices and a bound's share only where
 // node j attains it (with the raw shares, the volumes and the bounds read per
-// neighbour it took 462 us at 64^3, 161 now).
+// neighbour it took 462 us at 64^3, 161 now; with the bounds' shares always
+// read, 270: the two more lines a neighbour cost more than the branches).
 template <int SUB>
 __global__ __launch_bounds__(NTHR) void k_grad_adjoint(LevelDev<double> L, const double *gbn, const int *amin, double *qb) {
   int j, sub, bb_;
