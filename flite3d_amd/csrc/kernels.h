@@ -1,6 +1,6 @@
 // Device kernels of the MI355X flow-solver hot path (gfx950, wave64).
 //
-// Layout (device numbering, RCM order, see solver.hip):
+// Layout (device numbering, nested Morton order, see solver.hip):
 //   node state      u[c*n+i] (SoA, 6 comps), uprev, p, dt, dtt, mu, vort,
 //                   divg, diss[5], src[6], tdiff
 //   rec0[8*i]       AoS per node: rho, u, v, w, rhoE, p, nu~, mu  (gathers)
@@ -17,8 +17,9 @@
 // Every edge loop of the reference (scatter to both ends) is evaluated here
 // as a gather at each node over its incidence list in a fixed order, so
 // results are deterministic and no atomics are used.  The HLLC flux is the
-// exception: it is evaluated once per edge into fbuf and gathered by the
-// stage-update kernel.
+// exception: it is evaluated once per edge, in blocks of sides whose per-node
+// sums the stage kernel adds, or, on small first-order levels, in the stage's
+// own blocks of nodes (k_stage_blk).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -35,7 +36,8 @@ constexpr int GREC = 26;
 // viscosity | nodal cb2 term | pad.  (Stress, velocity, grad nu~ and the
 // diffusion coefficient's three factors took this line and the neighbour's
 // gather record: the second pass, staged, took 838 us with the SA time steps
-// and 767 without on 2.1M nodes, 601 and 441 now.)
+// and 767 without on 2.1M nodes; 601 and 441 with this record, 535 and 419
+// since the staging's loads are in flight together.)
 constexpr int VREC = 16;
 constexpr int NTHR = 256;
 
@@ -496,9 +498,8 @@ __global__ void k_pack(LevelDev<R> L, DevParams P) {
 // of a walk part (init / edge / bside / reduce / finish, like the gather
 // parts below): Green-Gauss sums over the interior sides (q_i + q_j) w and
 // the boundary sides (3 q_i + q_o) w, and the minimum and maximum of the
-// neighbours' values.  Carried along the viscous pass 1's walk it made that
-// walk slower than a walk of its own (register pressure), so the gradient
-// kernels walk it alone.
+// neighbours' values.  GradViscPart carries it along the viscous pass 1 where
+// both are due; elsewhere the gradient kernels walk it alone.
 template <typename R>
 struct GradPart {
   static constexpr int AUXW = 0;
@@ -2576,6 +2577,22 @@ __device__ __forceinline__ void visc_vort_divg(const T *g, TV vol, T &vort, T &d
   divg = dudx + dvdy + dwdz;
 }
 
+// viscosity and conductivity of the stress law, the eddy viscosity's shares
+// included with Spalart-Allmaras
+template <typename T>
+__device__ __forceinline__ void visc_coef(const DevParams &P, T Traw, T rho, T nu, T &mu, T &k) {
+  mu = sutherland(P, Traw);
+  k = T(1.0 / P.Pr) * mu;
+  if (P.sa) {
+    T tvc = T(1.0 / P.Re) * rho * nu;
+    T ksi = tvc / mu;
+    T k3 = ksi * ksi * ksi;
+    tvc = tvc * k3 / (k3 + T(357.9));
+    mu = mu + tvc;
+    k = k + tvc * T(1.0 / P.Prt);
+  }
+}
+
 // stress and heat flux of a node; with Spalart-Allmaras the eddy viscosity
 // of (rho, nu~) is added to both (DEF:5556-5566).  The volume and the wall
 // normal are of type TV (double, or dual numbers for the mesh derivatives).
@@ -2586,16 +2603,8 @@ __device__ __forceinline__ void visc_tau(const DevParams &P, const T *g, TV vol,
   T dudx = g[0] * vt, dvdx = g[1] * vt, dwdx = g[2] * vt, dTdx = g[3] * vt;
   T dudy = g[4] * vt, dvdy = g[5] * vt, dwdy = g[6] * vt, dTdy = g[7] * vt;
   T dudz = g[8] * vt, dvdz = g[9] * vt, dwdz = g[10] * vt, dTdz = g[11] * vt;
-  T mu = sutherland(P, Traw);
-  T k = T(1.0 / P.Pr) * mu;
-  if (P.sa) {
-    T tvc = T(1.0 / P.Re) * rho * nu;
-    T ksi = tvc / mu;
-    T k3 = ksi * ksi * ksi;
-    tvc = tvc * k3 / (k3 + T(357.9));
-    mu = mu + tvc;
-    k = k + tvc * T(1.0 / P.Prt);
-  }
+  T mu, k;
+  visc_coef(P, Traw, rho, nu, mu, k);
   T two3 = T(2.0 / 3.0), four3 = T(4.0 / 3.0);
   t[0] = mu * (four3 * dudx - two3 * (dvdy + dwdz));
   t[1] = mu * (dudy + dvdx);
@@ -2919,8 +2928,10 @@ __global__ __launch_bounds__(NTHR) void k_visc_adjoint_tau(LevelDev<double> L, D
 // Green-Gauss sums and tbar on T (through the viscosity).  With
 // Spalart-Allmaras the stress reads the eddy viscosity of (rho, nu~) and
 // the node's SA source (multiplier lam(6)) reads rho, nu~, the laminar
-// viscosity of T and the vorticity and divergence of the same sums: two more
-// passes, rnbar[2 i ..] = the shares on (rho, nu~).  lam may be null (no
+// viscosity of T and the vorticity and divergence of the same sums;
+// rnbar[2 i ..] = the shares on (rho, nu~).  The shares on the sums are closed
+// forms, the others a dual pass each (with a pass for each sum too: 213 us at
+// 275k nodes, NOWVN now).  lam may be null (no
 // source term: the drag's friction alone drives taub).  With mbar (5 per
 // node) also the shares on the mesh quantities the node reads: its volume,
 // its wall normal (wall nodes, the adiabatic projection) and, with
@@ -2939,16 +2950,56 @@ __global__ __launch_bounds__(NTHR) void k_visc_adjoint_node(LevelDev<double> L, 
   const double l6 = (P.sa && lam) ? lam[5 * (size_t)L.n + i] : 0.0;
   const double *nr = L.nrm + 3 * (size_t)i;
   double m[5] = {0, 0, 0, 0, 0};
-  // seeds: 0-11 the sums, 12 T, 13 rho, 14 nu~, 15 V, 16-18 the normal,
-  // 19 the wall distance
+  const double vt = 1.0 / L.vol[i];
+  {
+    // the sums: the stress and heat flux are linear in them, the source reads
+    // the vorticity (one dual pass for its share) and the divergence
+    double mu, k, gb[12];
+    visc_coef(P, Tv, qi[0], qi[6], mu, k);
+    mu *= vt;
+    k *= vt;
+    const double tr = 2.0 / 3.0 * (tb[0] + tb[3] + tb[5]);
+    gb[0] = mu * (2.0 * tb[0] - tr);
+    gb[5] = mu * (2.0 * tb[3] - tr);
+    gb[10] = mu * (2.0 * tb[5] - tr);
+    gb[1] = gb[4] = mu * tb[1];
+    gb[2] = gb[8] = mu * tb[2];
+    gb[6] = gb[9] = mu * tb[4];
+    const double nt = wall ? tb[6] * nr[0] + tb[7] * nr[1] + tb[8] * nr[2] : 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) gb[4 * d + 3] = k * (wall ? tb[6 + d] - nt * nr[d] : tb[6 + d]);
+    if (l6 != 0.0) {
+      double vort, divg, ml = sutherland(P, Tv);
+      visc_vort_divg(gv, L.vol[i], vort, divg);
+      if (ml < 0.1 / P.Re) ml = 0.1 * P.Re;
+      const Dual S = sa_source_t<Dual, Dual>(P, Dual(qi[0]), Dual(qi[6]), Dual(ml), Dual(vort, 1.0), Dual(divg),
+                                             Dual(L.wd[i]), Dual(L.vol[i]));
+      const double sv = vort > 0.0 ? l6 * S.d * vt * vt / vort : 0.0;
+      const double sd = -l6 * (qi[6] > 0.0 ? qi[6] : 0.0);
+      const double c1 = sv * (gv[4] - gv[1]), c2 = sv * (gv[9] - gv[6]), c3 = sv * (gv[2] - gv[8]);
+      gb[4] += c1;
+      gb[1] -= c1;
+      gb[9] += c2;
+      gb[6] -= c2;
+      gb[2] += c3;
+      gb[8] -= c3;
+      gb[0] += sd;
+      gb[5] += sd;
+      gb[10] += sd;
+    }
+    double2 *o = reinterpret_cast<double2 *>(gbar + 12 * (size_t)i);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) o[c] = make_double2(gb[2 * c], gb[2 * c + 1]);
+  }
+  // seeds: 12 T, 13 rho, 14 nu~, 15 V, 16-18 the normal, 19 the wall distance
   const int passes = mbar ? 20 : (P.sa ? 15 : 13);
 #pragma unroll 1
-  for (int k = 0; k < passes; ++k) {
+  for (int k = 12; k < passes; ++k) {
     if ((k == 13 || k == 14 || k == 19) && !P.sa) continue;
     if (k >= 16 && k <= 18 && !wall) continue;
     Dual gs[12], t[9];
 #pragma unroll
-    for (int c = 0; c < 12; ++c) gs[c] = Dual(gv[c], k == c ? 1.0 : 0.0);
+    for (int c = 0; c < 12; ++c) gs[c] = Dual(gv[c]);
     const Dual T(Tv, k == 12 ? 1.0 : 0.0), R(qi[0], k == 13 ? 1.0 : 0.0), N(qi[6], k == 14 ? 1.0 : 0.0);
     const Dual Vd(L.vol[i], k == 15 ? 1.0 : 0.0), Wd(L.wd[i], k == 19 ? 1.0 : 0.0);
     const Dual nd[3] = {Dual(nr[0], k == 16 ? 1.0 : 0.0), Dual(nr[1], k == 17 ? 1.0 : 0.0),
@@ -2965,8 +3016,7 @@ __global__ __launch_bounds__(NTHR) void k_visc_adjoint_node(LevelDev<double> L, 
       visc_vort_divg(gs, Vd, vort, divg);
       acc += l6 * sa_source_t<Dual, Dual>(P, R, N, mu, vort, divg, Wd, Vd).d;
     }
-    if (k < 12) gbar[12 * (size_t)i + k] = acc;
-    else if (k == 12) tbar[i] = acc;
+    if (k == 12) tbar[i] = acc;
     else if (k < 15) rnbar[2 * (size_t)i + (k - 13)] = acc;
     else if (k == 15) m[0] = acc;
     else if (k == 16) m[1] = acc;
