@@ -1,0 +1,121 @@
+"""Sizes at which a launch shape or a kernel's split changes, on the GPU
+against the oracle, and the lanes-per-node variants of the linearised
+kernels against each other.
+
+Bars as in test_gpu_parity: 1e-11 of the component scale for single
+operations, 1e-9 for states after whole V-cycles, 1e-8 for monitor sums and
+forces.  The lanes of the linearised kernels only change the order of sums of
+at most a few dozen terms, each combined once per stage of the chain, so their
+results are held to the single operations' 1e-11.
+"""
+import numpy as np
+import pytest
+
+from flite3d_amd.device import Solver
+
+from cases import euler, levels, rans
+from test_gpu_parity import jst_case, pair, perturb, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def cycles_match(iv, lv, n=3):
+    s, o = pair(iv, lv)
+    s.init_freestream(); o.init_freestream()
+    for c in range(1, n + 1):
+        s.cycle(c); o.cycle(c)
+    ms, mo = s.monitor(), o.monitor()
+    assert np.allclose(ms["res"], mo["res"], rtol=1e-8, atol=1e-16), (ms["res"], mo["res"])
+    assert np.allclose(ms["forces"], mo["forces"], rtol=1e-8, atol=1e-14), (ms["forces"], mo["forces"])
+    nc = 6 if iv.turbulencemodel == 1 else 5
+    e = rel_err(s.get(1, "U")[:nc], o.get(1, "U")[:nc])
+    s.close(); o.close()
+    assert e.max() < 1e-9, e
+
+
+@pytest.mark.parametrize("n,nl", [(2, 1), (3, 2), (4, 2), (9, 3), (17, 3)])
+@pytest.mark.parametrize("kind", ["euler1", "euler2", "rans"])
+def test_cycles_at_block_remainders(kind, n, nl):
+    """The smallest meshes (less than one wavefront of nodes), node and side
+    blocks with remainders on each level, and 324 wall nodes (n = 17), beyond
+    the force integral's one-wavefront order."""
+    print(f"[case] {kind} n={n} levels={nl}", flush=True)
+    iv = rans(multigridscheme=3) if kind == "rans" else euler(int(kind[-1]), multigridscheme=3)
+    cycles_match(iv, levels(n, nl, first_cell=0.01 if kind == "rans" else None))
+
+
+@pytest.mark.parametrize("n", [25, 40])
+def test_first_order_stage_rule(n):
+    """Both sides of the size rule of the one-launch first-order stage without
+    a turbulence equation (17.6k and 68.9k level-1 nodes): the state after two
+    cycles as the oracle has it."""
+    print(f"[case] first-order stage rule n={n}", flush=True)
+    cycles_match(euler(1, multigridscheme=3), levels(n, 2), 2)
+
+
+@pytest.mark.parametrize("lanes", ["1", "4", "16"])
+@pytest.mark.parametrize("name", ["llf", "roe_matrix"])
+def test_jst_lanes(name, lanes, monkeypatch):
+    print(f"[case] jst {name} lanes {lanes}", flush=True)
+    monkeypatch.setenv("FLITE_GATHER_LANES", lanes)
+    s, o = pair(jst_case(name), levels(9, 2))
+    s.init_freestream(); o.init_freestream()
+    perturb(s, o, 1, np.random.default_rng(5), amp=0.05)
+    for x in (s, o):
+        x.apply(1, "PRESSURE_ABS")
+        x.apply(1, "TIMESTEPS")
+        x.apply(1, "DISSIPATION")
+        x.apply(1, "RHS")
+    for f in ("DT", "DISSIPATION", "RHS"):
+        e = rel_err(s.get(1, f), o.get(1, f))
+        assert e.max() < 1e-11, (f, e)
+    s.close(); o.close()
+
+
+@pytest.mark.parametrize("order,fp32", [(1, False), (2, True)])
+def test_fields_round_trip(order, fp32):
+    """Fields renumbered on the device come back as they went in, on each
+    level: bit for bit in FP64, as the nearest FP32 on FP32 levels."""
+    print(f"[case] field round trip order={order} fp32={fp32}", flush=True)
+    lv = levels(9, 3)
+    s, o = pair(euler(order), lv, fp32)
+    o.close()
+    s.init_freestream()
+    rng = np.random.default_rng(8)
+    for k in range(1, 4):
+        u = s.get(k, "U")
+        u = u * (1.0 + 0.1 * rng.uniform(-1, 1, size=u.shape))
+        s.set(k, "U", u)
+        want = u.astype(np.float32).astype(np.float64) if fp32 and k > 1 else u
+        assert np.array_equal(s.get(k, "U")[:5], want[:5]), k
+    s.close()
+
+
+@pytest.mark.parametrize("kind", ["euler1", "euler2", "rans1", "rans2"])
+def test_linearised_lanes(kind, monkeypatch):
+    print(f"[case] linearised lanes {kind}", flush=True)
+    order = int(kind[-1])
+    sa = kind.startswith("rans")
+    iv = rans(hllcfluxorder=order) if sa else euler(order)
+    lv = levels(9, 1, first_cell=0.01 if sa else None)
+    nc = 6 if sa else 5
+    got = {}
+    for lanes in ("1", "4", "16"):
+        monkeypatch.setenv("FLITE_GATHER_LANES", lanes)
+        s = Solver(iv.to_struct(), list(lv))
+        s.init_freestream()
+        rng = np.random.default_rng(9)
+        u = s.get(1, "U")
+        u = u * (1.0 + 0.02 * rng.uniform(-1, 1, size=u.shape))
+        if sa:
+            u[5] = 0.1 + 5.0 * rng.uniform(0, 1, size=u.shape[1])
+        s.set(1, "U", u)
+        s.apply(1, "PRESSURE")
+        v = rng.standard_normal((nc, u.shape[1]))
+        got[lanes] = s.tangent(v), s.adjoint(v)
+        s.close()
+    for lanes in ("1", "4"):
+        for a, b in zip(got[lanes], got["16"]):
+            assert np.abs(b).max() > 0
+            e = rel_err(a, b)
+            assert e.max() < 1e-11, (lanes, e)
