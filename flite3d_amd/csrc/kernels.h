@@ -23,6 +23,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../include/flite3d_amd.h"
 
 namespace fk {
@@ -351,8 +353,9 @@ __device__ __forceinline__ void for_edges(const LevelDev<R> &L, int i, int sub, 
 // side's first end, -w when it is the second): f(nbr, wx, wy, wz).  A
 // reference scatter "+f to i1, -f to i2" with f linear in w becomes "+f(w_s)"
 // here, with the same rounding since the sign flip is exact.
+// for_slots also passes the slot, for the side and the node's role in it.
 template <int SUB, typename R, typename F>
-__device__ __forceinline__ void for_edges_w(const LevelDev<R> &L, int i, int sub, F f) {
+__device__ __forceinline__ void for_slots(const LevelDev<R> &L, int i, int sub, F f) {
   int s = i / SLICE, lane = i % SLICE;
   int base = L.ell_ptr[s], K = L.ell_k[s];
   const long long ns = L.nslot;
@@ -360,8 +363,12 @@ __device__ __forceinline__ void for_edges_w(const LevelDev<R> &L, int i, int sub
     int slot = base + k * SLICE + lane;
     int j = ldnt(L.ell_nbr + slot);
     if (j < 0) continue;
-    f(j, ldnt(L.ellw + slot), ldnt(L.ellw + ns + slot), ldnt(L.ellw + 2 * ns + slot));
+    f(slot, j, ldnt(L.ellw + slot), ldnt(L.ellw + ns + slot), ldnt(L.ellw + 2 * ns + slot));
   }
+}
+template <int SUB, typename R, typename F>
+__device__ __forceinline__ void for_edges_w(const LevelDev<R> &L, int i, int sub, F f) {
+  for_slots<SUB>(L, i, sub, [&](int, int j, R wx, R wy, R wz) { f(j, wx, wy, wz); });
 }
 
 // ---------------------------------------------------------------------------
@@ -706,6 +713,21 @@ __device__ __forceinline__ R led(R a, R ilo, R ihi) {
 // too when their derivatives are wanted.
 // upwinded SA convection of one side (makeSARHS, DEF:6873-6880) from the
 // ends' gather records
+//
+// Its linearisation takes the upwind term's sign from sa_upwind alone: x =
+// w.(m_b - m_a) of m = nu~ v against nu~_a - nu~_b, 0 where either vanishes
+// (fluid at rest at both ends, say), which counts as positive seen from the
+// side's first end.  Without contraction x has the same bits from either end
+// (differences and weights change sign together), so the tangent and both
+// ends' shares of the adjoint take one branch.
+__device__ __forceinline__ int sa_upwind(const double *ma, const double *mb, double ta, double tb, double wx, double wy,
+                                         double wz) {
+#pragma clang fp contract(off)
+  const double x = wx * (mb[0] * tb - ma[0] * ta) + wy * (mb[1] * tb - ma[1] * ta) + wz * (mb[2] * tb - ma[2] * ta);
+  const double dt = ta - tb;
+  if (x == 0.0 || dt == 0.0) return 0;
+  return (x < 0.0) == (dt < 0.0) ? 1 : -1;
+}
 template <typename T>
 __device__ __forceinline__ T sa_side_convection(const T *A, const T *B, T wx, T wy, T wz) {
   T u1 = A[1], v1 = A[2], w1 = A[3], t1 = A[6];
@@ -715,7 +737,14 @@ __device__ __forceinline__ T sa_side_convection(const T *A, const T *B, T wx, T 
   if (fabs(dtt) > T(1e-20)) {
     T id = frcp(dtt);
     T ax = (u2 * t2 - u1 * t1) * id, ay = (v2 * t2 - v1 * t1) * id, az = (w2 * t2 - w1 * t1) * id;
-    fsa = fsa + fabs(wx * ax + wy * ay + wz * az) * dtt;
+    T y = wx * ax + wy * ay + wz * az;
+    if constexpr (std::is_same_v<T, ad::Dual>) {
+      const double ma[3] = {u1.v, v1.v, w1.v}, mb[3] = {u2.v, v2.v, w2.v};
+      y = sa_upwind(ma, mb, t1.v, t2.v, wx.v, wy.v, wz.v) < 0 ? -y : y;
+    } else {
+      y = fabs(y);
+    }
+    fsa = fsa + y * dtt;
   }
   return fsa;
 }
@@ -1836,9 +1865,12 @@ __global__ __launch_bounds__(NTHR) void k_adjoint_gather(LevelDev<double> L, con
 // the velocities): node i's share of sum over sides of (lam6_ea - lam6_eb) f6,
 // added to out.  With m = nu~ v, X = w.(m_b - m_a) and s the sign of X / (nu~_a
 // - nu~_b), f6 = w.(m_a + m_b) + s X, so with the node-signed weight node i's
-// own m enters a side's term as (lam_i - lam_j)(1 - s) w.m_i: the walk sums
-// that one vector, and its shares on v and nu~ follow at the end.  (Six dual
-// passes of every side took 168 us at 275k nodes, 73 now.)
+// own m enters a side's term as (lam_i - lam_j)(1 - s) w.m_i from the first
+// end and (1 + s) from the second: the walk sums that one vector, and its
+// shares on v and nu~ follow at the end.  sa_upwind from the node has the sign
+// of s at the first end and of -s at the second, so the role is read only
+// where it is 0.  (Six dual passes of every side took 168 us at 275k nodes,
+// 73 now.)
 template <int SUB>
 __global__ __launch_bounds__(NTHR) void k_sa_conv_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *out) {
   int i, sub, bb_;
@@ -1848,15 +1880,13 @@ __global__ __launch_bounds__(NTHR) void k_sa_conv_adjoint(LevelDev<double> L, De
   double qi[8], z[3] = {0, 0, 0};
   ldrec<8>(L.rec0 + 8 * (size_t)i, qi);
   const double li = lam[5 * n + i];
-  for_edges_w<SUB>(L, i, sub, [&](int j, double wx, double wy, double wz) {
+  for_slots<SUB>(L, i, sub, [&](int slot, int j, double wx, double wy, double wz) {
     double qj[8];
     ldrec<8>(L.rec0 + 8 * (size_t)j, qj);
-    const double dt = qi[6] - qj[6];
     double c = li - lam[5 * n + j];
-    if (::fabs(dt) > 1e-20) {
-      const double x = wx * (qj[1] * qj[6] - qi[1] * qi[6]) + wy * (qj[2] * qj[6] - qi[2] * qi[6]) +
-                       wz * (qj[3] * qj[6] - qi[3] * qi[6]);
-      c *= x / dt < 0.0 ? 2.0 : 0.0;
+    if (::fabs(qi[6] - qj[6]) > 1e-20) {
+      const int s = sa_upwind(qi + 1, qj + 1, qi[6], qj[6], wx, wy, wz);
+      c *= s < 0 || (s == 0 && (L.ell_e[slot] & 1)) ? 2.0 : 0.0;
     }
     z[0] += c * wx;
     z[1] += c * wy;

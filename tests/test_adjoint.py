@@ -569,3 +569,38 @@ def test_device_vector_applies_equal_host_ones(kind):
     with pytest.raises(DeviceError):
         s.tangent_device(x.ctypes.data, x.ctypes.data)
     s.close()
+
+
+@pytest.mark.parametrize("state", ["rest", "uniform"])
+@pytest.mark.parametrize("order", [1, 2])
+def test_rans_adjoint_dot_product_where_the_upwind_term_vanishes(order, state):
+    """The SA convection's upwind term is exactly zero on a side whose ends
+    are at rest, or whose weight is normal to a uniform flow, while nu~
+    differs: tangent and adjoint take the same branch there too.  nu~'s row
+    against the velocities and density holds the convection; the bar is that
+    of the other states."""
+    from cases import rans
+    print(f"[case] RANS-SA adjoint at vanishing upwind terms order={order} {state}", flush=True)
+    lv = levels(8, 2, jitter=0.0)
+    iv = rans(hllcfluxorder=order, reynoldsnumber=1.0e4)
+    s = Solver(iv.to_struct(), list(lv))
+    s.init_freestream()
+    inf = np.array(iv.inflowfield[0])
+    x, y, z = lv[0].coords
+    u = np.zeros((6, lv[0].n_nodes))
+    u[0], u[4] = inf[0], inf[4]
+    if state == "uniform":
+        u[1] = inf[0]
+    u[5] = 3.0 * (1.0 + 0.3 * np.sin(1.7 * x + 0.9 * y - 1.3 * z + 0.2))
+    s.set(1, "U", u)
+    s.apply(1, "PRESSURE")
+    rng = np.random.default_rng(59)
+    for rows, cols in [(range(6), range(6)), ([5], [0]), ([5], [1, 2, 3]), ([5], [5])]:
+        du, lam = rng.standard_normal((2, 6, u.shape[1]))
+        du[[c for c in range(6) if c not in cols]] = 0.0
+        lam[[c for c in range(6) if c not in rows]] = 0.0
+        terms = lam * s.tangent(du)
+        a, b = np.sum(terms), np.sum(s.adjoint(lam) * du)
+        scale = np.sqrt(np.sum(terms ** 2))
+        assert abs(a - b) <= 1e-12 * max(abs(a), abs(b), scale), (list(rows), list(cols), a, b)
+    s.close()
