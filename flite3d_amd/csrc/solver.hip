@@ -1727,8 +1727,9 @@ int do_cycle(flite_ctx *c, int cycle) {
     for (int i = 1; i < ng; ++i) {
       TRY(do_time_iterations(c, i, nrs, i == 1, more && i > 1, true));
       TRY(do_restrict(c, i, more));
-      Level &F = *c->lev[i - 1];
-      TRY(op_map_state(c, F, *c->lev[i]));
+      Level &F = *c->lev[i - 1], &K = *c->lev[i];
+      // without a smoothing step to start, the coarse level keeps its pressure and previous state
+      TRY(more ? op_map_state(c, F, K) : op_restrict_array(c, F, K, F.u, K.u));
     }
     TRY(do_time_iterations(c, ng, nrs, ng == 1, more && ng > 1));
     for (int i = ng; i >= 2; --i) {

@@ -119,3 +119,24 @@ def test_linearised_lanes(kind, monkeypatch):
             assert np.abs(b).max() > 0
             e = rel_err(a, b)
             assert e.max() < 1e-11, (lanes, e)
+
+
+@pytest.mark.parametrize("order", [1, 2])
+def test_cycle_without_smoothing_steps(order):
+    """numberOfRelaxationSteps 0: the transfers alone, from a state and time
+    steps that one smoothing step left.  The restricted state keeps the
+    pressure the restriction formed, which the prolongation's far field reads."""
+    print(f"[case] no smoothing steps, order={order}", flush=True)
+    iv = euler(order, multigridscheme=1, numberofrelaxationsteps=0)
+    s, o = pair(iv, levels(8, 3))
+    s.init_freestream(); o.init_freestream()
+    perturb(s, o, 1, np.random.default_rng(3), amp=0.05)
+    for x in (s, o):
+        x.do_time_iterations(1, 1, True)
+        x.cycle(1)
+        x.cycle(2)
+    for k in (1, 2, 3):
+        for f in ("U", "PRESSURE"):
+            e = rel_err(s.get(k, f)[:5], o.get(k, f)[:5])
+            assert e.max() < 1e-9, (k, f, e)
+    s.close(); o.close()
