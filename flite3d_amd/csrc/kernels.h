@@ -4,6 +4,7 @@
 //   node state      u[c*n+i] (SoA, 6 comps), uprev, p, dt, dtt, mu, vort,
 //                   divg, diss[5], src[6], tdiff
 //   rec0[8*i]       AoS per node: rho, u, v, w, rhoE, p, nu~, mu  (gathers)
+//   mom[4*i]        AoS per node: the state's momenta, pad (levels with JST or fluxType 1-3)
 //   grec[GREC*i]    AoS per node (HLLC-2): grad 15 | 1/lo 5 | 1/hi 5 | pad
 //                   (lo/hi = nodeHelpArray 16-25: min/max over sides - q)
 //   edges           ea[e], eb[e] (ends in reference orientation), w[3*e] AoS
@@ -146,6 +147,9 @@ struct LevelDev {
   R *u, *uprev, *rhs, *diss, *src, *p, *dt, *dtt, *mu, *vort, *divg, *tdiff;
   R *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;  // tau, dnu = tau + 9: VREC-strided, one shared record
   R *rec1;  // the next state's gather records while a walking stage reads rec0 (null: no such stage)
+  // the conserved momenta beside the records, for differences of neighbouring
+  // states: rho (m / rho) is not m (null: no such terms), and those of rec1
+  R *mom, *mom1;
   R *jst;  // JST node record (8 per node): L(U) 5, pressure switch, side count, volume / time step
   R *uold, *uold2;  // solutions at the last two physical times (6 per node, unsteady only)
   // moving meshes (null on a fixed mesh): GCL weight per side and 2 per
@@ -172,6 +176,8 @@ struct LevelDev {
     tdiff += bn;
     rec0 += 8 * bn;
     if (rec1) rec1 += 8 * bn;
+    if (mom) mom += 4 * bn;
+    if (mom1) mom1 += 4 * bn;
     grec += (size_t)b * (size_t)gstride;
     tau += VREC * bn;
     dnu += VREC * bn;
@@ -380,13 +386,20 @@ template <> struct Pair<float> { using type = float2; };
 
 // Neighbour walks of node i: f(qj, tj, wx, wy, wz) per interior side with w
 // the node-signed side weights and either qj the neighbour's gather record
-// (AUXW = 0) or tj the first AUXW words of its viscous record, in registers.
-// walk_global reads the neighbours' records from memory; walk_staged the
-// viscous records from the LDS slots a node block staged.
-template <int SUB, int AUXW = 0, typename R, typename F>
+// (AUXW = 0; MOM: with its momenta as tj) or tj the first AUXW words of its
+// viscous record, in registers.  walk_global reads the neighbours' records
+// from memory; walk_staged the viscous records from the LDS slots a node block
+// staged.
+template <int SUB, int AUXW = 0, bool MOM = false, typename R, typename F>
 __device__ __forceinline__ void walk_global(const LevelDev<R> &L, int i, int sub, F f) {
+  static_assert(!(MOM && AUXW > 0), "one of the two");
   for_edges_w<SUB>(L, i, sub, [&](int j, R wx, R wy, R wz) {
-    if constexpr (AUXW == 0) {
+    if constexpr (MOM) {
+      R qj[8], mj[4];
+      ldrec<8>(L.rec0 + 8 * (size_t)j, qj);
+      ldrec<4>(L.mom + 4 * (size_t)j, mj);
+      f(qj, mj, wx, wy, wz);
+    } else if constexpr (AUXW == 0) {
       R qj[8];
       ldrec<8>(L.rec0 + 8 * (size_t)j, qj);
       f(qj, (const R *)nullptr, wx, wy, wz);
@@ -431,12 +444,23 @@ __device__ __forceinline__ R state_pressure(const DevParams &P, const R *q) {
   return pp > R(0.1) ? pp : R(0.1);
 }
 
-// pressure and gather record (into rec) of node i for the state q[6]
+template <typename R>
+__device__ __forceinline__ void write_momenta(R *mom, int i, R m1, R m2, R m3) {
+  if (!mom) return;
+  R *m = mom + 4 * (size_t)i;
+  m[0] = m1;
+  m[1] = m2;
+  m[2] = m3;
+}
+
+// pressure, gather record (into rec) and momenta (into mom) of node i for the
+// state q[6]
 template <typename R>
 __device__ __forceinline__ void write_record(const LevelDev<R> &L, const DevParams &P, int i, const R *q, R mu,
-                                             R *rec) {
+                                             R *rec, R *mom) {
   R pp = state_pressure(P, q);
   L.p[i] = pp;
+  write_momenta(mom, i, q[1], q[2], q[3]);
   R *g = rec + 8 * (size_t)i;
   g[0] = q[0];
   g[1] = q[1] / q[0];
@@ -457,7 +481,7 @@ template <typename R>
 __device__ __forceinline__ void begin_step(const LevelDev<R> &L, const DevParams &P, int i, const R *q, R mu,
                                            int ncopy, int zero) {
   const size_t n = L.n;
-  write_record(L, P, i, q, mu, L.rec0);
+  write_record(L, P, i, q, mu, L.rec0, L.mom);
   for (int c = 0; c < ncopy; ++c) L.uprev[c * n + i] = q[c];
   if (zero)
     for (int c = 0; c < 5; ++c) L.diss[c * n + i] = R(0);
@@ -487,6 +511,7 @@ __global__ void k_pack(LevelDev<R> L, DevParams P) {
   if (i >= L.n) return;
   int n = L.n;
   R r = L.u[i];
+  write_momenta(L.mom, i, L.u[n + i], L.u[2 * n + i], L.u[3 * n + i]);
   R *q = L.rec0 + 8 * (size_t)i;
   q[0] = r;
   q[1] = L.u[n + i] / r;
@@ -3916,23 +3941,24 @@ template <typename R>
 struct JstSumsPart {
   static constexpr int AUXW = 0;
   R U[5], p, h[5], h7, h8, conn;
-  static __device__ __forceinline__ void state(const R *q, R *u) {
+  // the conserved state from the gather record and the momenta
+  static __device__ __forceinline__ void state(const R *q, const R *m, R *u) {
     u[0] = q[0];
-    u[1] = q[0] * q[1];
-    u[2] = q[0] * q[2];
-    u[3] = q[0] * q[3];
+    u[1] = m[0];
+    u[2] = m[1];
+    u[3] = m[2];
     u[4] = q[4];
   }
-  __device__ void init(const LevelDev<R> &, const DevParams &, int, const R *qi) {
-    state(qi, U);
+  __device__ void init(const LevelDev<R> &L, const DevParams &, int i, const R *qi) {
+    state(qi, L.mom + 4 * (size_t)i, U);
     p = qi[5];
 #pragma unroll
     for (int c = 0; c < 5; ++c) h[c] = 0;
     h7 = h8 = conn = 0;
   }
-  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *, const R *qj, R, R, R) {
+  __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *mj, const R *qj, R, R, R) {
     R V[5];
-    state(qj, V);
+    state(qj, mj, V);
 #pragma unroll
     for (int c = 0; c < 4; ++c) h[c] += V[c] - U[c];
     h[4] += (V[4] - U[4]) + (qj[5] - p);
@@ -3959,6 +3985,11 @@ struct JstSumsPart {
     o[7] = L.vol[i] / L.dt[i];
   }
 };
+
+template <typename T>
+constexpr bool reads_momenta = false;
+template <typename R>
+constexpr bool reads_momenta<JstSumsPart<R>> = true;
 
 constexpr int max3(int a, int b, int c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
 
@@ -4008,7 +4039,8 @@ __global__ __launch_bounds__(NTHR) void k_gather(LevelDev<R> L, DevParams P) {
   L.to_batch(bb_);
   P.to_batch(bb_);
   if (i >= L.n) return;
-  gather_body<R, SUB, A, B, C>(L, P, i, sub, [&](auto f) { walk_global<SUB, W>(L, i, sub, f); });
+  constexpr bool MOM = reads_momenta<A> || reads_momenta<B> || reads_momenta<C>;
+  gather_body<R, SUB, A, B, C>(L, P, i, sub, [&](auto f) { walk_global<SUB, W, MOM>(L, i, sub, f); });
 }
 
 template <typename R, typename A, typename B, typename C>
@@ -4075,10 +4107,11 @@ __global__ void k_jst_flux(LevelDev<R> L, DevParams P, int add) {
   if (i >= L.n) return;
   const size_t n = L.n;
   const R k2 = R(P.k2), k4 = R(L.gnum == 1 ? P.k4 : P.k4c);
-  R qi[8], ji[8], Ui[5], acc[5] = {0, 0, 0, 0, 0};
+  R qi[8], mi[4], ji[8], Ui[5], acc[5] = {0, 0, 0, 0, 0};
   ldrec<8>(L.rec0 + 8 * (size_t)i, qi);
+  ldrec<4>(L.mom + 4 * (size_t)i, mi);
   ldrec<8>(L.jst + 8 * (size_t)i, ji);
-  JstSumsPart<R>::state(qi, Ui);
+  JstSumsPart<R>::state(qi, mi, Ui);
   const int s = i / SLICE, lane = i % SLICE;
   const int base = L.ell_ptr[s], K = L.ell_k[s];
   const long long ns = L.nslot;
@@ -4087,10 +4120,11 @@ __global__ void k_jst_flux(LevelDev<R> L, DevParams P, int add) {
     const int e = L.ell_e[slot];
     if (e < 0) continue;
     const size_t j = L.ell_nbr[slot];
-    R qj[8], jj[8], Uj[5];
+    R qj[8], mj[4], jj[8], Uj[5];
     ldrec<8>(L.rec0 + 8 * j, qj);
+    ldrec<4>(L.mom + 4 * j, mj);
     ldrec<8>(L.jst + 8 * j, jj);
-    JstSumsPart<R>::state(qj, Uj);
+    JstSumsPart<R>::state(qj, mj, Uj);
     R d4v[5], d2v[5];
 #pragma unroll
     for (int c = 0; c < 5; ++c) {
@@ -4367,11 +4401,11 @@ __device__ __forceinline__ double sa_source(const LevelDev<R> &L, const DevParam
                              double(in.vol));
 }
 
-// the stage at node i from its convective residual r[6]; rec: where the
-// next state's gather record goes
+// the stage at node i from its convective residual r[6]; rec, mom: where the
+// next state's gather record and momenta go
 template <typename R, int MODE, bool SA>
 __device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams &P, const StageArgs &S, int i,
-                                           NodeIn<R> &in, R *r, R *rec) {
+                                           NodeIn<R> &in, R *r, R *rec, R *mom) {
   const int n = L.n;
   bool sa_on = SA && S.calc_turb;
   if (sa_on) r[5] += R(sa_source(L, P, i, in));
@@ -4452,7 +4486,7 @@ __device__ __forceinline__ void stage_node(const LevelDev<R> &L, const DevParams
     if (!S.next_record) return;
     // pressure and gather record of the new state, as k_prep forms them, so
     // the next stage starts without a separate pass
-    write_record(L, P, i, q, in.mu, rec);
+    write_record(L, P, i, q, in.mu, rec, mom);
   } else if (MODE == MODE_COARSE) {
     outer_bc(P, in.bc, q, in.p);
     for (int c = 0; c < 6; ++c) {
@@ -4486,7 +4520,7 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
   gather_rhs<R, SA, SUB>(L, i, sub, S.partials, r);
   if (sub) return;
   NodeIn<R> in = node_in<R, SA>(L, S, i);
-  stage_node<R, MODE, SA>(L, P, S, i, in, r, L.rec0);
+  stage_node<R, MODE, SA>(L, P, S, i, in, r, L.rec0, L.mom);
 }
 
 // One launch per stage: the residual of a block of consecutive nodes and
@@ -4511,14 +4545,16 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
 // more than the launches.
 // STEP: the nodes' local time steps (makeTimeSteps, inviscid) from the same
 // tasks.
-constexpr int SB_S = 7;  // LDS stride of a record (not mu) and of a task's result, odd
+constexpr int SB_S = 7;    // LDS stride of a record (not mu) and of a task's result, odd
+constexpr int SB_SM = 11;  // of a record with the momenta (fluxType 1-3)
 
 constexpr int SB_IN = 32;  // rows of the update's inputs
 
 template <typename R, int MODE, bool SA, bool HLLC, bool STEP>
 __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, StageArgs S) {
   static_assert(SB_CAP <= SB_TASKS && !(SA && STEP), "one LDS area serves the records and the results");
-  __shared__ R sn[SB_TASKS * SB_S];
+  constexpr int RS = HLLC ? SB_S : SB_SM;
+  __shared__ R sn[SB_CAP * RS > SB_TASKS * SB_S ? SB_CAP * RS : SB_TASKS * SB_S];
   __shared__ R own[SB_IN * SB_NODES];
   __shared__ unsigned short sinc[SB_INC];
   const int lb = xcd_block(), bb_ = lb % L.nb, blk = lb / L.nb, t = threadIdx.x;
@@ -4537,18 +4573,23 @@ __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, 
   for (int q = 0; q < SB_INC / NTHR; ++q) sinc[t + q * NTHR] = L.sb_inc[(size_t)SB_INC * blk + t + q * NTHR];
   // the nodes' records, two words a load
   {
-    constexpr int PER = (SB_CAP * 4 + NTHR - 1) / NTHR;
+    constexpr int U = HLLC ? 4 : 6;  // two-word units of a record, with the momenta's
+    constexpr int PER = (SB_CAP * U + NTHR - 1) / NTHR;
     using P2 = typename Pair<R>::type;
     int g[PER];
     P2 v[PER];
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
-      const int k = (t + q * NTHR) / 4;
+      const int k = (t + q * NTHR) / U;
       g[q] = k < SB_CAP ? nodes[k] : -1;
     }
 #pragma unroll
     for (int q = 0; q < PER; ++q)
-      if (g[q] >= 0) v[q] = reinterpret_cast<const P2 *>(L.rec0 + 8 * (size_t)g[q])[t % 4];
+      if (g[q] >= 0) {
+        const int j = (t + q * NTHR) % U;
+        const R *rec = j < 4 ? L.rec0 + 8 * (size_t)g[q] + 2 * j : L.mom + 4 * (size_t)g[q] + 2 * (j - 4);
+        v[q] = *reinterpret_cast<const P2 *>(rec);
+      }
     // and the own nodes' inputs of the update: row r of thread group r
     const int m = t % SB_NODES, r8 = t / SB_NODES, oi = nodes[0] + m < (int)n ? nodes[0] + m : (int)n - 1;
     R x0 = r8 < 6 ? L.uprev[r8 * n + oi] : r8 == 6 ? L.vol[oi] : L.dt[oi];
@@ -4559,9 +4600,10 @@ __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, 
 #pragma unroll
     for (int q = 0; q < PER; ++q)
       if (g[q] >= 0) {
-        R *o = sn + SB_S * ((t + q * NTHR) / 4) + 2 * (t % 4);
+        const int k = (t + q * NTHR) / U, j = (t + q * NTHR) % U;
+        R *o = sn + RS * k + (j < 4 ? 2 * j : 2 * j - 1);  // the momenta follow nu~
         o[0] = v[q].x;
-        if (t % 4 < 3) o[1] = v[q].y;  // not mu
+        if (j != 3 && j != 5) o[1] = v[q].y;  // not mu, not the pad
       }
     own[t] = x0;
     own[NTHR + t] = x1;
@@ -4572,14 +4614,13 @@ __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, 
   const int kind = loc >> 24;
   R f[7] = {0, 0, 0, 0, 0, 0, 0};
   if (kind != 255) {
-    const R *A = sn + (loc & 0xfffu) * SB_S, *B = sn + ((loc >> 12) & 0xfffu) * SB_S;
+    const R *A = sn + (loc & 0xfffu) * RS, *B = sn + ((loc >> 12) & 0xfffu) * RS;
     if (kind == 0) {
       if constexpr (HLLC) {
         side_flux<R, R, 1, SA, 2>(P, (const R *)nullptr, (const R *)nullptr, (const R *)nullptr, (const R *)nullptr, A,
                                   B, wx, wy, wz, f);
       } else {
-        const R UA[5] = {A[0], A[0] * A[1], A[0] * A[2], A[0] * A[3], A[4]};
-        const R UB[5] = {B[0], B[0] * B[1], B[0] * B[2], B[0] * B[3], B[4]};
+        const R UA[5] = {A[0], A[7], A[8], A[9], A[4]}, UB[5] = {B[0], B[7], B[8], B[9], B[4]};
         simple_flux(P, P.ftype, UA, A[5], UB, B[5], wx, wy, wz, R(0), f);
         f[5] = SA ? sa_side_convection(A, B, wx, wy, wz) : R(0);
       }
@@ -4643,7 +4684,7 @@ __global__ __launch_bounds__(NTHR) void k_stage_blk(LevelDev<R> L, DevParams P, 
   in.dtt = row(30);
   in.tdiff = row(31);
   if constexpr (STEP) L.dt[i] = in.dt = R(0.5) / (lam / in.vol);
-  stage_node<R, MODE, SA>(L, P, S, i, in, r, L.rec1);
+  stage_node<R, MODE, SA>(L, P, S, i, in, r, L.rec1, HLLC ? L.mom : L.mom1);
 }
 
 // ---------------------------------------------------------------------------

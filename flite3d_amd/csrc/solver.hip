@@ -160,6 +160,7 @@ struct Level {
   void *u, *uprev, *rhs, *diss, *src, *p, *dt, *dtt, *mu, *vort, *divg, *tdiff;
   void *rec0, *grec, *tau, *dnu, *fbuf, *bbuf, *ws;
   void *rec1 = nullptr;  // second record buffer of the one-launch stages (levels that use them)
+  void *mom = nullptr, *mom1 = nullptr;  // momenta beside rec0 and rec1 (levels with JST or fluxType 1-3)
   void *jst = nullptr;  // JST node records (levels with the JST dissipation)
   void *uold = nullptr, *uold2 = nullptr;  // unsteady only
   void *gcl = nullptr, *bgcl = nullptr, *volp = nullptr, *volp2 = nullptr, *cmv = nullptr;  // moving mesh only
@@ -224,7 +225,7 @@ struct Level {
     v.p = (R *)p; v.dt = (R *)dt; v.dtt = (R *)dtt; v.mu = (R *)mu; v.vort = (R *)vort;
     v.divg = (R *)divg; v.tdiff = (R *)tdiff; v.rec0 = (R *)rec0; v.rec1 = (R *)rec1; v.grec = (R *)grec;
     v.tau = (R *)tau; v.dnu = (R *)dnu; v.fbuf = (R *)fbuf; v.bbuf = (R *)bbuf; v.ws = (R *)ws;
-    v.jst = (R *)jst;
+    v.mom = (R *)mom; v.mom1 = (R *)mom1; v.jst = (R *)jst;
     v.uold = (R *)uold;
     v.uold2 = (R *)uold2;
     v.gcl = (const R *)gcl; v.bgcl = (const R *)bgcl;
@@ -1105,8 +1106,10 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
       TRY(P.upload(&L.sb_inc, T.inc));
       TRY(up_real(&L.sb_w, T.w));
       TRY(al_real(&L.rec1, (size_t)(8 * (size_t)n) * NB));
+      if (c->hp.flux_type != 4) TRY(al_real(&L.mom1, (size_t)(4 * (size_t)n) * NB));
     }
   }
+  if (c->hp.flux_type != 4 || jst_active(c, L)) TRY(al_real(&L.mom, (size_t)(4 * (size_t)n) * NB));
   L.gstride = need_grad ? GREC * (long long)n : 0;
   TRY(al_real(&L.grec, need_grad ? GREC * (size_t)n * NB : 1));
   TRY(al_real(&L.tau, (size_t)(VREC * (size_t)n) * NB));  // tau and dnu share the record
@@ -1418,7 +1421,10 @@ int op_stage(flite_ctx *c, Level &L, int mode, const StageArgs &S0, bool step = 
       else go(std::false_type{});
     });
   }));
-  if (mode == MODE_STAGE && S.next_record) std::swap(L.rec0, L.rec1);
+  if (mode == MODE_STAGE && S.next_record) {
+    std::swap(L.rec0, L.rec1);
+    if (L.mom1) std::swap(L.mom, L.mom1);
+  }
   return 0;
 }
 
@@ -3128,7 +3134,7 @@ int flite_autotune(flite_ctx *c, int repeats, int *lanes_out) {
         {L.p, nb * es},        {L.rec0, 8 * nb * es},  {L.dt, nb * es},         {L.dtt, nb * es},
         {L.mu, nb * es},       {L.vort, nb * es},      {L.divg, nb * es},       {L.tdiff, nb * es},
         {L.diss, 5 * nb * es}, {L.tau, VREC * nb * es}, {L.ws, 3 * nb * es},     {L.rhs, 6 * nb * es},
-        {L.grec, (size_t)L.gstride * L.nbatch * es}};
+        {L.grec, (size_t)L.gstride * L.nbatch * es}, {L.mom, L.mom ? 4 * nb * es : 0}};
     size_t total = 0;
     for (auto &k : kept) total += k.second;
     char *save = nullptr;

@@ -8,6 +8,8 @@ forces.  The lanes of the linearised kernels only change the order of sums of
 at most a few dozen terms, each combined once per stage of the chain, so their
 results are held to the single operations' 1e-11.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -140,3 +142,56 @@ def test_cycle_without_smoothing_steps(order):
             e = rel_err(s.get(k, f)[:5], o.get(k, f)[:5])
             assert e.max() < 1e-9, (k, f, e)
     s.close(); o.close()
+
+
+@pytest.mark.parametrize("name", ["llf", "roe"])
+@pytest.mark.parametrize("level", [1, 2])
+def test_jst_reads_the_stored_momenta(name, level):
+    """Equal momenta on unequal densities: the dissipation's momentum
+    differences are exactly zero."""
+    print(f"[case] jst momenta {name} level={level}", flush=True)
+    s, o = pair(jst_case(name), levels(8, 2))
+    o.close()
+    s.init_freestream()
+    rng = np.random.default_rng(12)
+    u = s.get(level, "U")
+    u[0] = rng.uniform(0.8, 1.2, u.shape[1])
+    u[1:4] = np.array([0.7, 0.3, -0.2])[:, None]
+    s.set(level, "U", u)
+    for op in ("PRESSURE", "TIMESTEPS", "DISSIPATION"):
+        s.apply(level, op)
+    d = s.get(level, "DISSIPATION")
+    s.close()
+    assert np.abs(d[0]).max() > 0
+    assert np.all(d[1:4] == 0.0), np.abs(d[1:4]).max()
+
+
+def test_central_flux_reads_the_stored_momenta():
+    """Side weights and momenta of few bits, unequal densities: the central
+    mass fluxes and their sums are exact, away from the boundary sides."""
+    print("[case] central flux momenta", flush=True)
+    lv = levels(8, 1)
+    w = np.round(lv[0].side_w * 2.0 ** 20) / 2.0 ** 20
+    lv = [dataclasses.replace(lv[0], side_w=w)]
+    s = Solver(jst_case("central").to_struct(), lv)
+    s.init_freestream()
+    rng = np.random.default_rng(13)
+    u = s.get(1, "U")
+    m = np.array([0.75, 0.25, -0.375])
+    u[0] = rng.uniform(0.8, 1.2, u.shape[1])
+    u[1:4] = m[:, None]
+    s.set(1, "U", u)
+    s.apply(1, "PRESSURE")
+    s.apply(1, "RHS")
+    r = s.get(1, "RHS")[0]
+    s.close()
+    want = np.zeros(u.shape[1])
+    f = 2.0 * (m @ w)
+    base = lv[0].side_index.min()
+    a, b = lv[0].side_index - base
+    np.add.at(want, a, f)
+    np.add.at(want, b, -f)
+    inner = np.ones(u.shape[1], bool)
+    inner[lv[0].bside_index[:2] - base] = False
+    assert inner.sum() > 100 and np.abs(want[inner]).max() > 0
+    assert np.array_equal(r[inner], want[inner]), np.abs(r - want)[inner].max()
