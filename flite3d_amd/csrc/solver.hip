@@ -256,10 +256,9 @@ struct flite_ctx {
   std::vector<flite_params> hp_b;  // per condition (batched contexts)
   double *cond_dev = nullptr;      // per-condition Mach and inflow state on the device
   int sel = 0;                     // condition that field/state/monitor calls act on
-  // columns of a field in host numbering on their way in or out (grown to the
-  // largest field asked for, released with the context)
+  // up to XFER_COLS columns of a field in host numbering on their way in or
+  // out: part of the built levels, so that access to a field allocates nothing
   double *xfer = nullptr;
-  size_t xfer_cap = 0;
   double *mon_host = nullptr;      // the monitor's MON_REC results, in pinned host memory the kernel writes
   std::vector<std::unique_ptr<Level>> lev;
   // coarse levels of the other precision (flite_set_coarse_precision),
@@ -1208,6 +1207,10 @@ int carry_in(const Level &L, void *d, int nc, const std::vector<double> &h) {
   return 0;
 }
 
+// columns of a field that the staging holds: a state.  Wider fields (the
+// gradient's 25) go through it in turns.
+constexpr int XFER_COLS = 6;
+
 // builds the device levels once every level is staged
 int ensure_built(flite_ctx *c) {
   if (c->built) return 0;
@@ -1215,8 +1218,14 @@ int ensure_built(flite_ctx *c) {
     if (!c->staged_ok[l]) return fail(FLITE_E_STATE, "not all levels uploaded");
   c->orders = nested_orders(c->staged);
   c->lev_alt.clear();
-  for (int l = 0; l < c->nl; ++l)
+  int most = 0;
+  for (int l = 0; l < c->nl; ++l) {
     TRY(build_level(c, l + 1, c->staged[l], c->orders[l], c->hp.coarse_fp32 != 0, c->lev[l]));
+    most = std::max(most, c->lev[l]->n);
+  }
+  if (c->xfer) (void)hipFree(c->xfer);
+  c->xfer = nullptr;
+  HIPTRY(hipMalloc((void **)&c->xfer, (size_t)XFER_COLS * most * sizeof(double)));
   c->built = true;
   if (!c->carry.empty()) {  // a moved mesh: the solution arrays carry over
     auto carry = std::move(c->carry);
@@ -1827,16 +1836,6 @@ void *field_ptr(Level &L, int field, int *ncomp, size_t *stride_nodes) {
   }
 }
 
-int need_xfer(flite_ctx *c, size_t count) {
-  if (c->xfer_cap >= count) return 0;
-  if (c->xfer) (void)hipFree(c->xfer);
-  c->xfer = nullptr;
-  c->xfer_cap = 0;
-  HIPTRY(hipMalloc((void **)&c->xfer, count * sizeof(double)));
-  c->xfer_cap = count;
-  return 0;
-}
-
 // nc columns of n doubles, the host's at leading dimension ld
 int copy_columns(flite_ctx *c, double *dst, const double *src, int n, int ld, int nc, bool to_host) {
   const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
@@ -1850,6 +1849,17 @@ int copy_columns(flite_ctx *c, double *dst, const double *src, int n, int ld, in
     HIPTRY(hipMemcpyAsync(d, s, (size_t)n * sizeof(double), kind, c->stream));
   }
   return 0;
+}
+
+// f(first column, columns) over nc columns, XFER_COLS at a time; the copies
+// queued on the caller's buffer have ended on return, also after an error
+template <typename F>
+int by_columns(flite_ctx *c, int nc, F f) {
+  int rc = 0;
+  for (int k = 0; k < nc && rc == 0; k += XFER_COLS) rc = f(k, std::min(XFER_COLS, nc - k));
+  if (rc == 0) return sync(c);
+  (void)hipStreamSynchronize(c->stream);
+  return rc;
 }
 
 }  // namespace
@@ -2042,16 +2052,16 @@ int flite_field_get(flite_ctx *c, int level, int field, double *out, int ld) {
   const long long n = L.n;
   // nc components, component k of device node d at p + base + sk k + si d
   auto fetch = [&](const void *p, size_t base, long long sk, long long si, int nc, int inv) -> int {
-    TRY(need_xfer(c, (size_t)nc * L.n));
-    auto go = [&](auto zero) -> int {
-      using R = decltype(zero);
-      hipLaunchKernelGGL(k_field_out<R>, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, (const R *)p + base, sk, si,
-                         (const int *)L.host_index, L.n, nc, inv, c->xfer);
-      return check_launch();
-    };
-    TRY(L.fp32 ? go(0.0f) : go(0.0));
-    TRY(copy_columns(c, out, c->xfer, L.n, ld, nc, true));
-    return sync(c);
+    return by_columns(c, nc, [&](int k, int cols) -> int {
+      auto go = [&](auto zero) -> int {
+        using R = decltype(zero);
+        hipLaunchKernelGGL(k_field_out<R>, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, (const R *)p + base + sk * k, sk,
+                           si, (const int *)L.host_index, L.n, cols, inv - k, c->xfer);
+        return check_launch();
+      };
+      TRY(L.fp32 ? go(0.0f) : go(0.0));
+      return copy_columns(c, out + (size_t)k * ld, c->xfer, L.n, ld, cols, true);
+    });
   };
   if (field == FLITE_FIELD_GRADIENT) {
     if (!(L.has_coords && c->hp.hllc_flux_order > 1)) return fail(FLITE_E_STATE, "no gradient on this level");
@@ -2078,16 +2088,16 @@ int flite_field_set(flite_ctx *c, int level, int field, const double *in, int ld
   void *p = field_ptr(L, field, &nc, &stride);
   if (!p) return fail(FLITE_E_ARG, "field cannot be set");
   p = (char *)p + (size_t)c->sel * nc * stride * (L.fp32 ? 4 : 8);
-  TRY(need_xfer(c, (size_t)nc * L.n));
-  TRY(copy_columns(c, c->xfer, in, L.n, ld, nc, false));
-  auto go = [&](auto zero) -> int {
-    using R = decltype(zero);
-    hipLaunchKernelGGL(k_field_in<R>, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, (const double *)c->xfer,
-                       (const int *)L.host_index, L.n, nc, (R *)p);
-    return check_launch();
-  };
-  TRY(L.fp32 ? go(0.0f) : go(0.0));
-  return sync(c);
+  return by_columns(c, nc, [&](int k, int cols) -> int {
+    TRY(copy_columns(c, c->xfer, in + (size_t)k * ld, L.n, ld, cols, false));
+    auto go = [&](auto zero) -> int {
+      using R = decltype(zero);
+      hipLaunchKernelGGL(k_field_in<R>, dim3(nblk(L.n)), dim3(NTHR), 0, c->stream, (const double *)c->xfer,
+                         (const int *)L.host_index, L.n, cols, (R *)p + (size_t)k * stride);
+      return check_launch();
+    };
+    return L.fp32 ? go(0.0f) : go(0.0);
+  });
 }
 
 int flite_state_set(flite_ctx *c, int level, const double *u, int ld, int ncomp, int batch) {

@@ -8,12 +8,13 @@ forces.  The lanes of the linearised kernels only change the order of sums of
 at most a few dozen terms, each combined once per stage of the chain, so their
 results are held to the single operations' 1e-11.
 """
+import ctypes
 import dataclasses
 
 import numpy as np
 import pytest
 
-from flite3d_amd.device import Solver
+from flite3d_amd.device import Solver, lib
 
 from cases import euler, levels, rans
 from test_gpu_parity import jst_case, pair, perturb, rel_err
@@ -195,3 +196,27 @@ def test_central_flux_reads_the_stored_momenta():
     inner[lv[0].bside_index[:2] - base] = False
     assert inner.sum() > 100 and np.abs(want[inner]).max() > 0
     assert np.array_equal(r[inner], want[inner]), np.abs(r - want)[inner].max()
+
+
+def free_device_memory():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_field_access_takes_no_device_memory():
+    """Fields of any width go through the context's own staging: reading 25
+    components of 68.9k nodes (14 MB) leaves the device's free memory as it
+    was."""
+    print("[case] field access and device memory", flush=True)
+    s = Solver(euler(2).to_struct(), list(levels(40, 1)))
+    s.init_freestream()
+    s.cycle(1)
+    s.get(1, "PRESSURE")
+    before = free_device_memory()
+    g = s.get(1, "GRADIENT")
+    s.set(1, "U", s.get(1, "U"))
+    after = free_device_memory()
+    s.close()
+    assert g.shape[0] == 25 and np.abs(g[:15]).max() > 0
+    assert after == before, before - after
