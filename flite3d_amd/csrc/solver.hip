@@ -1611,21 +1611,24 @@ int op_map_state(flite_ctx *c, Level &F, Level &K) {
   });
 }
 
+// what a smoothing step with its own dissipation forms before its first stage
+// (with a viscous term that stage's gradients too)
+int op_first_terms(flite_ctx *c, Level &L) {
+  if (viscous(c)) {
+    // makeTimeSteps, makeViscosityTerm, makeTurbulentTimeSteps, makeSADiffusion
+    TRY(op_step_terms(c, L, true, true, has_gradients(c, L)));
+    return op_jst(c, L, true);
+  }
+  return stage_steps(c, L) ? 0 : op_jst(c, L, false, true);
+}
+
 // begun: an earlier launch has done the step's start (begin_step).
 // record_last: the last stage leaves the records of its state too, for a
 // restriction that follows within the cycle.
 int do_single_iteration(flite_ctx *c, Level &L, bool calc_diss, bool begun, bool record_last) {
   const flite_params &hp = c->hp;
   if (!begun) TRY(op_prep(c, L, true, c->P.sa ? 6 : 5, calc_diss && zero_dissipation(c, L)));
-  if (calc_diss) {
-    if (viscous(c)) {
-      // makeTimeSteps, makeViscosityTerm, makeTurbulentTimeSteps, makeSADiffusion
-      TRY(op_step_terms(c, L, true, true, has_gradients(c, L)));
-      TRY(op_jst(c, L, true));
-    } else if (!stage_steps(c, L)) {
-      TRY(op_jst(c, L, false, true));
-    }
-  }
+  if (calc_diss) TRY(op_first_terms(c, L));
   for (int k = 1; k <= hp.rk_stages; ++k) {
     // stage k > 1 starts from the pressure and records the previous stage
     // kernel wrote with the new state
@@ -3110,9 +3113,12 @@ int flite_set_coarse_precision(flite_ctx *c, int fp32) {
 
 // Per level, the lanes per node (1, 4 or 16) of the gather and stage
 // kernels that run fastest on this context's current state: each candidate
-// runs the level's lane-dependent kernels (pressure and records, time steps
-// and viscous/SA passes, gradient, residual gather) `repeats` times after one
-// untimed run, timed with HIP events on the context's stream.
+// runs a smoothing step's launches of the level that depend on the lanes
+// (records, time steps, viscous/SA passes and JST as op_first_terms makes
+// them, the later stages' gradient, residual gather) `repeats` times after one
+// untimed run, timed with HIP events on the context's stream.  A level whose
+// step has none of them (the one-launch stages with their time steps) keeps
+// its lanes.
 int flite_autotune(flite_ctx *c, int repeats, int *lanes_out) {
   TRY(check_ctx(c));
   if (repeats < 1 || !lanes_out) return fail(FLITE_E_ARG, "repeats must be >= 1 and lanes_out non-null");
@@ -3123,12 +3129,10 @@ int flite_autotune(flite_ctx *c, int repeats, int *lanes_out) {
   hipEvent_t a = nullptr, b = nullptr;
   int rc = 0;
   if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) rc = fail(FLITE_E_HIP, "hipEventCreate");
-  const bool visc = c->hp.reynolds_number > 0.0;
   auto run = [&](Level &L) -> int {
     TRY(op_prep(c, L, true));
-    if (visc) TRY(op_step_terms(c, L, true, c->P.sa));
-    else TRY(op_timesteps(c, L));
-    TRY(op_grad(c, L));
+    TRY(op_first_terms(c, L));
+    if (!viscous(c) || c->hp.rk_stages > 1) TRY(op_grad(c, L));
     StageArgs S{};
     S.calc_turb = 1;
     return op_stage(c, L, MODE_RHS, S);
@@ -3161,7 +3165,7 @@ int flite_autotune(flite_ctx *c, int repeats, int *lanes_out) {
     if (rc == 0) rc = op_prep(c, L, true);
     if (rc == 0) rc = op_flux(c, L);
     for (int lanes : {1, 4, 16}) {
-      if (rc != 0) break;
+      if (rc != 0 || stage_steps(c, L)) break;
       L.lanes = lanes;
       rc = run(L);
       if (rc == 0 && hipEventRecord(a, c->stream) != hipSuccess) rc = fail(FLITE_E_HIP, "hipEventRecord");

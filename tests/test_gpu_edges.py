@@ -220,3 +220,24 @@ def test_field_access_takes_no_device_memory():
     s.close()
     assert g.shape[0] == 25 and np.abs(g[:15]).max() > 0
     assert after == before, before - after
+
+
+@pytest.mark.parametrize("kind", ["euler1", "jst", "rans"])
+def test_autotune_times_the_cycle(kind, monkeypatch):
+    """Autotuning times the launches a cycle makes.  Where no launch of a
+    level depends on its lanes (the one-launch stages with their time steps)
+    the lanes stay as they were; elsewhere one lane a node, the slowest on
+    levels this small, gives way.  The cycles that follow are the oracle's."""
+    print(f"[case] autotune {kind}", flush=True)
+    monkeypatch.setenv("FLITE_GATHER_LANES", "1")
+    iv = {"euler1": euler(1, multigridscheme=3), "jst": jst_case("roe", multigridscheme=3),
+          "rans": rans(multigridscheme=3)}[kind]
+    s, o = pair(iv, levels(8, 2, first_cell=0.005 if kind == "rans" else None))
+    s.init_freestream(); o.init_freestream()
+    lanes = s.autotune(5)
+    assert lanes == [1, 1] if kind == "euler1" else lanes[0] in (4, 16), lanes
+    for c in (1, 2):
+        s.cycle(c); o.cycle(c)
+    e = rel_err(s.get(1, "U")[:5], o.get(1, "U")[:5])
+    s.close(); o.close()
+    assert e.max() < 1e-9, e
