@@ -4706,22 +4706,19 @@ __global__ void k_fill(R *dst, R v, size_t cnt) {
   if (i < cnt) dst[i] = v;
 }
 
-// node BC application on a state array (setBCsOnSolutionField + outer)
+// node boundary conditions on the level's state (setBCsOnSolutionField)
 template <typename R>
-__global__ void k_bc_state(LevelDev<R> L, DevParams P, R *a, int outer) {
+__global__ void k_bc_state(LevelDev<R> L, DevParams P) {
   int bb_;
   int i = btid(L.nb, bb_);
   L.to_batch(bb_);
   P.to_batch(bb_);
-  a += (size_t)bb_ * 6 * (size_t)L.n;
   if (i >= L.n) return;
-  int n = L.n;
+  const size_t n = L.n;
   R q[6];
-  for (int c = 0; c < 6; ++c) q[c] = a[(size_t)c * n + i];
-  const NodeBc<R> b = node_bc(L, i);
-  bc_solution(L, P, i, b, q, a == L.u ? q[0] : L.u[i]);
-  if (outer) outer_bc(P, b, q, L.p[i]);
-  for (int c = 0; c < 6; ++c) a[(size_t)c * n + i] = q[c];
+  for (int c = 0; c < 6; ++c) q[c] = L.u[c * n + i];
+  bc_solution(L, P, i, node_bc(L, i), q, q[0]);
+  for (int c = 0; c < 6; ++c) L.u[c * n + i] = q[c];
 }
 
 // restriction (mapFineToCoarse, DEF:12572-12690) as a gather over the fine

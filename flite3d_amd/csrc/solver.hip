@@ -1564,11 +1564,11 @@ int op_copy(flite_ctx *c, Level &L, void *dst, const void *src, int ncomp) {
   });
 }
 
-int op_bc_state(flite_ctx *c, Level &L, void *a, int outer) {
+int op_bc_state(flite_ctx *c, Level &L) {
   DevParams P = c->P;
   return with_level(L, [&](auto V) {
     using R = std::remove_pointer_t<decltype(V.u)>;
-    hipLaunchKernelGGL(k_bc_state<R>, dim3(nblk(L.n) * L.nbatch), dim3(NTHR), 0, c->stream, V, P, (R *)a, outer);
+    hipLaunchKernelGGL(k_bc_state<R>, dim3(nblk(L.n) * L.nbatch), dim3(NTHR), 0, c->stream, V, P);
     return check_launch();
   });
 }
@@ -1937,7 +1937,7 @@ int flite_ctx_create(const flite_params *p, int n_levels, int n_batch, flite_ctx
   int dev = 0;
   HIPTRY(hipGetDevice(&dev));
   TRY(scratch_setup(dev));  // this device's copy of the monitor scratch, once per device
-  auto c = std::make_unique<flite_ctx>();
+  std::unique_ptr<flite_ctx, void (*)(flite_ctx *)> c(new flite_ctx, flite_ctx_destroy);  // whole on every error path
   c->device = dev;
   c->hp = *p;
   c->P = make_dev_params(*p);
@@ -2170,7 +2170,7 @@ int flite_init_freestream(flite_ctx *c) {
   // on u (DEF:3980-3994)
   TRY(set_old_states(c, L.u, L.u));
   TRY(op_prep(c, L, true));
-  TRY(op_bc_state(c, L, L.u, 0));
+  TRY(op_bc_state(c, L));
   return preamble(c);
 }
 
@@ -2573,12 +2573,14 @@ bool second_order(const flite_ctx *c, const Level &L) {
   return L.has_coords && c->hp.hllc_flux_order > 1 && c->hp.flux_type == 4;
 }
 
-// second-order linearisation scratch: per node DQ + 52 doubles (tangent: dq
-// DQ + dual (G, B) 52; adjoint: state shares 5, (G, B) shares 25, record
-// shares 5)
-// and 10 extremal-neighbour indices
+// second-order linearisation scratch: per node LIN_NODE doubles (tangent: dq
+// DQ, gradient records' tangents GREC; adjoint: scaled (G, B) shares GREC,
+// state shares 5, record shares 5; mesh adjoint: state shares 5, (G, B) shares
+// LIN_G, volume share 1) and 10 extremal-neighbour indices
+constexpr int LIN_NODE = GREC + 10;
+static_assert(LIN_NODE >= DQ + GREC && LIN_NODE >= 6 + LIN_G, "every user fits");
 int alloc_lin(Level &L) {
-  if (!L.lin) TRY(L.pool.alloc(&L.lin, (DQ + 52) * (size_t)std::max(1, L.n)));
+  if (!L.lin) TRY(L.pool.alloc(&L.lin, LIN_NODE * (size_t)std::max(1, L.n)));
   if (!L.amin) TRY(L.pool.alloc(&L.amin, 10 * (size_t)std::max(1, L.n)));
   return 0;
 }
