@@ -150,6 +150,7 @@ struct LevelDev {
   // the conserved momenta beside the records, for differences of neighbouring
   // states: rho (m / rho) is not m (null: no such terms), and those of rec1
   R *mom, *mom1;
+  const R *wsum;  // 3 per node: sum w + 2 sum_b w over the node's sides (levels with gradients)
   R *jst;  // JST node record (8 per node): L(U) 5, pressure switch, side count, volume / time step
   R *uold, *uold2;  // solutions at the last two physical times (6 per node, unsteady only)
   // moving meshes (null on a fixed mesh): GCL weight per side and 2 per
@@ -526,12 +527,17 @@ __global__ void k_pack(LevelDev<R> L, DevParams P) {
 // ---------------------------------------------------------------------------
 // computeGradient (DEF:2923-3245) + LocalMinMax (DEF:3248-3459), gathered
 // ---------------------------------------------------------------------------
-// computeGradient (DEF:2923-3245) + LocalMinMax (DEF:3248-3459) in the form
-// of a walk part (init / edge / bside / reduce / finish, like the gather
-// parts below): Green-Gauss sums over the interior sides (q_i + q_j) w and
-// the boundary sides (3 q_i + q_o) w, and the minimum and maximum of the
+// In the form of a walk part (init / edge / bside / reduce / finish, like the
+// gather parts below): Green-Gauss sums over the interior sides (q_i + q_j) w
+// and the boundary sides (3 q_i + q_o) w, and the minimum and maximum of the
 // neighbours' values.  GradViscPart carries it along the viscous pass 1 where
 // both are due; elsewhere the gradient kernels walk it alone.
+// The sums are taken as sum (q_j - q_i) w + sum_b (q_o - q_i) w + 2 q_i W with
+// W = sum w + 2 sum_b w, the node's own weights summed without rounding at
+// upload (wsum): the terms of q_i cancel over a node's sides, and summed
+// with the rest they left a rounding of q_i, not of the differences, that
+// depended on the lanes (tangent of RANS 64^3: 1.0e-13 with 4 lanes, 1.2e-13
+// with 1; 1.0e-13 so with 1, 4 and 16, at the same time).
 template <typename R>
 struct GradPart {
   static constexpr int AUXW = 0;
@@ -549,10 +555,10 @@ struct GradPart {
   __device__ void edge(const LevelDev<R> &, const DevParams &, const R *, const R *, const R *qj, R wx, R wy, R wz) {
 #pragma unroll
     for (int c = 0; c < 5; ++c) {
-      R s = q0[c] + qj[c];
-      g[c] += s * wx;
-      g[5 + c] += s * wy;
-      g[10 + c] += s * wz;
+      R d = qj[c] - q0[c];
+      g[c] += d * wx;
+      g[5 + c] += d * wy;
+      g[10 + c] += d * wz;
       R lo = rmin(q0[c], qj[c]);
       R hi = rmin(-q0[c], -qj[c]);
       mn[c] = rmin(mn[c], lo);
@@ -563,10 +569,10 @@ struct GradPart {
                         R wz) {
 #pragma unroll
     for (int c = 0; c < 5; ++c) {
-      R t = R(2) * q0[c] + (q0[c] + qo[c]);
-      g[c] += t * wx;
-      g[5 + c] += t * wy;
-      g[10 + c] += t * wz;
+      R d = qo[c] - q0[c];
+      g[c] += d * wx;
+      g[5 + c] += d * wy;
+      g[10 + c] += d * wz;
     }
   }
   template <int SUB>
@@ -579,8 +585,17 @@ struct GradPart {
       mx[c] = lmin<SUB>(mx[c]);
     }
   }
-  // the node's record: gradient 15, reciprocal bounds 5 + 5, pad
-  __device__ void values(const LevelDev<R> &L, int i, R *out) const {
+  // the node's own terms, then its record: gradient 15, reciprocal bounds 5 +
+  // 5, pad
+  __device__ void values(const LevelDev<R> &L, int i, R *out) {
+    const R *W = L.wsum + 3 * (size_t)i;
+    R wx = R(2) * W[0], wy = R(2) * W[1], wz = R(2) * W[2];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      g[c] += q0[c] * wx;
+      g[5 + c] += q0[c] * wy;
+      g[10 + c] += q0[c] * wz;
+    }
     R vt = R(1) / L.vol[i];
 #pragma unroll
     for (int c = 0; c < 15; ++c) out[c] = g[c] * vt;

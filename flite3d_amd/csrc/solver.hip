@@ -166,7 +166,7 @@ struct Level {
   void *gcl = nullptr, *bgcl = nullptr, *volp = nullptr, *volp2 = nullptr, *cmv = nullptr;  // moving mesh only
   int *ea, *eb, *ba, *bb, *bind, *ell_ptr, *ell_k, *bs_ptr, *bs_list, *ncls, *host_index, *wall_nodes;
   int *ell_e, *ell_nbr;
-  void *ellw;
+  void *ellw, *wsum = nullptr;  // wsum: each node's own weights summed (levels with gradients)
   long long nslot = 0;
   // side blocks of the LDS-staged flux kernel, one table set per shape
   // (FB_SHAPE_THR / FB_SHAPE_NODES); fb_shape is the one in use
@@ -220,7 +220,7 @@ struct Level {
     v.nsb = nsb; v.sb_node = sb_node; v.sb_loc = sb_loc; v.sb_inc = sb_inc; v.sb_iptr = sb_iptr;
     v.sb_w = (const R *)sb_w;
     v.vol = (const R *)vol; v.xyz = has_coords ? (const R *)xyz : nullptr;
-    v.wd = (const R *)wd; v.nrm = (const R *)nrm; v.ncls = ncls;
+    v.wsum = (const R *)wsum; v.wd = (const R *)wd; v.nrm = (const R *)nrm; v.ncls = ncls;
     v.u = (R *)u; v.uprev = (R *)uprev; v.rhs = (R *)rhs; v.diss = (R *)diss; v.src = (R *)src;
     v.p = (R *)p; v.dt = (R *)dt; v.dtt = (R *)dtt; v.mu = (R *)mu; v.vort = (R *)vort;
     v.divg = (R *)divg; v.tdiff = (R *)tdiff; v.rec0 = (R *)rec0; v.rec1 = (R *)rec1; v.grec = (R *)grec;
@@ -1109,6 +1109,29 @@ int build_level(flite_ctx *c, int level, const Staged &S, const std::vector<int>
     }
   }
   if (c->hp.flux_type != 4 || jst_active(c, L)) TRY(al_real(&L.mom, (size_t)(4 * (size_t)n) * NB));
+  if (need_grad) {
+    // the weights of a node cancel to their rounding: summed with the error of
+    // every addition kept
+    std::vector<double> sum(3 * (size_t)n, 0.0), err(3 * (size_t)n, 0.0);
+    auto add = [&](int i, int q, double x) {
+      const size_t k = 3 * (size_t)i + q;
+      const double t = sum[k] + x, b = t - sum[k];
+      err[k] += (sum[k] - (t - b)) + (x - b);
+      sum[k] = t;
+    };
+    for (int q = 0; q < 3; ++q) {
+      for (int k = 0; k < ne; ++k) {
+        add(ea[k], q, w[3 * (size_t)k + q]);
+        add(eb[k], q, -w[3 * (size_t)k + q]);
+      }
+      for (int s = 0; s < nbs; ++s) {
+        add(ba[s], q, 2.0 * wb[3 * (size_t)s + q]);
+        add(bb[s], q, 2.0 * wb[3 * (size_t)s + q]);
+      }
+    }
+    for (size_t k = 0; k < sum.size(); ++k) sum[k] += err[k];
+    TRY(up_real(&L.wsum, sum));
+  }
   L.gstride = need_grad ? GREC * (long long)n : 0;
   TRY(al_real(&L.grec, need_grad ? GREC * (size_t)n * NB : 1));
   TRY(al_real(&L.tau, (size_t)(VREC * (size_t)n) * NB));  // tau and dnu share the record

@@ -10,6 +10,7 @@ results are held to the single operations' 1e-11.
 """
 import ctypes
 import dataclasses
+import math
 
 import numpy as np
 import pytest
@@ -241,3 +242,49 @@ def test_autotune_times_the_cycle(kind, monkeypatch):
     e = rel_err(s.get(1, "U")[:5], o.get(1, "U")[:5])
     s.close(); o.close()
     assert e.max() < 1e-9, e
+
+
+@pytest.mark.parametrize("lanes", ["1", "4", "16"])
+def test_gradient_rounds_the_differences(lanes, monkeypatch):
+    """The Green-Gauss sums' rounding is one of the neighbours' differences,
+    not of the values, whatever the lanes: against extended precision, at most
+    (terms + 4) 2^-53 of the sum of |differences times weights| with up to 40
+    terms a node, hence 32 x 2^-52 of it."""
+    print(f"[case] gradient rounding lanes={lanes}", flush=True)
+    monkeypatch.setenv("FLITE_GATHER_LANES", lanes)
+    lv = levels(9, 1)
+    s = Solver(euler(2).to_struct(), list(lv))
+    s.init_freestream()
+    x, y, z = lv[0].coords
+    u = s.get(1, "U")
+    wave = np.sin(1.3 * x + 0.7 * y - 0.9 * z)
+    u[0] = 1.0 + 1e-3 * wave
+    u[1:4] = u[0] * np.array([0.9, 0.1, 0.2])[:, None] * (1.0 + 1e-3 * wave)
+    u[4] = 1e3 + 1e-2 * wave
+    s.set(1, "U", u)
+    s.apply(1, "PRESSURE")
+    s.apply(1, "RHS")
+    got = s.get(1, "GRADIENT")[:15].reshape(3, 5, -1)
+    s.close()
+    q = np.concatenate([u[:1], u[1:4] / u[0], u[4:5]]).astype(np.longdouble)
+    base = lv[0].side_index.min()
+    a, b = lv[0].side_index - base
+    ba, bb = lv[0].bside_index[:2] - base
+    want, size = np.zeros((2, 3, 5, u.shape[1]), np.longdouble)
+    for d in range(3):
+        w, wb = lv[0].side_w[d].astype(np.longdouble), lv[0].bside_w[d].astype(np.longdouble)
+        terms = [[] for _ in range(u.shape[1])]  # a node's weights cancel: summed exactly
+        for node, sign, weight in ((a, 1, w), (b, -1, w), (ba, 2, wb), (bb, 2, wb)):
+            for k, v in zip(node, sign * weight):
+                terms[k].append(float(v))
+        own = np.array([math.fsum(t) for t in terms], np.longdouble)
+        for c in range(5):
+            for i, j, weight in ((a, b, w), (b, a, -w), (ba, bb, wb), (bb, ba, wb)):
+                np.add.at(want[d, c], i, (q[c][j] - q[c][i]) * weight)
+                np.add.at(size[d, c], i, abs((q[c][j] - q[c][i]) * weight))
+            want[d, c] += 2 * q[c] * own
+            size[d, c] += abs(2 * q[c] * own)
+    vol = lv[0].volume.astype(np.longdouble)
+    e = abs(got - want / vol) / (size / vol)
+    assert np.abs(want).max() > 0
+    assert e.max() <= 32 * 2.0 ** -52, e.max()
