@@ -288,3 +288,24 @@ def test_gradient_rounds_the_differences(lanes, monkeypatch):
     e = abs(got - want / vol) / (size / vol)
     assert np.abs(want).max() > 0
     assert e.max() <= 32 * 2.0 ** -52, e.max()
+
+
+@pytest.mark.parametrize("env", [{"FLITE_FLUX_KERNEL": "block"},
+                                 {"FLITE_FLUX_KERNEL": "block", "FLITE_SIDE_BLOCK": "512"}])
+@pytest.mark.parametrize("kind", ["euler1", "rans"])
+def test_first_order_side_blocks(kind, env, monkeypatch):
+    """Side blocks of both shapes on the first-order levels, which run their
+    stages in one launch unless told otherwise."""
+    print(f"[case] first-order side blocks {kind} {env}", flush=True)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    iv = rans(multigridscheme=3) if kind == "rans" else euler(1, multigridscheme=3)
+    cycles_match(iv, levels(8, 3, first_cell=0.005 if kind == "rans" else None))
+
+
+@pytest.mark.parametrize("n", [24, 25])
+def test_first_order_stage_rule_with_sa(n):
+    """Both sides of the one-launch stage's size rule with a turbulence
+    equation (15.6k and 17.6k level-1 nodes)."""
+    print(f"[case] first-order SA stage rule n={n}", flush=True)
+    cycles_match(rans(hllcfluxorder=1, multigridscheme=3), levels(n, 2, first_cell=0.005), 2)
