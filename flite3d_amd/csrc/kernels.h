@@ -4927,7 +4927,11 @@ __global__ void k_prolong(LevelDev<RF> F, LevelDev<RC> K, DevParams P, Transfer 
 // DEF:14710-14806), all on the device: up to MON_BLOCKS blocks stride over
 // the nodes and the wall nodes, each thread accumulating its share in stride
 // order; wavefront butterflies and one LDS step reduce the block to a record
-// of MON_REC doubles; k_monitor_final reduces the records.  The order of
+// of MON_REC doubles; k_monitor_final reduces the records.  The wall's terms
+// are summed one after another in the register's order, a chunk of NTHR nodes
+// a block, and without contraction: a wall of one chunk has the bits of the
+// serial loop this stands for (the drag tests compare them with the oracle's),
+// which a tree has for some states only.  The order of
 // every sum is fixed, so the results are reproducible bit for bit.  Record:
 // sum (u - uprev)^2 [7], max |u - uprev| [7], host index of that maximum [7]
 // (smallest index on ties), force integrals [8] (lift, drag, latF,
@@ -5019,8 +5023,9 @@ __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParam
                                                          const R *warea, double *part, int bsel) {
   L.to_batch(bsel);
   P.to_batch(bsel);
-  constexpr int NW = NTHR / 64;
-  __shared__ double lds[MON_REC][NW];
+  constexpr int NW = NTHR / 64, FIRST_FORCE = 21;
+  __shared__ double lds[FIRST_FORCE][NW];
+  __shared__ double terms[8][NTHR + 1];  // odd stride: the eight summing lanes read different banks
   const int n = L.n, stride = gridDim.x * NTHR;
   double sum[7], mx[7];
   int mi[7];
@@ -5040,20 +5045,22 @@ __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParam
       maxloc(mx[j], mi[j], fabs(d), hi);
     }
   }
-  // force integrals; walls of up to NTHR nodes are summed in the register's
-  // order, as the loop this stands for, and without contraction, so that an
-  // inviscid drag has the bits of a serial program's whatever the state
-  double f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const bool serial = nw <= NTHR;
-  __shared__ double terms[8][NTHR];
-  for (int k = blockIdx.x * NTHR + threadIdx.x; k < nw; k += stride) {
-    double o[8];
-    force_terms(L, P, F, wall_nodes[k], warea, o);
+  // force integrals: quantity q's sum on thread q
+  const int q = threadIdx.x;
+  const bool force = q >= FIRST_FORCE && q < MON_REC;
+  double v = 0;
+  for (int k0 = blockIdx.x * NTHR; k0 < nw; k0 += stride) {
+    const int cnt = nw - k0 < NTHR ? nw - k0 : NTHR;
+    if (q < cnt) {
+      double o[8];
+      force_terms(L, P, F, wall_nodes[k0 + q], warea, o);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      if (serial) terms[c][threadIdx.x] = o[c];
-      else f[c] += o[c];
+      for (int c = 0; c < 8; ++c) terms[c][q] = o[c];
     }
+    __syncthreads();
+    if (force)
+      for (int k = 0; k < cnt; ++k) v += terms[q - FIRST_FORCE][k];
+    __syncthreads();
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
@@ -5066,28 +5073,17 @@ __global__ __launch_bounds__(NTHR) void k_monitor_reduce(LevelDev<R> L, DevParam
       lds[14 + j][wave] = double(mi[j]);
     }
   }
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const double t = wave_sum(f[c]);
-    if (lane == 0) lds[21 + c][wave] = t;
-  }
   __syncthreads();
-  const int q = threadIdx.x;
-  if (q < MON_REC) {
-    double v = 0;
-    if (q >= 7 && q < 21) {  // the maxima, and the indices that go with them
-      const int j = q < 14 ? q : q - 7;
-      double m = lds[j][0];
-      int k = (int)lds[j + 7][0];
-      for (int w = 1; w < NW; ++w) maxloc(m, k, lds[j][w], (int)lds[j + 7][w]);
-      v = q < 14 ? m : double(k);
-    } else {
-      for (int w = 0; w < NW; ++w) v += lds[q][w];
-      if (serial && blockIdx.x == 0 && q >= 21)
-        for (int k = 0; k < nw; ++k) v += terms[q - 21][k];
-    }
-    part[(size_t)MON_BLOCKS * q + blockIdx.x] = v;
+  if (q >= 7 && q < FIRST_FORCE) {  // the maxima, and the indices that go with them
+    const int j = q < 14 ? q : q - 7;
+    double m = lds[j][0];
+    int k = (int)lds[j + 7][0];
+    for (int w = 1; w < NW; ++w) maxloc(m, k, lds[j][w], (int)lds[j + 7][w]);
+    v = q < 14 ? m : double(k);
+  } else if (q < 7) {
+    for (int w = 0; w < NW; ++w) v += lds[q][w];
   }
+  if (q < MON_REC) part[(size_t)MON_BLOCKS * q + blockIdx.x] = v;
 }
 
 // wavefront w of one block takes quantities w, w + FIN_NW, ..; all of a
