@@ -226,8 +226,9 @@ __device__ __forceinline__ R rmin(R a, R b) { return a < b ? a : b; }
 // Forward-mode dual number: a value and one directional derivative.  The
 // residual's side and boundary fluxes are templated on their arithmetic
 // type; evaluated on Dual they give the exact derivative along the seeded
-// direction (the tangent), and seeded along each input in turn the rows of
-// the transposed Jacobian products (the adjoint).  Comparisons and
+// direction (the tangent), and seeded along an input its row of the
+// transposed Jacobian products (the metric and mesh adjoints; the state
+// adjoint's side flux has a reverse sweep of its own).  Comparisons and
 // selections act on the value, so the derivative is that of the branch the
 // value takes.  Kept in its own namespace so that its sqrt/fabs/fmin/fmax
 // are found by argument lookup only and never hide the double versions.
@@ -748,7 +749,7 @@ __device__ __forceinline__ R led(R a, R ilo, R ihi) {
 // 1/lo 5 | 1/hi 5), of type TG (R, or dual numbers for the linearisation),
 // and coordinates X1, X2; first order ignores them.
 // T is the arithmetic type: the level's R for the residual, a dual number
-// for its tangent and adjoint; with T a dual number the second-order branch
+// for its tangent and its mesh adjoint; with T a dual number the second-order branch
 // takes the gradient records (TG) and the coordinates (TX) as dual numbers
 // too when their derivatives are wanted.
 // upwinded SA convection of one side (makeSARHS, DEF:6873-6880) from the
@@ -1148,9 +1149,11 @@ __global__ __launch_bounds__(NTHR) void k_bflux(LevelDev<R> L, DevParams P) {
 // 14.8M sides (second order, SA), 656 now; 219 and 165 on 3.6M.
 // BND: blocks spread evenly among the side blocks evaluate the boundary sides,
 // one a thread, instead of a launch of their own (k_bflux).  That saves the
-// launch where it is the cost: us merged / apart, 13.4 / 18 with 19k boundary
-// sides, 114 / 120 with 74k, but 72 / 68 with 89k, 230 / 227 with 115k and
-// 914 / 907 with 295k (the longer code takes registers from the sides).
+// launch where it is the cost: us merged / apart, first order 16 / 24 with 19k
+// boundary sides and 72 / 71 with 89k; second order with SA 46 / 52 with 41k,
+// 87 / 93 with 74k, 125 / 127 with 93k, 164 / 165 with 115k, but 343 / 341
+// with 195k and 676 / 663 with 295k (the longer code takes registers from the
+// sides).
 // side-block shapes: FB_SHAPE_THR[k] sides per block (one thread each)
 // touching at most FB_SHAPE_NODES[k] distinct nodes; the autotuner picks
 // one per level (shape 0 unless it finds another faster)
@@ -1468,8 +1471,9 @@ __device__ __forceinline__ T sa_source_t(const DevParams &P, T rho, T nu, T mu, 
 // Tangent and adjoint of the level-1 convective residual R(U) (makeRHS,
 // DEF:1525-2512: interior HLLC sides + boundary sides) for first-order
 // HLLC without viscous or turbulence terms.  The side and boundary fluxes
-// are re-evaluated on dual numbers from the conserved state, so nothing per
-// side is stored between the forward and the reverse sweeps.
+// are re-evaluated from the conserved state (the tangent and the boundary
+// adjoint on dual numbers, the side adjoint by a reverse sweep), so nothing
+// per side is stored between the forward and the reverse sweeps.
 // ---------------------------------------------------------------------------
 // gather record of a conserved state exactly as k_prep forms it
 template <typename T>
@@ -1910,7 +1914,7 @@ __global__ __launch_bounds__(NTHR) void k_adjoint_gather(LevelDev<double> L, con
 // shares on v and nu~ follow at the end.  sa_upwind from the node has the sign
 // of s at the first end and of -s at the second, so the role is read only
 // where it is 0.  (Six dual passes of every side took 168 us at 275k nodes,
-// 73 now.)
+// 71 now.)
 template <int SUB>
 __global__ __launch_bounds__(NTHR) void k_sa_conv_adjoint(LevelDev<double> L, DevParams P, const double *lam, double *out) {
   int i, sub, bb_;
@@ -2032,10 +2036,11 @@ __global__ __launch_bounds__(NTHR) void k_bflux_metric_adjoint(LevelDev<double> 
 // Tangent and adjoint of the second-order (MUSCL + LED) inviscid residual.
 // Side (a, b)'s flux depends on both ends' gather records q, their
 // Green-Gauss gradients G and reciprocal limiter bounds B (grad_minmax_body),
-// and G and B on the neighbours' q.  The tangent runs that chain forward on
-// dual numbers.  The adjoint seeds each side's flux on its 60 inputs (both
-// ends' conserved states, gradients and bounds), sums the shares per node,
-// and transposes the gradient (a linear node gather) and the bounds (a
+// and G and B on the neighbours' q.  The tangent forms dG and dB in plain sums
+// and the slopes' tangents in closed form, and evaluates the HLLC flux on dual
+// numbers.  The adjoint runs that flux's reverse sweep once a side, sums the
+// shares per node, and transposes the gradient (a linear node gather) and the
+// bounds (a
 // bound 1/(q_k* - q_i) moves with the neighbour k* that attains the
 // extremum and with the node itself).
 // ---------------------------------------------------------------------------
@@ -2621,8 +2626,8 @@ __global__ __launch_bounds__(NTHR) void k_vol_mesh_adjoint(LevelDev<double> L, c
 // Sutherland viscosity of max(T, 0.001) and the adiabatic-wall projection;
 // A = sum over sides of E(tau_i, tau_j, u_i, u_j; w) and over non-symmetry
 // boundary sides of B(tau_i, tau_o, u_i, u_o; w_b).  The functions below
-// follow ViscNodePart / ViscFluxPart operation for operation, on any
-// arithmetic type.
+// form the terms of visc_node and ViscFluxPart on any arithmetic type, the
+// energy flux from both ends' stresses and velocities instead of their sums.
 // ---------------------------------------------------------------------------
 constexpr int VLIN = 66;  // scratch doubles per node of the viscous linearisation
 
@@ -3001,7 +3006,7 @@ __global__ __launch_bounds__(NTHR) void k_visc_adjoint_tau(LevelDev<double> L, D
 // viscosity of T and the vorticity and divergence of the same sums;
 // rnbar[2 i ..] = the shares on (rho, nu~).  The shares on the sums are closed
 // forms, the others a dual pass each (with a pass for each sum too: 213 us at
-// 275k nodes, NOWVN now).  lam may be null (no
+// 275k nodes, 103 now).  lam may be null (no
 // source term: the drag's friction alone drives taub).  With mbar (5 per
 // node) also the shares on the mesh quantities the node reads: its volume,
 // its wall normal (wall nodes, the adiabatic projection) and, with
@@ -3165,8 +3170,8 @@ __global__ __launch_bounds__(NTHR) void k_visc_adjoint_record(LevelDev<double> L
   }
 }
 
-// adjoint of the SA diffusion (k_sa_diff1_tangent / k_sa_tangent
-// transposed), multipliers m = lam(6).  Forward, node k: g_k = sum_j
+// adjoint of the SA diffusion (SADiff1Part and SADiff2Part transposed),
+// multipliers m = lam(6).  Forward, node k: g_k = sum_j
 // (nu_k + nu_j) w_kj + boundary terms, d_k = g_k / V_k, the nodal term
 // -f1 g_k.d_k, and the side terms -f2 (v_k w.d_k + v_j w.d_j) with
 // v = Re mu_lam / rho + nu~.  Pass 1, node k: W_k = sum_j (m_k - m_j) w_kj
@@ -4111,7 +4116,7 @@ __global__ __launch_bounds__(NTHR) void k_gather_blk(LevelDev<R> L, DevParams P)
 // Both passes read the 64-byte records of the neighbours with the level's
 // lanes per node; with one lane per node and the conserved state's seven
 // scattered words per neighbour they took 19 + 27 us on 9k nodes and 23 + 40
-// us on 160, now 8.5 + 6.6 and 6.6 + 5.8 (the first with the time steps).
+// us on 160, now 8.2 + 6.0 and 6.4 + 5.7 (the first with the time steps).
 template <typename R, bool MATRIX, int SUB>
 __global__ void k_jst_flux(LevelDev<R> L, DevParams P, int add) {
   int i, sub;
@@ -4554,8 +4559,9 @@ __global__ void k_stage(LevelDev<R> L, DevParams P, StageArgs S) {
 // and what the update reads of the block's own nodes staged beside the
 // records.  Per stage, FP64 without SA,
 // against the three launches: 8.8 us for 18 on 1.3k nodes, 23.5 for 27 on
-// 33k.  (A walk of each node's own sides, every flux at both ends, measured
-// 14 and 40 us.)  Second-order sides stay with k_flux_blk: their records are
+// 33k; with the central, LLF and Roe fluxes, whose records carry the momenta
+// too, 8.7 on 1.3k and 10.6 on 9k.  (A walk of each node's own sides, every
+// flux at both ends, measured 14 and 40 us.)  Second-order sides stay with k_flux_blk: their records are
 // five times as long and their arithmetic twice, so the repeated sides cost
 // more than the launches.
 // STEP: the nodes' local time steps (makeTimeSteps, inviscid) from the same

@@ -1313,7 +1313,12 @@ bool viscous(const flite_ctx *c) { return c->hp.reynolds_number > 0.0; }
 // with SA and 64k without (build_level): the repeated sides cost little where
 // latency is the time.  Per stage, us in one launch / as fluxes and stage: SA
 // 14 / 20 at 5k nodes, 33 / 26 at 31k, 193 / 103 at 255k; inviscid 8 / 14 at
-// 1.3k, 10 / 15 at 9k, 23 / 26 at 33k.
+// 1.3k, 10 / 15 at 9k, 23 / 26 at 33k.  As the lanes, the rule looks at the
+// level's own nodes: a condition of a batch keeps its single run's bits.
+// Batched, ms a cycle of such a level, one launch / apart: 64 x 1.3k 0.43 /
+// 0.64, 48 x 4.8k 1.03 / 1.38, 64 x 9.3k 0.89 / 1.35, 32 x 15.6k with SA 1.09 /
+// 1.39; from 33k nodes it loses 5 to 15% of that level (48 x 35.9k 2.51 /
+// 2.38, 16 x 33k in FP32 1.41 / 1.23) and the whole cycle still gains.
 bool stage_blocks(const flite_ctx *c, const Level &L) { return L.nsb > 0 && !c->flux_apart; }
 
 // ... whose first stage also forms the time steps: nothing else of the step
@@ -1322,7 +1327,8 @@ bool stage_steps(const flite_ctx *c, const Level &L) {
   return stage_blocks(c, L) && !viscous(c) && !jst_active(c, L);
 }
 
-// boundary sides up to which k_flux_blk evaluates them too (its BND)
+// boundary sides up to which k_flux_blk evaluates them too (its BND): between
+// the 74k where it gains at either order and the 89k where first order loses
 constexpr int BND_MERGED = 80000;
 
 int op_flux(flite_ctx *c, Level &L) {

@@ -255,9 +255,8 @@ int flite_apply(flite_ctx *ctx, int level, int op);
  * Both recompute the level's pressure, gather records and (second order)
  * gradients from the current state.
  *   flite_tangent_apply:  out = (dR/dU) du
- *   flite_adjoint_apply:  out = (dR/dU)^T lam  (a reversed side loop that
- *                         re-evaluates each side's inputs on dual numbers;
- *                         no Jacobian is stored)
+ *   flite_adjoint_apply:  out = (dR/dU)^T lam  (a reverse sweep of each
+ *                         side's flux; no Jacobian is stored)
  *   flite_drag_state_gradient: the drag of calculateLiftAndDrag
  *                         (mgnsg3d_def_par.F90:14757-14803: the pressure
  *                         term and, with ReynoldsNumber > 0, the friction
